@@ -38,10 +38,10 @@ namespace lal
                       const double* v, int* trp, int* tci, double* tv);
     // nnz_a: A's nonzeros, which pick the lanes per row of the product count
     int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a = 0);
+                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a, long nnz_b);
     int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                           const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv);
+                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b);
 }
 
 using lal::alloc_n;
@@ -494,21 +494,21 @@ namespace
             AP.n = nc;
             LAL_TRY(alloc_n(&AP.rp, Af.m + 1));
             LAL_TRY(lal::csrgemm_nnz(c, Af.m, Af.n, nc, Af.rp, Af.ci, P.rp, P.ci, AP.rp,
-                                     &AP.nnz, Af.nnz));
+                                     &AP.nnz, Af.nnz, P.nnz));
             LAL_TRY(alloc_n(&AP.ci, AP.nnz));
             LAL_TRY(alloc_n(&AP.v, AP.nnz));
             LAL_TRY(lal::csrgemm_solve_f64(c, Af.m, Af.n, nc, Af.rp, Af.ci, Af.v, P.rp, P.ci,
-                                           P.v, AP.rp, AP.ci, AP.v));
+                                           P.v, AP.rp, AP.ci, AP.v, Af.nnz, P.nnz));
             // A_c = R (A P)
             Ac.m = nc;
             Ac.n = nc;
             LAL_TRY(alloc_n(&Ac.rp, nc + 1));
             LAL_TRY(lal::csrgemm_nnz(c, nc, Af.m, nc, R.rp, R.ci, AP.rp, AP.ci, Ac.rp, &Ac.nnz,
-                                     R.nnz));
+                                     R.nnz, AP.nnz));
             LAL_TRY(alloc_n(&Ac.ci, Ac.nnz));
             LAL_TRY(alloc_n(&Ac.v, Ac.nnz));
             LAL_TRY(lal::csrgemm_solve_f64(c, nc, Af.m, nc, R.rp, R.ci, R.v, AP.rp, AP.ci, AP.v,
-                                           Ac.rp, Ac.ci, Ac.v));
+                                           Ac.rp, Ac.ci, Ac.v, R.nnz, AP.nnz));
             (void)hipStreamSynchronize(c->stream);
             AP.free_all();
             level++;

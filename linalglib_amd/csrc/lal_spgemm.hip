@@ -7,12 +7,12 @@
 // SpGEMM: rows of C are binned on the device by their product count into LDS
 // hash tables of H = 64 ... 4096 slots (open addressing, linear probing,
 // slots claimed with atomicCAS); rows beyond that get a table in global
-// memory.  Tables of up to 256 slots are built by H / 8 lanes per row (and
-// the symbolic pass's key-only tables of 512 and 1024 slots by 32), larger
-// ones by a wavefront per row.  The numeric pass walks the A row
-// sequentially and lets the lanes take the B row in parallel; the columns of one B row are distinct, so
-// every C entry receives at most one contribution per step and is folded in
-// A-row-then-B-row order from its first product -- the exact accumulation of
+// memory.  A table is built by 8 to 64 lanes (the symbolic pass's large
+// key-only ones by a workgroup).  The numeric pass searches the slots of
+// several A entries' B rows at once but adds their products in A-row order;
+// the columns of one B row are distinct, so every C entry receives at most one
+// contribution per A entry and is folded in A-row-then-B-row order from its
+// first product -- the exact accumulation of
 // backend/host/host_csrgemm.cpp:91-183.  The table is then compacted and each
 // entry is placed by its rank, giving ascending columns.
 #include "lal_internal.h"
@@ -279,45 +279,80 @@ namespace
         }
     }
 
-    // Rows of C in LDS tables of H slots: G lanes per row, NT / G rows per
-    // workgroup (G = H / 8 up to 256 slots, 32 for the symbolic pass's 512-
-    // and 1024-slot key-only tables, a wavefront otherwise).  The steps and
-    // the accumulation order are those of spgemm_row -- A-row entries one
-    // after another, the lanes of the group over the entries of that entry's
-    // B row -- but the group first loads up to G entries of the A row and
-    // their B-row bounds at once, one entry per lane, and each step takes its
-    // bounds from the owning lane, so a step waits on one load (the B row)
-    // instead of three dependent ones; each lane's first entry of the next
-    // step's B row is loaded during the current step.  Rows of P and A P hold
-    // a few to a few tens of entries, which a full wavefront per row would
-    // leave mostly idle.
-    template <int H, int G, int NT, bool NUMERIC>
-    __global__ void __launch_bounds__(NT)
-        spgemm_group_kernel(int nrows, const int* __restrict__ rows, const int* __restrict__ arp,
-                            const int* __restrict__ aci, const double* __restrict__ av,
-                            const int* __restrict__ brp, const int* __restrict__ bci,
-                            const double* __restrict__ bv, const int* __restrict__ crp,
-                            int* __restrict__ cout_, double* __restrict__ cval,
-                            int* __restrict__ err)
+    // v of lane t (the same t in every lane of the wavefront)
+    __device__ __forceinline__ int wave_lane(int v, int t)
     {
-        static_assert(G >= 2 && G <= 64 && (G & (G - 1)) == 0 && H % G == 0 && NT % G == 0);
-        constexpr int RPB   = NT / G;
+        return __builtin_amdgcn_readlane(v, t);
+    }
+    __device__ __forceinline__ double wave_lane(double v, int t)
+    {
+        const long long b  = __builtin_bit_cast(long long, v);
+        const unsigned  lo = (unsigned)__builtin_amdgcn_readlane((int)b, t);
+        const unsigned  hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), t);
+        return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+    }
+
+    // Rows of C in LDS tables of H slots (a power of two, at least 64): G lanes
+    // per row, L of them per B row.
+    //
+    // Bound by latency: a step (one A entry and its B row) is a chain of
+    // dependent loads and LDS round trips, and the coarse levels have few and
+    // long rows.  So G lanes load G entries of the A row with their B-row
+    // bounds at once, and S * U steps are taken together: S = G / L groups of
+    // lanes side by side, U steps per group in flight, first their B-row loads,
+    // then their slot searches (which slot a column gets does not depend on
+    // the order), and only then, in A-row order, their additions, as LDS adds
+    // without a return value.  The LDS executes one wave's instructions in
+    // order and the columns of one step are distinct, so every C entry is
+    // folded in A-row-then-B-row order; slots start at -0.0, to which adding
+    // the first product is exact, so the fold is the one from the first
+    // product.  A B row longer than L is several steps.
+    //
+    // AHEAD: the next batch's B-row loads are issued before this batch's LDS
+    // work.  It shortens a row's chain and costs registers and occupancy, so
+    // it is for launches of few rows (launch_group).
+    template <int G, int L, bool NUMERIC, bool AHEAD>
+    __global__ void __launch_bounds__(256)
+        spgemm_group_kernel(int nrows, int H, const int* __restrict__ rows,
+                            const int* __restrict__ arp, const int* __restrict__ aci,
+                            const double* __restrict__ av, const int* __restrict__ brp,
+                            const int* __restrict__ bci, const double* __restrict__ bv,
+                            const int* __restrict__ crp, int* __restrict__ cout_,
+                            double* __restrict__ cval, int* __restrict__ err)
+    {
+        static_assert(G <= 64 && L <= G && (G & (G - 1)) == 0 && (L & (L - 1)) == 0);
+        constexpr int S = G / L, U = S >= 4 ? 2 : 4;
         constexpr unsigned long long GMASK = G == 64 ? ~0ull : (1ull << (G % 64)) - 1ull;
-        constexpr int hmask = H - 1;
-        __shared__ int    s_keys[RPB][H];
-        __shared__ double s_vals[NUMERIC ? RPB : 1][NUMERIC ? H : 1];
-        const int         grp = (int)threadIdx.x / G;
-        const int         gl  = (int)threadIdx.x % G;       // lane in the group
-        const int         gb  = ((int)threadIdx.x & 63) - gl; // the group's first lane
-        const int         r   = blockIdx.x * RPB + grp;
+        typedef int   int4v __attribute__((ext_vector_type(4)));
+        // per row of the workgroup: H values (numeric pass), H keys
+        extern __shared__ __attribute__((aligned(16))) unsigned char s_tab[];
+        const int hmask = H - 1;
+        const int rpb   = (int)blockDim.x / G;
+        const int grp   = (int)threadIdx.x / G;
+        const int gl    = (int)threadIdx.x % G;         // lane in the group
+        const int gb    = ((int)threadIdx.x & 63) - gl; // the group's first lane
+        const int sl    = gl % L, sg = gl / L;          // lane of the step, step of the batch
+        const int r     = blockIdx.x * rpb + grp;
         if(r >= nrows)
             return;
         const int row  = rows[r];
-        int*      keys = s_keys[grp];
-        double*   vals = NUMERIC ? s_vals[grp] : nullptr;
-        for(int s = gl; s < H; s += G)
-            keys[s] = -1;
+        double*   vals = NUMERIC ? reinterpret_cast<double*>(s_tab) + (size_t)grp * H : nullptr;
+        int*      keys = reinterpret_cast<int*>(s_tab + (NUMERIC ? sizeof(double) * rpb * H : 0)) +
+                    (size_t)grp * H;
+        for(int s = gl; s < H / 4; s += G)
+            reinterpret_cast<int4v*>(keys)[s] = int4v{-1, -1, -1, -1};
+        if(NUMERIC)
+            for(int s = gl; s < H; s += G)
+                vals[s] = -0.0;
         wave_sync_mem<false>();
+        // lane t's value of v, for the whole group (a wavefront taking its
+        // steps one by one reads the lane as a scalar)
+        auto lane_value = [&](auto v, int t) {
+            if constexpr(S == 1 && G == 64)
+                return wave_lane(v, __builtin_amdgcn_readfirstlane(t));
+            else
+                return __shfl(v, gb + t, 64);
+        };
         int       local = 0;
         const int rs = arp[row], re = arp[row + 1];
         for(int j0 = rs; j0 < re; j0 += G)
@@ -333,60 +368,117 @@ namespace
                 bs = brp[ca];
                 be = brp[ca + 1];
             }
-            const int cnt = min(G, re - j0);
-            // each lane's first entry of step t's B row is loaded during step
-            // t - 1, so the step's inserts do not wait on it
-            int    nbs = __shfl(bs, gb, 64), nbe = __shfl(be, gb, 64);
-            double nva  = NUMERIC ? __shfl(va, gb, 64) : 0.0;
-            int    ncol = nbs + gl < nbe ? bci[nbs + gl] : -1;
-            double nbv  = NUMERIC && nbs + gl < nbe ? bv[nbs + gl] : 0.0;
-            for(int t = 0; t < cnt; t++)
+            // steps of this chunk: one per A entry, or more where a B row is
+            // longer than L (then `upto` counts the steps through each entry)
+            const bool wide  = ((__ballot(be - bs > L) >> gb) & GMASK) != 0;
+            int        steps = min(G, re - j0);
+            int        upto  = 0;
+            if(wide)
             {
-                const int    tbs = nbs, tbe = nbe;
-                const double tva = nva;
-                const int    col0 = ncol;
-                const double bv0  = nbv;
-                if(t + 1 < cnt)
+                upto = (be - bs + L - 1) / L;
+#pragma unroll
+                for(int o = 1; o < G; o <<= 1)
                 {
-                    nbs = __shfl(bs, gb + t + 1, 64);
-                    nbe = __shfl(be, gb + t + 1, 64);
-                    if(NUMERIC)
-                        nva = __shfl(va, gb + t + 1, 64);
-                    ncol = nbs + gl < nbe ? bci[nbs + gl] : -1;
-                    if(NUMERIC)
-                        nbv = nbs + gl < nbe ? bv[nbs + gl] : 0.0;
+                    const int t = __shfl(upto, gb + max(gl - o, 0), 64);
+                    upto += gl >= o ? t : 0;
                 }
-                for(int p = tbs + gl; p < tbe; p += G)
+                steps = __shfl(upto, gb + G - 1, 64);
+            }
+            // entries of the steps s0 .. s0 + S U - 1: columns (-1: none), the
+            // B values and the A value of their step
+            auto fetch = [&](int s0, int (&col)[U], double (&bval)[U], double (&aval)[U]) {
+#pragma unroll
+                for(int u = 0; u < U; u++)
                 {
-                    const bool   first = p == tbs + gl;
-                    const int    col   = first ? col0 : bci[p];
-                    const double bp    = NUMERIC ? (first ? bv0 : bv[p]) : 0.0;
-                    int          h     = slot_of(col, hmask);
-                    for(int probe = 0;; probe++)
+                    const int s = s0 + u * S + sg;
+                    int       t = min(s, G - 1), off = 0; // A entry, chunk of its B row
+                    if(wide)
                     {
-                        if(probe == H)
+                        // t: the entries that end at or before step s
+                        if(G == 64 && S == 1)
+                            t = min(__popcll(__ballot(upto <= s)), G - 1);
+                        else
                         {
-                            *err = 1; // table full: the row pointer undercounts this row
-                            break;
+                            t = 0;
+#pragma unroll
+                            for(int o = G / 2; o > 0; o >>= 1)
+                            {
+                                const int v = __shfl(upto, gb + t + o - 1, 64);
+                                t += v <= s ? o : 0;
+                            }
                         }
-                        int old = atomicCAS(&keys[h], -1, col);
-                        if(old == -1)
-                        {
-                            local++;
-                            if(NUMERIC)
-                                vals[h] = tva * bp;
-                            break;
-                        }
-                        if(old == col)
-                        {
-                            if(NUMERIC)
-                                vals[h] += tva * bp;
-                            break;
-                        }
-                        h = (h + 1) & hmask;
+                        const int before = lane_value(upto, max(t - 1, 0));
+                        off              = (s - (t > 0 ? before : 0)) * L;
                     }
+                    const int  p  = lane_value(bs, t) + off + sl;
+                    const int  pe = lane_value(be, t); // every lane takes part
+                    const bool ok = s < steps && p < pe;
+                    aval[u]       = NUMERIC ? lane_value(va, t) : 0.0;
+                    col[u]        = ok ? bci[p] : -1;
+                    bval[u]       = NUMERIC && ok ? bv[p] : 0.0;
                 }
-                wave_sync_mem<false>();
+            };
+            int    ncol[U];
+            double nbv[U], nav[U];
+            if(AHEAD)
+                fetch(0, ncol, nbv, nav);
+            for(int s0 = 0; s0 < steps; s0 += S * U)
+            {
+                int      col[U], h[U];
+                double   prod[U];
+                unsigned pend = 0;
+                if(!AHEAD)
+                    fetch(s0, ncol, nbv, nav);
+#pragma unroll
+                for(int u = 0; u < U; u++)
+                {
+                    prod[u] = nav[u] * nbv[u];
+                    col[u]  = ncol[u];
+                    h[u]    = slot_of(col[u], hmask);
+                    pend |= col[u] >= 0 ? 1u << u : 0u;
+                }
+                if(AHEAD && s0 + S * U < steps)
+                    fetch(s0 + S * U, ncol, nbv, nav);
+                const unsigned all = pend;
+                for(int probe = 0; pend != 0; probe++)
+                {
+                    if(probe == H)
+                    {
+                        *err = 1; // table full: the row pointer undercounts this row
+                        break;
+                    }
+                    int old[U];
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+                        if(pend >> u & 1)
+                            old[u] = atomicCAS(&keys[h[u]], -1, col[u]);
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+                        if(pend >> u & 1)
+                        {
+                            if(old[u] == -1)
+                                local++;
+                            if(old[u] == -1 || old[u] == col[u])
+                                pend &= ~(1u << u);
+                            else
+                                h[u] = (h[u] + 1) & hmask;
+                        }
+                }
+                if(NUMERIC)
+                {
+                    const unsigned got = all & ~pend;
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+#pragma unroll
+                        for(int k = 0; k < S; k++)
+                        {
+                            if(sg == k && (got >> u & 1))
+                                (void)__hip_atomic_fetch_add(&vals[h[u]], prod[u],
+                                                             __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                }
             }
         }
         if(!NUMERIC)
@@ -398,43 +490,142 @@ namespace
                 cout_[row] = local;
             return;
         }
-        // compact the occupied slots into [0, nnz) in place
+        wave_sync_mem<false>();
+        // compact the occupied slots into [0, nnz) in place, eight per lane at
+        // a time (an entry never moves up, so the slots a later pass reads
+        // are still untouched)
         int                      base  = 0;
         const unsigned long long below = (1ull << gl) - 1ull;
-        for(int s0 = 0; s0 < H; s0 += G)
+        for(int s0 = 0; s0 < H; s0 += 8 * G)
         {
-            const int                s     = s0 + gl;
-            const int                k     = keys[s];
-            const double             v     = vals[s];
-            const bool               valid = k != -1;
-            const unsigned long long mask  = (__ballot(valid) >> gb) & GMASK;
-            wave_sync_mem<false>();
-            if(valid)
+            int    k[8];
+            double v[8];
+#pragma unroll
+            for(int u = 0; u < 8; u++)
             {
-                int pos   = base + __popcll(mask & below);
-                keys[pos] = k;
-                vals[pos] = v;
+                const int t = s0 + u * G + gl;
+                k[u]        = t < H ? keys[t] : -1;
+                v[u]        = t < H ? vals[t] : 0.0;
             }
-            base += __popcll(mask);
+            wave_sync_mem<false>();
+#pragma unroll
+            for(int u = 0; u < 8; u++)
+            {
+                const unsigned long long mask = (__ballot(k[u] != -1) >> gb) & GMASK;
+                if(k[u] != -1)
+                {
+                    const int pos = base + __popcll(mask & below);
+                    keys[pos]     = k[u];
+                    vals[pos]     = v[u];
+                }
+                base += __popcll(mask);
+            }
             wave_sync_mem<false>();
         }
-        const int nnz = base;
+        const int nnz  = base;
+        const int nnz4 = (nnz + 3) & ~3; // at most H, a multiple of 4
+        if(nnz + gl < nnz4)
+            keys[nnz + gl] = INT_MAX;
+        wave_sync_mem<false>();
         const int out = crp[row];
         const int len = crp[row + 1] - out;
         if(nnz != len && gl == 0)
             *err = 1;
+        // an entry's place is the number of smaller columns, four per read
         for(int e = gl; e < nnz; e += G)
         {
-            const int k  = keys[e];
-            int       rk = 0;
-            for(int t = 0; t < nnz; t++)
-                rk += keys[t] < k;
+            const int    k  = keys[e];
+            int          rk = 0;
+            const int4v* k4 = reinterpret_cast<const int4v*>(keys);
+            for(int t = 0; t < nnz4 / 4; t++)
+            {
+                const int4v q = k4[t];
+                rk += (q.x < k) + (q.y < k) + (q.z < k) + (q.w < k);
+            }
             if(rk < len)
             {
                 cout_[out + rk] = k;
                 cval[out + rk]  = vals[e];
             }
         }
+    }
+
+    // Distinct columns of one row of C per workgroup, in a key table of H
+    // slots: the symbolic pass's rows of more than 512 products or so.  The
+    // count does not depend on the order, so 32 groups of 8 lanes take the A
+    // row's entries side by side, four B-row entries per lane in flight; a
+    // wavefront walking such a row alone was a chain of some hundred
+    // dependent steps on a tenth of the chip.
+    template <int H>
+    __global__ void __launch_bounds__(256)
+        spgemm_count_kernel(const int* __restrict__ rows, const int* __restrict__ arp,
+                            const int* __restrict__ aci, const int* __restrict__ brp,
+                            const int* __restrict__ bci, int* __restrict__ cout_,
+                            int* __restrict__ err)
+    {
+        constexpr int G = 8, U = 4, hmask = H - 1;
+        __shared__ int s_keys[H];
+        __shared__ int s_sum[4];
+        const int tid = (int)threadIdx.x, gl = tid % G;
+        const int row = rows[blockIdx.x];
+        const int re  = arp[row + 1];
+        int       j   = arp[row] + tid / G;
+        for(int s = tid; s < H; s += 256)
+            s_keys[s] = -1;
+        __syncthreads();
+        int local = 0;
+        for(; j < re; j += 256 / G)
+        {
+            const int ca = aci[j];
+            const int be = brp[ca + 1];
+            for(int p0 = brp[ca] + gl; p0 < be; p0 += U * G)
+            {
+                int      col[U], h[U];
+                unsigned pend = 0;
+#pragma unroll
+                for(int u = 0; u < U; u++)
+                {
+                    const int p = p0 + u * G;
+                    col[u]      = p < be ? bci[p] : -1;
+                }
+#pragma unroll
+                for(int u = 0; u < U; u++)
+                {
+                    h[u] = slot_of(col[u], hmask);
+                    pend |= col[u] >= 0 ? 1u << u : 0u;
+                }
+                for(int probe = 0; pend != 0; probe++)
+                {
+                    if(probe == H)
+                    {
+                        *err = 1;
+                        break;
+                    }
+                    int old[U];
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+                        if(pend >> u & 1)
+                            old[u] = atomicCAS(&s_keys[h[u]], -1, col[u]);
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+                        if(pend >> u & 1)
+                        {
+                            if(old[u] == -1)
+                                local++;
+                            if(old[u] == -1 || old[u] == col[u])
+                                pend &= ~(1u << u);
+                            else
+                                h[u] = (h[u] + 1) & hmask;
+                        }
+                }
+            }
+        }
+        local = lal::wave_sum(local);
+        if((tid & 63) == 0)
+            s_sum[tid >> 6] = local;
+        __syncthreads();
+        if(tid == 0)
+            cout_[row] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
     }
 
     template <bool NUMERIC>
@@ -481,6 +672,8 @@ namespace
         std::vector<int>  bin_start; // per LDS bin (H = 64 << b), into d_rows
         int               n_lds    = 0;
         int               n_global = 0;
+        int               g        = 8; // lanes per A row and per B row
+        int               l        = 8; // (launch_group)
         std::vector<long long> toff; // global table offsets (n_global + 1)
         int*              d_rows   = nullptr; // LDS-bin rows, then global rows
         long long*        d_toff   = nullptr;
@@ -674,6 +867,64 @@ namespace
         return LAL_OK;
     }
 
+    // Smallest power of two of 8 .. 64 that holds n entries.
+    inline int lanes_for(long n)
+    {
+        int g = 8;
+        while(g < 64 && g < n)
+            g <<= 1;
+        return g;
+    }
+
+    // Rows of C with H-slot tables: l lanes take a B row (its mean length),
+    // g lanes the A row (its mean length).  Below 262,144 such lanes (half of
+    // what the chip holds) the rows' own chains are the time: they take a
+    // wavefront each and load a batch ahead.  121^3 diffusion, numeric pass:
+    // level 3's R (A P), 4,400 rows, takes 502 us with the batch ahead and 648
+    // without (960 with one step at a time); level 0's, 300,000 rows, 606 with
+    // and 484 without (790 with one step at a time).
+    template <bool NUMERIC>
+    void launch_group(lal_context* c, int nr, int H, int g, int l, const int* rows,
+                      const int* arp, const int* aci, const double* av, const int* brp,
+                      const int* bci, const double* bv, const int* crp, int* cout_, double* cval)
+    {
+        const bool few = (long)nr * g < 256L * 1024;
+        if(few)
+            g = 64;
+        g = std::max(g, l);
+        // up to 256 lanes and 48 KB of tables per workgroup
+        const size_t row_bytes = (size_t)H * (NUMERIC ? 12 : 4);
+        int          nt        = 256;
+        while(nt > 64 && row_bytes * (nt / g) > 48 * 1024)
+            nt >>= 1;
+        const int    rpb = nt / g;
+        const size_t lds = row_bytes * rpb;
+        const int    nb  = (nr + rpb - 1) / rpb;
+#define LAL_SPGEMM_GROUP(GG, LL, AHEAD)                                                      \
+    case (AHEAD ? 65536 : 0) + GG * 128 + LL:                                                \
+        spgemm_group_kernel<GG, LL, NUMERIC, AHEAD><<<nb, nt, lds, c->stream>>>(             \
+            nr, H, rows, arp, aci, av, brp, bci, bv, crp, cout_, cval, c->d_flag);           \
+        break;
+        switch((few ? 65536 : 0) + g * 128 + l)
+        {
+            LAL_SPGEMM_GROUP(8, 8, false)
+            LAL_SPGEMM_GROUP(16, 8, false)
+            LAL_SPGEMM_GROUP(16, 16, false)
+            LAL_SPGEMM_GROUP(32, 8, false)
+            LAL_SPGEMM_GROUP(32, 16, false)
+            LAL_SPGEMM_GROUP(32, 32, false)
+            LAL_SPGEMM_GROUP(64, 8, false)
+            LAL_SPGEMM_GROUP(64, 16, false)
+            LAL_SPGEMM_GROUP(64, 32, false)
+            LAL_SPGEMM_GROUP(64, 64, false)
+            LAL_SPGEMM_GROUP(64, 8, true)
+            LAL_SPGEMM_GROUP(64, 16, true)
+            LAL_SPGEMM_GROUP(64, 32, true)
+            LAL_SPGEMM_GROUP(64, 64, true)
+        }
+#undef LAL_SPGEMM_GROUP
+    }
+
     template <bool NUMERIC>
     int run_plan(lal_context* c, const spgemm_plan& P, const int* arp, const int* aci,
                  const double* av, const int* brp, const int* bci, const double* bv,
@@ -685,38 +936,27 @@ namespace
             if(nr == 0)
                 continue;
             const int* rows = P.d_rows + n0;
-#define LAL_SPGEMM_GROUP(HH, G, NT, NUM)                                                     \
-    spgemm_group_kernel<HH, G, NT, NUM><<<(nr + NT / G - 1) / (NT / G), NT, 0, c->stream>>>(  \
-        nr, rows, arp, aci, av, brp, bci, bv, crp, cout_, cval, c->d_flag)
-            switch(b)
-            {
-            case 0: LAL_SPGEMM_GROUP(64, 8, 256, NUMERIC); break;
-            case 1: LAL_SPGEMM_GROUP(128, 16, 256, NUMERIC); break;
-            case 2: LAL_SPGEMM_GROUP(256, 32, 256, NUMERIC); break;
-            // 512 and 1024 slots: a wavefront per row for the numeric pass
-            // (24 / 48 KB for four rows), 32 lanes for the symbolic pass's
-            // key-only tables (sized by products; 8 rows hold 16 / 32 KB)
-            case 3:
-                if constexpr(NUMERIC)
-                    LAL_SPGEMM_GROUP(512, 64, 256, true);
-                else
-                    LAL_SPGEMM_GROUP(512, 32, 256, false);
-                break;
-            case 4:
-                if constexpr(NUMERIC)
-                    LAL_SPGEMM_GROUP(1024, 64, 256, true);
-                else
-                    LAL_SPGEMM_GROUP(1024, 32, 256, false);
-                break;
-            // one row (a wavefront) per workgroup from 2048 slots on
-            case 5: LAL_SPGEMM_GROUP(2048, 64, 64, NUMERIC); break;
-            case 6: LAL_SPGEMM_GROUP(4096, 64, 64, NUMERIC); break;
-            // key-only tables of the symbolic pass (the numeric pass never bins here)
-            case 7: LAL_SPGEMM_GROUP(8192, 64, 64, false); break;
-            case 8: LAL_SPGEMM_GROUP(16384, 64, 64, false); break;
-            case 9: LAL_SPGEMM_GROUP(32768, 64, 64, false); break;
-            }
-#undef LAL_SPGEMM_GROUP
+            const int H = 64 << b;
+#define LAL_SPGEMM_COUNT(HH)                                                                 \
+    spgemm_count_kernel<HH><<<nr, 256, 0, c->stream>>>(rows, arp, aci, brp, bci, cout_, c->d_flag)
+            // the symbolic pass's tables of 2048 slots and more (alone beyond
+            // 4096), and smaller ones of so few rows that the chip holds a
+            // workgroup for each: a workgroup per row
+            if(!NUMERIC && (H >= 2048 || (H >= 512 && nr <= 2048)))
+                switch(b)
+                {
+                case 3: LAL_SPGEMM_COUNT(512); break;
+                case 4: LAL_SPGEMM_COUNT(1024); break;
+                case 5: LAL_SPGEMM_COUNT(2048); break;
+                case 6: LAL_SPGEMM_COUNT(4096); break;
+                case 7: LAL_SPGEMM_COUNT(8192); break;
+                case 8: LAL_SPGEMM_COUNT(16384); break;
+                default: LAL_SPGEMM_COUNT(32768); break;
+                }
+            else
+                launch_group<NUMERIC>(c, nr, H, P.g, P.l, rows, arp, aci, av, brp, bci, bv, crp,
+                                      cout_, cval);
+#undef LAL_SPGEMM_COUNT
             LAL_LAUNCHED();
         }
         if(P.n_global)
@@ -764,11 +1004,13 @@ namespace lal
     }
 
     int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a)
+                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a,
+                    long nnz_b)
     {
-        (void)k;
         LAL_HIP(hipMemsetAsync(crp, 0, sizeof(int) * (m + 1), c->stream));
         spgemm_plan P;
+        P.g = lanes_for(m > 0 ? nnz_a / m : 0);
+        P.l = lanes_for(k > 0 ? nnz_b / k : 0);
         LAL_TRY(make_plan(c, m, n, arp, aci, brp, nullptr, false, P, nnz_a));
         int st = run_plan<false>(c, P, arp, aci, nullptr, brp, bci, nullptr, nullptr, crp,
                                  nullptr);
@@ -784,10 +1026,11 @@ namespace lal
 
     int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                           const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv)
+                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b)
     {
-        (void)k;
         spgemm_plan P;
+        P.g = lanes_for(m > 0 ? nnz_a / m : 0);
+        P.l = lanes_for(k > 0 ? nnz_b / k : 0);
         LAL_TRY(make_plan(c, m, n, arp, aci, brp, crp, true, P));
         LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
         int st = run_plan<true>(c, P, arp, aci, av, brp, bci, bv, crp, cci, cv);
@@ -883,7 +1126,7 @@ extern "C" int lal_csrgemm_nnz(lal_handle c, int m, int k, int n, int nnz_A, con
     LAL_REQUIRE(crp != nullptr && nnz_C != nullptr && arp != nullptr && brp != nullptr);
     LAL_REQUIRE((nnz_A == 0 || aci) && (nnz_B == 0 || bci));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
-    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A);
+    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A, nnz_B);
 }
 
 extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_A,
@@ -895,5 +1138,6 @@ extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_
     LAL_REQUIRE(crp != nullptr && arp != nullptr && brp != nullptr);
     LAL_REQUIRE((nnz_A == 0 || (aci && av)) && (nnz_B == 0 || (bci && bv)));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
-    return lal::csrgemm_solve_f64(c, m, k, n, arp, aci, av, brp, bci, bv, crp, cci, cv);
+    return lal::csrgemm_solve_f64(c, m, k, n, arp, aci, av, brp, bci, bv, crp, cci, cv, nnz_A,
+                                  nnz_B);
 }
