@@ -567,12 +567,13 @@ namespace lal
                      double* d);
 
     int sa_strength(lal_context* c, int m, int nnz, const int* rp, const int* ci,
-                    const double* v, double eps, int* conn)
+                    const double* v, double eps, int* conn, arena* a)
     {
         if(m == 0)
             return LAL_OK;
+        temps   tmp(c, a);
         double* d = nullptr;
-        LAL_HIP(hipMallocAsync((void**)&d, sizeof(double) * m, c->stream));
+        LAL_TRY(tmp.get(&d, m));
         LAL_HIP(hipMemsetAsync(d, 0, sizeof(double) * m, c->stream));
         const int lanes = setup_row_lanes(nnz, m);
         if(lanes == 64)
@@ -595,19 +596,19 @@ namespace lal
             strength_kernel<<<grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, v, d, eps, conn);
         }
         LAL_LAUNCHED();
-        LAL_HIP(hipFreeAsync(d, c->stream));
         return LAL_OK;
     }
 
     int pmis_aggregate(lal_context* c, int m, int nnz, const int* rp, const int* ci,
-                       const int* conn, int64_t* agg)
+                       const int* conn, int64_t* agg, arena* a)
     {
         if(m == 0)
             return LAL_OK;
-        int *state = nullptr, *max_state = nullptr, *hash = nullptr;
-        LAL_HIP(hipMallocAsync((void**)&state, sizeof(int) * m, c->stream));
-        LAL_HIP(hipMallocAsync((void**)&max_state, sizeof(int) * m, c->stream));
-        LAL_HIP(hipMallocAsync((void**)&hash, sizeof(int) * m, c->stream));
+        temps tmp(c, a);
+        int * state = nullptr, *max_state = nullptr, *hash = nullptr;
+        LAL_TRY(tmp.get(&state, m));
+        LAL_TRY(tmp.get(&max_state, m));
+        LAL_TRY(tmp.get(&hash, m));
         LAL_HIP(hipMemsetAsync(agg, 0, sizeof(int64_t) * m, c->stream));
         const int g     = grid_for(m, 256);
         const int lanes = setup_row_lanes(nnz, m);
@@ -662,7 +663,7 @@ namespace lal
         if(buf[cur] != max_state)
             LAL_HIP(hipMemcpyAsync(max_state, buf[cur], sizeof(int) * m, hipMemcpyDeviceToDevice,
                                    c->stream));
-        LAL_TRY(scan_i64_dev(c, m, agg));
+        LAL_TRY(scan_i64_dev(c, m, agg, a));
         for(int k = 0; k < 2; k++)
         {
             LAL_HIP(hipMemcpyAsync(state, max_state, sizeof(int) * m, hipMemcpyDeviceToDevice,
@@ -678,15 +679,12 @@ namespace lal
                                                            max_state);
             LAL_LAUNCHED();
         }
-        LAL_HIP(hipFreeAsync(state, c->stream));
-        LAL_HIP(hipFreeAsync(max_state, c->stream));
-        LAL_HIP(hipFreeAsync(hash, c->stream));
         return LAL_OK;
     }
 
     int sa_prolongator_nnz(lal_context* c, int m, int nnz, const int* rp, const int* ci,
                            const int* conn, const int64_t* agg, int* prp, int* nnz_P,
-                           int* n_c)
+                           int* n_c, arena* a)
     {
         // count[m] = 0 is written by the group of row m, so m + 1 groups
         if(m > 0 && nnz >= PROLONG_WAVE_MIN_ROW * (long)m)
@@ -696,7 +694,7 @@ namespace lal
             prolong_count_group_kernel<8><<<(m + 1 + 31) / 32, 256, 0, c->stream>>>(m, rp, ci,
                                                                                     conn, agg, prp);
         LAL_LAUNCHED();
-        LAL_TRY(scan_i32_dev(c, m + 1, prp));
+        LAL_TRY(scan_i32_dev(c, m + 1, prp, a));
         int64_t mx = LLONG_MIN;
         LAL_TRY(max_i64_dev(c, m, agg, &mx));
         int64_t nc = std::max<int64_t>(mx, -1) + 1;
@@ -753,11 +751,11 @@ namespace
 namespace lal
 {
     int ua_prolongator_nnz(lal_context* c, int m, const int64_t* agg, int* prp, int* nnz_P,
-                           int* n_c)
+                           int* n_c, arena* a)
     {
         ua_count_kernel<<<grid_for(m + 1, 256), 256, 0, c->stream>>>(m, agg, prp);
         LAL_LAUNCHED();
-        LAL_TRY(scan_i32_dev(c, m + 1, prp));
+        LAL_TRY(scan_i32_dev(c, m + 1, prp, a));
         int64_t mx = LLONG_MIN;
         LAL_TRY(max_i64_dev(c, m, agg, &mx));
         const int64_t nc = std::max<int64_t>(mx, -1) + 1;
@@ -785,7 +783,7 @@ extern "C" int lal_sa_strength_f64(lal_handle c, int m, int nnz, const int* rp, 
 {
     LAL_REQUIRE(c != nullptr && m >= 0 && nnz >= 0);
     LAL_REQUIRE(m == 0 || (rp && (nnz == 0 || (ci && v && conn))));
-    return lal::sa_strength(c, m, nnz, rp, ci, v, eps, conn);
+    return lal::sa_strength(c, m, nnz, rp, ci, v, eps, conn, nullptr);
 }
 
 extern "C" int lal_pmis_aggregate(lal_handle c, int m, int nnz, const int* rp, const int* ci,
@@ -793,7 +791,7 @@ extern "C" int lal_pmis_aggregate(lal_handle c, int m, int nnz, const int* rp, c
 {
     LAL_REQUIRE(c != nullptr && m >= 0 && nnz >= 0);
     LAL_REQUIRE(m == 0 || (rp && agg && (nnz == 0 || (ci && conn))));
-    return lal::pmis_aggregate(c, m, nnz, rp, ci, conn, agg);
+    return lal::pmis_aggregate(c, m, nnz, rp, ci, conn, agg, nullptr);
 }
 
 extern "C" int lal_pmis_init(lal_handle c, int m, int nnz, const int* rp, const int* conn,
@@ -846,7 +844,7 @@ extern "C" int lal_sa_prolongator_nnz(lal_handle c, int m, int nnz, const int* r
 {
     LAL_REQUIRE(c != nullptr && m >= 0 && nnz >= 0 && prp && nnz_P && n_c);
     LAL_REQUIRE(m == 0 || (rp && agg && (nnz == 0 || (ci && conn))));
-    return lal::sa_prolongator_nnz(c, m, nnz, rp, ci, conn, agg, prp, nnz_P, n_c);
+    return lal::sa_prolongator_nnz(c, m, nnz, rp, ci, conn, agg, prp, nnz_P, n_c, nullptr);
 }
 
 extern "C" int lal_sa_prolongator_fill_f64(lal_handle c, int m, int nnz, const int* rp,

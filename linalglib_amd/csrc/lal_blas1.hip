@@ -326,16 +326,15 @@ namespace
     }
 
     template <typename T>
-    int scan_dev(lal_context* c, int n, T* x)
+    int scan_dev(lal_context* c, int n, T* x, lal::arena* a)
     {
         if(n <= 0)
             return LAL_OK;
-        int ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-        T*  sums   = nullptr;
-        LAL_HIP(hipMallocAsync((void**)&sums, sizeof(T) * ntiles, c->stream));
-        const int st = scan_passes<T>(c, n, x, sums);
-        LAL_HIP(hipFreeAsync(sums, c->stream));
-        return st;
+        int        ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+        T*         sums   = nullptr;
+        lal::temps tmp(c, a);
+        LAL_TRY(tmp.get(&sums, ntiles));
+        return scan_passes<T>(c, n, x, sums);
     }
 
     __global__ void __launch_bounds__(256)
@@ -394,13 +393,13 @@ namespace lal
     {
         return reduce_dev<double, 1>(c, n, x, x, d_out);
     }
-    int scan_i32_dev(lal_context* c, int n, int32_t* x)
+    int scan_i32_dev(lal_context* c, int n, int32_t* x, arena* a)
     {
-        return scan_dev<int32_t>(c, n, x);
+        return scan_dev<int32_t>(c, n, x, a);
     }
-    int scan_i64_dev(lal_context* c, int n, int64_t* x)
+    int scan_i64_dev(lal_context* c, int n, int64_t* x, arena* a)
     {
-        return scan_dev<int64_t>(c, n, x);
+        return scan_dev<int64_t>(c, n, x, a);
     }
 
     // Called by lal_create with `device` current: the device address of that

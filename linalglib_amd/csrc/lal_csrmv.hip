@@ -242,7 +242,8 @@ namespace lal
     }
 
     int csrmv_analysis_dev(lal_context* c, int m, int n, int nnz, const int* rp,
-                           const int* ci, int exact, lal_csrmv_info** out, bool trusted)
+                           const int* ci, int exact, lal_csrmv_info** out, bool trusted,
+                           arena* mem)
     {
         if(!trusted)
             LAL_TRY(check_columns(c, nnz, n, ci));
@@ -287,7 +288,11 @@ namespace lal
             packed[meta_at + 4 * k + 3] = h[blocks[k + 1]];
         }
         d->win = win;
-        if(hipMalloc(&d->d_blocks, sizeof(int) * packed.size()) != hipSuccess)
+        d->owned = mem == nullptr;
+        if((mem ? mem->get(&d->d_blocks, packed.size())
+                : hipMalloc(&d->d_blocks, sizeof(int) * packed.size()) == hipSuccess
+                      ? LAL_OK
+                      : LAL_ERR_OOM) != LAL_OK)
         {
             delete d;
             return LAL_ERR_OOM;
@@ -299,41 +304,27 @@ namespace lal
         return LAL_OK;
     }
 
-    int compact_columns(lal_context* c, lal_csrmv_info* d, int nnz, const int* ci)
+    int compact_columns(lal_context* c, lal_csrmv_info* d, int nnz, const int* ci, arena* mem)
     {
         if(!d || d->exact || nnz <= 0 || d->nblocks <= 0 || d->d_c16)
             return LAL_OK;
         unsigned short* c16   = nullptr;
         int*            cbase = nullptr;
         int*            fail  = c->d_flag; // the context's flag word, read back below
-        auto release = [&]() {
-            (void)hipFree(c16);
-            (void)hipFree(cbase);
-        };
+        const auto      mark  = mem->mark();
         // rounded up to whole 16-byte lines: the kernels load four entries at a time
-        if(hipMalloc(&c16, ((size_t)nnz * sizeof(unsigned short) + 15) & ~(size_t)15) !=
-               hipSuccess ||
-           hipMalloc(&cbase, sizeof(int) * d->nblocks) != hipSuccess)
+        LAL_TRY(mem->get(&c16, ((size_t)nnz + 7) & ~(size_t)7));
+        LAL_TRY(mem->get(&cbase, d->nblocks));
+        LAL_HIP(hipMemsetAsync(fail, 0, sizeof(int), c->stream));
+        c16_kernel<<<d->nblocks, 256, 0, c->stream>>>(d->d_blocks, d->nblocks, ci, cbase, c16,
+                                                      fail);
+        LAL_LAUNCHED();
+        LAL_HIP(hipMemcpyAsync(c->h_flag, fail, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        LAL_HIP(hipStreamSynchronize(c->stream));
+        if(c->h_flag[0])
         {
-            release();
-            return LAL_ERR_OOM;
-        }
-        int rc = hipMemsetAsync(fail, 0, sizeof(int), c->stream) == hipSuccess ? LAL_OK : LAL_ERR_HIP;
-        if(rc == LAL_OK)
-        {
-            c16_kernel<<<d->nblocks, 256, 0, c->stream>>>(d->d_blocks, d->nblocks, ci, cbase, c16,
-                                                         fail);
-            if(hipGetLastError() != hipSuccess ||
-               hipMemcpyAsync(c->h_flag, fail, sizeof(int), hipMemcpyDeviceToHost, c->stream) !=
-                   hipSuccess ||
-               hipStreamSynchronize(c->stream) != hipSuccess)
-                rc = LAL_ERR_HIP;
-        }
-        const int h_fail = rc == LAL_OK ? c->h_flag[0] : 1;
-        if(rc != LAL_OK || h_fail)
-        {
-            release();
-            return rc;
+            mem->release(mark);
+            return LAL_OK;
         }
         d->d_c16   = c16;
         d->d_cbase = cbase;
@@ -389,16 +380,16 @@ extern "C" int lal_csrmv_analysis(lal_handle c, int m, int n, int nnz, const int
     LAL_REQUIRE(c != nullptr && descr != nullptr && m >= 0 && n >= 0 && nnz >= 0);
     LAL_REQUIRE(row_ptr != nullptr && (nnz == 0 || col_ind != nullptr));
     *descr = nullptr;
-    return lal::csrmv_analysis_dev(c, m, n, nnz, row_ptr, col_ind, exact, descr, false);
+    return lal::csrmv_analysis_dev(c, m, n, nnz, row_ptr, col_ind, exact, descr, false,
+                                   nullptr);
 }
 
 extern "C" int lal_csrmv_descr_destroy(lal_csrmv_descr d)
 {
     if(!d)
         return LAL_OK;
-    (void)hipFree(d->d_blocks);
-    (void)hipFree(d->d_c16);
-    (void)hipFree(d->d_cbase);
+    if(d->owned)
+        (void)hipFree(d->d_blocks);
     delete d;
     return LAL_OK;
 }

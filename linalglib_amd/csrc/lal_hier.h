@@ -20,19 +20,6 @@ namespace lal
         double*         v   = nullptr;
         float*          v32 = nullptr;
         lal_csrmv_info* d   = nullptr;
-
-        void free_all()
-        {
-            (void)hipFree(rp);
-            (void)hipFree(ci);
-            (void)hipFree(v);
-            (void)hipFree(v32);
-            lal_csrmv_descr_destroy(d);
-            rp = ci = nullptr;
-            v       = nullptr;
-            v32     = nullptr;
-            d       = nullptr;
-        }
     };
 
     template <typename T>
@@ -131,6 +118,9 @@ struct lal_hierarchy_t
     lal_context*      c = nullptr;
     lal_saamg_options opts{};
     int               levels = 0;
+    // every device array of the build lies in here (the Gauss-Seidel
+    // schedules, built on first use, have their own)
+    lal::arena        mem;
     lal::level_t      L[21];
     // coarsest level
     int     coarse_kind = 0; // 0 scalar, 1 Gauss-Seidel, 2 dense inverse
@@ -185,28 +175,19 @@ struct lal_hierarchy_t
             (void)hipStreamDestroy(capture_stream);
         for(int l = 0; l <= 20; l++)
         {
-            L[l].A.free_all();
-            L[l].P.free_all();
-            L[l].R.free_all();
-            for(double* ptr : {L[l].w64.x, L[l].w64.t, L[l].w64.b, L[l].w64.r, L[l].w64.diag,
-                               L[l].w64.dinv})
-                (void)hipFree(ptr);
-            for(float* ptr : {L[l].w32.x, L[l].w32.t, L[l].w32.b, L[l].w32.r, L[l].w32.diag,
-                              L[l].w32.dinv})
-                (void)hipFree(ptr);
+            for(lal::csr_dev* M : {&L[l].A, &L[l].P, &L[l].R})
+                lal_csrmv_descr_destroy(M->d);
             for(lal::gs_sched* g : {&L[l].gs_fwd, &L[l].gs_bwd})
                 for(void* ptr : {(void*)g->perm, (void*)g->off_d, (void*)g->prp, (void*)g->pci,
                                  (void*)g->pv, (void*)g->pdiag, (void*)g->tiles})
-                    (void)hipFree(ptr);
+                    if(ptr)
+                        (void)hipFree(ptr);
             for(void* ptr : {(void*)L[l].mc.off_d, (void*)L[l].mc.perm, (void*)L[l].mc.prp,
                              (void*)L[l].mc.pci, (void*)L[l].mc.pv, (void*)L[l].mc.pdinv,
                              (void*)L[l].mc.plan})
-                (void)hipFree(ptr);
+                if(ptr)
+                    (void)hipFree(ptr);
         }
-        for(void* ptr : {(void*)coarse_inv, (void*)res, (void*)z, (void*)p, (void*)q,
-                         (void*)res32, (void*)z32, (void*)p32, (void*)q32, (void*)d32, (void*)s,
-                         (void*)part, (void*)tail_img64, (void*)tail_img32})
-            (void)hipFree(ptr);
         if(h_note)
             (void)hipHostFree(h_note);
     }

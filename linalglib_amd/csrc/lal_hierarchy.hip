@@ -22,29 +22,30 @@
 namespace lal
 {
     int sa_strength(lal_context* c, int m, int nnz, const int* rp, const int* ci,
-                    const double* v, double eps, int* conn);
+                    const double* v, double eps, int* conn, arena* a);
     int pmis_aggregate(lal_context* c, int m, int nnz, const int* rp, const int* ci,
-                       const int* conn, int64_t* agg);
+                       const int* conn, int64_t* agg, arena* a);
     int sa_prolongator_nnz(lal_context* c, int m, int nnz, const int* rp, const int* ci,
-                           const int* conn, const int64_t* agg, int* prp, int* nnz_P, int* n_c);
+                           const int* conn, const int64_t* agg, int* prp, int* nnz_P, int* n_c,
+                           arena* a);
     int sa_prolongator_fill(lal_context* c, int m, int nnz, const int* rp, const int* ci,
                             const double* v, const int* conn, const int64_t* agg, double relax,
                             const int* prp, int* pci, double* pv);
     int ua_prolongator_nnz(lal_context* c, int m, const int64_t* agg, int* prp, int* nnz_P,
-                           int* n_c);
+                           int* n_c, arena* a);
     int ua_prolongator_fill(lal_context* c, int m, const int64_t* agg, const int* prp, int* pci,
                             double* pv);
     int transpose_f64(lal_context* c, int m, int n, int nnz, const int* rp, const int* ci,
-                      const double* v, int* trp, int* tci, double* tv);
+                      const double* v, int* trp, int* tci, double* tv, arena* a);
     // nnz_a: A's nonzeros, which pick the lanes per row of the product count
     int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a, long nnz_b);
+                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a, long nnz_b,
+                    arena* a);
     int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                           const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b);
+                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b, arena* a);
 }
 
-using lal::alloc_n;
 using lal::converges;
 using lal::post_scalar;
 using lal::wait_scalar;
@@ -235,7 +236,7 @@ namespace
             return false;
         if(img)
         {
-            *status = alloc_n(img, (size_t)d->img_words);
+            *status = h->mem.get(img, (size_t)d->img_words);
             if(*status != LAL_OK)
                 return false;
             for(const piece& p : pieces)
@@ -253,11 +254,11 @@ namespace
         return true;
     }
 
-    int to_f32(lal_context* c, const double* x, float** y, size_t n)
+    int to_f32(lal_hierarchy_t* h, const double* x, float** y, size_t n)
     {
-        LAL_TRY(alloc_n(y, n));
+        LAL_TRY(h->mem.get(y, n));
         if(n)
-            LAL_TRY(lal_convert_f64_f32(c, x, *y, n));
+            LAL_TRY(lal_convert_f64_f32(h->c, x, *y, n));
         return LAL_OK;
     }
 
@@ -272,7 +273,7 @@ namespace
             // same row pointer, copied); the rest are this setup's products
             if(!L.A.d)
                 LAL_TRY(lal::csrmv_analysis_dev(c, L.A.m, L.A.n, L.A.nnz, L.A.rp, L.A.ci, exact,
-                                                &L.A.d, true));
+                                                &L.A.d, true, &h->mem));
             L.A.d->exact = exact;
             // The finest operator is read three times per PCG iteration
             // (residual, post-sweep, the Krylov product), the last two with
@@ -284,41 +285,41 @@ namespace
             // columns (offsets from each row block's smallest column) where
             // the blocks allow it: 2 bytes per nonzero less, same results
             if(!exact)
-                LAL_TRY(lal::compact_columns(c, L.A.d, L.A.nnz, L.A.ci));
-            LAL_TRY(alloc_n(&L.w64.x, L.A.m));
-            LAL_TRY(alloc_n(&L.w64.t, L.A.m));
-            LAL_TRY(alloc_n(&L.w64.b, L.A.m));
-            LAL_TRY(alloc_n(&L.w64.r, L.A.m));
-            LAL_TRY(alloc_n(&L.w64.diag, L.A.m));
-            LAL_TRY(alloc_n(&L.w64.dinv, L.A.m));
+                LAL_TRY(lal::compact_columns(c, L.A.d, L.A.nnz, L.A.ci, &h->mem));
+            LAL_TRY(h->mem.get(&L.w64.x, L.A.m));
+            LAL_TRY(h->mem.get(&L.w64.t, L.A.m));
+            LAL_TRY(h->mem.get(&L.w64.b, L.A.m));
+            LAL_TRY(h->mem.get(&L.w64.r, L.A.m));
+            LAL_TRY(h->mem.get(&L.w64.diag, L.A.m));
+            LAL_TRY(h->mem.get(&L.w64.dinv, L.A.m));
             LAL_TRY(lal::diag_inv<double>(c, L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag,
                                           L.w64.dinv, L.A.nnz));
             if(l < h->levels)
             {
                 LAL_TRY(lal::csrmv_analysis_dev(c, L.P.m, L.P.n, L.P.nnz, L.P.rp, L.P.ci, exact,
-                                                &L.P.d, true));
+                                                &L.P.d, true, &h->mem));
                 LAL_TRY(lal::csrmv_analysis_dev(c, L.R.m, L.R.n, L.R.nnz, L.R.rp, L.R.ci, exact,
-                                                &L.R.d, true));
+                                                &L.R.d, true, &h->mem));
                 if(!exact)
                 {
-                    LAL_TRY(lal::compact_columns(c, L.P.d, L.P.nnz, L.P.ci));
-                    LAL_TRY(lal::compact_columns(c, L.R.d, L.R.nnz, L.R.ci));
+                    LAL_TRY(lal::compact_columns(c, L.P.d, L.P.nnz, L.P.ci, &h->mem));
+                    LAL_TRY(lal::compact_columns(c, L.R.d, L.R.nnz, L.R.ci, &h->mem));
                 }
             }
             if(h->opts.build_f32)
             {
-                LAL_TRY(to_f32(c, L.A.v, &L.A.v32, L.A.nnz));
+                LAL_TRY(to_f32(h, L.A.v, &L.A.v32, L.A.nnz));
                 if(l < h->levels)
                 {
-                    LAL_TRY(to_f32(c, L.P.v, &L.P.v32, L.P.nnz));
-                    LAL_TRY(to_f32(c, L.R.v, &L.R.v32, L.R.nnz));
+                    LAL_TRY(to_f32(h, L.P.v, &L.P.v32, L.P.nnz));
+                    LAL_TRY(to_f32(h, L.R.v, &L.R.v32, L.R.nnz));
                 }
-                LAL_TRY(alloc_n(&L.w32.x, L.A.m));
-                LAL_TRY(alloc_n(&L.w32.t, L.A.m));
-                LAL_TRY(alloc_n(&L.w32.b, L.A.m));
-                LAL_TRY(alloc_n(&L.w32.r, L.A.m));
-                LAL_TRY(alloc_n(&L.w32.diag, L.A.m));
-                LAL_TRY(alloc_n(&L.w32.dinv, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.x, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.t, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.b, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.r, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.diag, L.A.m));
+                LAL_TRY(h->mem.get(&L.w32.dinv, L.A.m));
                 LAL_TRY(lal::diag_inv<float>(c, L.A.m, L.A.rp, L.A.ci, L.A.v32, L.w32.diag,
                                              L.w32.dinv, L.A.nnz));
             }
@@ -350,7 +351,7 @@ namespace
             LAL_HIP(hipStreamSynchronize(c->stream));
             if(dense_inverse(Ac.m, rp, ci, v, inv))
             {
-                LAL_TRY(alloc_n(&h->coarse_inv, inv.size()));
+                LAL_TRY(h->mem.get(&h->coarse_inv, inv.size()));
                 LAL_HIP(hipMemcpyAsync(h->coarse_inv, inv.data(), sizeof(double) * inv.size(),
                                        hipMemcpyHostToDevice, c->stream));
                 LAL_HIP(hipStreamSynchronize(c->stream));
@@ -389,12 +390,12 @@ namespace
         }
 
         const int n = h->L[0].A.m;
-        LAL_TRY(alloc_n(&h->res, n));
-        LAL_TRY(alloc_n(&h->z, n));
-        LAL_TRY(alloc_n(&h->p, n));
-        LAL_TRY(alloc_n(&h->q, n));
-        LAL_TRY(alloc_n(&h->s, lal::LAL_SOLVER_SLOTS));
-        LAL_TRY(alloc_n(&h->part, 4 * lal::PCG_BLOCKS));
+        LAL_TRY(h->mem.get(&h->res, n));
+        LAL_TRY(h->mem.get(&h->z, n));
+        LAL_TRY(h->mem.get(&h->p, n));
+        LAL_TRY(h->mem.get(&h->q, n));
+        LAL_TRY(h->mem.get(&h->s, lal::LAL_SOLVER_SLOTS));
+        LAL_TRY(h->mem.get(&h->part, 4 * lal::PCG_BLOCKS));
         LAL_HIP(hipHostMalloc((void**)&h->h_note, 64, hipHostMallocMapped | hipHostMallocCoherent));
         std::memset(h->h_note, 0, 64);
         h->h_seq = reinterpret_cast<unsigned*>(h->h_note + 1);
@@ -402,11 +403,11 @@ namespace
         h->d_seq = reinterpret_cast<unsigned*>(h->d_note + 1);
         if(h->opts.build_f32)
         {
-            LAL_TRY(alloc_n(&h->res32, n));
-            LAL_TRY(alloc_n(&h->z32, n));
-            LAL_TRY(alloc_n(&h->p32, n));
-            LAL_TRY(alloc_n(&h->q32, n));
-            LAL_TRY(alloc_n(&h->d32, n));
+            LAL_TRY(h->mem.get(&h->res32, n));
+            LAL_TRY(h->mem.get(&h->z32, n));
+            LAL_TRY(h->mem.get(&h->p32, n));
+            LAL_TRY(h->mem.get(&h->q32, n));
+            LAL_TRY(h->mem.get(&h->d32, n));
             h->has32 = true;
         }
         LAL_HIP(hipStreamSynchronize(c->stream));
@@ -426,9 +427,11 @@ namespace
         A0.m = m;
         A0.n = n;
         A0.nnz = nnz;
-        LAL_TRY(alloc_n(&A0.rp, m + 1));
-        LAL_TRY(alloc_n(&A0.ci, nnz));
-        LAL_TRY(alloc_n(&A0.v, nnz));
+        lal::arena tmp; // a level's temporary arrays
+        tmp.reserve((size_t)nnz * 30 + (size_t)m * 60);
+        LAL_TRY(h->mem.get(&A0.rp, m + 1));
+        LAL_TRY(h->mem.get(&A0.ci, nnz));
+        LAL_TRY(h->mem.get(&A0.v, nnz));
         LAL_HIP(hipMemcpyAsync(A0.rp, rp, sizeof(int) * (m + 1), hipMemcpyDeviceToDevice,
                                c->stream));
         if(nnz)
@@ -449,73 +452,70 @@ namespace
             csr_dev& Ac = h->L[level + 1].A;
             int*     conn = nullptr;
             int64_t* agg  = nullptr;
-            LAL_TRY(alloc_n(&conn, Af.nnz));
-            LAL_TRY(alloc_n(&agg, Af.m));
-            LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn));
-            LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg));
-            LAL_TRY(alloc_n(&P.rp, Af.m + 1));
+            tmp.release(lal::arena::mark_t{});
+            LAL_TRY(tmp.get(&conn, Af.nnz));
+            LAL_TRY(tmp.get(&agg, Af.m));
+            LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn, &tmp));
+            LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, &tmp));
+            LAL_TRY(h->mem.get(&P.rp, Af.m + 1));
             int nnzP = 0, nc = 0;
             if(unsmoothed)
-                LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc));
+                LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc, &tmp));
             else
                 LAL_TRY(lal::sa_prolongator_nnz(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, P.rp,
-                                                &nnzP, &nc));
+                                                &nnzP, &nc, &tmp));
             if(nc == 0)
             {
-                (void)hipFree(conn);
-                (void)hipFree(agg);
-                P.free_all();
+                P = csr_dev{};
                 break;
             }
             P.m   = Af.m;
             P.n   = nc;
             P.nnz = nnzP;
-            LAL_TRY(alloc_n(&P.ci, nnzP));
-            LAL_TRY(alloc_n(&P.v, nnzP));
+            LAL_TRY(h->mem.get(&P.ci, nnzP));
+            LAL_TRY(h->mem.get(&P.v, nnzP));
             if(unsmoothed)
                 LAL_TRY(lal::ua_prolongator_fill(c, Af.m, agg, P.rp, P.ci, P.v));
             else
                 LAL_TRY(lal::sa_prolongator_fill(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, conn, agg,
                                                  o.relax, P.rp, P.ci, P.v));
-            (void)hipStreamSynchronize(c->stream);
-            (void)hipFree(conn);
-            (void)hipFree(agg);
             // R = P^T
             R.m   = nc;
             R.n   = Af.m;
             R.nnz = nnzP;
-            LAL_TRY(alloc_n(&R.rp, nc + 1));
-            LAL_TRY(alloc_n(&R.ci, nnzP));
-            LAL_TRY(alloc_n(&R.v, nnzP));
-            LAL_TRY(lal::transpose_f64(c, P.m, P.n, P.nnz, P.rp, P.ci, P.v, R.rp, R.ci, R.v));
+            LAL_TRY(h->mem.get(&R.rp, nc + 1));
+            LAL_TRY(h->mem.get(&R.ci, nnzP));
+            LAL_TRY(h->mem.get(&R.v, nnzP));
+            LAL_TRY(lal::transpose_f64(c, P.m, P.n, P.nnz, P.rp, P.ci, P.v, R.rp, R.ci, R.v,
+                                       &tmp));
             // AP = A P
             csr_dev AP;
             AP.m = Af.m;
             AP.n = nc;
-            LAL_TRY(alloc_n(&AP.rp, Af.m + 1));
+            LAL_TRY(tmp.get(&AP.rp, Af.m + 1));
             LAL_TRY(lal::csrgemm_nnz(c, Af.m, Af.n, nc, Af.rp, Af.ci, P.rp, P.ci, AP.rp,
-                                     &AP.nnz, Af.nnz, P.nnz));
-            LAL_TRY(alloc_n(&AP.ci, AP.nnz));
-            LAL_TRY(alloc_n(&AP.v, AP.nnz));
+                                     &AP.nnz, Af.nnz, P.nnz, &tmp));
+            LAL_TRY(tmp.get(&AP.ci, AP.nnz));
+            LAL_TRY(tmp.get(&AP.v, AP.nnz));
             LAL_TRY(lal::csrgemm_solve_f64(c, Af.m, Af.n, nc, Af.rp, Af.ci, Af.v, P.rp, P.ci,
-                                           P.v, AP.rp, AP.ci, AP.v, Af.nnz, P.nnz));
+                                           P.v, AP.rp, AP.ci, AP.v, Af.nnz, P.nnz, &tmp));
             // A_c = R (A P)
             Ac.m = nc;
             Ac.n = nc;
-            LAL_TRY(alloc_n(&Ac.rp, nc + 1));
+            LAL_TRY(h->mem.get(&Ac.rp, nc + 1));
             LAL_TRY(lal::csrgemm_nnz(c, nc, Af.m, nc, R.rp, R.ci, AP.rp, AP.ci, Ac.rp, &Ac.nnz,
-                                     R.nnz, AP.nnz));
-            LAL_TRY(alloc_n(&Ac.ci, Ac.nnz));
-            LAL_TRY(alloc_n(&Ac.v, Ac.nnz));
+                                     R.nnz, AP.nnz, &tmp));
+            LAL_TRY(h->mem.get(&Ac.ci, Ac.nnz));
+            LAL_TRY(h->mem.get(&Ac.v, Ac.nnz));
             LAL_TRY(lal::csrgemm_solve_f64(c, nc, Af.m, nc, R.rp, R.ci, R.v, AP.rp, AP.ci, AP.v,
-                                           Ac.rp, Ac.ci, Ac.v, R.nnz, AP.nnz));
-            (void)hipStreamSynchronize(c->stream);
-            AP.free_all();
+                                           Ac.rp, Ac.ci, Ac.v, R.nnz, AP.nnz, &tmp));
             level++;
             eps *= 0.5;
         }
-        h->levels = level;
-        return finish_setup(h);
+        h->levels    = level;
+        const int st = finish_setup(h);
+        (void)hipStreamSynchronize(c->stream); // before tmp goes
+        return st;
     }
 
     // One V-cycle at level l for rhs b with the initial guess zero.  The
@@ -1074,11 +1074,14 @@ namespace
         // validate the input pattern before any setup kernel gathers through
         // it; the analysis describes the finest operator (a copy of the same
         // pattern), so the hierarchy keeps it for level 0
-        lal_csrmv_info* d0 = nullptr;
-        LAL_TRY(lal::csrmv_analysis_dev(c, m, n, nnz, rp, ci, 0, &d0));
-        auto* h      = new lal_hierarchy_t;
-        h->L[0].A.d  = d0;
-        int   s = setup(c, m, n, nnz, rp, ci, v, o, h, unsmoothed);
+        auto* h = new lal_hierarchy_t;
+        // The whole hierarchy takes about 80 bytes per nonzero (120 with the
+        // FP32 levels) and 200 per row: the first chunk is half of that, and
+        // the arena grows by half its size.
+        h->mem.reserve((size_t)nnz * (o.build_f32 ? 60 : 40) + (size_t)m * 100);
+        int s = lal::csrmv_analysis_dev(c, m, n, nnz, rp, ci, 0, &h->L[0].A.d, false, &h->mem);
+        if(s == LAL_OK)
+            s = setup(c, m, n, nnz, rp, ci, v, o, h, unsmoothed);
         if(s != LAL_OK)
         {
             (void)hipStreamSynchronize(c->stream);

@@ -17,6 +17,48 @@
 
 struct lal_hierarchy_t;
 
+namespace lal
+{
+    // Device memory handed out from a few large allocations and freed with
+    // the object.  A hierarchy build makes several hundred arrays; one
+    // hipMalloc and hipFree each cost more than the build's kernels.
+    struct arena
+    {
+        struct mark_t
+        {
+            size_t chunk = 0, used = 0;
+        };
+        arena() = default;
+        arena(const arena&) = delete;
+        arena& operator=(const arena&) = delete;
+        ~arena();
+        // `first` bytes for the first allocation (rounded up as needed)
+        void reserve(size_t first)
+        {
+            next_ = first;
+        }
+        int get_bytes(void** p, size_t bytes);
+        template <typename T>
+        int get(T** p, size_t n)
+        {
+            return get_bytes(reinterpret_cast<void**>(p), sizeof(T) * (n > 0 ? n : 1));
+        }
+        // release(mark()) gives back what was taken since, for later work on
+        // the same stream
+        mark_t mark() const;
+        void   release(const mark_t& m);
+
+    private:
+        struct chunk
+        {
+            char*  p;
+            size_t cap, used;
+        };
+        std::vector<chunk> chunks_;
+        size_t             cur_ = 0, next_ = 0, total_ = 0;
+    };
+}
+
 // Devices the per-device static scratch table covers.
 #define LAL_MAX_DEVICES 64
 
@@ -186,6 +228,36 @@ namespace lal
         return v;
     }
 
+    // Temporary device arrays of one call: from `a` when given (marked and
+    // released by whoever owns it), else stream-ordered allocations freed at
+    // the end of the scope.
+    struct temps
+    {
+        temps(lal_context* c, arena* a) : c_(c), a_(a) {}
+        temps(const temps&) = delete;
+        ~temps()
+        {
+            for(void* p : own_)
+                (void)hipFreeAsync(p, c_->stream);
+        }
+        template <typename T>
+        int get(T** p, size_t n)
+        {
+            if(a_)
+                return a_->get(p, n);
+            *p = nullptr;
+            LAL_HIP(hipMallocAsync(reinterpret_cast<void**>(p), sizeof(T) * (n > 0 ? n : 1),
+                                   c_->stream));
+            own_.push_back(*p);
+            return LAL_OK;
+        }
+
+    private:
+        lal_context*       c_;
+        arena*             a_;
+        std::vector<void*> own_;
+    };
+
     // Internal launchers shared across translation units (device-resident
     // results; nothing is copied to the host).
     int dot_f64_dev(lal_context* c, int n, const double* x, const double* y, double* d_out,
@@ -193,8 +265,8 @@ namespace lal
     int dot_f32_dev(lal_context* c, int n, const float* x, const float* y, double* d_out,
                     int slot);
     int norm_inf_f64_dev(lal_context* c, int n, const double* x, double* d_out, int slot);
-    int scan_i32_dev(lal_context* c, int n, int32_t* x);
-    int scan_i64_dev(lal_context* c, int n, int64_t* x);
+    int scan_i32_dev(lal_context* c, int n, int32_t* x, arena* a = nullptr);
+    int scan_i64_dev(lal_context* c, int n, int64_t* x, arena* a = nullptr);
     // Device address of the allocation-free scan's static scratch for
     // `device` (which must be current), looked up once per device.
     int noalloc_scratch_init(int device);

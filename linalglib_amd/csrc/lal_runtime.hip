@@ -1,6 +1,7 @@
 // Context, memory and elementwise utilities of the C ABI.
 #include "lal_internal.h"
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -12,6 +13,58 @@ namespace lal
     void set_last_error(const char* msg)
     {
         g_last_error = msg;
+    }
+
+    arena::~arena()
+    {
+        for(chunk& k : chunks_)
+            (void)hipFree(k.p);
+    }
+
+    int arena::get_bytes(void** p, size_t bytes)
+    {
+        *p    = nullptr;
+        bytes = (bytes + 255) & ~(size_t)255;
+        for(; cur_ < chunks_.size(); cur_++)
+        {
+            chunk& k = chunks_[cur_];
+            if(k.cap - k.used >= bytes)
+            {
+                *p = k.p + k.used;
+                k.used += bytes;
+                return LAL_OK;
+            }
+        }
+        // a new chunk: half of what there is, within 1 MiB .. 512 MiB
+        size_t cap = std::max(next_, std::min(std::max(total_ / 2, (size_t)1 << 20),
+                                              (size_t)512 << 20));
+        cap        = std::max((cap + 255) & ~(size_t)255, bytes);
+        next_      = 0;
+        char* q    = nullptr;
+        if(cap > bytes && hipMalloc(&q, cap) != hipSuccess)
+        {
+            (void)hipGetLastError(); // no room to spare: just this array
+            q   = nullptr;
+            cap = bytes;
+        }
+        if(q == nullptr)
+            LAL_HIP(hipMalloc(&q, cap));
+        chunks_.push_back({q, cap, bytes});
+        total_ += cap;
+        *p = q;
+        return LAL_OK;
+    }
+
+    arena::mark_t arena::mark() const
+    {
+        return {cur_, cur_ < chunks_.size() ? chunks_[cur_].used : 0};
+    }
+
+    void arena::release(const mark_t& m)
+    {
+        for(size_t k = m.chunk; k < chunks_.size(); k++)
+            chunks_[k].used = k == m.chunk ? m.used : 0;
+        cur_ = m.chunk;
     }
 
     int hip_status(hipError_t e, const char* what, const char* file, int line)

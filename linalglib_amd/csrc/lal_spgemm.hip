@@ -679,23 +679,6 @@ namespace
         long long*        d_toff   = nullptr;
         int*              d_keys   = nullptr;
         double*           d_vals   = nullptr;
-
-        int release(hipStream_t s)
-        {
-            if(d_rows)
-                LAL_HIP(hipFreeAsync(d_rows, s));
-            if(d_toff)
-                LAL_HIP(hipFreeAsync(d_toff, s));
-            if(d_keys)
-                LAL_HIP(hipFreeAsync(d_keys, s));
-            if(d_vals)
-                LAL_HIP(hipFreeAsync(d_vals, s));
-            d_rows = nullptr;
-            d_toff = nullptr;
-            d_keys = nullptr;
-            d_vals = nullptr;
-            return LAL_OK;
-        }
     };
 
     constexpr int kBins = 10; // 64 .. 32768 (above 4096 only for the symbolic pass)
@@ -786,7 +769,7 @@ namespace
     // eleven bin counts (and, when some rows need global tables, their table
     // sizes) to size the launches and the global tables.
     int make_plan(lal_context* c, int m, int n, const int* arp, const int* aci, const int* brp,
-                  const int* crp, bool numeric, spgemm_plan& P, long nnz_a = 0)
+                  const int* crp, bool numeric, spgemm_plan& P, lal::temps& tmp, long nnz_a = 0)
     {
         constexpr int nb = kBins + 1;
         static_assert(nb <= 16, "the bin counts are read back through the context's flags");
@@ -802,7 +785,7 @@ namespace
         long long* d_gsl  = nullptr;
         if(!numeric)
         {
-            LAL_HIP(hipMallocAsync((void**)&d_prod, sizeof(int) * m, c->stream));
+            LAL_TRY(tmp.get(&d_prod, m));
             // rows of A averaging 16 or more entries: 16 lanes per row
             if(nnz_a >= 16L * m)
                 products_group_kernel<16><<<(int)(((long)m * 16 + 255) / 256), 256, 0,
@@ -811,7 +794,7 @@ namespace
                 products_kernel<<<grid, 256, 0, c->stream>>>(m, arp, aci, brp, d_prod);
             LAL_LAUNCHED();
         }
-        LAL_HIP(hipMallocAsync((void**)&d_bins, sizeof(int) * 2 * nb, c->stream));
+        LAL_TRY(tmp.get(&d_bins, 2 * nb));
         LAL_HIP(hipMemsetAsync(d_bins, 0, sizeof(int) * 2 * nb, c->stream));
         bin_count_kernel<<<grid, 256, 0, c->stream>>>(m, d_prod, numeric ? crp : nullptr, n,
                                                       max_h, d_bins);
@@ -831,10 +814,9 @@ namespace
         total += P.n_global;
         if(total)
         {
-            LAL_HIP(hipMallocAsync((void**)&P.d_rows, sizeof(int) * total, c->stream));
+            LAL_TRY(tmp.get(&P.d_rows, total));
             if(P.n_global)
-                LAL_HIP(hipMallocAsync((void**)&d_gsl, sizeof(long long) * P.n_global,
-                                       c->stream));
+                LAL_TRY(tmp.get(&d_gsl, P.n_global));
             bin_scatter_kernel<<<grid, 256, 0, c->stream>>>(m, d_prod, numeric ? crp : nullptr, n,
                                                             max_h, d_bins, d_bins + nb, P.d_rows,
                                                             d_gsl);
@@ -849,21 +831,15 @@ namespace
             for(int r = 0; r < P.n_global; r++)
                 P.toff[r + 1] += P.toff[r];
             const long long slots = P.toff[P.n_global];
-            LAL_HIP(hipMallocAsync((void**)&P.d_toff, sizeof(long long) * P.toff.size(),
-                                   c->stream));
+            LAL_TRY(tmp.get(&P.d_toff, P.toff.size()));
             LAL_HIP(hipMemcpyAsync(P.d_toff, P.toff.data(), sizeof(long long) * P.toff.size(),
                                    hipMemcpyHostToDevice, c->stream));
-            LAL_HIP(hipMallocAsync((void**)&P.d_keys, sizeof(int) * slots, c->stream));
+            LAL_TRY(tmp.get(&P.d_keys, slots));
             if(numeric)
-                LAL_HIP(hipMallocAsync((void**)&P.d_vals, sizeof(double) * slots, c->stream));
+                LAL_TRY(tmp.get(&P.d_vals, slots));
             // P.toff must outlive the copy to the device
             LAL_HIP(hipStreamSynchronize(c->stream));
         }
-        if(d_prod)
-            LAL_HIP(hipFreeAsync(d_prod, c->stream));
-        if(d_gsl)
-            LAL_HIP(hipFreeAsync(d_gsl, c->stream));
-        LAL_HIP(hipFreeAsync(d_bins, c->stream));
         return LAL_OK;
     }
 
@@ -974,49 +950,49 @@ namespace lal
 {
     template <typename T>
     int transpose_t(lal_context* c, int m, int n, int nnz, const int* rp, const int* ci,
-                    const T* v, int* trp, int* tci, T* tv)
+                    const T* v, int* trp, int* tci, T* tv, arena* a)
     {
+        temps tmp(c, a);
         LAL_HIP(hipMemsetAsync(trp, 0, sizeof(int) * (n + 1), c->stream));
         if(nnz > 0)
         {
             col_count_kernel<<<grid_for(nnz, 256), 256, 0, c->stream>>>(nnz, ci, trp);
             LAL_LAUNCHED();
         }
-        LAL_TRY(scan_i32_dev(c, n + 1, trp));
+        LAL_TRY(scan_i32_dev(c, n + 1, trp, a));
         if(nnz == 0)
             return LAL_OK;
         int* cursor = nullptr;
-        LAL_HIP(hipMallocAsync((void**)&cursor, sizeof(int) * std::max(n, 1), c->stream));
+        LAL_TRY(tmp.get(&cursor, n));
         LAL_HIP(hipMemcpyAsync(cursor, trp, sizeof(int) * n, hipMemcpyDeviceToDevice, c->stream));
         transpose_scatter_kernel<T><<<grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, v,
                                                                              cursor, tci, tv);
         LAL_LAUNCHED();
         row_sort_wave_kernel<T><<<(n + 3) / 4, 256, 0, c->stream>>>(n, trp, tci, tv);
         LAL_LAUNCHED();
-        LAL_HIP(hipFreeAsync(cursor, c->stream));
         return LAL_OK;
     }
 
     int transpose_f64(lal_context* c, int m, int n, int nnz, const int* rp, const int* ci,
-                      const double* v, int* trp, int* tci, double* tv)
+                      const double* v, int* trp, int* tci, double* tv, arena* a)
     {
-        return transpose_t<double>(c, m, n, nnz, rp, ci, v, trp, tci, tv);
+        return transpose_t<double>(c, m, n, nnz, rp, ci, v, trp, tci, tv, a);
     }
 
     int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                     const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a,
-                    long nnz_b)
+                    long nnz_b, arena* a)
     {
+        temps tmp(c, a);
         LAL_HIP(hipMemsetAsync(crp, 0, sizeof(int) * (m + 1), c->stream));
         spgemm_plan P;
         P.g = lanes_for(m > 0 ? nnz_a / m : 0);
         P.l = lanes_for(k > 0 ? nnz_b / k : 0);
-        LAL_TRY(make_plan(c, m, n, arp, aci, brp, nullptr, false, P, nnz_a));
+        LAL_TRY(make_plan(c, m, n, arp, aci, brp, nullptr, false, P, tmp, nnz_a));
         int st = run_plan<false>(c, P, arp, aci, nullptr, brp, bci, nullptr, nullptr, crp,
                                  nullptr);
-        P.release(c->stream);
         LAL_TRY(st);
-        LAL_TRY(scan_i32_dev(c, m + 1, crp));
+        LAL_TRY(scan_i32_dev(c, m + 1, crp, a));
         LAL_HIP(hipMemcpyAsync(c->h_flag, crp + m, sizeof(int), hipMemcpyDeviceToHost,
                                c->stream));
         LAL_HIP(hipStreamSynchronize(c->stream));
@@ -1026,15 +1002,15 @@ namespace lal
 
     int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                           const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b)
+                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b, arena* a)
     {
+        temps       tmp(c, a);
         spgemm_plan P;
         P.g = lanes_for(m > 0 ? nnz_a / m : 0);
         P.l = lanes_for(k > 0 ? nnz_b / k : 0);
-        LAL_TRY(make_plan(c, m, n, arp, aci, brp, crp, true, P));
+        LAL_TRY(make_plan(c, m, n, arp, aci, brp, crp, true, P, tmp));
         LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
         int st = run_plan<true>(c, P, arp, aci, av, brp, bci, bv, crp, cci, cv);
-        P.release(c->stream);
         LAL_TRY(st);
         LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost,
                                c->stream));
@@ -1107,7 +1083,7 @@ extern "C" int lal_transpose_f64(lal_handle c, int m, int n, int nnz, const int*
 {
     LAL_REQUIRE(c != nullptr && m >= 0 && n >= 0 && nnz >= 0 && trp != nullptr);
     LAL_REQUIRE(nnz == 0 || (rp && ci && v && tci && tv));
-    return lal::transpose_f64(c, m, n, nnz, rp, ci, v, trp, tci, tv);
+    return lal::transpose_f64(c, m, n, nnz, rp, ci, v, trp, tci, tv, nullptr);
 }
 
 extern "C" int lal_transpose_f32(lal_handle c, int m, int n, int nnz, const int* rp,
@@ -1115,7 +1091,7 @@ extern "C" int lal_transpose_f32(lal_handle c, int m, int n, int nnz, const int*
 {
     LAL_REQUIRE(c != nullptr && m >= 0 && n >= 0 && nnz >= 0 && trp != nullptr);
     LAL_REQUIRE(nnz == 0 || (rp && ci && v && tci && tv));
-    return lal::transpose_t<float>(c, m, n, nnz, rp, ci, v, trp, tci, tv);
+    return lal::transpose_t<float>(c, m, n, nnz, rp, ci, v, trp, tci, tv, nullptr);
 }
 
 extern "C" int lal_csrgemm_nnz(lal_handle c, int m, int k, int n, int nnz_A, const int* arp,
@@ -1126,7 +1102,8 @@ extern "C" int lal_csrgemm_nnz(lal_handle c, int m, int k, int n, int nnz_A, con
     LAL_REQUIRE(crp != nullptr && nnz_C != nullptr && arp != nullptr && brp != nullptr);
     LAL_REQUIRE((nnz_A == 0 || aci) && (nnz_B == 0 || bci));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
-    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A, nnz_B);
+    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A, nnz_B,
+                            nullptr);
 }
 
 extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_A,
@@ -1139,5 +1116,5 @@ extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_
     LAL_REQUIRE((nnz_A == 0 || (aci && av)) && (nnz_B == 0 || (bci && bv)));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
     return lal::csrgemm_solve_f64(c, m, k, n, arp, aci, av, brp, bci, bv, crp, cci, cv, nnz_A,
-                                  nnz_B);
+                                  nnz_B, nullptr);
 }

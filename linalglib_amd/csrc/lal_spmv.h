@@ -32,6 +32,8 @@ struct lal_csrmv_info
     // null when not built or a block's columns span more than 65535
     unsigned short* d_c16   = nullptr;
     int*            d_cbase = nullptr;
+    bool owned = true; // d_blocks is this descriptor's to free (else, as the
+                       // 16-bit columns always, it lies in a hierarchy's arena)
 };
 
 namespace lal
