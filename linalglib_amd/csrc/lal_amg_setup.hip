@@ -122,6 +122,9 @@ namespace
             *incomplete = 1;
     }
 
+    // PASS: every row's state goes to max_state, changed or not, so that the
+    // setup's two joins alternate the buffers.
+    template <bool PASS>
     __global__ void __launch_bounds__(256)
         pmis_join_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                          const int* __restrict__ conn, const int* __restrict__ state,
@@ -131,6 +134,8 @@ namespace
         if(i >= m)
             return;
         const int si = state[i];
+        if(PASS)
+            max_state[i] = si;
         if(si == -1)
         {
             for(int j = rp[i]; j < rp[i + 1]; j++)
@@ -513,7 +518,7 @@ namespace
             *incomplete = 1;
     }
 
-    template <int G>
+    template <int G, bool PASS>
     __global__ void __launch_bounds__(256)
         pmis_join_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                                const int* __restrict__ conn, const int* __restrict__ state,
@@ -524,6 +529,8 @@ namespace
         if(i >= m)
             return;
         const int si = state[i];
+        if(PASS && gl == 0)
+            max_state[i] = si;
         if(si == -1)
         {
             // the first strong neighbour (in CSR order) with state 1
@@ -545,6 +552,54 @@ namespace
         }
         else if(si == -2 && gl == 0)
             agg[i] = -2;
+    }
+
+    __device__ __forceinline__ long long wave_max_i64(long long v)
+    {
+#pragma unroll
+        for(int o = 32; o > 0; o >>= 1)
+        {
+            const long long t = __shfl_xor(v, o, 64);
+            v                 = t > v ? t : v;
+        }
+        return v;
+    }
+
+    // Largest of the workgroup's values, in thread 0.
+    __device__ __forceinline__ long long block_max_i64(long long v)
+    {
+        __shared__ long long s_m[4];
+        v = wave_max_i64(v);
+        if((threadIdx.x & 63) == 0)
+            s_m[threadIdx.x >> 6] = v;
+        __syncthreads();
+        const long long a = s_m[0] > s_m[1] ? s_m[0] : s_m[1];
+        const long long b = s_m[2] > s_m[3] ? s_m[2] : s_m[3];
+        return a > b ? a : b;
+    }
+
+    __global__ void __launch_bounds__(256)
+        max_agg_kernel(int m, const int64_t* __restrict__ agg, long long* __restrict__ part)
+    {
+        long long v = LLONG_MIN;
+        for(int i = blockIdx.x * 256 + threadIdx.x; i < m; i += gridDim.x * 256)
+            v = agg[i] > v ? agg[i] : v;
+        v = block_max_i64(v);
+        if(threadIdx.x == 0)
+            part[blockIdx.x] = v;
+    }
+
+    // out: {largest of the 256 partials, *nnz}
+    __global__ void __launch_bounds__(256)
+        max_agg_finish_kernel(const long long* __restrict__ part, const int* __restrict__ nnz,
+                              long long* __restrict__ out)
+    {
+        const long long v = block_max_i64(part[threadIdx.x]);
+        if(threadIdx.x == 0)
+        {
+            out[0] = v;
+            out[1] = *nnz;
+        }
     }
 
     // Lanes per row for the row-walking setup passes: one for short rows (the
@@ -625,9 +680,11 @@ namespace lal
         // Here the rounds alternate between two buffers (the round kernel
         // writes every decided row through, and a row still undecided was
         // undecided in the older buffer too, so it reads 0 there as in the
-        // copy), and the host checks after every second round: a round after
-        // a complete one finds no undecided row and changes nothing, so the
-        // aggregates are those of the reference's loop.
+        // copy), and the host checks after an even number of rounds: a round
+        // after a complete one finds no undecided row and changes nothing, so
+        // the aggregates are those of the reference's loop.
+        // (the first round reads max_state and writes every row of state that
+        // it decides; rows it leaves undecided must read 0 there)
         LAL_HIP(hipMemcpyAsync(state, max_state, sizeof(int) * m, hipMemcpyDeviceToDevice,
                                c->stream));
         int* buf[2] = {max_state, state}; // buf[cur]: the latest state
@@ -648,37 +705,58 @@ namespace lal
             cur ^= 1;
             return LAL_OK;
         };
-        for(int iter = 0; iter < 20; iter += 2)
+        // Six rounds suffice nearly always; a flag per round, read together.
+        for(int iter = 0; iter < 20;)
         {
-            LAL_HIP(hipMemsetAsync(c->d_flag, 0, 2 * sizeof(int), c->stream));
-            LAL_TRY(round(c->d_flag));
-            LAL_TRY(round(c->d_flag + 1));
-            LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag + 1, sizeof(int), hipMemcpyDeviceToHost,
-                                   c->stream));
-            LAL_HIP(hipStreamSynchronize(c->stream));
-            if(c->h_flag[0] == 0)
+            const int n = iter == 0 ? 6 : 2;
+            int       flags[6];
+            for(int k = 0; k < n; k++)
+                LAL_TRY(round(c->d_flag + k));
+            LAL_TRY(read_ints(c, c->d_flag, n, flags, true));
+            iter += n;
+            if(flags[n - 1] == 0)
                 break;
         }
-        // the joins below read max_state: the latest state must be there
-        if(buf[cur] != max_state)
-            LAL_HIP(hipMemcpyAsync(max_state, buf[cur], sizeof(int) * m, hipMemcpyDeviceToDevice,
-                                   c->stream));
+        // (an even number of rounds: the latest state is in max_state again)
         LAL_TRY(scan_i64_dev(c, m, agg, a));
         for(int k = 0; k < 2; k++)
         {
-            LAL_HIP(hipMemcpyAsync(state, max_state, sizeof(int) * m, hipMemcpyDeviceToDevice,
-                                   c->stream));
+            const int* in  = buf[k];
+            int*       out = buf[k ^ 1];
             if(lanes == 64)
-                pmis_join_group_kernel<64>
-                    <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, state, agg, max_state);
+                pmis_join_group_kernel<64, true>
+                    <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             else if(lanes == 16)
-                pmis_join_group_kernel<16>
-                    <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, state, agg, max_state);
+                pmis_join_group_kernel<16, true>
+                    <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             else
-                pmis_join_kernel<<<g, 256, 0, c->stream>>>(m, rp, ci, conn, state, agg,
-                                                           max_state);
+                pmis_join_kernel<true><<<g, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             LAL_LAUNCHED();
         }
+        return LAL_OK;
+    }
+
+    // Entries (prp[m]) and columns (the largest aggregate id + 1) of a
+    // prolongator whose row pointer has been scanned.
+    static int prolongator_size(lal_context* c, int m, const int64_t* agg, const int* prp,
+                                int* nnz_P, int* n_c, arena* a)
+    {
+        constexpr int MAXB = 256;
+        temps         tmp(c, a);
+        long long*    part = nullptr;
+        int           got[3];
+        LAL_TRY(tmp.get(&part, MAXB + 2));
+        max_agg_kernel<<<MAXB, 256, 0, c->stream>>>(m, agg, part);
+        LAL_LAUNCHED();
+        max_agg_finish_kernel<<<1, MAXB, 0, c->stream>>>(part, prp + m, part + MAXB);
+        LAL_LAUNCHED();
+        LAL_TRY(read_ints(c, reinterpret_cast<int*>(part + MAXB), 3, got, false));
+        const int64_t mx = (int64_t)(((uint64_t)(uint32_t)got[1] << 32) | (uint32_t)got[0]);
+        const int64_t nc = std::max<int64_t>(mx, -1) + 1;
+        if(nc > INT_MAX)
+            return LAL_ERR_UNSUPPORTED;
+        *nnz_P = got[2];
+        *n_c   = (int)nc;
         return LAL_OK;
     }
 
@@ -695,15 +773,7 @@ namespace lal
                                                                                     conn, agg, prp);
         LAL_LAUNCHED();
         LAL_TRY(scan_i32_dev(c, m + 1, prp, a));
-        int64_t mx = LLONG_MIN;
-        LAL_TRY(max_i64_dev(c, m, agg, &mx));
-        int64_t nc = std::max<int64_t>(mx, -1) + 1;
-        if(nc > INT_MAX)
-            return LAL_ERR_UNSUPPORTED;
-        LAL_HIP(hipMemcpyAsync(nnz_P, prp + m, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        *n_c = (int)nc;
-        return LAL_OK;
+        return prolongator_size(c, m, agg, prp, nnz_P, n_c, a);
     }
 
     int sa_prolongator_fill(lal_context* c, int m, int nnz, const int* rp, const int* ci,
@@ -756,15 +826,7 @@ namespace lal
         ua_count_kernel<<<grid_for(m + 1, 256), 256, 0, c->stream>>>(m, agg, prp);
         LAL_LAUNCHED();
         LAL_TRY(scan_i32_dev(c, m + 1, prp, a));
-        int64_t mx = LLONG_MIN;
-        LAL_TRY(max_i64_dev(c, m, agg, &mx));
-        const int64_t nc = std::max<int64_t>(mx, -1) + 1;
-        if(nc > INT_MAX)
-            return LAL_ERR_UNSUPPORTED;
-        LAL_HIP(hipMemcpyAsync(nnz_P, prp + m, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        *n_c = (int)nc;
-        return LAL_OK;
+        return prolongator_size(c, m, agg, prp, nnz_P, n_c, a);
     }
 
     int ua_prolongator_fill(lal_context* c, int m, const int64_t* agg, const int* prp, int* pci,
@@ -815,13 +877,12 @@ extern "C" int lal_pmis_round(lal_handle c, int m, int nnz, const int* rp, const
     *complete = 1;
     if(m == 0)
         return LAL_OK;
-    LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
     pmis_round_kernel<false><<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
         m, rp, ci, conn, state, hash, agg, max_state, c->d_flag);
     LAL_LAUNCHED();
-    LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    LAL_HIP(hipStreamSynchronize(c->stream));
-    *complete = c->h_flag[0] == 0;
+    int undecided = 0;
+    LAL_TRY(lal::read_ints(c, c->d_flag, 1, &undecided, true));
+    *complete = undecided == 0;
     return LAL_OK;
 }
 
@@ -832,8 +893,8 @@ extern "C" int lal_pmis_join(lal_handle c, int m, int nnz, const int* rp, const 
     LAL_REQUIRE(m == 0 || (rp && state && agg && max_state && (nnz == 0 || (ci && conn))));
     if(m == 0)
         return LAL_OK;
-    pmis_join_kernel<<<lal::grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, conn, state, agg,
-                                                                   max_state);
+    pmis_join_kernel<false><<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
+        m, rp, ci, conn, state, agg, max_state);
     LAL_LAUNCHED();
     return LAL_OK;
 }

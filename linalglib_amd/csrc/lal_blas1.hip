@@ -337,22 +337,6 @@ namespace
         return scan_passes<T>(c, n, x, sums);
     }
 
-    __global__ void __launch_bounds__(256)
-        max_i64_kernel(int n, const int64_t* __restrict__ x, unsigned long long* out)
-    {
-        long long m = LLONG_MIN;
-        for(int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
-            m = x[i] > m ? x[i] : m;
-#pragma unroll
-        for(int o = 32; o > 0; o >>= 1)
-        {
-            long long t = __shfl_xor(m, o, 64);
-            m           = t > m ? t : m;
-        }
-        if((threadIdx.x & 63) == 0)
-            atomicMax((long long*)out, m);
-    }
-
     template <typename T>
     int axpy_t(lal_context* c, int n, T alpha, const T* x, T* y)
     {
@@ -422,20 +406,6 @@ namespace lal
             return LAL_ERR_HIP;
         }
         g_scratch[device] = static_cast<int64_t*>(p);
-        return LAL_OK;
-    }
-    int max_i64_dev(lal_context* c, int n, const int64_t* x, int64_t* h_out)
-    {
-        long long init = LLONG_MIN;
-        auto*     slot = reinterpret_cast<unsigned long long*>(c->d_slots + (LAL_NUM_SLOTS - 1));
-        LAL_HIP(hipMemcpyAsync(slot, &init, sizeof(init), hipMemcpyHostToDevice, c->stream));
-        if(n > 0)
-        {
-            max_i64_kernel<<<lal::grid_for(n, 256, 2048), 256, 0, c->stream>>>(n, x, slot);
-            LAL_LAUNCHED();
-        }
-        LAL_HIP(hipMemcpyAsync(h_out, slot, sizeof(long long), hipMemcpyDeviceToHost, c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
         return LAL_OK;
     }
 }

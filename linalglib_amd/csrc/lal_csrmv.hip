@@ -85,10 +85,11 @@ namespace
         }
     }
 
-    // Flags 1 in *bad if a column index lies outside [0, n): an invalid matrix
+    // Sets `bit` in *bad if a column index lies outside [0, n): an invalid matrix
     // is refused before any gather can run off the end of x.
     __global__ void __launch_bounds__(256)
-        check_cols_kernel(int nnz, int n, const int* __restrict__ ci, int* __restrict__ bad)
+        check_cols_kernel(int nnz, int n, const int* __restrict__ ci, int* __restrict__ bad,
+                          int bit = 1)
     {
         int k = blockIdx.x * 256 + threadIdx.x;
         int stride = gridDim.x * 256;
@@ -96,7 +97,7 @@ namespace
         for(; k < nnz; k += stride)
             b |= (unsigned)ci[k] >= (unsigned)n;
         if(__any(b) && (threadIdx.x & 63) == 0)
-            atomicOr(bad, 1);
+            atomicOr(bad, bit);
     }
 
     __global__ void __launch_bounds__(256)
@@ -114,29 +115,199 @@ namespace
             }
     }
 
-    // One workgroup per row block: the block's column range, its base (the
-    // smallest column) and every entry's offset from it as 16 bits; *fail
-    // is set when a block spans more than 65535 columns.
+    // ------------------------------------------------------ row-block analysis
+    // Rows are packed greedily: a block closes at 256 rows or when the next
+    // row would push it past `cap` nonzeros; a row longer than cap is a block of
+    // its own.  The packing starts anew every RB_TILE rows, so that a workgroup
+    // packs each tile by itself: all rows' "next block" are found at once in
+    // LDS (a binary search in the staged row pointer) and one lane follows
+    // them.  Several operators share a launch (a hierarchy analyses all of its
+    // own at once, without a copy of a row pointer to the host).
+    constexpr int RB_TILE  = 2048;
+    constexpr int RB_BATCH = 24; // operators per launch (their table is a kernel argument)
+
+    struct rb_table
+    {
+        int           n;
+        lal::rb_op op[RB_BATCH];
+    };
+
+    // results of one operator, in the order read back
+    enum
+    {
+        RB_NBLOCKS = 0,
+        RB_WIN     = 1, // widest 4-aligned nonzero window of a block (<= 2052)
+        RB_BAD     = 2, // 1: row pointer not from 0 to nnz, 2: not monotone, 4: column range
+        RB_WIDE    = 3, // a block spans more than 65535 columns
+        RB_RES     = 4
+    };
+
+    // Position of `at` among the operators' starts (ascending).
+    template <typename F>
+    __device__ __forceinline__ int rb_find(const rb_table& t, int at, F start)
+    {
+        int k = 0;
+        while(k + 1 < t.n && start(t.op[k + 1]) <= at)
+            k++;
+        return k;
+    }
+
+    // WRITE false: blocks per tile into tcount, the widest window and the row
+    // pointer's faults into res.  WRITE true: the block table, at the tile's
+    // offset that the scan left in tcount.
+    template <bool WRITE>
     __global__ void __launch_bounds__(256)
-        c16_kernel(const int* __restrict__ blocks, int nb, const int* __restrict__ ci,
-                   int* __restrict__ cbase, unsigned short* __restrict__ c16, int* fail)
+        rb_tile_kernel(rb_table tab, int* __restrict__ tcount, int* __restrict__ res)
+    {
+        __shared__ int            s_rp[RB_TILE + 1];
+        __shared__ unsigned short s_next[RB_TILE];
+        __shared__ int            s_n;
+        const int    k   = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.tile0; });
+        const lal::rb_op o = tab.op[k];
+        int*         out = res + RB_RES * k;
+        if(WRITE && (out[RB_BAD] != 0 || out[RB_NBLOCKS] > o.ub))
+            return;
+        const int tid = (int)threadIdx.x;
+        const int r0  = ((int)blockIdx.x - o.tile0) * RB_TILE;
+        const int n   = min(RB_TILE, o.m - r0);
+        for(int i = tid; i <= n; i += 256)
+            s_rp[i] = o.rp[r0 + i];
+        __syncthreads();
+        if(!WRITE)
+        {
+            int bad = 0;
+            for(int i = tid; i < n; i += 256)
+                bad |= s_rp[i + 1] < s_rp[i] ? 2 : 0;
+            if(tid == 0)
+                bad |= (r0 == 0 && s_rp[0] != 0) || (r0 + n == o.m && s_rp[n] != o.nnz) ? 1 : 0;
+            if(bad)
+                atomicOr(out + RB_BAD, bad);
+        }
+        // the block from row i ends before the first row t (at most 256 on)
+        // with rp[t + 1] - rp[i] > cap
+        for(int i = tid; i < n; i += 256)
+        {
+            const long long top = (long long)s_rp[i] + o.cap;
+            int             lo = i, hi = min(n, i + SPMV_THREADS); // rp[lo] <= top
+            while(lo < hi)
+            {
+                const int mid = (lo + hi + 1) >> 1;
+                if(s_rp[mid] <= top)
+                    lo = mid;
+                else
+                    hi = mid - 1;
+            }
+            s_next[i] = (unsigned short)max(lo, i + 1);
+        }
+        __syncthreads();
+        if(tid == 0)
+        {
+            int cnt = 0, win = 4;
+            for(int r = 0; r < n;)
+            {
+                const int nx   = s_next[r];
+                const int span = ((s_rp[nx] + 3) & ~3) - (s_rp[r] & ~3);
+                win            = max(win, min(span, 2052));
+                // reached rows are read once: the list of block starts
+                // replaces the links behind the walk
+                s_next[cnt++] = (unsigned short)r;
+                r             = nx;
+            }
+            s_n = cnt;
+            if(!WRITE)
+            {
+                tcount[blockIdx.x] = cnt;
+                atomicMax(out + RB_WIN, win);
+            }
+        }
+        if(!WRITE)
+            return;
+        __syncthreads();
+        const int nb   = s_n;
+        const int at   = tcount[blockIdx.x];
+        const int all  = out[RB_NBLOCKS];
+        int*      meta = o.blocks + lal::block_meta_offset(all);
+        for(int b = tid; b < nb; b += 256)
+        {
+            const int i = s_next[b], e = b + 1 < nb ? (int)s_next[b + 1] : n;
+            o.blocks[at + b]           = r0 + i;
+            meta[4 * (size_t)(at + b)]     = r0 + i;
+            meta[4 * (size_t)(at + b) + 1] = r0 + e;
+            meta[4 * (size_t)(at + b) + 2] = s_rp[i];
+            meta[4 * (size_t)(at + b) + 3] = s_rp[e];
+        }
+        if(tid == 0 && r0 + n == o.m)
+            o.blocks[all] = o.m;
+    }
+
+    // One workgroup per operator: its tiles' block counts become offsets.
+    __global__ void __launch_bounds__(256)
+        rb_scan_kernel(rb_table tab, int* __restrict__ tcount, int* __restrict__ res)
+    {
+        __shared__ int  s_w[4];
+        const int       k    = (int)blockIdx.x;
+        const lal::rb_op o   = tab.op[k];
+        const int       lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
+        int             carry = 0;
+        for(int t0 = 0; t0 < o.ntiles; t0 += 256)
+        {
+            const int i   = t0 + (int)threadIdx.x;
+            const int v   = i < o.ntiles ? tcount[o.tile0 + i] : 0;
+            int       inc = v;
+#pragma unroll
+            for(int d = 1; d < 64; d <<= 1)
+            {
+                const int q = __shfl_up(inc, d, 64);
+                inc += lane >= d ? q : 0;
+            }
+            if(lane == 63)
+                s_w[wid] = inc;
+            __syncthreads();
+            int off = carry, tot = 0;
+            for(int w = 0; w < 4; w++)
+            {
+                off += w < wid ? s_w[w] : 0;
+                tot += s_w[w];
+            }
+            if(i < o.ntiles)
+                tcount[o.tile0 + i] = off + inc - v;
+            carry += tot;
+            __syncthreads();
+        }
+        if(threadIdx.x == 0)
+            res[RB_RES * k + RB_NBLOCKS] = carry;
+    }
+
+    // One workgroup per row block (the grid holds every operator's largest
+    // possible number of blocks): the block's column range, its base (the
+    // smallest column) and every entry's offset from it as 16 bits; RB_WIDE is
+    // set when a block spans more than 65535 columns.
+    __global__ void __launch_bounds__(256)
+        rb_columns_kernel(rb_table tab, int* __restrict__ res)
     {
         typedef int int4v __attribute__((ext_vector_type(4)));
         __shared__ int sh_mn[4], sh_mx[4];
-        const int4v mt = reinterpret_cast<const int4v*>(blocks + lal::block_meta_offset(nb))[blockIdx.x];
+        const int k  = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.blk0; });
+        const lal::rb_op o = tab.op[k];
+        int*      out = res + RB_RES * k;
+        const int nb  = out[RB_NBLOCKS];
+        const int b   = (int)blockIdx.x - o.blk0;
+        if(o.c16 == nullptr || out[RB_BAD] != 0 || nb > o.ub || b >= nb)
+            return;
+        const int4v mt = reinterpret_cast<const int4v*>(o.blocks + lal::block_meta_offset(nb))[b];
         const int   e0 = mt.z, e1 = mt.w;
         int         mn = INT_MAX, mx = INT_MIN;
-        for(int k = e0 + (int)threadIdx.x; k < e1; k += 256)
+        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
         {
-            const int col = ci[k];
+            const int col = o.ci[e];
             mn            = min(mn, col);
             mx            = max(mx, col);
         }
 #pragma unroll
-        for(int o = 32; o > 0; o >>= 1)
+        for(int d = 32; d > 0; d >>= 1)
         {
-            mn = min(mn, __shfl_xor(mn, o, 64));
-            mx = max(mx, __shfl_xor(mx, o, 64));
+            mn = min(mn, __shfl_xor(mn, d, 64));
+            mx = max(mx, __shfl_xor(mx, d, 64));
         }
         if((threadIdx.x & 63) == 0)
         {
@@ -149,12 +320,12 @@ namespace
         const int base = e1 > e0 ? mn : 0;
         if(threadIdx.x == 0)
         {
-            cbase[blockIdx.x] = base;
+            o.cbase[b] = base;
             if(e1 > e0 && (long long)mx - mn > 65535)
-                atomicOr(fail, 1);
+                atomicOr(out + RB_WIDE, 1);
         }
-        for(int k = e0 + (int)threadIdx.x; k < e1; k += 256)
-            c16[k] = (unsigned short)(ci[k] - base);
+        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
+            o.c16[e] = (unsigned short)(o.ci[e] - base);
     }
 
     template <typename T, typename ACC, int MODE>
@@ -189,145 +360,127 @@ namespace
 
 namespace lal
 {
-    // Greedy row packing: a block closes at 256 rows or when the next row
-    // would push it past `cap` nonzeros; a row longer than cap is a block of
-    // its own.  cap is 2048 (the kernels' LDS chunk) for large matrices; for
-    // small ones it shrinks, down to 256, so that a launch still has about
-    // 1024 workgroups: their time is one latency chain per workgroup, and
-    // more, shorter chains spread over all CUs finish sooner.
-    int csrmv_analysis_host(const int* h_rp, int m, std::vector<int>& blocks)
-    {
-        const long nnz = m > 0 ? h_rp[m] : 0;
-        int        cap = spmv_cap<double>::value;
-        while(cap > 256 && nnz / 1024 < cap)
-            cap >>= 1;
-        blocks.clear();
-        blocks.push_back(0);
-        int r = 0;
-        while(r < m)
-        {
-            // the block ends before the first row r (at most SPMV_THREADS rows
-            // on) with row_ptr[r + 1] - row_ptr[start] > cap; row_ptr is
-            // non-decreasing, so that row is a binary search away
-            const int       start = r;
-            const int       lim   = std::min(m, start + SPMV_THREADS);
-            const long long top   = (long long)h_rp[start] + cap;
-            r = (int)(std::upper_bound(h_rp + start + 1, h_rp + lim + 1, top) - h_rp) - 1;
-            if(r == start)
-                r++;
-            blocks.push_back(r);
-        }
-        return LAL_OK;
-    }
-
-    int check_columns(lal_context* c, int nnz, int n, const int* ci)
+    int raise_bad_columns(lal_context* c, int nnz, int n, const int* ci, int* flag)
     {
         if(nnz == 0)
             return LAL_OK;
-        if(ci == nullptr)
-            return LAL_ERR_INVALID;
-        LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
-        check_cols_kernel<<<grid_for(nnz, 256, 4096), 256, 0, c->stream>>>(nnz, n, ci,
-                                                                            c->d_flag);
+        check_cols_kernel<<<grid_for(nnz, 256, 4096), 256, 0, c->stream>>>(nnz, n, ci, flag);
         LAL_LAUNCHED();
-        LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        if(c->h_flag[0])
+        return LAL_OK;
+    }
+
+    // Nonzeros per row block: 2048 (the kernels' LDS chunk) for large
+    // matrices; for small ones it shrinks, down to 256, so that a launch still
+    // has about 1024 workgroups: their time is one latency chain per
+    // workgroup, and more, shorter chains spread over all CUs finish sooner.
+    static int block_cap(int nnz)
+    {
+        int cap = spmv_cap<double>::value;
+        while(cap > 256 && nnz / 1024 < cap)
+            cap >>= 1;
+        return cap;
+    }
+
+    int analyse(lal_context* c, const std::vector<rb_request>& req, arena* mem, arena* tmp)
+    {
+        for(size_t first = 0; first < req.size(); first += RB_BATCH)
         {
-            set_last_error("column index outside [0, n)");
-            return LAL_ERR_INVALID;
+            temps    t(c, tmp);
+            rb_table tab{};
+            int      tiles = 0, blocks = 0;
+            tab.n          = (int)std::min(req.size() - first, (size_t)RB_BATCH);
+            for(int k = 0; k < tab.n; k++)
+            {
+                const rb_request& q = req[first + k];
+                rb_op&            o = tab.op[k];
+                o.rp     = q.rp;
+                o.ci     = q.ci;
+                o.m      = q.m;
+                o.nnz    = q.nnz;
+                o.cap    = block_cap(q.nnz);
+                o.tile0  = tiles;
+                o.ntiles = std::max((q.m + RB_TILE - 1) / RB_TILE, 1);
+                o.blk0   = blocks;
+                // a block that is neither of 256 rows nor a tile's last holds
+                // more than cap nonzeros together with its successor
+                o.ub = q.m / SPMV_THREADS + (int)(2LL * q.nnz / o.cap) + o.ntiles + 1;
+                tiles += o.ntiles;
+                blocks += o.ub;
+                LAL_TRY(q.d->arrays(mem, o.ub));
+                o.blocks = q.d->d_blocks;
+                if(mem && q.want16 && q.nnz > 0)
+                {
+                    // whole 16-byte lines: the kernels load four entries at a time
+                    LAL_TRY(mem->get(&q.d->d_c16, ((size_t)q.nnz + 7) & ~(size_t)7));
+                    LAL_TRY(mem->get(&q.d->d_cbase, o.ub));
+                    o.c16   = q.d->d_c16;
+                    o.cbase = q.d->d_cbase;
+                }
+            }
+            int *tcount = nullptr, *res = nullptr;
+            int  h[RB_RES * RB_BATCH] = {};
+            LAL_TRY(t.get(&res, RB_RES * RB_BATCH));
+            LAL_TRY(t.get(&tcount, tiles));
+            LAL_TRY(lal_fill_i32(c, res, RB_RES * RB_BATCH, 0));
+            rb_tile_kernel<false><<<tiles, 256, 0, c->stream>>>(tab, tcount, res);
+            LAL_LAUNCHED();
+            rb_scan_kernel<<<tab.n, 256, 0, c->stream>>>(tab, tcount, res);
+            LAL_LAUNCHED();
+            rb_tile_kernel<true><<<tiles, 256, 0, c->stream>>>(tab, tcount, res);
+            LAL_LAUNCHED();
+            if(mem)
+            {
+                rb_columns_kernel<<<blocks, 256, 0, c->stream>>>(tab, res);
+                LAL_LAUNCHED();
+            }
+            for(int k = 0; k < tab.n; k++)
+                if(req[first + k].check_n >= 0 && tab.op[k].nnz > 0)
+                {
+                    check_cols_kernel<<<grid_for(tab.op[k].nnz, 256, 4096), 256, 0, c->stream>>>(
+                        tab.op[k].nnz, req[first + k].check_n, tab.op[k].ci,
+                        res + RB_RES * k + RB_BAD, 4);
+                    LAL_LAUNCHED();
+                }
+            LAL_TRY(read_ints(c, res, RB_RES * tab.n, h, false));
+            for(int k = 0; k < tab.n; k++)
+            {
+                const rb_request& q = req[first + k];
+                const int*        r = h + RB_RES * k;
+                if(r[RB_BAD] & 4)
+                    set_last_error("column index outside [0, n)");
+                else if(r[RB_BAD] & 1)
+                    set_last_error("row_ptr does not start at 0 or end at nnz");
+                else if(r[RB_BAD] & 2 || r[RB_NBLOCKS] > tab.op[k].ub)
+                    set_last_error("row_ptr is not monotone");
+                else
+                {
+                    q.d->nblocks = r[RB_NBLOCKS];
+                    q.d->win     = std::max(r[RB_WIN], 4);
+                    if(r[RB_WIDE])
+                        q.d->d_c16 = nullptr;
+                    continue;
+                }
+                return LAL_ERR_INVALID;
+            }
         }
         return LAL_OK;
     }
 
     int csrmv_analysis_dev(lal_context* c, int m, int n, int nnz, const int* rp,
-                           const int* ci, int exact, lal_csrmv_info** out, bool trusted,
-                           arena* mem)
+                           const int* ci, int exact, lal_csrmv_info** out)
     {
-        if(!trusted)
-            LAL_TRY(check_columns(c, nnz, n, ci));
-        std::vector<int> h(m + 1);
-        LAL_HIP(hipMemcpyAsync(h.data(), rp, sizeof(int) * (m + 1), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        if(h[0] != 0 || h[m] != nnz)
+        auto* d   = new lal_csrmv_info;
+        d->m      = m;
+        d->nnz    = nnz;
+        d->exact  = exact;
+        d->by_nnz = m != n;
+        const int st = analyse(c, {{d, rp, ci, m, nnz, false, n}}, nullptr, nullptr);
+        if(st != LAL_OK)
         {
-            set_last_error("row_ptr does not start at 0 or end at nnz");
-            return LAL_ERR_INVALID;
+            lal_csrmv_descr_destroy(d);
+            return st;
         }
-        // (a pattern this library built is monotone by construction)
-        for(int i = 0; i < m && !trusted; i++)
-            if(h[i + 1] < h[i])
-            {
-                set_last_error("row_ptr is not monotone");
-                return LAL_ERR_INVALID;
-            }
-        std::vector<int> blocks;
-        csrmv_analysis_host(h.data(), m, blocks);
-        auto* d    = new lal_csrmv_info;
-        d->m       = m;
-        d->nnz     = nnz;
-        d->exact   = exact;
-        d->by_nnz  = m != n;
-        d->nblocks = (int)blocks.size() - 1;
-        // the row offsets, then (16-byte aligned) one {r0, r1, row_ptr[r0],
-        // row_ptr[r1]} quadruple per block: a block learns its rows and its
-        // nonzero window from a single load
-        const size_t meta_at = lal::block_meta_offset(d->nblocks);
-        std::vector<int> packed(meta_at + 4 * (size_t)d->nblocks);
-        std::copy(blocks.begin(), blocks.end(), packed.begin());
-        int win = 4;
-        for(int k = 0; k < d->nblocks; k++)
-        {
-            const int span = ((h[blocks[k + 1]] + 3) & ~3) - (h[blocks[k]] & ~3);
-            win            = std::max(win, std::min(span, 2052));
-            packed[meta_at + 4 * k + 0] = blocks[k];
-            packed[meta_at + 4 * k + 1] = blocks[k + 1];
-            packed[meta_at + 4 * k + 2] = h[blocks[k]];
-            packed[meta_at + 4 * k + 3] = h[blocks[k + 1]];
-        }
-        d->win = win;
-        d->owned = mem == nullptr;
-        if((mem ? mem->get(&d->d_blocks, packed.size())
-                : hipMalloc(&d->d_blocks, sizeof(int) * packed.size()) == hipSuccess
-                      ? LAL_OK
-                      : LAL_ERR_OOM) != LAL_OK)
-        {
-            delete d;
-            return LAL_ERR_OOM;
-        }
-        LAL_HIP(hipMemcpyAsync(d->d_blocks, packed.data(), sizeof(int) * packed.size(),
-                               hipMemcpyHostToDevice, c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
         *out = d;
-        return LAL_OK;
-    }
-
-    int compact_columns(lal_context* c, lal_csrmv_info* d, int nnz, const int* ci, arena* mem)
-    {
-        if(!d || d->exact || nnz <= 0 || d->nblocks <= 0 || d->d_c16)
-            return LAL_OK;
-        unsigned short* c16   = nullptr;
-        int*            cbase = nullptr;
-        int*            fail  = c->d_flag; // the context's flag word, read back below
-        const auto      mark  = mem->mark();
-        // rounded up to whole 16-byte lines: the kernels load four entries at a time
-        LAL_TRY(mem->get(&c16, ((size_t)nnz + 7) & ~(size_t)7));
-        LAL_TRY(mem->get(&cbase, d->nblocks));
-        LAL_HIP(hipMemsetAsync(fail, 0, sizeof(int), c->stream));
-        c16_kernel<<<d->nblocks, 256, 0, c->stream>>>(d->d_blocks, d->nblocks, ci, cbase, c16,
-                                                      fail);
-        LAL_LAUNCHED();
-        LAL_HIP(hipMemcpyAsync(c->h_flag, fail, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        if(c->h_flag[0])
-        {
-            mem->release(mark);
-            return LAL_OK;
-        }
-        d->d_c16   = c16;
-        d->d_cbase = cbase;
         return LAL_OK;
     }
 
@@ -374,21 +527,30 @@ namespace lal
     }
 }
 
+int lal_csrmv_info::arrays(lal::arena* mem, int nb)
+{
+    const size_t ints = lal::block_meta_offset(nb) + 4 * (size_t)nb;
+    owned             = mem == nullptr;
+    if(mem)
+        return mem->get(&d_blocks, ints);
+    LAL_HIP(hipMalloc(&d_blocks, sizeof(int) * ints));
+    return LAL_OK;
+}
+
 extern "C" int lal_csrmv_analysis(lal_handle c, int m, int n, int nnz, const int* row_ptr,
                                   const int* col_ind, int exact, lal_csrmv_descr* descr)
 {
     LAL_REQUIRE(c != nullptr && descr != nullptr && m >= 0 && n >= 0 && nnz >= 0);
     LAL_REQUIRE(row_ptr != nullptr && (nnz == 0 || col_ind != nullptr));
     *descr = nullptr;
-    return lal::csrmv_analysis_dev(c, m, n, nnz, row_ptr, col_ind, exact, descr, false,
-                                   nullptr);
+    return lal::csrmv_analysis_dev(c, m, n, nnz, row_ptr, col_ind, exact, descr);
 }
 
 extern "C" int lal_csrmv_descr_destroy(lal_csrmv_descr d)
 {
     if(!d)
         return LAL_OK;
-    if(d->owned)
+    if(d->owned && d->d_blocks)
         (void)hipFree(d->d_blocks);
     delete d;
     return LAL_OK;

@@ -38,12 +38,9 @@ namespace lal
     int transpose_f64(lal_context* c, int m, int n, int nnz, const int* rp, const int* ci,
                       const double* v, int* trp, int* tci, double* tv, arena* a);
     // nnz_a: A's nonzeros, which pick the lanes per row of the product count
-    int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a, long nnz_b,
-                    arena* a);
-    int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                          const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b, arena* a);
+    int product(lal_context* c, int m, int k, int n, int nnz_a, const int* arp, const int* aci,
+                const double* av, int nnz_b, const int* brp, const int* bci, const double* bv,
+                int** crp, int** cci, double** cv, int* nnz_c, arena* mem, arena* work);
 }
 
 using lal::converges;
@@ -262,30 +259,42 @@ namespace
         return LAL_OK;
     }
 
-    int finish_setup(lal_hierarchy_t* h)
+    // A fresh descriptor for an m x n operator of a hierarchy.
+    lal_csrmv_info* descr(csr_dev& A, int m, int nnz, int n, int exact)
+    {
+        A.d         = new lal_csrmv_info;
+        A.d->m      = m;
+        A.d->nnz    = nnz;
+        A.d->exact  = exact;
+        A.d->by_nnz = m != n;
+        return A.d;
+    }
+
+    int finish_setup(lal_hierarchy_t* h, lal::arena* tmp)
     {
         lal_context* c     = h->c;
         const int    exact = h->opts.exact;
+        // level 0 carries the descriptor of the input's validation (the same
+        // pattern, copied); the rest are this setup's products.  The fast path
+        // reads the operators with 16-bit columns (offsets from each row
+        // block's smallest column) where the blocks allow it: 2 bytes per
+        // nonzero less, same results.
+        std::vector<lal::rb_request> req;
+        for(int l = 0; l <= h->levels; l++)
+            for(csr_dev* A : {&h->L[l].A, &h->L[l].P, &h->L[l].R})
+                if(A->d == nullptr && (A == &h->L[l].A || l < h->levels))
+                    req.push_back({descr(*A, A->m, A->nnz, A->n, exact), A->rp, A->ci, A->m,
+                                   A->nnz, exact == 0, -1});
+        LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
         for(int l = 0; l <= h->levels; l++)
         {
             level_t& L = h->L[l];
-            // level 0 carries the descriptor of the input's validation (the
-            // same row pointer, copied); the rest are this setup's products
-            if(!L.A.d)
-                LAL_TRY(lal::csrmv_analysis_dev(c, L.A.m, L.A.n, L.A.nnz, L.A.rp, L.A.ci, exact,
-                                                &L.A.d, true, &h->mem));
-            L.A.d->exact = exact;
             // The finest operator is read three times per PCG iteration
             // (residual, post-sweep, the Krylov product), the last two with
             // only vector passes between them: it may stay in the Infinity
             // Cache when it fits (decided per precision at launch).  Keeping
             // a coarser level as well overflows the cache and slows the solve.
             L.A.d->keep = l == 0;
-            // the fast path reads the hierarchy's operators with 16-bit
-            // columns (offsets from each row block's smallest column) where
-            // the blocks allow it: 2 bytes per nonzero less, same results
-            if(!exact)
-                LAL_TRY(lal::compact_columns(c, L.A.d, L.A.nnz, L.A.ci, &h->mem));
             LAL_TRY(h->mem.get(&L.w64.x, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.t, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.b, L.A.m));
@@ -294,18 +303,6 @@ namespace
             LAL_TRY(h->mem.get(&L.w64.dinv, L.A.m));
             LAL_TRY(lal::diag_inv<double>(c, L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag,
                                           L.w64.dinv, L.A.nnz));
-            if(l < h->levels)
-            {
-                LAL_TRY(lal::csrmv_analysis_dev(c, L.P.m, L.P.n, L.P.nnz, L.P.rp, L.P.ci, exact,
-                                                &L.P.d, true, &h->mem));
-                LAL_TRY(lal::csrmv_analysis_dev(c, L.R.m, L.R.n, L.R.nnz, L.R.rp, L.R.ci, exact,
-                                                &L.R.d, true, &h->mem));
-                if(!exact)
-                {
-                    LAL_TRY(lal::compact_columns(c, L.P.d, L.P.nnz, L.P.ci, &h->mem));
-                    LAL_TRY(lal::compact_columns(c, L.R.d, L.R.nnz, L.R.ci, &h->mem));
-                }
-            }
             if(h->opts.build_f32)
             {
                 LAL_TRY(to_f32(h, L.A.v, &L.A.v32, L.A.nnz));
@@ -492,28 +489,18 @@ namespace
             csr_dev AP;
             AP.m = Af.m;
             AP.n = nc;
-            LAL_TRY(tmp.get(&AP.rp, Af.m + 1));
-            LAL_TRY(lal::csrgemm_nnz(c, Af.m, Af.n, nc, Af.rp, Af.ci, P.rp, P.ci, AP.rp,
-                                     &AP.nnz, Af.nnz, P.nnz, &tmp));
-            LAL_TRY(tmp.get(&AP.ci, AP.nnz));
-            LAL_TRY(tmp.get(&AP.v, AP.nnz));
-            LAL_TRY(lal::csrgemm_solve_f64(c, Af.m, Af.n, nc, Af.rp, Af.ci, Af.v, P.rp, P.ci,
-                                           P.v, AP.rp, AP.ci, AP.v, Af.nnz, P.nnz, &tmp));
+            LAL_TRY(lal::product(c, Af.m, Af.n, nc, Af.nnz, Af.rp, Af.ci, Af.v, P.nnz, P.rp,
+                                 P.ci, P.v, &AP.rp, &AP.ci, &AP.v, &AP.nnz, &tmp, &tmp));
             // A_c = R (A P)
             Ac.m = nc;
             Ac.n = nc;
-            LAL_TRY(h->mem.get(&Ac.rp, nc + 1));
-            LAL_TRY(lal::csrgemm_nnz(c, nc, Af.m, nc, R.rp, R.ci, AP.rp, AP.ci, Ac.rp, &Ac.nnz,
-                                     R.nnz, AP.nnz, &tmp));
-            LAL_TRY(h->mem.get(&Ac.ci, Ac.nnz));
-            LAL_TRY(h->mem.get(&Ac.v, Ac.nnz));
-            LAL_TRY(lal::csrgemm_solve_f64(c, nc, Af.m, nc, R.rp, R.ci, R.v, AP.rp, AP.ci, AP.v,
-                                           Ac.rp, Ac.ci, Ac.v, R.nnz, AP.nnz, &tmp));
+            LAL_TRY(lal::product(c, nc, Af.m, nc, R.nnz, R.rp, R.ci, R.v, AP.nnz, AP.rp, AP.ci,
+                                 AP.v, &Ac.rp, &Ac.ci, &Ac.v, &Ac.nnz, &h->mem, &tmp));
             level++;
             eps *= 0.5;
         }
         h->levels    = level;
-        const int st = finish_setup(h);
+        const int st = finish_setup(h, &tmp);
         (void)hipStreamSynchronize(c->stream); // before tmp goes
         return st;
     }
@@ -1079,7 +1066,8 @@ namespace
         // FP32 levels) and 200 per row: the first chunk is half of that, and
         // the arena grows by half its size.
         h->mem.reserve((size_t)nnz * (o.build_f32 ? 60 : 40) + (size_t)m * 100);
-        int s = lal::csrmv_analysis_dev(c, m, n, nnz, rp, ci, 0, &h->L[0].A.d, false, &h->mem);
+        int s = lal::analyse(c, {{descr(h->L[0].A, m, nnz, n, o.exact), rp, ci, m, nnz,
+                                  o.exact == 0, n}}, &h->mem, nullptr);
         if(s == LAL_OK)
             s = setup(c, m, n, nnz, rp, ci, v, o, h, unsmoothed);
         if(s != LAL_OK)

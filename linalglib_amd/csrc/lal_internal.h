@@ -59,6 +59,10 @@ namespace lal
     };
 }
 
+// Flag words of a context, and integers one read_ints hands back at most.
+#define LAL_FLAGS 32
+#define LAL_NOTE_INTS 192
+
 // Devices the per-device static scratch table covers.
 #define LAL_MAX_DEVICES 64
 
@@ -73,8 +77,14 @@ struct lal_context
     unsigned* d_ticket = nullptr; // LAL_NUM_SLOTS
     double*   d_slots  = nullptr; // LAL_NUM_SLOTS device scalars
     double*   h_slots  = nullptr; // pinned mirror
+    // flag words of the checks and setup passes: zero between calls (whoever
+    // raises one reads it back with read_ints, which clears it)
     int*      d_flag   = nullptr;
-    int*      h_flag   = nullptr;
+    // small results reach the host through mapped pinned memory: LAL_NOTE_INTS
+    // values and, after them, a sequence number that the host polls
+    int*      h_note   = nullptr;
+    int*      d_note   = nullptr;
+    unsigned  note_seq = 0;
     // hierarchies built on this context: lal_destroy detaches them, so that
     // one destroyed after its context no longer touches it
     std::vector<lal_hierarchy_t*> hierarchies;
@@ -270,9 +280,11 @@ namespace lal
     // Device address of the allocation-free scan's static scratch for
     // `device` (which must be current), looked up once per device.
     int noalloc_scratch_init(int device);
-    int max_i64_dev(lal_context* c, int n, const int64_t* x, int64_t* h_out);
+    // The n ints at src once the stream has come to them (blocks); clear: they
+    // are zeroed behind the read.
+    int read_ints(lal_context* c, int* src, int n, int* out, bool clear);
     // Clears the context pointer of every hierarchy built on c (lal_destroy).
     void detach_hierarchies(lal_context* c);
-    // LAL_ERR_INVALID unless every ci[0..nnz) lies in [0, n) (blocks until known).
-    int check_columns(lal_context* c, int nnz, int n, const int* ci);
+    // Sets *flag (on the device) unless every ci[0..nnz) lies in [0, n).
+    int raise_bad_columns(lal_context* c, int nnz, int n, const int* ci, int* flag);
 }

@@ -70,12 +70,6 @@ namespace lal
         const int*            cbase = nullptr;
     };
 
-    // Builds the 16-bit column copy of a fast-path descriptor's matrix
-    // (d->d_c16, d->d_cbase) when every row block's columns span at most
-    // 65535; otherwise leaves the descriptor as it is.  Results of the row
-    // kernels are the same either way: only the bytes read change.
-    int compact_columns(lal_context* c, lal_csrmv_info* d, int nnz, const int* ci, arena* mem);
-
     // The descriptor's 16-bit columns into a's fields.
     inline void use_c16(rv_args& a, const lal_csrmv_info* d)
     {

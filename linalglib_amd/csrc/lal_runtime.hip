@@ -81,6 +81,57 @@ namespace lal
     }
 }
 
+namespace
+{
+    // One wavefront: n ints to mapped host memory, then the sequence number.
+    // The system-scope release waits for the wave's stores before it.
+    __global__ void __launch_bounds__(64)
+        note_kernel(int* __restrict__ src, int n, int clear, int* note, unsigned seq)
+    {
+        for(int i = threadIdx.x; i < n; i += 64)
+        {
+            __hip_atomic_store(note + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if(clear)
+                src[i] = 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+        if(threadIdx.x == 0)
+            __hip_atomic_store(reinterpret_cast<unsigned*>(note + LAL_NOTE_INTS), seq,
+                               __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+namespace lal
+{
+    int read_ints(lal_context* c, int* src, int n, int* out, bool clear)
+    {
+        LAL_REQUIRE(n >= 0 && n <= LAL_NOTE_INTS);
+        const unsigned seq = ++c->note_seq;
+        note_kernel<<<1, 64, 0, c->stream>>>(src, n, clear ? 1 : 0, c->d_note, seq);
+        LAL_LAUNCHED();
+        const unsigned* h_seq = reinterpret_cast<const unsigned*>(c->h_note + LAL_NOTE_INTS);
+        // poll, and look at the stream now and then so that a failed kernel
+        // turns into an error instead of a hang
+        for(long spins = 1; __atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq; spins++)
+            if((spins & 1023) == 0)
+            {
+                const hipError_t e = hipStreamQuery(c->stream);
+                if(e == hipSuccess)
+                    break; // drained: the note is there
+                if(e != hipErrorNotReady)
+                    LAL_HIP(e);
+            }
+        if(__atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq)
+        {
+            set_last_error("a result did not reach the host");
+            return LAL_ERR_HIP;
+        }
+        for(int i = 0; i < n; i++)
+            out[i] = __atomic_load_n(c->h_note + i, __ATOMIC_RELAXED);
+        return LAL_OK;
+    }
+}
+
 extern "C" const char* lal_last_error(void)
 {
     return lal::g_last_error.c_str();
@@ -139,12 +190,15 @@ extern "C" int lal_create(lal_handle* handle)
     LAL_HIP(hipMalloc(&c->d_part, sizeof(double) * LAL_RED_BLOCKS * 2));
     LAL_HIP(hipMalloc(&c->d_ticket, sizeof(unsigned) * LAL_NUM_SLOTS));
     LAL_HIP(hipMalloc(&c->d_slots, sizeof(double) * LAL_NUM_SLOTS));
-    LAL_HIP(hipMalloc(&c->d_flag, sizeof(int) * 16));
+    LAL_HIP(hipMalloc(&c->d_flag, sizeof(int) * LAL_FLAGS));
     LAL_HIP(hipHostMalloc(&c->h_slots, sizeof(double) * LAL_NUM_SLOTS, hipHostMallocDefault));
-    LAL_HIP(hipHostMalloc(&c->h_flag, sizeof(int) * 16, hipHostMallocDefault));
+    LAL_HIP(hipHostMalloc(&c->h_note, sizeof(int) * (LAL_NOTE_INTS + 1),
+                          hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(c->h_note, 0, sizeof(int) * (LAL_NOTE_INTS + 1));
+    LAL_HIP(hipHostGetDevicePointer((void**)&c->d_note, c->h_note, 0));
     LAL_HIP(hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned) * LAL_NUM_SLOTS, c->stream));
     LAL_HIP(hipMemsetAsync(c->d_slots, 0, sizeof(double) * LAL_NUM_SLOTS, c->stream));
-    LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int) * 16, c->stream));
+    LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int) * LAL_FLAGS, c->stream));
     LAL_HIP(hipStreamSynchronize(c->stream));
     *handle = c;
     return LAL_OK;
@@ -162,7 +216,7 @@ extern "C" int lal_destroy(lal_handle c)
     (void)hipFree(c->d_slots);
     (void)hipFree(c->d_flag);
     (void)hipHostFree(c->h_slots);
-    (void)hipHostFree(c->h_flag);
+    (void)hipHostFree(c->h_note);
     if(c->own_stream)
         (void)hipStreamDestroy(c->stream);
     delete c;

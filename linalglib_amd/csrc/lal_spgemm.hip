@@ -675,6 +675,8 @@ namespace
         int               g        = 8; // lanes per A row and per B row
         int               l        = 8; // (launch_group)
         std::vector<long long> toff; // global table offsets (n_global + 1)
+        int*              d_prod   = nullptr; // products per row (symbolic plan)
+        int*              d_part   = nullptr; // row offsets per bin and workgroup
         int*              d_rows   = nullptr; // LDS-bin rows, then global rows
         long long*        d_toff   = nullptr;
         int*              d_keys   = nullptr;
@@ -705,123 +707,168 @@ namespace
         return H > max_h ? kBins : b;
     }
 
-    // Rows per bin, gathered per workgroup in LDS.
+    // Rows of a workgroup of the binning kernels (each takes one contiguous
+    // range; at most BIN_GROUPS of them, so that one workgroup adds them up).
+    constexpr int BIN_GROUPS = 1024;
+    inline int bin_rows(int m)
+    {
+        return std::max(256, ((m + BIN_GROUPS - 1) / BIN_GROUPS + 255) / 256 * 256);
+    }
+
+    // part[bin * groups + workgroup] = the workgroup's rows in the bin.  The
+    // symbolic pass also clears its counts (rows without products keep the 0).
     __global__ void __launch_bounds__(256)
-        bin_count_kernel(int m, const int* __restrict__ prod, const int* __restrict__ crp,
-                         int ncols, int max_h, int* __restrict__ hist)
+        bin_count_kernel(int m, int per, const int* __restrict__ prod,
+                         const int* __restrict__ crp, int ncols, int max_h,
+                         int* __restrict__ part, int* __restrict__ clear)
     {
         __shared__ int s_n[kBins + 1];
         if(threadIdx.x <= kBins)
             s_n[threadIdx.x] = 0;
         __syncthreads();
-        const int i = blockIdx.x * 256 + threadIdx.x;
-        long long H = 0;
-        const int b = i < m ? row_bin(i, prod, crp, ncols, max_h, &H) : -1;
-        if(b >= 0)
-            atomicAdd(&s_n[b], 1);
+        const int r0 = blockIdx.x * per, r1 = min(m, r0 + per);
+        for(int i = r0 + (int)threadIdx.x; i < r1; i += 256)
+        {
+            long long H = 0;
+            const int b = row_bin(i, prod, crp, ncols, max_h, &H);
+            if(b >= 0)
+                atomicAdd(&s_n[b], 1);
+            if(clear)
+                clear[i] = 0;
+        }
+        if(clear && r1 == m && threadIdx.x == 0)
+            clear[m] = 0;
         __syncthreads();
-        if(threadIdx.x <= kBins && s_n[threadIdx.x])
-            atomicAdd(&hist[threadIdx.x], s_n[threadIdx.x]);
+        if(threadIdx.x <= kBins)
+            part[threadIdx.x * gridDim.x + blockIdx.x] = s_n[threadIdx.x];
     }
 
-    // Rows into their bins: bin b follows the rows of bins 0 .. b-1, and
-    // within a bin the workgroups take their places in order of arrival (each
-    // row of C is computed on its own, so the order changes no result).  A
-    // row of the global bin also records its table size in gslots.
+    // One workgroup: the counts, bin after bin, become row offsets; out[b] =
+    // rows of bin b, out[kBins + 1] = *tail when given.
     __global__ void __launch_bounds__(256)
-        bin_scatter_kernel(int m, const int* __restrict__ prod, const int* __restrict__ crp,
-                           int ncols, int max_h, const int* __restrict__ hist,
-                           int* __restrict__ cursor, int* __restrict__ rows,
+        bin_scan_kernel(int groups, int* __restrict__ part, int* __restrict__ out,
+                        const int* __restrict__ tail)
+    {
+        __shared__ int s_w[4];
+        const int      lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
+        int            carry = 0;
+        for(int b = 0; b <= kBins; b++)
+        {
+            const int before = carry;
+            for(int g0 = 0; g0 < groups; g0 += 256)
+            {
+                const int i   = g0 + (int)threadIdx.x;
+                const int v   = i < groups ? part[b * groups + i] : 0;
+                int       inc = v;
+#pragma unroll
+                for(int o = 1; o < 64; o <<= 1)
+                {
+                    const int q = __shfl_up(inc, o, 64);
+                    inc += lane >= o ? q : 0;
+                }
+                if(lane == 63)
+                    s_w[wid] = inc;
+                __syncthreads();
+                int off = carry, tot = 0;
+                for(int w = 0; w < 4; w++)
+                {
+                    off += w < wid ? s_w[w] : 0;
+                    tot += s_w[w];
+                }
+                if(i < groups)
+                    part[b * groups + i] = off + inc - v;
+                carry += tot;
+                __syncthreads();
+            }
+            if(threadIdx.x == 0)
+                out[b] = carry - before;
+        }
+        if(threadIdx.x == 0)
+            out[kBins + 1] = tail ? *tail : 0;
+    }
+
+    // Rows into their bins, at the workgroup's offsets (each row of C is
+    // computed on its own, so the order within a workgroup changes no
+    // result).  A row of the global bin, whose first position is g0, also
+    // records its table size in gslots.
+    __global__ void __launch_bounds__(256)
+        bin_scatter_kernel(int m, int per, const int* __restrict__ prod,
+                           const int* __restrict__ crp, int ncols, int max_h,
+                           const int* __restrict__ part, int* __restrict__ rows, int g0,
                            long long* __restrict__ gslots)
     {
-        __shared__ int s_n[kBins + 1], s_base[kBins + 1];
+        __shared__ int s_at[kBins + 1];
         if(threadIdx.x <= kBins)
-            s_n[threadIdx.x] = 0;
+            s_at[threadIdx.x] = part[threadIdx.x * gridDim.x + blockIdx.x];
         __syncthreads();
-        const int i     = blockIdx.x * 256 + threadIdx.x;
-        long long H     = 0;
-        const int b     = i < m ? row_bin(i, prod, crp, ncols, max_h, &H) : -1;
-        const int local = b >= 0 ? atomicAdd(&s_n[b], 1) : 0;
-        __syncthreads();
-        if(threadIdx.x <= kBins && s_n[threadIdx.x])
+        const int r0 = blockIdx.x * per, r1 = min(m, r0 + per);
+        for(int i = r0 + (int)threadIdx.x; i < r1; i += 256)
         {
-            int start = 0;
-            for(int q = 0; q < (int)threadIdx.x; q++)
-                start += hist[q];
-            s_base[threadIdx.x] = start + atomicAdd(&cursor[threadIdx.x], s_n[threadIdx.x]);
-        }
-        __syncthreads();
-        if(b >= 0)
-        {
-            const int pos = s_base[b] + local;
+            long long H = 0;
+            const int b = row_bin(i, prod, crp, ncols, max_h, &H);
+            if(b < 0)
+                continue;
+            const int pos = atomicAdd(&s_at[b], 1);
             rows[pos]     = i;
             if(b == kBins)
-            {
-                int n_lds = 0;
-                for(int q = 0; q < kBins; q++)
-                    n_lds += hist[q];
-                gslots[pos - n_lds] = H;
-            }
+                gslots[pos - g0] = H;
         }
     }
 
-    // Rows of C binned by table size on the device; the host reads back the
-    // eleven bin counts (and, when some rows need global tables, their table
-    // sizes) to size the launches and the global tables.
-    int make_plan(lal_context* c, int m, int n, const int* arp, const int* aci, const int* brp,
-                  const int* crp, bool numeric, spgemm_plan& P, lal::temps& tmp, long nnz_a = 0)
+    // Rows of C binned by table size on the device: counts the rows of each
+    // bin and hands the host the eleven counts (and, for the numeric plan,
+    // *tail, which it wants at the same time).
+    int plan_count(lal_context* c, int m, int n, const int* crp, bool numeric, spgemm_plan& P,
+                   lal::temps& tmp, int* clear, const int* tail, int* tail_out)
     {
         constexpr int nb = kBins + 1;
-        static_assert(nb <= 16, "the bin counts are read back through the context's flags");
         P.bin_start.assign(nb, 0);
-        P.n_lds    = 0;
-        P.n_global = 0;
+        P.n_lds = P.n_global = 0;
         if(m <= 0)
             return LAL_OK;
-        const int  max_h  = numeric ? kLdsMaxH : kLdsMaxHSym;
-        const int  grid   = lal::grid_for(m, 256);
-        int*       d_prod = nullptr;
-        int*       d_bins = nullptr; // counts, then cursors
-        long long* d_gsl  = nullptr;
-        if(!numeric)
-        {
-            LAL_TRY(tmp.get(&d_prod, m));
-            // rows of A averaging 16 or more entries: 16 lanes per row
-            if(nnz_a >= 16L * m)
-                products_group_kernel<16><<<(int)(((long)m * 16 + 255) / 256), 256, 0,
-                                            c->stream>>>(m, arp, aci, brp, d_prod);
-            else
-                products_kernel<<<grid, 256, 0, c->stream>>>(m, arp, aci, brp, d_prod);
-            LAL_LAUNCHED();
-        }
-        LAL_TRY(tmp.get(&d_bins, 2 * nb));
-        LAL_HIP(hipMemsetAsync(d_bins, 0, sizeof(int) * 2 * nb, c->stream));
-        bin_count_kernel<<<grid, 256, 0, c->stream>>>(m, d_prod, numeric ? crp : nullptr, n,
-                                                      max_h, d_bins);
+        const int per    = bin_rows(m);
+        const int groups = (m + per - 1) / per;
+        int*      out    = nullptr;
+        LAL_TRY(tmp.get(&P.d_part, (size_t)nb * groups));
+        LAL_TRY(tmp.get(&out, nb + 1));
+        bin_count_kernel<<<groups, 256, 0, c->stream>>>(m, per, P.d_prod, numeric ? crp : nullptr,
+                                                        n, numeric ? kLdsMaxH : kLdsMaxHSym,
+                                                        P.d_part, clear);
         LAL_LAUNCHED();
-        LAL_HIP(hipMemcpyAsync(c->h_flag, d_bins, sizeof(int) * nb, hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        long long total = 0;
-        for(int b = 0; b < kBins; b++)
+        bin_scan_kernel<<<1, 256, 0, c->stream>>>(groups, P.d_part, out, tail);
+        LAL_LAUNCHED();
+        int got[nb + 1];
+        LAL_TRY(lal::read_ints(c, out, nb + 1, got, false));
+        int total = 0;
+        for(int b = 0; b < nb; b++)
         {
-            P.bin_start[b] = (int)total;
-            total += c->h_flag[b];
+            P.bin_start[b] = total;
+            total += got[b];
         }
-        P.bin_start[kBins] = (int)total;
-        P.n_lds            = (int)total;
-        P.n_global         = c->h_flag[kBins];
-        total += P.n_global;
-        if(total)
-        {
-            LAL_TRY(tmp.get(&P.d_rows, total));
-            if(P.n_global)
-                LAL_TRY(tmp.get(&d_gsl, P.n_global));
-            bin_scatter_kernel<<<grid, 256, 0, c->stream>>>(m, d_prod, numeric ? crp : nullptr, n,
-                                                            max_h, d_bins, d_bins + nb, P.d_rows,
-                                                            d_gsl);
-            LAL_LAUNCHED();
-        }
+        P.n_lds    = P.bin_start[kBins];
+        P.n_global = got[kBins];
+        if(tail_out)
+            *tail_out = got[kBins + 1];
+        return LAL_OK;
+    }
+
+    // The rows' lists, and the tables of those that need global memory.
+    int plan_rows(lal_context* c, int m, int n, const int* crp, bool numeric, spgemm_plan& P,
+                  lal::temps& tmp)
+    {
+        const int total = P.n_lds + P.n_global;
+        if(total == 0)
+            return LAL_OK;
+        const int  per    = bin_rows(m);
+        const int  groups = (m + per - 1) / per;
+        long long* d_gsl  = nullptr;
+        LAL_TRY(tmp.get(&P.d_rows, total));
+        if(P.n_global)
+            LAL_TRY(tmp.get(&d_gsl, P.n_global));
+        bin_scatter_kernel<<<groups, 256, 0, c->stream>>>(
+            m, per, P.d_prod, numeric ? crp : nullptr, n, numeric ? kLdsMaxH : kLdsMaxHSym,
+            P.d_part, P.d_rows, P.n_lds, d_gsl);
+        LAL_LAUNCHED();
         if(P.n_global)
         {
             P.toff.assign(P.n_global + 1, 0);
@@ -840,6 +887,24 @@ namespace
             // P.toff must outlive the copy to the device
             LAL_HIP(hipStreamSynchronize(c->stream));
         }
+        return LAL_OK;
+    }
+
+    // Products of every row of C, for the symbolic plan (rows of A averaging
+    // 16 or more entries: 16 lanes per row).
+    int count_products(lal_context* c, int m, const int* arp, const int* aci, const int* brp,
+                       long nnz_a, spgemm_plan& P, lal::temps& tmp)
+    {
+        if(m <= 0)
+            return LAL_OK;
+        LAL_TRY(tmp.get(&P.d_prod, m));
+        if(nnz_a >= 16L * m)
+            products_group_kernel<16><<<(int)(((long)m * 16 + 255) / 256), 256, 0, c->stream>>>(
+                m, arp, aci, brp, P.d_prod);
+        else
+            products_kernel<<<lal::grid_for(m, 256), 256, 0, c->stream>>>(m, arp, aci, brp,
+                                                                          P.d_prod);
+        LAL_LAUNCHED();
         return LAL_OK;
     }
 
@@ -979,48 +1044,80 @@ namespace lal
         return transpose_t<double>(c, m, n, nnz, rp, ci, v, trp, tci, tv, a);
     }
 
-    int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
-                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a,
-                    long nnz_b, arena* a)
+    // The symbolic pass: row_ptr of C, its entry count, and in `num` the plan
+    // of the numeric pass over it (its bin counts come with the entry count).
+    static int symbolic(lal_context* c, int m, int n, const int* arp, const int* aci,
+                        const int* brp, const int* bci, int* crp, int* nnz_c, int g, int l,
+                        long nnz_a, spgemm_plan& num, temps& tmp, arena* a)
     {
-        temps tmp(c, a);
-        LAL_HIP(hipMemsetAsync(crp, 0, sizeof(int) * (m + 1), c->stream));
+        if(m <= 0)
+        {
+            LAL_HIP(hipMemsetAsync(crp, 0, sizeof(int), c->stream));
+            *nnz_c = 0;
+            return LAL_OK;
+        }
         spgemm_plan P;
-        P.g = lanes_for(m > 0 ? nnz_a / m : 0);
-        P.l = lanes_for(k > 0 ? nnz_b / k : 0);
-        LAL_TRY(make_plan(c, m, n, arp, aci, brp, nullptr, false, P, tmp, nnz_a));
-        int st = run_plan<false>(c, P, arp, aci, nullptr, brp, bci, nullptr, nullptr, crp,
-                                 nullptr);
-        LAL_TRY(st);
+        P.g = g;
+        P.l = l;
+        LAL_TRY(count_products(c, m, arp, aci, brp, nnz_a, P, tmp));
+        LAL_TRY(plan_count(c, m, n, nullptr, false, P, tmp, crp, nullptr, nullptr));
+        LAL_TRY(plan_rows(c, m, n, nullptr, false, P, tmp));
+        LAL_TRY(run_plan<false>(c, P, arp, aci, nullptr, brp, bci, nullptr, nullptr, crp,
+                                nullptr));
         LAL_TRY(scan_i32_dev(c, m + 1, crp, a));
-        LAL_HIP(hipMemcpyAsync(c->h_flag, crp + m, sizeof(int), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        *nnz_c = c->h_flag[0];
-        return LAL_OK;
+        num.g = g;
+        num.l = l;
+        return plan_count(c, m, n, crp, true, num, tmp, nullptr, crp + m, nnz_c);
+    }
+
+    int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
+                    const int* brp, const int* bci, int* crp, int* nnz_c, long nnz_a, long nnz_b)
+    {
+        temps       tmp(c, nullptr);
+        spgemm_plan num;
+        return symbolic(c, m, n, arp, aci, brp, bci, crp, nnz_c, lanes_for(m > 0 ? nnz_a / m : 0),
+                        lanes_for(k > 0 ? nnz_b / k : 0), nnz_a, num, tmp, nullptr);
     }
 
     int csrgemm_solve_f64(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
                           const double* av, const int* brp, const int* bci, const double* bv,
-                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b, arena* a)
+                          const int* crp, int* cci, double* cv, long nnz_a, long nnz_b)
     {
-        temps       tmp(c, a);
+        temps       tmp(c, nullptr);
         spgemm_plan P;
         P.g = lanes_for(m > 0 ? nnz_a / m : 0);
         P.l = lanes_for(k > 0 ? nnz_b / k : 0);
-        LAL_TRY(make_plan(c, m, n, arp, aci, brp, crp, true, P, tmp));
-        LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
-        int st = run_plan<true>(c, P, arp, aci, av, brp, bci, bv, crp, cci, cv);
-        LAL_TRY(st);
-        LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        if(c->h_flag[0])
+        LAL_TRY(plan_count(c, m, n, crp, true, P, tmp, nullptr, nullptr, nullptr));
+        LAL_TRY(plan_rows(c, m, n, crp, true, P, tmp));
+        LAL_TRY(run_plan<true>(c, P, arp, aci, av, brp, bci, bv, crp, cci, cv));
+        int bad = 0;
+        LAL_TRY(read_ints(c, c->d_flag, 1, &bad, true));
+        if(bad)
         {
             set_last_error("csrgemm_solve: row_ptr of C does not match the product's pattern");
             return LAL_ERR_INVALID;
         }
         return LAL_OK;
+    }
+
+    // C = A B for a hierarchy build: C's arrays (nnz entries, m + 1 row
+    // pointers) lie in `mem`, the work arrays in `work`.  The operands are the
+    // build's own, so the numeric pass's row check cannot fail and is not
+    // waited for.
+    int product(lal_context* c, int m, int k, int n, int nnz_a, const int* arp, const int* aci,
+                const double* av, int nnz_b, const int* brp, const int* bci, const double* bv,
+                int** crp, int** cci, double** cv, int* nnz_c, arena* mem, arena* work)
+    {
+        temps       tmp(c, work);
+        spgemm_plan num;
+        LAL_TRY(mem->get(crp, (size_t)m + 1));
+        LAL_TRY(symbolic(c, m, n, arp, aci, brp, bci, *crp, nnz_c,
+                         lanes_for(m > 0 ? nnz_a / m : 0), lanes_for(k > 0 ? nnz_b / k : 0),
+                         nnz_a, num, tmp, work));
+        LAL_TRY(mem->get(cci, *nnz_c));
+        LAL_TRY(mem->get(cv, *nnz_c));
+        LAL_TRY(plan_rows(c, m, n, *crp, true, num, tmp));
+        return run_plan<true>(c, num, arp, aci, av, brp, bci, bv, *crp, *cci, *cv);
     }
 }
 
@@ -1059,17 +1156,23 @@ namespace
     int check_product_operands(lal_context* c, int k, int n, int nnz_A, const int* aci,
                                int nnz_B, const int* brp, const int* bci)
     {
-        LAL_TRY(lal::check_columns(c, nnz_A, k, aci));
-        LAL_TRY(lal::check_columns(c, nnz_B, n, bci));
-        if(k == 0 || nnz_B == 0)
-            return LAL_OK;
-        LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int), c->stream));
-        dup_cols_kernel<<<lal::grid_for(k, 256), 256, 0, c->stream>>>(k, brp, bci, c->d_flag);
-        LAL_LAUNCHED();
-        LAL_HIP(hipMemcpyAsync(c->h_flag, c->d_flag, sizeof(int), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        if(c->h_flag[0])
+        // three flags, read together
+        LAL_TRY(lal::raise_bad_columns(c, nnz_A, k, aci, c->d_flag));
+        LAL_TRY(lal::raise_bad_columns(c, nnz_B, n, bci, c->d_flag + 1));
+        if(k > 0 && nnz_B > 0)
+        {
+            dup_cols_kernel<<<lal::grid_for(k, 256), 256, 0, c->stream>>>(k, brp, bci,
+                                                                          c->d_flag + 2);
+            LAL_LAUNCHED();
+        }
+        int bad[3];
+        LAL_TRY(lal::read_ints(c, c->d_flag, 3, bad, true));
+        if(bad[0] || bad[1])
+        {
+            lal::set_last_error("column index outside [0, n)");
+            return LAL_ERR_INVALID;
+        }
+        if(bad[2])
         {
             lal::set_last_error("csrgemm: a row of B repeats a column index");
             return LAL_ERR_UNSUPPORTED;
@@ -1102,8 +1205,7 @@ extern "C" int lal_csrgemm_nnz(lal_handle c, int m, int k, int n, int nnz_A, con
     LAL_REQUIRE(crp != nullptr && nnz_C != nullptr && arp != nullptr && brp != nullptr);
     LAL_REQUIRE((nnz_A == 0 || aci) && (nnz_B == 0 || bci));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
-    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A, nnz_B,
-                            nullptr);
+    return lal::csrgemm_nnz(c, m, k, n, arp, aci, brp, bci, crp, nnz_C, nnz_A, nnz_B);
 }
 
 extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_A,
@@ -1116,5 +1218,5 @@ extern "C" int lal_csrgemm_solve_f64(lal_handle c, int m, int k, int n, int nnz_
     LAL_REQUIRE((nnz_A == 0 || (aci && av)) && (nnz_B == 0 || (bci && bv)));
     LAL_TRY(check_product_operands(c, k, n, nnz_A, aci, nnz_B, brp, bci));
     return lal::csrgemm_solve_f64(c, m, k, n, arp, aci, av, brp, bci, bv, crp, cci, cv, nnz_A,
-                                  nnz_B, nullptr);
+                                  nnz_B);
 }

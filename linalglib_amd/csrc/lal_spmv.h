@@ -12,6 +12,8 @@
 
 #include "lal_internal.h"
 
+#include <vector>
+
 struct lal_csrmv_info
 {
     int  m        = 0;
@@ -27,11 +29,13 @@ struct lal_csrmv_info
     int* d_blocks = nullptr; // nblocks + 1 row offsets, then per block
                              // {r0, r1, row_ptr[r0], row_ptr[r1]} at
                              // lal::block_meta_offset(nblocks)
-    // 16-bit columns (fast path of the operators a hierarchy owns, set by
-    // lal::compact_columns): entry k of block b stores col_ind[k] - d_cbase[b];
-    // null when not built or a block's columns span more than 65535
+    // 16-bit columns (fast path of the operators a hierarchy owns): entry k of
+    // block b stores col_ind[k] - d_cbase[b]; null when not built or a block's
+    // columns span more than 65535
     unsigned short* d_c16   = nullptr;
     int*            d_cbase = nullptr;
+    // room for nb blocks, in the arena or an allocation of its own
+    int arrays(lal::arena* mem, int nb);
     bool owned = true; // d_blocks is this descriptor's to free (else, as the
                        // 16-bit columns always, it lies in a hierarchy's arena)
 };
@@ -46,6 +50,35 @@ namespace lal
     }
 
     constexpr int SPMV_THREADS = 256;
+
+    // A matrix pattern to analyse: d gets its row blocks and, with want16 and
+    // where the blocks allow it, its 16-bit columns; check_n >= 0: every
+    // column must lie in [0, check_n).
+    struct rb_request
+    {
+        lal_csrmv_info* d;
+        const int*      rp;
+        const int*      ci;
+        int             m, nnz;
+        bool            want16;
+        int             check_n;
+    };
+    // The same as the analysis kernels see it.
+    struct rb_op
+    {
+        const int*      rp;
+        const int*      ci;
+        int*            blocks;
+        unsigned short* c16;
+        int*            cbase;
+        int             m, nnz, cap;
+        int             tile0, ntiles; // its row tiles
+        int             blk0, ub;      // its blocks at most, in the columns' grid
+    };
+    // Analyses every request in one pass over the device (blocks until the
+    // results are known).  mem: where the descriptors' arrays lie (null: their
+    // own allocations, without 16-bit columns).
+    int analyse(lal_context* c, const std::vector<rb_request>& req, arena* mem, arena* tmp);
 
     // Largest matrix (values and column indices at the precision of the call)
     // that a descriptor marked `keep` reads with cache-allocating loads: three
