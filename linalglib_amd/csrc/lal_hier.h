@@ -164,15 +164,12 @@ struct lal_hierarchy_t
         hipGraphExec_t exec;
     };
     std::vector<cycle_graph> cycle_graphs;
-    hipStream_t              capture_stream = nullptr; // where they are captured
 
     ~lal_hierarchy_t()
     {
         for(auto& g : cycle_graphs)
             if(g.exec)
                 (void)hipGraphExecDestroy(g.exec);
-        if(capture_stream)
-            (void)hipStreamDestroy(capture_stream);
         for(int l = 0; l <= 20; l++)
         {
             for(lal::csr_dev* M : {&L[l].A, &L[l].P, &L[l].R})
@@ -233,9 +230,9 @@ namespace lal
 
     // Runs body() -- launches on h->c->stream only: no allocation, memset or
     // host synchronisation -- eagerly on the first use of its key, captures it
-    // as a HIP graph on the hierarchy's own non-blocking stream on the second
+    // as a HIP graph on the context's own non-blocking stream on the second
     // (the caller's stream may be the null stream, which cannot be captured;
-    // the context's stream points at the capture stream meanwhile) and
+    // the context's stream points at its own meanwhile) and
     // replays the graph on the caller's stream from then on.  A capture that
     // fails leaves the key eager.
     template <typename Body>
@@ -261,24 +258,16 @@ namespace lal
         }
         if(g->failed)
             return body();
-        if(h->capture_stream == nullptr &&
-           hipStreamCreateWithFlags(&h->capture_stream, hipStreamNonBlocking) != hipSuccess)
-        {
-            (void)hipGetLastError();
-            h->capture_stream = nullptr;
-            g->failed         = true;
-            return body();
-        }
         hipGraph_t        graph = nullptr;
         hipGraphExec_t    exec  = nullptr;
         const hipStream_t user  = c->stream;
-        if(hipStreamBeginCapture(h->capture_stream, hipStreamCaptureModeThreadLocal) ==
+        if(hipStreamBeginCapture(c->side, hipStreamCaptureModeThreadLocal) ==
            hipSuccess)
         {
-            c->stream          = h->capture_stream;
+            c->stream          = c->side;
             const int        st = body();
             c->stream          = user;
-            const hipError_t e  = hipStreamEndCapture(h->capture_stream, &graph);
+            const hipError_t e  = hipStreamEndCapture(c->side, &graph);
             if(st == LAL_OK && e == hipSuccess && graph != nullptr &&
                hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess)
                 g->exec = exec;

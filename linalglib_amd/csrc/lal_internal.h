@@ -68,8 +68,9 @@ namespace lal
 
 struct lal_context
 {
-    hipStream_t stream     = nullptr;
-    bool        own_stream = false;
+    hipStream_t stream     = nullptr; // where the work goes: `side` or the caller's
+    hipStream_t side       = nullptr; // the context's own, non-blocking; graphs are
+                                      // captured on it
     int         device     = 0;
     int         num_cu     = 0;
     // reduction workspace: partials, a ticket counter per reduction slot

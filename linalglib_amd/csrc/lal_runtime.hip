@@ -185,8 +185,8 @@ extern "C" int lal_create(lal_handle* handle)
             return st;
         }
     }
-    LAL_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    c->own_stream = true;
+    LAL_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+    c->stream = c->side;
     LAL_HIP(hipMalloc(&c->d_part, sizeof(double) * LAL_RED_BLOCKS * 2));
     LAL_HIP(hipMalloc(&c->d_ticket, sizeof(unsigned) * LAL_NUM_SLOTS));
     LAL_HIP(hipMalloc(&c->d_slots, sizeof(double) * LAL_NUM_SLOTS));
@@ -208,8 +208,7 @@ extern "C" int lal_destroy(lal_handle c)
 {
     if(!c)
         return LAL_OK;
-    if(c->stream)
-        (void)hipStreamSynchronize(c->stream);
+    (void)hipStreamSynchronize(c->stream);
     lal::detach_hierarchies(c);
     (void)hipFree(c->d_part);
     (void)hipFree(c->d_ticket);
@@ -217,8 +216,7 @@ extern "C" int lal_destroy(lal_handle c)
     (void)hipFree(c->d_flag);
     (void)hipHostFree(c->h_slots);
     (void)hipHostFree(c->h_note);
-    if(c->own_stream)
-        (void)hipStreamDestroy(c->stream);
+    (void)hipStreamDestroy(c->side);
     delete c;
     return LAL_OK;
 }
@@ -227,10 +225,7 @@ extern "C" int lal_set_stream(lal_handle c, void* stream)
 {
     LAL_REQUIRE(c != nullptr);
     LAL_HIP(hipStreamSynchronize(c->stream));
-    if(c->own_stream)
-        LAL_HIP(hipStreamDestroy(c->stream));
-    c->stream     = static_cast<hipStream_t>(stream);
-    c->own_stream = false;
+    c->stream = static_cast<hipStream_t>(stream);
     return LAL_OK;
 }
 
