@@ -18,23 +18,6 @@
 
 namespace
 {
-    __global__ void __launch_bounds__(256)
-        strength_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                        const double* __restrict__ val, const double* __restrict__ d, double eps,
-                        int* __restrict__ conn)
-    {
-        int i = blockIdx.x * 256 + threadIdx.x;
-        if(i >= m)
-            return;
-        const double di = fabs(d[i]);
-        for(int j = rp[i]; j < rp[i + 1]; j++)
-        {
-            int    c = ci[j];
-            double v = val[j];
-            conn[j]  = (c != i) && (fabs(v) >= eps * sqrt(di * fabs(d[c])));
-        }
-    }
-
     __device__ __forceinline__ int hash1(unsigned x)
     {
         x = ((x >> 16) ^ x) * 0x45d9f3bu;
@@ -73,11 +56,8 @@ namespace
         }
     }
 
-    // PASS: decided rows also copy their state into max_state, so that the
-    // setup's own loop can alternate two buffers instead of copying state
-    // from max_state before every round (the C ABI round leaves them alone,
-    // as the reference's kernel does).
-    template <bool PASS>
+    // The C ABI's single steps, a lane per row: a decided row's max_state is
+    // left alone, as the reference's kernel does.
     __global__ void __launch_bounds__(256)
         pmis_round_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                           const int* __restrict__ conn, const int* __restrict__ state,
@@ -89,11 +69,7 @@ namespace
             return;
         const int si = state[i];
         if(si != 0)
-        {
-            if(PASS)
-                max_state[i] = si;
             return; // only undecided rows change anything
-        }
         int ms = si, mh = hash[i], mr = i;
         for(int j = rp[i]; j < rp[i + 1]; j++)
             if(conn[j] == 1)
@@ -122,9 +98,6 @@ namespace
             *incomplete = 1;
     }
 
-    // PASS: every row's state goes to max_state, changed or not, so that the
-    // setup's two joins alternate the buffers.
-    template <bool PASS>
     __global__ void __launch_bounds__(256)
         pmis_join_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                          const int* __restrict__ conn, const int* __restrict__ state,
@@ -134,8 +107,6 @@ namespace
         if(i >= m)
             return;
         const int si = state[i];
-        if(PASS)
-            max_state[i] = si;
         if(si == -1)
         {
             for(int j = rp[i]; j < rp[i + 1]; j++)
@@ -165,47 +136,74 @@ namespace
 namespace
 {
     // The prolongator P = (I - relax D^-1 A_F) T (saamg.cpp:51-207) with G lanes
-    // per row: a wavefront (G = 64) for the long rows of the coarse Galerkin
-    // levels, 8 lanes for the finest level's stencil rows.  Row i's entries
+    // per row (setup_row_lanes).  Row i's entries
     // are its candidates' distinct aggregates >= 0 (the diagonal and the
     // strong neighbours) in ascending order, each the CSR-order fold of its
     // contributions from the first one, with the weak couplings lumped into
-    // the diagonal.  Lanes read the row in coalesced chunks of G, the next
-    // aggregate in ascending order is a group-wide minimum, and every fold
-    // runs over the lanes in entry order.
+    // the diagonal.  The next aggregate in ascending order is a group-wide
+    // minimum, and every fold runs over the lanes in entry order.
+    //
+    // A row's candidates stay in registers, PROLONG_KEEP entries per lane: one
+    // read of the row, then every output column is a group minimum and a fold
+    // over registers.  The fills of a 121^3 diffusion hierarchy take 0.64 ms;
+    // rescanning the row from memory for every column (rows beyond
+    // G * PROLONG_KEEP entries still do) they took 1.77.
+    constexpr int PROLONG_KEEP = 4;
+
     template <int G>
-    __device__ __forceinline__ int64_t group_min_i64(int64_t v)
+    __device__ __forceinline__ int group_min_i32(int v)
     {
 #pragma unroll
         for(int o = G / 2; o > 0; o >>= 1)
-        {
-            const int64_t t = __shfl_xor(v, o, 64);
-            v               = t < v ? t : v;
-        }
+            v = min(v, __shfl_xor(v, o, 64));
         return v;
     }
 
-    // Smallest aggregate id above `last` among the row's candidates (LLONG_MAX
-    // when there is none); group-uniform.
-    template <int G>
-    __device__ __forceinline__ int64_t next_aggregate(int i, int rs, int re, int gl,
-                                                      const int* __restrict__ ci,
-                                                      const int* __restrict__ conn,
-                                                      const int64_t* __restrict__ agg,
-                                                      int64_t last)
+    // Aggregate of entry j's column when it is a candidate of row i (aggregate
+    // ids are below the row count, so 32 bits hold them); INT_MAX otherwise.
+    __device__ __forceinline__ int candidate_aggregate(int i, int c, int cn,
+                                                       const int64_t* __restrict__ agg)
     {
-        int64_t best = LLONG_MAX;
-        for(int j = rs + gl; j < re; j += G)
-        {
-            const int c = ci[j];
-            if(p_candidate(i, c, conn[j]))
+        if(!p_candidate(i, c, cn))
+            return INT_MAX;
+        const int64_t a = agg[c];
+        return a >= 0 ? (int)a : INT_MAX;
+    }
+
+    // v of lane t of the group that starts at lane gb (t group-uniform; in a
+    // whole wavefront it is a scalar read).
+    template <int G, typename V>
+    __device__ __forceinline__ V group_lane(V v, int gb, int t)
+    {
+        if constexpr(G == 64)
+            return lal::wave_lane(v, __builtin_amdgcn_readfirstlane(t));
+        else
+            return __shfl(v, gb + t, 64);
+    }
+
+    // Smallest aggregate id above `last` among the row's candidates (INT_MAX
+    // when there is none); group-uniform.  key: the lane's first PROLONG_KEEP
+    // entries; entries beyond them come from memory.
+    template <int G>
+    __device__ __forceinline__ int next_aggregate(int i, int rs, int re, int gl, bool more,
+                                                  const int (&key)[PROLONG_KEEP],
+                                                  const int* __restrict__ ci,
+                                                  const int* __restrict__ conn,
+                                                  const int64_t* __restrict__ agg, int last)
+    {
+        int best = INT_MAX;
+#pragma unroll
+        for(int u = 0; u < PROLONG_KEEP; u++)
+            if(key[u] > last && key[u] < best)
+                best = key[u];
+        if(more)
+            for(int j = rs + G * PROLONG_KEEP + gl; j < re; j += G)
             {
-                const int64_t a = agg[c];
+                const int a = candidate_aggregate(i, ci[j], conn[j], agg);
                 if(a > last && a < best)
                     best = a;
             }
-        }
-        return group_min_i64<G>(best);
+        return group_min_i32<G>(best);
     }
 
     template <int G>
@@ -225,12 +223,20 @@ namespace
             return;
         }
         const int rs = rp[i], re = rp[i + 1];
-        int       k    = 0;
-        int64_t   last = -1; // aggregates >= 0 only
+        int       key[PROLONG_KEEP];
+#pragma unroll
+        for(int u = 0; u < PROLONG_KEEP; u++)
+        {
+            const int j = rs + u * G + gl;
+            key[u]      = j < re ? candidate_aggregate(i, ci[j], conn[j], agg) : INT_MAX;
+        }
+        const bool more = re - rs > G * PROLONG_KEEP;
+        int        k    = 0;
+        int        last = -1;
         for(;;)
         {
-            const int64_t best = next_aggregate<G>(i, rs, re, gl, ci, conn, agg, last);
-            if(best == LLONG_MAX)
+            const int best = next_aggregate<G>(i, rs, re, gl, more, key, ci, conn, agg, last);
+            if(best == INT_MAX)
                 break;
             k++;
             last = best;
@@ -253,90 +259,117 @@ namespace
         if(i >= m)
             return;
         const int rs = rp[i], re = rp[i + 1];
-        // a_ii minus the weak couplings, summed in CSR order
-        double diagonal = 0.0;
-        for(int j0 = rs; j0 < re; j0 += G)
+        const int p0 = prp[i], p1 = prp[i + 1];
+        int       key[PROLONG_KEEP];
+        double    v[PROLONG_KEEP];
+        int       kind[PROLONG_KEEP]; // 1: the diagonal, 2: weak, 0: strong or none
+#pragma unroll
+        for(int u = 0; u < PROLONG_KEEP; u++)
         {
-            const int j    = j0 + gl;
-            int       kind = 0;
-            double    v    = 0.0;
+            const int j = rs + u * G + gl;
+            key[u]      = INT_MAX;
+            v[u]        = 0.0;
+            kind[u]     = 0;
             if(j < re)
             {
-                const int c = ci[j];
-                if(c == i)
-                    kind = 1;
-                else if(conn[j] == 0)
-                    kind = 2;
-                v = val[j];
-            }
-            const int n = min(G, re - j0);
-            for(int t = 0; t < n; t++)
-            {
-                const int    kt = __shfl(kind, gb + t, 64);
-                const double vt = __shfl(v, gb + t, 64);
-                if(kt == 1)
-                    diagonal += vt;
-                else if(kt == 2)
-                    diagonal -= vt;
+                const int c = ci[j], cn = conn[j];
+                v[u]    = val[j];
+                kind[u] = c == i ? 1 : cn == 0 ? 2 : 0;
+                key[u]  = candidate_aggregate(i, c, cn, agg);
             }
         }
-        const double invd = 1.0 / diagonal;
-        int64_t      last = -1;
-        for(int out = prp[i]; out < prp[i + 1]; out++)
-        {
-            const int64_t best  = next_aggregate<G>(i, rs, re, gl, ci, conn, agg, last);
-            bool          first = true;
-            double        acc   = 0.0;
-            for(int j0 = rs; j0 < re; j0 += G)
+        const bool more = re - rs > G * PROLONG_KEEP;
+        // a_ii minus the weak couplings, summed in CSR order
+        double diagonal = 0.0;
+        auto   lump     = [&](int kd, double vv) {
+            unsigned long long mask = __ballot(kd != 0) >> gb;
+            if(G < 64)
+                mask &= (1ull << (G % 64)) - 1ull;
+            while(mask)
             {
-                const int j     = j0 + gl;
-                bool      match = false;
-                double    value = 0.0;
+                const int    t  = __ffsll((long long)mask) - 1;
+                const int    kt = group_lane<G>(kd, gb, t);
+                const double vt = group_lane<G>(vv, gb, t);
+                mask &= mask - 1;
+                diagonal = kt == 1 ? diagonal + vt : diagonal - vt;
+            }
+        };
+#pragma unroll
+        for(int u = 0; u < PROLONG_KEEP; u++)
+            lump(kind[u], v[u]);
+        if(more)
+            for(int j0 = rs + G * PROLONG_KEEP; j0 < re; j0 += G)
+            {
+                const int j  = j0 + gl;
+                int       kd = 0;
+                double    vv = 0.0;
                 if(j < re)
                 {
                     const int c = ci[j];
-                    if(p_candidate(i, c, conn[j]) && agg[c] == best)
-                    {
-                        match = true;
-                        value = (c == i) ? 1.0 - relax : -relax * invd * val[j];
-                    }
+                    kd          = c == i ? 1 : conn[j] == 0 ? 2 : 0;
+                    vv          = val[j];
                 }
+                lump(kd, vv);
+            }
+        const double invd = 1.0 / diagonal;
+        auto smoothed = [&](bool diag, double a) { return diag ? 1.0 - relax : -relax * invd * a; };
+#pragma unroll
+        for(int u = 0; u < PROLONG_KEEP; u++)
+            v[u] = smoothed(kind[u] == 1, v[u]);
+        int last = -1;
+        for(int out = p0; out < p1; out++)
+        {
+            const int best = next_aggregate<G>(i, rs, re, gl, more, key, ci, conn, agg, last);
+            bool      first = true;
+            double    acc   = 0.0;
+            auto      fold  = [&](bool match, double value) {
                 unsigned long long mask = __ballot(match) >> gb;
                 if(G < 64)
-                    mask &= (1ull << G) - 1ull;
+                    mask &= (1ull << (G % 64)) - 1ull;
                 while(mask)
                 {
                     const int    t  = __ffsll((long long)mask) - 1;
-                    const double vt = __shfl(value, gb + t, 64);
+                    const double vt = group_lane<G>(value, gb, t);
                     mask &= mask - 1;
-                    if(first)
-                    {
-                        acc   = vt;
-                        first = false;
-                    }
-                    else
-                        acc += vt;
+                    acc   = first ? vt : acc + vt;
+                    first = false;
                 }
-            }
+            };
+#pragma unroll
+            for(int u = 0; u < PROLONG_KEEP; u++)
+                fold(key[u] == best, v[u]);
+            if(more)
+                for(int j0 = rs + G * PROLONG_KEEP; j0 < re; j0 += G)
+                {
+                    const int j     = j0 + gl;
+                    bool      match = false;
+                    double    value = 0.0;
+                    if(j < re)
+                    {
+                        const int c = ci[j];
+                        if(candidate_aggregate(i, c, conn[j], agg) == best)
+                        {
+                            match = true;
+                            value = smoothed(c == i, val[j]);
+                        }
+                    }
+                    fold(match, value);
+                }
             if(gl == 0)
             {
-                pci[out] = (int)best;
+                pci[out] = best;
                 pv[out]  = acc;
             }
             last = best;
         }
     }
-
-    // Rows this long on average take a wavefront per row, shorter ones 8 lanes.
-    constexpr long PROLONG_WAVE_MIN_ROW = 24;
 }
 
 namespace
 {
-    // Strength, the diagonal and the PMIS passes with G lanes per row (G = 16
-    // or 64, 256 / G rows per workgroup) for the long rows of the coarse
-    // Galerkin levels, where a lane walking a row of 40-190 entries alone is
-    // a chain of dependent loads.  Each lane takes the row's entries
+    // Strength, the diagonal and the PMIS passes with G lanes per row (8,
+    // 16 or 64, 256 / G rows per workgroup): a lane walking a row alone is a
+    // chain of dependent, strided loads.  Each lane takes the row's entries
     // j = rs + gl, rs + gl + G, ... in order; every per-row result the
     // thread-per-row kernels form in CSR order -- the first (or last) match,
     // a lexicographic maximum that keeps its first occurrence -- is the
@@ -475,7 +508,9 @@ namespace
     // pmis_round_kernel with G lanes per row: the running maximum starts at
     // the row itself, takes the row's strong neighbours in order, then the
     // strong neighbours of the row that maximum names.
-    template <int G, bool PASS>
+    // Every row's state goes to max_state, decided or not, so that the rounds
+    // alternate two buffers.
+    template <int G>
     __global__ void __launch_bounds__(256)
         pmis_round_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                                 const int* __restrict__ conn, const int* __restrict__ state,
@@ -489,7 +524,7 @@ namespace
         const int si = state[i];
         if(si != 0)
         {
-            if(PASS && gl == 0)
+            if(gl == 0)
                 max_state[i] = si;
             return; // only undecided rows change anything
         }
@@ -518,7 +553,7 @@ namespace
             *incomplete = 1;
     }
 
-    template <int G, bool PASS>
+    template <int G>
     __global__ void __launch_bounds__(256)
         pmis_join_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                                const int* __restrict__ conn, const int* __restrict__ state,
@@ -529,7 +564,7 @@ namespace
         if(i >= m)
             return;
         const int si = state[i];
-        if(PASS && gl == 0)
+        if(gl == 0)
             max_state[i] = si;
         if(si == -1)
         {
@@ -602,12 +637,13 @@ namespace
         }
     }
 
-    // Lanes per row for the row-walking setup passes: one for short rows (the
-    // finest level's stencil), 16 or 64 for the coarse Galerkin levels.
+    // Lanes per row for the row-walking setup passes: 8 for short rows (the
+    // finest level's stencil, whose rows a lane alone would read one entry
+    // after another, strided), 16 or 64 for the coarse Galerkin levels.
     inline int setup_row_lanes(long nnz, int m)
     {
         const long avg = m > 0 ? nnz / m : 0;
-        return avg >= 48 ? 64 : avg >= 12 ? 16 : 1;
+        return avg >= 48 ? 64 : avg >= 12 ? 16 : 8;
     }
 
     inline int group_grid(int m, int lanes)
@@ -631,25 +667,20 @@ namespace lal
         LAL_TRY(tmp.get(&d, m));
         LAL_HIP(hipMemsetAsync(d, 0, sizeof(double) * m, c->stream));
         const int lanes = setup_row_lanes(nnz, m);
-        if(lanes == 64)
+        const int gg    = group_grid(m, lanes);
+#define LAL_LANES(G)                                                                         \
+    case G:                                                                                  \
+        diagonal_group_kernel<G><<<gg, 256, 0, c->stream>>>(m, rp, ci, v, d);                \
+        LAL_LAUNCHED();                                                                      \
+        strength_group_kernel<G><<<gg, 256, 0, c->stream>>>(m, rp, ci, v, d, eps, conn);     \
+        break;
+        switch(lanes)
         {
-            diagonal_group_kernel<64><<<group_grid(m, 64), 256, 0, c->stream>>>(m, rp, ci, v, d);
-            LAL_LAUNCHED();
-            strength_group_kernel<64>
-                <<<group_grid(m, 64), 256, 0, c->stream>>>(m, rp, ci, v, d, eps, conn);
+            LAL_LANES(64)
+            LAL_LANES(16)
+            LAL_LANES(8)
         }
-        else if(lanes == 16)
-        {
-            diagonal_group_kernel<16><<<group_grid(m, 16), 256, 0, c->stream>>>(m, rp, ci, v, d);
-            LAL_LAUNCHED();
-            strength_group_kernel<16>
-                <<<group_grid(m, 16), 256, 0, c->stream>>>(m, rp, ci, v, d, eps, conn);
-        }
-        else
-        {
-            LAL_TRY(diagonal_f64(c, m, rp, ci, v, d));
-            strength_kernel<<<grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, v, d, eps, conn);
-        }
+#undef LAL_LANES
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -665,7 +696,6 @@ namespace lal
         LAL_TRY(tmp.get(&max_state, m));
         LAL_TRY(tmp.get(&hash, m));
         LAL_HIP(hipMemsetAsync(agg, 0, sizeof(int64_t) * m, c->stream));
-        const int g     = grid_for(m, 256);
         const int lanes = setup_row_lanes(nnz, m);
         const int gg    = group_grid(m, lanes);
         if(lanes == 64)
@@ -673,7 +703,7 @@ namespace lal
         else if(lanes == 16)
             pmis_init_group_kernel<16><<<gg, 256, 0, c->stream>>>(m, rp, conn, max_state, hash);
         else
-            pmis_init_kernel<<<g, 256, 0, c->stream>>>(m, rp, conn, max_state, hash);
+            pmis_init_group_kernel<8><<<gg, 256, 0, c->stream>>>(m, rp, conn, max_state, hash);
         LAL_LAUNCHED();
         // The reference's loop (amg_aggregation.cpp:106-215): up to 20 rounds,
         // state = max_state before each, stop after the first complete one.
@@ -693,14 +723,14 @@ namespace lal
             const int* in  = buf[cur];
             int*       out = buf[cur ^ 1];
             if(lanes == 64)
-                pmis_round_group_kernel<64, true><<<gg, 256, 0, c->stream>>>(
-                    m, rp, ci, conn, in, hash, agg, out, flag);
+                pmis_round_group_kernel<64><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, hash,
+                                                                       agg, out, flag);
             else if(lanes == 16)
-                pmis_round_group_kernel<16, true><<<gg, 256, 0, c->stream>>>(
-                    m, rp, ci, conn, in, hash, agg, out, flag);
+                pmis_round_group_kernel<16><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, hash,
+                                                                       agg, out, flag);
             else
-                pmis_round_kernel<true><<<g, 256, 0, c->stream>>>(m, rp, ci, conn, in, hash, agg,
-                                                                  out, flag);
+                pmis_round_group_kernel<8><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, hash,
+                                                                      agg, out, flag);
             LAL_LAUNCHED();
             cur ^= 1;
             return LAL_OK;
@@ -724,13 +754,14 @@ namespace lal
             const int* in  = buf[k];
             int*       out = buf[k ^ 1];
             if(lanes == 64)
-                pmis_join_group_kernel<64, true>
+                pmis_join_group_kernel<64>
                     <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             else if(lanes == 16)
-                pmis_join_group_kernel<16, true>
+                pmis_join_group_kernel<16>
                     <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             else
-                pmis_join_kernel<true><<<g, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
+                pmis_join_group_kernel<8>
+                    <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             LAL_LAUNCHED();
         }
         return LAL_OK;
@@ -765,12 +796,14 @@ namespace lal
                            int* n_c, arena* a)
     {
         // count[m] = 0 is written by the group of row m, so m + 1 groups
-        if(m > 0 && nnz >= PROLONG_WAVE_MIN_ROW * (long)m)
-            prolong_count_group_kernel<64><<<(m + 1 + 3) / 4, 256, 0, c->stream>>>(m, rp, ci,
-                                                                                   conn, agg, prp);
+        const int lanes = setup_row_lanes(nnz, m);
+        const int gg    = group_grid(m + 1, lanes);
+        if(lanes == 64)
+            prolong_count_group_kernel<64><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, agg, prp);
+        else if(lanes == 16)
+            prolong_count_group_kernel<16><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, agg, prp);
         else
-            prolong_count_group_kernel<8><<<(m + 1 + 31) / 32, 256, 0, c->stream>>>(m, rp, ci,
-                                                                                    conn, agg, prp);
+            prolong_count_group_kernel<8><<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, agg, prp);
         LAL_LAUNCHED();
         LAL_TRY(scan_i32_dev(c, m + 1, prp, a));
         return prolongator_size(c, m, agg, prp, nnz_P, n_c, a);
@@ -782,12 +815,17 @@ namespace lal
     {
         if(m == 0)
             return LAL_OK;
-        if(nnz >= PROLONG_WAVE_MIN_ROW * (long)m)
-            prolong_fill_group_kernel<64><<<(m + 3) / 4, 256, 0, c->stream>>>(
-                m, rp, ci, v, conn, agg, relax, prp, pci, pv);
+        const int lanes = setup_row_lanes(nnz, m);
+        const int gg    = group_grid(m, lanes);
+        if(lanes == 64)
+            prolong_fill_group_kernel<64><<<gg, 256, 0, c->stream>>>(m, rp, ci, v, conn, agg,
+                                                                     relax, prp, pci, pv);
+        else if(lanes == 16)
+            prolong_fill_group_kernel<16><<<gg, 256, 0, c->stream>>>(m, rp, ci, v, conn, agg,
+                                                                     relax, prp, pci, pv);
         else
-            prolong_fill_group_kernel<8><<<(m + 31) / 32, 256, 0, c->stream>>>(
-                m, rp, ci, v, conn, agg, relax, prp, pci, pv);
+            prolong_fill_group_kernel<8><<<gg, 256, 0, c->stream>>>(m, rp, ci, v, conn, agg,
+                                                                    relax, prp, pci, pv);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -877,7 +915,7 @@ extern "C" int lal_pmis_round(lal_handle c, int m, int nnz, const int* rp, const
     *complete = 1;
     if(m == 0)
         return LAL_OK;
-    pmis_round_kernel<false><<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
+    pmis_round_kernel<<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
         m, rp, ci, conn, state, hash, agg, max_state, c->d_flag);
     LAL_LAUNCHED();
     int undecided = 0;
@@ -893,7 +931,7 @@ extern "C" int lal_pmis_join(lal_handle c, int m, int nnz, const int* rp, const 
     LAL_REQUIRE(m == 0 || (rp && state && agg && max_state && (nnz == 0 || (ci && conn))));
     if(m == 0)
         return LAL_OK;
-    pmis_join_kernel<false><<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
+    pmis_join_kernel<<<lal::grid_for(m, 256), 256, 0, c->stream>>>(
         m, rp, ci, conn, state, agg, max_state);
     LAL_LAUNCHED();
     return LAL_OK;

@@ -308,6 +308,46 @@ namespace
         }
     }
 
+    // Short arrays in one launch: one workgroup walks the tiles, the next
+    // tile's loads ahead of this one's scan.
+    constexpr int SCAN_SMALL = 8 * SCAN_TILE;
+
+    template <typename T>
+    __global__ void __launch_bounds__(SCAN_THREADS) scan_small(int n, T* __restrict__ x)
+    {
+        T   carry = 0;
+        T   v[SCAN_ITEMS];
+        int base = threadIdx.x * SCAN_ITEMS;
+#pragma unroll
+        for(int k = 0; k < SCAN_ITEMS; k++)
+            v[k] = base + k < n ? x[base + k] : 0;
+        for(int t0 = 0; t0 < n; t0 += SCAN_TILE, base += SCAN_TILE)
+        {
+            T next[SCAN_ITEMS];
+#pragma unroll
+            for(int k = 0; k < SCAN_ITEMS; k++)
+            {
+                const int at = base + SCAN_TILE + k;
+                next[k]      = at < n ? x[at] : 0;
+            }
+            T s = 0;
+#pragma unroll
+            for(int k = 0; k < SCAN_ITEMS; k++)
+                s += v[k];
+            T tot;
+            T e = block_exclusive_scan(s, &tot) + carry;
+#pragma unroll
+            for(int k = 0; k < SCAN_ITEMS; k++)
+            {
+                if(base + k < n)
+                    x[base + k] = e;
+                e += v[k];
+                v[k] = next[k];
+            }
+            carry += tot;
+        }
+    }
+
     static_assert(SCAN_TILE == 2048, "the no-allocation scratch holds one sum per 2048 entries");
 
     // The three passes of the scan with the tile sums in `sums` (ntiles
@@ -330,6 +370,12 @@ namespace
     {
         if(n <= 0)
             return LAL_OK;
+        if(n <= SCAN_SMALL)
+        {
+            scan_small<T><<<1, SCAN_THREADS, 0, c->stream>>>(n, x);
+            LAL_LAUNCHED();
+            return LAL_OK;
+        }
         int        ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
         T*         sums   = nullptr;
         lal::temps tmp(c, a);

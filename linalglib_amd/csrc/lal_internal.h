@@ -217,6 +217,19 @@ namespace lal
         return v;
     }
 
+    // v of lane t (the same t in every lane of the wavefront)
+    __device__ __forceinline__ int wave_lane(int v, int t)
+    {
+        return __builtin_amdgcn_readlane(v, t);
+    }
+    __device__ __forceinline__ double wave_lane(double v, int t)
+    {
+        const long long b  = __builtin_bit_cast(long long, v);
+        const unsigned  lo = (unsigned)__builtin_amdgcn_readlane((int)b, t);
+        const unsigned  hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), t);
+        return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+    }
+
     // Workgroup barrier that orders LDS accesses only: global loads issued
     // before it stay in flight (__syncthreads() waits for them).
     __device__ __forceinline__ void lds_barrier()

@@ -23,57 +23,65 @@
 namespace
 {
     // ------------------------------------------------------------ transpose
+    // Entries per column, and each entry's place among its column's (in order
+    // of arrival; the rows are sorted later): the atomic's return value, so
+    // that the scatter needs none of its own.
     __global__ void __launch_bounds__(256)
-        col_count_kernel(int nnz, const int* __restrict__ ci, int* __restrict__ cnt)
+        col_count_kernel(int nnz, const int* __restrict__ ci, int* __restrict__ cnt,
+                         int* __restrict__ place)
     {
         int k = blockIdx.x * 256 + threadIdx.x;
         if(k < nnz)
-            atomicAdd(&cnt[ci[k]], 1);
+            place[k] = atomicAdd(&cnt[ci[k]], 1);
     }
 
     template <typename T>
     __global__ void __launch_bounds__(256)
         transpose_scatter_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                                 const T* __restrict__ v, int* __restrict__ cursor,
-                                 int* __restrict__ tci, T* __restrict__ tv)
+                                 const T* __restrict__ v, const int* __restrict__ trp,
+                                 const int* __restrict__ place, int* __restrict__ tci,
+                                 T* __restrict__ tv)
     {
-        int i = blockIdx.x * 256 + threadIdx.x;
+        // 4 lanes per row
+        const int i = blockIdx.x * 64 + (int)(threadIdx.x >> 2);
         if(i >= m)
             return;
-        for(int j = rp[i]; j < rp[i + 1]; j++)
+        for(int j = rp[i] + (int)(threadIdx.x & 3); j < rp[i + 1]; j += 4)
         {
-            int pos  = atomicAdd(&cursor[ci[j]], 1);
-            tci[pos] = i;
-            tv[pos]  = v[j];
+            const int pos = trp[ci[j]] + place[j];
+            tci[pos]      = i;
+            tv[pos]       = v[j];
         }
     }
 
-    // Sorts each row by column, stably, with one wavefront per row: each lane
-    // ranks its entries (up to four) by counting the row's smaller columns,
-    // ties broken by position; every load of the row completes before the
-    // first store, so the row is permuted in place.  Rows longer than 256
-    // entries take lane 0's insertion sort.
-    template <typename T>
+    // Sorts each row by column, stably, with G lanes per row (16 for rows that
+    // are short on average, else a wavefront): each lane ranks its entries (up
+    // to four) by counting the row's smaller columns, ties broken by position;
+    // the columns pass from lane to lane in registers, and every load of the
+    // row completes before the first store, so the row is permuted in place.
+    // Rows longer than 4 G entries take the group's first lane's insertion sort.
+    template <int G, typename T>
     __global__ void __launch_bounds__(256)
-        row_sort_wave_kernel(int m, const int* __restrict__ rp, int* __restrict__ ci,
-                             T* __restrict__ v)
+        row_sort_kernel(int m, const int* __restrict__ rp, int* __restrict__ ci,
+                        T* __restrict__ v)
     {
-        const int lane = threadIdx.x & 63;
-        const int i    = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+        const int gl = (int)threadIdx.x % G;
+        const int gb = ((int)threadIdx.x & 63) - gl;
+        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
         if(i >= m)
             return;
-        const int s = rp[i], e = rp[i + 1];
-        if(e - s <= 1)
+        const int s = rp[i], n = rp[i + 1] - s;
+        if(n <= 1)
             return;
-        if(e - s > 256)
+        if(n > 4 * G)
         {
-            if(lane != 0)
+            if(gl != 0)
                 return;
-            for(int j = s + 1; j < e; j++)
+            for(int j = s + 1; j < s + n; j++)
             {
                 int kc = ci[j];
                 T   kv = v[j];
-                int    t  = j - 1;
+                int t  = j - 1;
                 while(t >= s && ci[t] > kc)
                 {
                     ci[t + 1] = ci[t];
@@ -90,24 +98,34 @@ namespace
 #pragma unroll
         for(int u = 0; u < 4; u++)
         {
-            const int j = s + lane + 64 * u;
-            key[u]      = j < e ? ci[j] : INT_MAX;
-            val[u]      = j < e ? v[j] : (T)0;
+            const int j = gl + G * u;
+            key[u]      = j < n ? ci[s + j] : INT_MAX;
+            val[u]      = j < n ? v[s + j] : (T)0;
             rank[u]     = 0;
         }
-        for(int t = s; t < e; t++)
-        {
-            const int kt = ci[t];
 #pragma unroll
-            for(int u = 0; u < 4; u++)
-                rank[u] += kt < key[u] || (kt == key[u] && t < s + lane + 64 * u);
+        for(int w = 0; w < 4; w++)
+        {
+            const int top = min(G, n - G * w);
+            for(int t = 0; t < top; t++)
+            {
+                int kt;
+                if constexpr(G == 64)
+                    kt = __builtin_amdgcn_readlane(key[w], t);
+                else
+                    kt = __shfl(key[w], gb + t, 64);
+#pragma unroll
+                for(int u = 0; u < 4; u++)
+                    if(G * u < n)
+                        rank[u] += kt < key[u] || (kt == key[u] && G * w + t < gl + G * u);
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for(int u = 0; u < 4; u++)
-            if(s + lane + 64 * u < e)
+            if(gl + G * u < n)
             {
                 ci[s + rank[u]] = key[u];
                 v[s + rank[u]]  = val[u];
@@ -279,19 +297,6 @@ namespace
         }
     }
 
-    // v of lane t (the same t in every lane of the wavefront)
-    __device__ __forceinline__ int wave_lane(int v, int t)
-    {
-        return __builtin_amdgcn_readlane(v, t);
-    }
-    __device__ __forceinline__ double wave_lane(double v, int t)
-    {
-        const long long b  = __builtin_bit_cast(long long, v);
-        const unsigned  lo = (unsigned)__builtin_amdgcn_readlane((int)b, t);
-        const unsigned  hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), t);
-        return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
-    }
-
     // Rows of C in LDS tables of H slots (a power of two, at least 64): G lanes
     // per row, L of them per B row.
     //
@@ -349,7 +354,7 @@ namespace
         // steps one by one reads the lane as a scalar)
         auto lane_value = [&](auto v, int t) {
             if constexpr(S == 1 && G == 64)
-                return wave_lane(v, __builtin_amdgcn_readfirstlane(t));
+                return lal::wave_lane(v, __builtin_amdgcn_readfirstlane(t));
             else
                 return __shfl(v, gb + t, 64);
         };
@@ -743,46 +748,52 @@ namespace
             part[threadIdx.x * gridDim.x + blockIdx.x] = s_n[threadIdx.x];
     }
 
-    // One workgroup: the counts, bin after bin, become row offsets; out[b] =
-    // rows of bin b, out[kBins + 1] = *tail when given.
-    __global__ void __launch_bounds__(256)
+    // One workgroup: the counts, bin after bin, become row offsets (one scan
+    // over all of them); out[b] = rows of bin b, out[kBins + 1] = *tail when
+    // given.
+    __global__ void __launch_bounds__(1024)
         bin_scan_kernel(int groups, int* __restrict__ part, int* __restrict__ out,
                         const int* __restrict__ tail)
     {
-        __shared__ int s_w[4];
+        __shared__ int s_w[16];
+        __shared__ int s_first[kBins + 2]; // offset of each bin's first row
         const int      lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
+        const int      n     = (kBins + 1) * groups;
         int            carry = 0;
-        for(int b = 0; b <= kBins; b++)
+        for(int i0 = 0; i0 < n; i0 += 1024)
         {
-            const int before = carry;
-            for(int g0 = 0; g0 < groups; g0 += 256)
-            {
-                const int i   = g0 + (int)threadIdx.x;
-                const int v   = i < groups ? part[b * groups + i] : 0;
-                int       inc = v;
+            const int i   = i0 + (int)threadIdx.x;
+            const int v   = i < n ? part[i] : 0;
+            int       inc = v;
 #pragma unroll
-                for(int o = 1; o < 64; o <<= 1)
-                {
-                    const int q = __shfl_up(inc, o, 64);
-                    inc += lane >= o ? q : 0;
-                }
-                if(lane == 63)
-                    s_w[wid] = inc;
-                __syncthreads();
-                int off = carry, tot = 0;
-                for(int w = 0; w < 4; w++)
-                {
-                    off += w < wid ? s_w[w] : 0;
-                    tot += s_w[w];
-                }
-                if(i < groups)
-                    part[b * groups + i] = off + inc - v;
-                carry += tot;
-                __syncthreads();
+            for(int o = 1; o < 64; o <<= 1)
+            {
+                const int q = __shfl_up(inc, o, 64);
+                inc += lane >= o ? q : 0;
             }
-            if(threadIdx.x == 0)
-                out[b] = carry - before;
+            if(lane == 63)
+                s_w[wid] = inc;
+            __syncthreads();
+            int off = carry, tot = 0;
+            for(int w = 0; w < 16; w++)
+            {
+                off += w < wid ? s_w[w] : 0;
+                tot += s_w[w];
+            }
+            if(i < n)
+            {
+                part[i] = off + inc - v;
+                if(i % groups == 0)
+                    s_first[i / groups] = off + inc - v;
+            }
+            carry += tot;
+            __syncthreads();
         }
+        if(threadIdx.x == 0)
+            s_first[kBins + 1] = carry;
+        __syncthreads();
+        if(threadIdx.x <= kBins)
+            out[threadIdx.x] = s_first[threadIdx.x + 1] - s_first[threadIdx.x];
         if(threadIdx.x == 0)
             out[kBins + 1] = tail ? *tail : 0;
     }
@@ -835,7 +846,7 @@ namespace
                                                         n, numeric ? kLdsMaxH : kLdsMaxHSym,
                                                         P.d_part, clear);
         LAL_LAUNCHED();
-        bin_scan_kernel<<<1, 256, 0, c->stream>>>(groups, P.d_part, out, tail);
+        bin_scan_kernel<<<1, 1024, 0, c->stream>>>(groups, P.d_part, out, tail);
         LAL_LAUNCHED();
         int got[nb + 1];
         LAL_TRY(lal::read_ints(c, out, nb + 1, got, false));
@@ -1019,21 +1030,24 @@ namespace lal
     {
         temps tmp(c, a);
         LAL_HIP(hipMemsetAsync(trp, 0, sizeof(int) * (n + 1), c->stream));
+        int* place = nullptr;
         if(nnz > 0)
         {
-            col_count_kernel<<<grid_for(nnz, 256), 256, 0, c->stream>>>(nnz, ci, trp);
+            LAL_TRY(tmp.get(&place, nnz));
+            col_count_kernel<<<grid_for(nnz, 256), 256, 0, c->stream>>>(nnz, ci, trp, place);
             LAL_LAUNCHED();
         }
         LAL_TRY(scan_i32_dev(c, n + 1, trp, a));
         if(nnz == 0)
             return LAL_OK;
-        int* cursor = nullptr;
-        LAL_TRY(tmp.get(&cursor, n));
-        LAL_HIP(hipMemcpyAsync(cursor, trp, sizeof(int) * n, hipMemcpyDeviceToDevice, c->stream));
-        transpose_scatter_kernel<T><<<grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, v,
-                                                                             cursor, tci, tv);
+        transpose_scatter_kernel<T><<<grid_for(m, 64), 256, 0, c->stream>>>(m, rp, ci, v, trp,
+                                                                            place, tci, tv);
         LAL_LAUNCHED();
-        row_sort_wave_kernel<T><<<(n + 3) / 4, 256, 0, c->stream>>>(n, trp, tci, tv);
+        // rows of up to 12 entries on average: 16 lanes, else a wavefront
+        if(nnz <= 12L * n)
+            row_sort_kernel<16, T><<<(n + 15) / 16, 256, 0, c->stream>>>(n, trp, tci, tv);
+        else
+            row_sort_kernel<64, T><<<(n + 3) / 4, 256, 0, c->stream>>>(n, trp, tci, tv);
         LAL_LAUNCHED();
         return LAL_OK;
     }
