@@ -80,6 +80,11 @@ namespace lal
     struct level_t
     {
         csr_dev      A, P, R;
+        // Q = P - D^-1 A P on the pattern of A P (fast path): prolongation and
+        // the first post-sweep in one operator.  With r = b - A x and
+        // y = x + D^-1 r already at hand, the sweep after x + P e is
+        // x + P e + D^-1 (b - A (x + P e)) = y + Q e.
+        csr_dev      Q;
         work<double> w64;
         work<float>  w32;
         gs_sched     gs_fwd, gs_bwd;
@@ -172,7 +177,7 @@ struct lal_hierarchy_t
                 (void)hipGraphExecDestroy(g.exec);
         for(int l = 0; l <= 20; l++)
         {
-            for(lal::csr_dev* M : {&L[l].A, &L[l].P, &L[l].R})
+            for(lal::csr_dev* M : {&L[l].A, &L[l].P, &L[l].R, &L[l].Q})
                 lal_csrmv_descr_destroy(M->d);
             for(lal::gs_sched* g : {&L[l].gs_fwd, &L[l].gs_bwd})
                 for(void* ptr : {(void*)g->perm, (void*)g->off_d, (void*)g->prp, (void*)g->pci,

@@ -281,8 +281,8 @@ namespace
         // nonzero less, same results.
         std::vector<lal::rb_request> req;
         for(int l = 0; l <= h->levels; l++)
-            for(csr_dev* A : {&h->L[l].A, &h->L[l].P, &h->L[l].R})
-                if(A->d == nullptr && (A == &h->L[l].A || l < h->levels))
+            for(csr_dev* A : {&h->L[l].A, &h->L[l].P, &h->L[l].R, &h->L[l].Q})
+                if(A->d == nullptr && (A == &h->L[l].A || (l < h->levels && A->rp)))
                     req.push_back({descr(*A, A->m, A->nnz, A->n, exact), A->rp, A->ci, A->m,
                                    A->nnz, exact == 0, -1});
         LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
@@ -303,11 +303,16 @@ namespace
             LAL_TRY(h->mem.get(&L.w64.dinv, L.A.m));
             LAL_TRY(lal::diag_inv<double>(c, L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag,
                                           L.w64.dinv, L.A.nnz));
+            if(L.Q.rp && l < h->levels)
+                LAL_TRY(lal::smoothed_prolongator(c, L.Q.m, L.Q.nnz, L.Q.rp, L.Q.ci, L.Q.v, L.P.rp,
+                                                  L.P.ci, L.P.v, L.w64.dinv));
             if(h->opts.build_f32)
             {
                 LAL_TRY(to_f32(h, L.A.v, &L.A.v32, L.A.nnz));
                 if(l < h->levels)
                 {
+                    if(L.Q.rp)
+                        LAL_TRY(to_f32(h, L.Q.v, &L.Q.v32, L.Q.nnz));
                     LAL_TRY(to_f32(h, L.P.v, &L.P.v32, L.P.nnz));
                     LAL_TRY(to_f32(h, L.R.v, &L.R.v32, L.R.nnz));
                 }
@@ -485,12 +490,14 @@ namespace
             LAL_TRY(h->mem.get(&R.v, nnzP));
             LAL_TRY(lal::transpose_f64(c, P.m, P.n, P.nnz, P.rp, P.ci, P.v, R.rp, R.ci, R.v,
                                        &tmp));
-            // AP = A P
-            csr_dev AP;
-            AP.m = Af.m;
-            AP.n = nc;
+            // AP = A P (the fast path makes Q of it)
+            csr_dev  ap_tmp;
+            csr_dev& AP = o.exact ? ap_tmp : h->L[level].Q;
+            AP.m        = Af.m;
+            AP.n        = nc;
             LAL_TRY(lal::product(c, Af.m, Af.n, nc, Af.nnz, Af.rp, Af.ci, Af.v, P.nnz, P.rp,
-                                 P.ci, P.v, &AP.rp, &AP.ci, &AP.v, &AP.nnz, &tmp, &tmp));
+                                 P.ci, P.v, &AP.rp, &AP.ci, &AP.v, &AP.nnz,
+                                 o.exact ? &tmp : &h->mem, &tmp));
             // A_c = R (A P)
             Ac.m = nc;
             Ac.n = nc;
@@ -543,6 +550,9 @@ namespace
         }
         T* cur   = W.x;
         T* other = W.t;
+        // one pre-sweep and a post-sweep: the residual pass also leaves
+        // y = x + r / a_ii in W.t, and the way up is y + Q e
+        const bool merged = fast && n2 >= 1 && L.Q.rp;
         if(n1 == 0)
         {
             // x = 0 and r = b - A*0, which is b bit for bit
@@ -553,7 +563,11 @@ namespace
         {
             if(!xinit)
                 LAL_TRY(lal::mul_elem<T>(c, A.m, b, W.dinv, cur));
-            LAL_TRY(residual_t<T>(c, A, Av, cur, b, W.r));
+            if(merged)
+                LAL_TRY(lal::residual_smoothed<T>(c, A.d, A.m, A.rp, A.ci, Av, cur, W.dinv, b, W.r,
+                                                  other));
+            else
+                LAL_TRY(residual_t<T>(c, A, Av, cur, b, W.r));
         }
         else
         {
@@ -581,10 +595,24 @@ namespace
                                Wc.b));
         T* ec = nullptr;
         LAL_TRY(vcycle<T>(h, l + 1, Wc.b, nullptr, n1, n2, fast, &ec));
-        // prolongation and correction: x += P ec
-        const csr_dev& P = L.P;
-        LAL_TRY(lal::csrmv(c, P.d, P.m, P.n, P.nnz, 1.0, P.rp, P.ci, vals<T>(P), ec, 1.0, cur));
-        for(int k = 0; k < n2; k++)
+        int done = 0; // post-sweeps behind us
+        if(merged)
+        {
+            // other = y; the result may go straight to dst
+            T* o = n2 == 1 && dst ? dst : cur;
+            LAL_TRY(lal::add_product<T>(c, L.Q.d, L.Q.m, L.Q.rp, L.Q.ci, vals<T>(L.Q), ec, other,
+                                        o));
+            cur  = o;
+            done = 1;
+        }
+        else
+        {
+            // prolongation and correction: x += P ec
+            const csr_dev& P = L.P;
+            LAL_TRY(lal::csrmv(c, P.d, P.m, P.n, P.nnz, 1.0, P.rp, P.ci, vals<T>(P), ec, 1.0,
+                               cur));
+        }
+        for(int k = done; k < n2; k++)
         {
             T* o = (k == n2 - 1 && dst) ? dst : other;
             LAL_TRY(lal::jacobi_sweep<T>(c, A.d, A.m, A.rp, A.ci, Av, W.diag, W.dinv, cur, b,

@@ -29,6 +29,9 @@
 //                                           fused with the residual)
 //   RESTRICT  y = A x and r = y * dinv     (restriction that also writes the
 //                                           coarse level's first sweep)
+//   SMOOTHED  y = b - A x and r = x + y * dinv  (residual, and the sweep that
+//                                           uses it)
+//   ADD       y = b + A x
 // dinv holds 1/a_ii, so no division is left in the inner loops.
 #pragma once
 
@@ -42,8 +45,10 @@ namespace lal
         RV_RESIDUAL = 1,
         RV_JACOBI   = 2,
         RV_JACOBI0  = 3,
-        RV_RESTRICT = 4 // y = A x and r = y * dinv: the coarse right-hand side
-                        // and the first Jacobi iterate from zero on it
+        RV_RESTRICT = 4, // y = A x and r = y * dinv: the coarse right-hand side
+                         // and the first Jacobi iterate from zero on it
+        RV_SMOOTHED = 5,
+        RV_ADD      = 6
     };
 
     struct rv_args

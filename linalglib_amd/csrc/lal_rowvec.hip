@@ -74,6 +74,69 @@ namespace
         return x[c];
     }
 
+    // What a row's epilogue reads besides its sum.  The staged kernels load it
+    // with the block's first window, so that the row sums end in a store and
+    // not in one more memory round trip.
+    template <typename T>
+    struct row_operands
+    {
+        T b = 0, d = 0, x = 0, y = 0;
+    };
+
+    template <typename T, int MODE>
+    __device__ __forceinline__ row_operands<T> load_operands(bool on, int row,
+                                                             const T* __restrict__ x,
+                                                             const T* __restrict__ d,
+                                                             const T* __restrict__ b, T beta,
+                                                             const T* __restrict__ y)
+    {
+        row_operands<T> o;
+        if(!on)
+            return o;
+        if(MODE == lal::RV_RESIDUAL || MODE == lal::RV_JACOBI || MODE == lal::RV_JACOBI0 ||
+           MODE == lal::RV_SMOOTHED || MODE == lal::RV_ADD)
+            o.b = b[row];
+        if(MODE == lal::RV_JACOBI || MODE == lal::RV_JACOBI0 || MODE == lal::RV_RESTRICT ||
+           MODE == lal::RV_SMOOTHED)
+            o.d = d[row];
+        if(MODE == lal::RV_JACOBI || MODE == lal::RV_SMOOTHED)
+            o.x = x[row];
+        if(MODE == lal::RV_SPMV && beta != (T)0)
+            o.y = y[row];
+        return o;
+    }
+
+    // y (and r) of one row from its sum acc = (A u)_row, per operation.
+    template <typename T, int MODE>
+    __device__ __forceinline__ void row_epilogue(int row, T acc, const row_operands<T>& o, T alpha,
+                                                 T beta, T* __restrict__ y, T* __restrict__ r)
+    {
+        if(MODE == lal::RV_SPMV)
+            y[row] = beta == (T)0 ? alpha * acc : fma(alpha, acc, beta * o.y);
+        else if(MODE == lal::RV_RESTRICT)
+        {
+            y[row] = acc;
+            r[row] = acc * o.d;
+        }
+        else if(MODE == lal::RV_RESIDUAL)
+            y[row] = o.b - acc;
+        else if(MODE == lal::RV_JACOBI)
+            y[row] = o.x + (o.b - acc) * o.d;
+        else if(MODE == lal::RV_SMOOTHED)
+        {
+            const T res = o.b - acc;
+            y[row]      = res;
+            r[row]      = o.x + res * o.d;
+        }
+        else if(MODE == lal::RV_ADD)
+            y[row] = o.b + acc;
+        else
+        {
+            y[row] = o.b * o.d;
+            r[row] = o.b - acc;
+        }
+    }
+
     template <typename T, int MODE>
     __global__ void __launch_bounds__(SPMV_THREADS)
         staged_kernel(int m, const int* __restrict__ blocks, int nb, const int* __restrict__ rp,
@@ -140,49 +203,8 @@ namespace
             acc = lal::group_sum(acc, g);
         if(!active || lig != 0)
             return;
-        if(MODE == lal::RV_SPMV)
-            y[row] = beta == (T)0 ? alpha * acc : fma(alpha, acc, beta * y[row]);
-        else if(MODE == lal::RV_RESTRICT)
-        {
-            y[row] = acc;
-            r[row] = acc * d[row];
-        }
-        else if(MODE == lal::RV_RESIDUAL)
-            y[row] = b[row] - acc;
-        else if(MODE == lal::RV_JACOBI)
-            y[row] = x[row] + (b[row] - acc) * d[row];
-        else
-        {
-            const T bi = b[row];
-            y[row]     = bi * d[row];
-            r[row]     = bi - acc;
-        }
-    }
-
-    // y (and r) of one row from its sum acc = (A u)_row, per operation.
-    template <typename T, int MODE>
-    __device__ __forceinline__ void row_epilogue(int row, T acc, const T* __restrict__ x,
-                                                 const T* __restrict__ d,
-                                                 const T* __restrict__ b, T alpha, T beta,
-                                                 T* __restrict__ y, T* __restrict__ r)
-    {
-        if(MODE == lal::RV_SPMV)
-            y[row] = beta == (T)0 ? alpha * acc : fma(alpha, acc, beta * y[row]);
-        else if(MODE == lal::RV_RESTRICT)
-        {
-            y[row] = acc;
-            r[row] = acc * d[row];
-        }
-        else if(MODE == lal::RV_RESIDUAL)
-            y[row] = b[row] - acc;
-        else if(MODE == lal::RV_JACOBI)
-            y[row] = x[row] + (b[row] - acc) * d[row];
-        else
-        {
-            const T bi = b[row];
-            y[row]     = bi * d[row];
-            r[row]     = bi - acc;
-        }
+        row_epilogue<T, MODE>(row, acc, load_operands<T, MODE>(true, row, x, d, b, beta, y), alpha,
+                              beta, y, r);
     }
 
     // Row sum over the staged nonzeros [j, e) (stride g): UR column indices
@@ -287,6 +309,8 @@ namespace
         // instead of being awaited before them: rp[r0] and rp[r1] are the
         // descriptor's base and end, lane i loads rp[r0 + i] for 0 < i < nrows.
         const int rpv = (tid > 0 && tid < nrows) ? rp[r0 + tid] : 0;
+        const row_operands<T> ops =
+            load_operands<T, MODE>(active && lig == 0, row, x, d, b, beta, y);
         int       rs = 0, re = 0;
         bool      bounds = false;
 
@@ -356,7 +380,7 @@ namespace
             acc = lal::group_sum(acc, g);
         if(!active || lig != 0)
             return;
-        row_epilogue<T, MODE>(row, acc, x, d, b, alpha, beta, y, r);
+        row_epilogue<T, MODE>(row, acc, ops, alpha, beta, y, r);
     }
 
     // Quad-staged kernel that gathers by nonzero (16-byte aligned ci and val):
@@ -395,6 +419,8 @@ namespace
         const int  cb     = C16 ? cbase[tile] : 0; // this block's 16-bit column base
         // row bounds through LDS, loaded with the first window (quad_kernel)
         const int rpv = (tid > 0 && tid < nrows) ? rp[r0 + tid] : 0;
+        const row_operands<T> ops =
+            load_operands<T, MODE>(active && lig == 0, row, x, d, b, beta, y);
         int       rs = 0, re = 0;
         bool      bounds = false;
 
@@ -476,7 +502,7 @@ namespace
             acc = lal::group_sum(acc, g);
         if(!active || lig != 0)
             return;
-        row_epilogue<T, MODE>(row, acc, x, d, b, alpha, beta, y, r);
+        row_epilogue<T, MODE>(row, acc, ops, alpha, beta, y, r);
     }
 
     template <typename T, int MODE, bool C16>
@@ -539,6 +565,8 @@ namespace lal
         case RV_RESTRICT: return launch<T, RV_RESTRICT>(c, a);
         case RV_RESIDUAL: return launch<T, RV_RESIDUAL>(c, a);
         case RV_JACOBI: return launch<T, RV_JACOBI>(c, a);
+        case RV_SMOOTHED: return launch<T, RV_SMOOTHED>(c, a);
+        case RV_ADD: return launch<T, RV_ADD>(c, a);
         default: return launch<T, RV_JACOBI0>(c, a);
         }
     }

@@ -53,6 +53,21 @@ namespace lal
     int jacobi_sweep(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                      const int* ci, const T* v, const T* diag, const T* dinv, const T* xold,
                      const T* b, T* xnew);
+    // r = b - A x and y = x + r / a_ii: the residual a V-cycle restricts and
+    // the Jacobi sweep that its post-smoothing builds on (fast descriptors).
+    template <typename T>
+    int residual_smoothed(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
+                          const int* ci, const T* v, const T* x, const T* dinv, const T* b, T* r,
+                          T* y);
+    // out = y + Q e (fast descriptors)
+    template <typename T>
+    int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
+                    const T* v, const T* e, const T* y, T* out);
+    // AP's values become those of Q = P - D^-1 A P (pattern of A P, a superset
+    // of P's; both with ascending columns).
+    int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
+                             double* v, const int* prp, const int* pci, const double* pv,
+                             const double* dinv);
     template <typename T>
     int jacobi0_residual(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                          const int* ci, const T* v, const T* diag, const T* dinv, const T* b,

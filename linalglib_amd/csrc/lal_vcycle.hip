@@ -439,6 +439,35 @@ namespace
             p[i] = beta == (T)0 ? (T)z[i] : (T)z[i] + beta * p[i];
     }
 
+    // One lane group per row: entry (i, c) of A P becomes P(i, c) - dinv_i (A P)(i, c).
+    __global__ void __launch_bounds__(256)
+        smoothed_prolongator_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
+                                    double* __restrict__ v, const int* __restrict__ prp,
+                                    const int* __restrict__ pci, const double* __restrict__ pv,
+                                    const double* __restrict__ dinv)
+    {
+        const int i = blockIdx.x * 16 + (int)(threadIdx.x >> 4);
+        if(i >= m)
+            return;
+        const double di = dinv[i];
+        const int    ps = prp[i], pe = prp[i + 1];
+        for(int j = rp[i] + (int)(threadIdx.x & 15); j < rp[i + 1]; j += 16)
+        {
+            const int c  = ci[j];
+            int       lo = ps, hi = pe; // first entry of P's row at or after c
+            while(lo < hi)
+            {
+                const int mid = (lo + hi) >> 1;
+                if(pci[mid] < c)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            const double p = lo < pe && pci[lo] == c ? pv[lo] : 0.0;
+            v[j]           = p - di * v[j];
+        }
+    }
+
     // x = b * dinv (first Jacobi iterate from zero)
     template <typename T>
     __global__ void __launch_bounds__(256)
@@ -504,6 +533,44 @@ namespace lal
             1); // no fast descriptor: one lane per row
         LAL_LAUNCHED();
         (void)diag;
+        return LAL_OK;
+    }
+
+    template <typename T>
+    int residual_smoothed(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
+                          const int* ci, const T* v, const T* x, const T* dinv, const T* b, T* r,
+                          T* y)
+    {
+        if(m == 0)
+            return LAL_OK;
+        rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, x, dinv, b, r, y, 0.0,
+                  0.0, d->win};
+        lal::use_c16(a, d);
+        a.keep = d->keep;
+        return rowvec_launch<T>(c, RV_SMOOTHED, a);
+    }
+
+    template <typename T>
+    int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
+                    const T* v, const T* e, const T* y, T* out)
+    {
+        if(m == 0)
+            return LAL_OK;
+        rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, e, nullptr, y, out,
+                  nullptr, 0.0, 0.0, d->win};
+        lal::use_c16(a, d);
+        return rowvec_launch<T>(c, RV_ADD, a);
+    }
+
+    int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
+                             double* v, const int* prp, const int* pci, const double* pv,
+                             const double* dinv)
+    {
+        if(m == 0 || nnz == 0)
+            return LAL_OK;
+        smoothed_prolongator_kernel<<<grid_for(m, 16), 256, 0, c->stream>>>(m, rp, ci, v, prp,
+                                                                            pci, pv, dinv);
+        LAL_LAUNCHED();
         return LAL_OK;
     }
 
@@ -681,6 +748,11 @@ namespace lal
     template int jacobi0_residual<T>(lal_context*, const lal_csrmv_info*, int, const int*,   \
                                      const int*, const T*, const T*, const T*, const T*, T*, \
                                      T*);                                                    \
+    template int residual_smoothed<T>(lal_context*, const lal_csrmv_info*, int, const int*,  \
+                                      const int*, const T*, const T*, const T*, const T*,    \
+                                      T*, T*);                                               \
+    template int add_product<T>(lal_context*, const lal_csrmv_info*, int, const int*,        \
+                                const int*, const T*, const T*, const T*, T*);               \
     template int diag_inv<T>(lal_context*, int, const int*, const int*, const T*, T*, T*,   \
                              long);                                                          \
     template int coarse_scalar<T>(lal_context*, const T*, const T*, T*);                     \
