@@ -123,6 +123,7 @@ namespace
     // LDS (a binary search in the staged row pointer) and one lane follows
     // them.  Several operators share a launch (a hierarchy analyses all of its
     // own at once, without a copy of a row pointer to the host).
+    constexpr int LIST_CAP = 2044; // nonzeros of a block with a column list
     constexpr int RB_TILE  = 2048;
     constexpr int RB_BATCH = 24; // operators per launch (their table is a kernel argument)
 
@@ -139,7 +140,10 @@ namespace
         RB_WIN     = 1, // widest 4-aligned nonzero window of a block (<= 2052)
         RB_BAD     = 2, // 1: row pointer not from 0 to nnz, 2: not monotone, 4: column range
         RB_WIDE    = 3, // a block spans more than 65535 columns
-        RB_RES     = 4
+        RB_LMAX    = 4, // longest list of distinct columns of a block
+        RB_LONG    = 5, // a block of more than LIST_CAP nonzeros (one long row) or 131072 columns
+        RB_FAR     = 6, // a list reaches beyond 65536 columns
+        RB_RES     = 7
     };
 
     // Position of `at` among the operators' starts (ascending).
@@ -281,10 +285,15 @@ namespace
     // One workgroup per row block (the grid holds every operator's largest
     // possible number of blocks): the block's column range, its base (the
     // smallest column) and every entry's offset from it as 16 bits; RB_WIDE is
-    // set when a block spans more than 65535 columns.
+    // set when a block spans more than 65535 columns.  Where asked for, also the
+    // block's distinct columns: a bitmap of the span in LDS, whose running
+    // population count is each column's place in the ascending list.
     __global__ void __launch_bounds__(256)
         rb_columns_kernel(rb_table tab, int* __restrict__ res)
     {
+        __shared__ unsigned s_bits[4096];
+        __shared__ int      s_place[4096];
+        __shared__ int      s_w[4];
         typedef int int4v __attribute__((ext_vector_type(4)));
         __shared__ int sh_mn[4], sh_mx[4];
         const int k  = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.blk0; });
@@ -326,6 +335,82 @@ namespace
         }
         for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
             o.c16[e] = (unsigned short)(o.ci[e] - base);
+        if(o.lpos == nullptr)
+            return;
+        if(e1 - e0 > LIST_CAP || (e1 > e0 && (long long)mx - mn > 131071))
+        {
+            if(threadIdx.x == 0)
+                atomicOr(out + RB_LONG, 1);
+            return;
+        }
+        const int words = e1 > e0 ? (mx - base) / 32 + 1 : 0; // at most 4096
+        for(int w = (int)threadIdx.x; w < words; w += 256)
+            s_bits[w] = 0;
+        __syncthreads();
+        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
+        {
+            const int off = o.ci[e] - base;
+            atomicOr(&s_bits[off >> 5], 1u << (off & 31));
+        }
+        __syncthreads();
+        unsigned short* list = o.list + lal::list_start(e0, b);
+        const int lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
+        int       carry = 0;
+        for(int w0 = 0; w0 < words; w0 += 256)
+        {
+            const int w   = w0 + (int)threadIdx.x;
+            const int n   = w < words ? __popc(s_bits[w]) : 0;
+            int       inc = n;
+#pragma unroll
+            for(int d = 1; d < 64; d <<= 1)
+            {
+                const int q = __shfl_up(inc, d, 64);
+                inc += lane >= d ? q : 0;
+            }
+            if(lane == 63)
+                s_w[wid] = inc;
+            __syncthreads();
+            int at = carry + inc - n, tot = 0;
+            for(int k2 = 0; k2 < 4; k2++)
+            {
+                at += k2 < wid ? s_w[k2] : 0;
+                tot += s_w[k2];
+            }
+            if(w < words)
+            {
+                s_place[w]    = at;
+                unsigned bits = s_bits[w];
+                while(bits)
+                {
+                    const int t = __ffs((int)bits) - 1;
+                    bits &= bits - 1;
+                    list[at++] = (unsigned short)(w * 32 + t);
+                }
+            }
+            carry += tot;
+            __syncthreads();
+        }
+        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
+        {
+            const int      off  = o.ci[e] - base;
+            const unsigned less = s_bits[off >> 5] & ((1u << (off & 31)) - 1u);
+            o.lpos[e]           = (unsigned short)(4 * (s_place[off >> 5] + __popc(less)));
+        }
+        // the last quad is read whole
+        if(b == nb - 1 && threadIdx.x < (unsigned)(-o.nnz & 3))
+            o.lpos[o.nnz + (int)threadIdx.x] = 0;
+        if(threadIdx.x == 0)
+        {
+            if(carry & 1)
+                list[carry] = (unsigned short)(mx - base); // (its low 16 bits)
+            // (words from 2048 on start the offsets of 65536 and more)
+            const int split = words > 2048 ? s_place[2048] : carry;
+            o.lmeta[2 * b]  = carry | split << 12 | lal::spmv_group_log(mt.y - mt.x) << 24;
+            o.lmeta[2 * b + 1] = base;
+            atomicMax(out + RB_LMAX, carry);
+            if(split < carry)
+                atomicOr(out + RB_FAR, 1);
+        }
     }
 
     template <typename T, typename ACC, int MODE>
@@ -397,7 +482,8 @@ namespace lal
                 o.ci     = q.ci;
                 o.m      = q.m;
                 o.nnz    = q.nnz;
-                o.cap    = block_cap(q.nnz);
+                // (the list kernel takes a block as 512 quads of four)
+                o.cap    = std::min(block_cap(q.nnz), q.want_list ? LIST_CAP : INT_MAX);
                 o.tile0  = tiles;
                 o.ntiles = std::max((q.m + RB_TILE - 1) / RB_TILE, 1);
                 o.blk0   = blocks;
@@ -415,6 +501,15 @@ namespace lal
                     LAL_TRY(mem->get(&q.d->d_cbase, o.ub));
                     o.c16   = q.d->d_c16;
                     o.cbase = q.d->d_cbase;
+                    if(q.want_list)
+                    {
+                        LAL_TRY(mem->get(&q.d->d_lpos, ((size_t)q.nnz + 7) & ~(size_t)7));
+                        LAL_TRY(mem->get(&q.d->d_list, list_start(q.nnz, o.ub) + 4));
+                        LAL_TRY(mem->get(&q.d->d_lmeta, 2 * (size_t)o.ub));
+                        o.lpos  = q.d->d_lpos;
+                        o.list  = q.d->d_list;
+                        o.lmeta = q.d->d_lmeta;
+                    }
                 }
             }
             int *tcount = nullptr, *res = nullptr;
@@ -458,6 +553,11 @@ namespace lal
                     q.d->win     = std::max(r[RB_WIN], 4);
                     if(r[RB_WIDE])
                         q.d->d_c16 = nullptr;
+                    if(q.d->d_lpos && !r[RB_LONG])
+                    {
+                        q.d->list_max = r[RB_LMAX];
+                        q.d->list_far = r[RB_FAR] != 0;
+                    }
                     continue;
                 }
                 return LAL_ERR_INVALID;

@@ -284,7 +284,8 @@ namespace
             for(csr_dev* A : {&h->L[l].A, &h->L[l].P, &h->L[l].R, &h->L[l].Q})
                 if(A->d == nullptr && (A == &h->L[l].A || (l < h->levels && A->rp)))
                     req.push_back({descr(*A, A->m, A->nnz, A->n, exact), A->rp, A->ci, A->m,
-                                   A->nnz, exact == 0, -1});
+                                   A->nnz, exact == 0, -1,
+                                   A == &h->L[l].Q || A == &h->L[l].A || A == &h->L[l].R});
         LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
         for(int l = 0; l <= h->levels; l++)
         {

@@ -73,13 +73,24 @@ namespace lal
         // 16-bit columns and their per-block bases (lal_csrmv_info::d_c16), or null
         const unsigned short* c16   = nullptr;
         const int*            cbase = nullptr;
+        // column lists (lal_csrmv_info::d_list), list_max 0: none
+        const unsigned short* lpos     = nullptr;
+        const unsigned short* list     = nullptr;
+        const int*            lmeta    = nullptr;
+        int                   list_max = 0;
+        bool                  list_far = false;
     };
 
-    // The descriptor's 16-bit columns into a's fields.
+    // The descriptor's 16-bit columns and column lists into a's fields.
     inline void use_c16(rv_args& a, const lal_csrmv_info* d)
     {
-        a.c16   = d->d_c16;
-        a.cbase = d->d_cbase;
+        a.c16      = d->d_c16;
+        a.cbase    = d->d_cbase;
+        a.lpos     = d->d_lpos;
+        a.list     = d->d_list;
+        a.lmeta    = d->d_lmeta;
+        a.list_max = d->list_max;
+        a.list_far = d->list_far;
     }
 
     template <typename T>

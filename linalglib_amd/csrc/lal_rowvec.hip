@@ -153,8 +153,9 @@ namespace
         int       r0, r1;
         lal::block_rows(blocks, m, tile, &r0, &r1);
         const int  nrows  = r1 - r0;
-        const int  g      = lal::spmv_group(nrows, 0);
-        const int  lrow   = tid / g;
+        const int  lg     = lal::spmv_group_log(nrows);
+        const int  g      = 1 << lg;
+        const int  lrow   = tid >> lg;
         const int  lig    = tid & (g - 1);
         const bool active = lrow < nrows;
         const int  row    = r0 + lrow;
@@ -296,8 +297,9 @@ namespace
         const int4v mt   = reinterpret_cast<const int4v*>(blocks + lal::block_meta_offset(nb))[tile];
         const int   r0 = mt.x, r1 = mt.y;
         const int  nrows  = r1 - r0;
-        const int  g      = lal::spmv_group(nrows, 0);
-        const int  lrow   = tid / g;
+        const int  lg     = lal::spmv_group_log(nrows);
+        const int  g      = 1 << lg;
+        const int  lrow   = tid >> lg;
         const int  lig    = tid & (g - 1);
         const bool active = lrow < nrows;
         const int  row    = r0 + lrow;
@@ -408,8 +410,9 @@ namespace
         const int4v mt   = reinterpret_cast<const int4v*>(blocks + lal::block_meta_offset(nb))[tile];
         const int   r0 = mt.x, r1 = mt.y;
         const int  nrows  = r1 - r0;
-        const int  g      = lal::spmv_group(nrows, 0);
-        const int  lrow   = tid / g;
+        const int  lg     = lal::spmv_group_log(nrows);
+        const int  g      = 1 << lg;
+        const int  lrow   = tid >> lg;
         const int  lig    = tid & (g - 1);
         const bool active = lrow < nrows;
         const int  row    = r0 + lrow;
@@ -505,6 +508,183 @@ namespace
         row_epilogue<T, MODE>(row, acc, ops, alpha, beta, y, r);
     }
 
+    // Sum of the staged products s_p[j], s_p[j + g], ... below e, four reads
+    // in flight.
+    template <typename T>
+    __device__ __forceinline__ T product_sum(const T* s_p, int j, int e, int g)
+    {
+        T acc = 0;
+        if(g == 1) // (uniform) constant offsets
+        {
+            for(; j + 3 < e; j += 4)
+            {
+                const T p0 = s_p[j], p1 = s_p[j + 1], p2 = s_p[j + 2], p3 = s_p[j + 3];
+                acc += p0;
+                acc += p1;
+                acc += p2;
+                acc += p3;
+            }
+            for(; j < e; j++)
+                acc += s_p[j];
+            return acc;
+        }
+        for(; j + 3 * g < e; j += 4 * g)
+        {
+            const T p0 = s_p[j], p1 = s_p[j + g], p2 = s_p[j + 2 * g], p3 = s_p[j + 3 * g];
+            acc += p0;
+            acc += p1;
+            acc += p2;
+            acc += p3;
+        }
+        for(; j < e; j += g)
+            acc += s_p[j];
+        return acc;
+    }
+
+    // p[i] with a 32-bit byte offset from a uniform base
+    template <typename V, typename T>
+    __device__ __forceinline__ V load_at(const T* p, unsigned byte)
+    {
+        return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + byte);
+    }
+    template <typename V, typename T>
+    __device__ __forceinline__ V stream_at(const T* p, unsigned byte)
+    {
+        return __builtin_nontemporal_load(
+            reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + byte));
+    }
+
+    // Row sums with x gathered through LDS, for operators whose blocks name
+    // each column several times (a hierarchy's long-row operators).
+    //
+    // A gather of 64 scattered entries keeps the L1 busy for 34-38 clocks, one
+    // of consecutive lanes' neighbouring entries for 5 (FP32) or 16 (FP64).  So
+    // the block gathers its distinct columns once, in ascending order, into
+    // LDS, while its values and the nonzeros' places in that list are on their
+    // way; the lanes then form the products of the quads they loaded out of
+    // LDS, and the rows sum theirs.  The instructions are what is left to pay
+    // (30 vector instructions per nonzero of a lane kept the SIMDs busy for
+    // half of the time): addresses are 32-bit offsets from the block's
+    // uniform bases, places are stored as byte offsets, lane groups are
+    // shifts.  Blocks hold at most 2044 nonzeros, 512 quads, so one window of two
+    // quads per lane always does.
+    // The lists are read two entries per lane: loads of 16 bits per lane cost as
+    // much as scattered ones (128^3 level 1 in FP32: 31 us with them, 26 with
+    // pairs).
+    constexpr int LIST_U = 4; // list pairs per lane: a list has at most 2044 entries
+
+    //
+    // FAR: some block's columns span more than 65536 (the finest restriction
+    // of a large grid), and its list's entries from `split` on are 65536 further.
+    template <typename T, int MODE, bool FAR>
+    __global__ void __launch_bounds__(SPMV_THREADS)
+        list_kernel(const int* __restrict__ blocks, int nb, int list_max,
+                    const int* __restrict__ rp, const unsigned short* __restrict__ lpos,
+                    const unsigned short* __restrict__ list, const int* __restrict__ lmeta,
+                    const T* __restrict__ val, const T* __restrict__ x, const T* __restrict__ d,
+                    const T* __restrict__ b, T alpha, T beta, T* __restrict__ y,
+                    T* __restrict__ r)
+    {
+        typedef int int2v __attribute__((ext_vector_type(2)));
+        // the block's row starts, its x entries, then its products
+        extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
+        int* s_rp = reinterpret_cast<int*>(s_raw);
+        T*   s_x  = reinterpret_cast<T*>(s_raw + RP_LDS_BYTES);
+        T*   s_p  = s_x + list_max; // list_max: a multiple of 4
+
+        const unsigned tid  = threadIdx.x;
+        const int      tile = lal::xcd_tile(blockIdx.x, nb);
+        const int4v mt = reinterpret_cast<const int4v*>(blocks + lal::block_meta_offset(nb))[tile];
+        const int2v lm = reinterpret_cast<const int2v*>(lmeta)[tile];
+        const int   r0 = mt.x, nrows = mt.y - mt.x, base = mt.z, end = mt.w;
+        const unsigned len   = (unsigned)lm.x & 0xfffu;
+        const unsigned split = (unsigned)lm.x >> 12 & 0xfffu; // entries from here on: 65536 further
+        const int      lg    = lm.x >> 24;                    // log2 of the lanes per row
+        const int      ws  = base & ~3;
+        const unsigned nq  = (unsigned)(end - ws + 3) >> 2;
+        const T*              xb = x + lm.y;
+        const T*              vb = val + ws;
+        const unsigned short* pb = lpos + ws;
+        const unsigned short* lb = list + lal::list_start(base, tile);
+        const unsigned        np = (len + 1) >> 1; // list pairs
+
+        unsigned lo[LIST_U];
+#pragma unroll
+        for(int u = 0; u < LIST_U; u++)
+            if(SPMV_THREADS * u < np) // (uniform)
+                lo[u] = stream_at<unsigned>(lb, 4u * min(tid + SPMV_THREADS * u, np - 1));
+        us4v    pq[2];
+        quad<T> vq[2];
+#pragma unroll
+        for(int u = 0; u < 2; u++)
+            if(SPMV_THREADS * u < nq) // (uniform)
+            {
+                const unsigned q = min(tid + SPMV_THREADS * u, nq - 1);
+                pq[u]            = stream_at<us4v>(pb, 8u * q);
+                vq[u].load(reinterpret_cast<const T*>(reinterpret_cast<const char*>(vb) +
+                                                      4u * sizeof(T) * q));
+            }
+        const int  lrow = (int)tid >> lg;
+        const bool on   = lrow < nrows;
+        const bool head = on && (tid & ((1u << lg) - 1u)) == 0;
+        const int  rpv  = rp[r0 + min((int)tid, nrows)];
+        const row_operands<T> ops = load_operands<T, MODE>(head, r0 + lrow, x, d, b, beta, y);
+        // (a list of odd length repeats its last column once more)
+        T xv[LIST_U][2];
+#pragma unroll
+        for(int u = 0; u < LIST_U; u++)
+            if(SPMV_THREADS * u < np)
+            {
+                unsigned o0 = lo[u] & 0xffffu, o1 = lo[u] >> 16;
+                if(FAR)
+                {
+                    const unsigned i = 2u * min(tid + SPMV_THREADS * u, np - 1);
+                    o0 += i >= split ? 65536u : 0u;
+                    o1 += i + 1 >= split ? 65536u : 0u;
+                }
+                xv[u][0] = load_at<T>(xb, (unsigned)sizeof(T) * o0);
+                xv[u][1] = load_at<T>(xb, (unsigned)sizeof(T) * o1);
+            }
+#pragma unroll
+        for(int u = 0; u < LIST_U; u++)
+            if(SPMV_THREADS * u < np)
+            {
+                T* at = s_x + 2u * min(tid + SPMV_THREADS * u, np - 1);
+                at[0] = xv[u][0];
+                at[1] = xv[u][1];
+            }
+        if((int)tid < nrows)
+            s_rp[tid] = rpv;
+        if(tid == 0)
+            s_rp[nrows] = end;
+        __syncthreads();
+        // (places of a neighbouring block's entries in the window's first and
+        // last quad are below list_max too; their products belong to no row
+        // here)
+#pragma unroll
+        for(int u = 0; u < 2; u++)
+            if(SPMV_THREADS * u < nq)
+            {
+                T v[4], p[4];
+                vq[u].store(v);
+#pragma unroll
+                for(int e = 0; e < 4; e++)
+                    p[e] = v[e] * load_at<T>(s_x, (unsigned)(sizeof(T) / 4) * pq[u][e]);
+                quad<T> out;
+                out.template load<true>(p);
+                out.store(s_p + 4u * min(tid + SPMV_THREADS * u, nq - 1));
+            }
+        __syncthreads();
+        T acc = 0;
+        if(on)
+            acc = product_sum(s_p, s_rp[lrow] - ws + (int)(tid & ((1u << lg) - 1u)),
+                              s_rp[lrow + 1] - ws, 1 << lg);
+        if(lg > 0)
+            acc = lal::group_sum(acc, 1 << lg);
+        if(head)
+            row_epilogue<T, MODE>(r0 + lrow, acc, ops, alpha, beta, y, r);
+    }
+
     template <typename T, int MODE, bool C16>
     void launch_staged(lal_context* c, const lal::rv_args& a, int nb)
     {
@@ -541,6 +721,19 @@ namespace
         if(nb == 0)
             return LAL_OK;
         const bool val16 = (reinterpret_cast<uintptr_t>(a.val) & 15) == 0;
+        if(a.blocks && val16 && a.list_max > 0)
+        {
+            const int    lm  = (a.list_max + 3) & ~3;
+            const size_t lds = RP_LDS_BYTES + sizeof(T) * (size_t)(lm + a.win);
+            auto*        fn  = a.list_far ? list_kernel<T, MODE, true>
+                                          : list_kernel<T, MODE, false>;
+            fn<<<nb, SPMV_THREADS, lds, c->stream>>>(
+                a.blocks, nb, lm, a.rp, a.lpos, a.list, a.lmeta, (const T*)a.val,
+                (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y,
+                (T*)a.r);
+            LAL_LAUNCHED();
+            return LAL_OK;
+        }
         if(a.blocks && val16 && a.c16 && a.cbase)
             launch_staged<T, MODE, true>(c, a, nb);
         else if(a.blocks && val16 && (reinterpret_cast<uintptr_t>(a.ci) & 15) == 0)

@@ -34,6 +34,18 @@ struct lal_csrmv_info
     // columns span more than 65535
     unsigned short* d_c16   = nullptr;
     int*            d_cbase = nullptr;
+    // Gathered x through LDS (operators a hierarchy asks it for): every block's
+    // distinct columns, ascending, as 16-bit offsets from its smallest one from
+    // d_list[lal::list_start()] on (an odd list's last one twice); per nonzero four times its
+    // column's place in that list; per block {list length | first entry whose
+    // offset is 65536 more than stored << 12 | log2 of the lanes per row << 24,
+    // smallest column}.  list_max: the longest list; 0 when not built (a block
+    // spans more than 131,072 columns or holds more than 2044 nonzeros).
+    unsigned short* d_lpos   = nullptr;
+    unsigned short* d_list   = nullptr;
+    int*            d_lmeta  = nullptr;
+    int             list_max = 0;
+    bool            list_far = false; // some offset is 65536 or more
     // room for nb blocks, in the arena or an allocation of its own
     int arrays(lal::arena* mem, int nb);
     bool owned = true; // d_blocks is this descriptor's to free (else, as the
@@ -62,6 +74,7 @@ namespace lal
         int             m, nnz;
         bool            want16;
         int             check_n;
+        bool            want_list = false; // with want16: the blocks' column lists too
     };
     // The same as the analysis kernels see it.
     struct rb_op
@@ -71,6 +84,9 @@ namespace lal
         int*            blocks;
         unsigned short* c16;
         int*            cbase;
+        unsigned short* lpos;
+        unsigned short* list;
+        int*            lmeta;
         int             m, nnz, cap;
         int             tile0, ntiles; // its row tiles
         int             blk0, ub;      // its blocks at most, in the columns' grid
@@ -91,15 +107,26 @@ namespace lal
         static constexpr int value = 2048;
     };
 
-    // Lanes per row for a block of `rows` rows.
+    // log2 of the lanes per row for a block of `rows` rows: the largest power
+    // of two up to 64 with which the rows fill at most SPMV_THREADS lanes, one
+    // from 128 rows on.
+    __device__ __forceinline__ int spmv_group_log(int rows)
+    {
+        const int up = 32 - __clz(rows - 1); // rows <= 2^up (rows 1: clz(0) is 32)
+        return rows >= 128 ? 0 : rows <= 4 ? 6 : 8 - up;
+    }
+
+    // Lanes per row; exact: always one.
     __device__ __forceinline__ int spmv_group(int rows, int exact)
     {
-        if(exact || rows >= 128)
-            return 1;
-        int g = 1;
-        while(g < 64 && 2 * g * rows <= SPMV_THREADS)
-            g <<= 1;
-        return g;
+        return exact ? 1 : 1 << spmv_group_log(rows);
+    }
+
+    // Where a block's column list starts: behind the lists of the blocks
+    // before it, which have no more entries than nonzeros, and 8-byte aligned.
+    __host__ __device__ inline size_t list_start(int base, int block)
+    {
+        return (size_t)(base & ~3) + 4 * (size_t)block;
     }
 
     template <typename T>
