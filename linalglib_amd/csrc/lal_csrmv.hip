@@ -282,84 +282,163 @@ namespace
             res[RB_RES * k + RB_NBLOCKS] = carry;
     }
 
+    // Four 16-bit values for entries e..e+3 (e a multiple of 4) of dst, those in
+    // [e0, e1) only: the quad at either end is shared with the next block.
+    __device__ __forceinline__ void store_quad16(unsigned short* __restrict__ dst, int e, int e0,
+                                                 int e1, const unsigned (&x)[4])
+    {
+        if(e >= e0 && e + 4 <= e1)
+            *reinterpret_cast<uint2*>(dst + e) = {x[0] | x[1] << 16, x[2] | x[3] << 16};
+        else
+#pragma unroll
+            for(int j = 0; j < 4; j++)
+                if(e + j >= e0 && e + j < e1)
+                    dst[e + j] = (unsigned short)x[j];
+    }
+
     // One workgroup per row block (the grid holds every operator's largest
     // possible number of blocks): the block's column range, its base (the
     // smallest column) and every entry's offset from it as 16 bits; RB_WIDE is
     // set when a block spans more than 65535 columns.  Where asked for, also the
     // block's distinct columns: a bitmap of the span in LDS, whose running
     // population count is each column's place in the ascending list.
+    // Every lane holds its two quads of columns in registers from the first read
+    // on (reading them again for each of the four passes, a two-byte store per
+    // entry and one lane unpacking a bitmap word took 770 us over the operators
+    // of a 121^3 diffusion hierarchy; now 460 us, bound by the chain of
+    // barriers).
     __global__ void __launch_bounds__(256)
         rb_columns_kernel(rb_table tab, int* __restrict__ res)
     {
-        __shared__ unsigned s_bits[4096];
-        __shared__ int      s_place[4096];
-        __shared__ int      s_w[4];
-        typedef int int4v __attribute__((ext_vector_type(4)));
-        __shared__ int sh_mn[4], sh_mx[4];
-        const int k  = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.blk0; });
-        const lal::rb_op o = tab.op[k];
-        int*      out = res + RB_RES * k;
-        const int nb  = out[RB_NBLOCKS];
-        const int b   = (int)blockIdx.x - o.blk0;
+        typedef int            int4v __attribute__((ext_vector_type(4)));
+        typedef unsigned       uint4v __attribute__((ext_vector_type(4)));
+        typedef unsigned short ushort4v __attribute__((ext_vector_type(4)));
+        __shared__ uint4v   s_bits4[1024];
+        __shared__ ushort4v s_place4[1024];
+        __shared__ unsigned s_list2[(LIST_CAP + 4) / 2];
+        __shared__ int      s_w[2][4];
+        __shared__ int      sh_mn[4], sh_mx[4];
+        unsigned* const       s_bits  = reinterpret_cast<unsigned*>(s_bits4);
+        unsigned short* const s_place = reinterpret_cast<unsigned short*>(s_place4);
+        unsigned short* const s_list  = reinterpret_cast<unsigned short*>(s_list2);
+        const int k = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.blk0; });
+        const lal::rb_op o   = tab.op[k];
+        int*             out = res + RB_RES * k;
+        const int        nb  = out[RB_NBLOCKS];
+        const int        b   = (int)blockIdx.x - o.blk0;
         if(o.c16 == nullptr || out[RB_BAD] != 0 || nb > o.ub || b >= nb)
             return;
         const int4v mt = reinterpret_cast<const int4v*>(o.blocks + lal::block_meta_offset(nb))[b];
-        const int   e0 = mt.z, e1 = mt.w;
+        const int   e0 = mt.z, e1 = mt.w, tid = (int)threadIdx.x;
+        const int   q0 = e0 & ~3;
+        const bool  held = e1 - q0 <= 2048; // else: one long row, or an unlucky 2048
+        const bool  al   = ((size_t)o.ci & 15) == 0;
+        int         col[2][4];
         int         mn = INT_MAX, mx = INT_MIN;
-        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
+        if(held)
         {
-            const int col = o.ci[e];
-            mn            = min(mn, col);
-            mx            = max(mx, col);
+#pragma unroll
+            for(int h = 0; h < 2; h++)
+            {
+                const int e = q0 + 4 * (tid + 256 * h);
+                if(al && e >= e0 && e + 4 <= e1)
+                {
+                    const int4v q = *reinterpret_cast<const int4v*>(o.ci + e);
+                    col[h][0] = q.x, col[h][1] = q.y, col[h][2] = q.z, col[h][3] = q.w;
+                }
+                else
+#pragma unroll
+                    for(int j = 0; j < 4; j++)
+                        col[h][j] = e + j >= e0 && e + j < e1 ? o.ci[e + j] : 0;
+            }
+#pragma unroll
+            for(int h = 0; h < 2; h++)
+#pragma unroll
+                for(int j = 0; j < 4; j++)
+                {
+                    const int e = q0 + 4 * (tid + 256 * h) + j;
+                    if(e >= e0 && e < e1)
+                    {
+                        mn = min(mn, col[h][j]);
+                        mx = max(mx, col[h][j]);
+                    }
+                }
         }
+        else
+            for(int e = e0 + tid; e < e1; e += 256)
+            {
+                mn = min(mn, o.ci[e]);
+                mx = max(mx, o.ci[e]);
+            }
 #pragma unroll
         for(int d = 32; d > 0; d >>= 1)
         {
             mn = min(mn, __shfl_xor(mn, d, 64));
             mx = max(mx, __shfl_xor(mx, d, 64));
         }
-        if((threadIdx.x & 63) == 0)
+        const int lane = tid & 63, wid = tid >> 6;
+        if(lane == 0)
         {
-            sh_mn[threadIdx.x >> 6] = mn;
-            sh_mx[threadIdx.x >> 6] = mx;
+            sh_mn[wid] = mn;
+            sh_mx[wid] = mx;
         }
         __syncthreads();
         mn = min(min(sh_mn[0], sh_mn[1]), min(sh_mn[2], sh_mn[3]));
         mx = max(max(sh_mx[0], sh_mx[1]), max(sh_mx[2], sh_mx[3]));
-        const int base = e1 > e0 ? mn : 0;
-        if(threadIdx.x == 0)
+        const int       base = e1 > e0 ? mn : 0;
+        const long long span = e1 > e0 ? (long long)mx - mn : 0;
+        if(tid == 0)
         {
             o.cbase[b] = base;
-            if(e1 > e0 && (long long)mx - mn > 65535)
+            if(span > 65535)
                 atomicOr(out + RB_WIDE, 1);
         }
-        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
-            o.c16[e] = (unsigned short)(o.ci[e] - base);
+        if(held)
+        {
+#pragma unroll
+            for(int h = 0; h < 2; h++)
+            {
+                unsigned x[4];
+#pragma unroll
+                for(int j = 0; j < 4; j++)
+                    x[j] = (unsigned)(col[h][j] - base) & 0xffffu;
+                store_quad16(o.c16, q0 + 4 * (tid + 256 * h), e0, e1, x);
+            }
+        }
+        else
+            for(int e = e0 + tid; e < e1; e += 256)
+                o.c16[e] = (unsigned short)(o.ci[e] - base);
         if(o.lpos == nullptr)
             return;
-        if(e1 - e0 > LIST_CAP || (e1 > e0 && (long long)mx - mn > 131071))
+        if(e1 - e0 > LIST_CAP || span > 131071)
         {
-            if(threadIdx.x == 0)
+            if(tid == 0)
                 atomicOr(out + RB_LONG, 1);
             return;
         }
-        const int words = e1 > e0 ? (mx - base) / 32 + 1 : 0; // at most 4096
-        for(int w = (int)threadIdx.x; w < words; w += 256)
-            s_bits[w] = 0;
+        const int words = e1 > e0 ? (int)(span >> 5) + 1 : 0; // at most 4096
+        const int w4    = (words + 3) >> 2;
+        for(int w = tid; w < w4; w += 256)
+            s_bits4[w] = uint4v{0, 0, 0, 0};
         __syncthreads();
-        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
-        {
-            const int off = o.ci[e] - base;
-            atomicOr(&s_bits[off >> 5], 1u << (off & 31));
-        }
+#pragma unroll
+        for(int h = 0; h < 2; h++)
+#pragma unroll
+            for(int j = 0; j < 4; j++)
+            {
+                const int e = q0 + 4 * (tid + 256 * h) + j;
+                const int off = col[h][j] - base;
+                if(e >= e0 && e < e1)
+                    atomicOr(&s_bits[off >> 5], 1u << (off & 31));
+            }
         __syncthreads();
-        unsigned short* list = o.list + lal::list_start(e0, b);
-        const int lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
-        int       carry = 0;
-        for(int w0 = 0; w0 < words; w0 += 256)
+        int carry = 0, turn = 0;
+        for(int w0 = 0; w0 < w4; w0 += 256, turn ^= 1)
         {
-            const int w   = w0 + (int)threadIdx.x;
-            const int n   = w < words ? __popc(s_bits[w]) : 0;
+            const int    w    = w0 + tid;
+            const uint4v bits = w < w4 ? s_bits4[w] : uint4v{0, 0, 0, 0};
+            const int n0 = __popc(bits.x), n1 = n0 + __popc(bits.y), n2 = n1 + __popc(bits.z);
+            const int n  = n2 + __popc(bits.w);
             int       inc = n;
 #pragma unroll
             for(int d = 1; d < 64; d <<= 1)
@@ -368,49 +447,61 @@ namespace
                 inc += lane >= d ? q : 0;
             }
             if(lane == 63)
-                s_w[wid] = inc;
+                s_w[turn][wid] = inc;
             __syncthreads();
-            int at = carry + inc - n, tot = 0;
-            for(int k2 = 0; k2 < 4; k2++)
+            int at = carry + inc - n;
+#pragma unroll
+            for(int v = 0; v < 4; v++)
             {
-                at += k2 < wid ? s_w[k2] : 0;
-                tot += s_w[k2];
+                at += v < wid ? s_w[turn][v] : 0;
+                carry += s_w[turn][v];
             }
-            if(w < words)
+            if(w < w4)
+                s_place4[w] = ushort4v{(unsigned short)at, (unsigned short)(at + n0),
+                                       (unsigned short)(at + n1), (unsigned short)(at + n2)};
+        }
+        __syncthreads();
+#pragma unroll
+        for(int h = 0; h < 2; h++)
+        {
+            const int eq = q0 + 4 * (tid + 256 * h);
+            unsigned  x[4];
+#pragma unroll
+            for(int j = 0; j < 4; j++)
             {
-                s_place[w]    = at;
-                unsigned bits = s_bits[w];
-                while(bits)
+                x[j] = 0;
+                if(eq + j >= e0 && eq + j < e1)
                 {
-                    const int t = __ffs((int)bits) - 1;
-                    bits &= bits - 1;
-                    list[at++] = (unsigned short)(w * 32 + t);
+                    const int      off  = col[h][j] - base;
+                    const unsigned less = s_bits[off >> 5] & ((1u << (off & 31)) - 1u);
+                    const int      at   = s_place[off >> 5] + __popc(less);
+                    s_list[at]          = (unsigned short)off;
+                    x[j]                = 4u * (unsigned)at;
                 }
             }
-            carry += tot;
-            __syncthreads();
-        }
-        for(int e = e0 + (int)threadIdx.x; e < e1; e += 256)
-        {
-            const int      off  = o.ci[e] - base;
-            const unsigned less = s_bits[off >> 5] & ((1u << (off & 31)) - 1u);
-            o.lpos[e]           = (unsigned short)(4 * (s_place[off >> 5] + __popc(less)));
+            store_quad16(o.lpos, eq, e0, e1, x);
         }
         // the last quad is read whole
-        if(b == nb - 1 && threadIdx.x < (unsigned)(-o.nnz & 3))
-            o.lpos[o.nnz + (int)threadIdx.x] = 0;
-        if(threadIdx.x == 0)
+        if(b == nb - 1 && tid < (-o.nnz & 3))
+            o.lpos[o.nnz + tid] = 0;
+        if(tid == 0)
         {
             if(carry & 1)
-                list[carry] = (unsigned short)(mx - base); // (its low 16 bits)
+                s_list[carry] = (unsigned short)span; // (its low 16 bits)
             // (words from 2048 on start the offsets of 65536 and more)
-            const int split = words > 2048 ? s_place[2048] : carry;
-            o.lmeta[2 * b]  = carry | split << 12 | lal::spmv_group_log(mt.y - mt.x) << 24;
+            const int split    = words > 2048 ? s_place[2048] : carry;
+            o.lmeta[2 * b]     = carry | split << 12 | lal::spmv_group_log(mt.y - mt.x) << 24;
             o.lmeta[2 * b + 1] = base;
-            atomicMax(out + RB_LMAX, carry);
-            if(split < carry)
+            // (one address for all blocks: few of them raise it)
+            if(carry > *(volatile int*)(out + RB_LMAX))
+                atomicMax(out + RB_LMAX, carry);
+            if(split < carry && *(volatile int*)(out + RB_FAR) == 0)
                 atomicOr(out + RB_FAR, 1);
         }
+        __syncthreads();
+        unsigned* const list = reinterpret_cast<unsigned*>(o.list + lal::list_start(e0, b));
+        for(int i = tid; i < (carry + 1) >> 1; i += 256)
+            list[i] = s_list2[i];
     }
 
     template <typename T, typename ACC, int MODE>

@@ -305,15 +305,17 @@ namespace
             LAL_TRY(lal::diag_inv<double>(c, L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag,
                                           L.w64.dinv, L.A.nnz));
             if(L.Q.rp && l < h->levels)
+            {
+                if(h->opts.build_f32)
+                    LAL_TRY(h->mem.get(&L.Q.v32, L.Q.nnz));
                 LAL_TRY(lal::smoothed_prolongator(c, L.Q.m, L.Q.nnz, L.Q.rp, L.Q.ci, L.Q.v, L.P.rp,
-                                                  L.P.ci, L.P.v, L.w64.dinv));
+                                                  L.P.ci, L.P.v, L.w64.dinv, L.Q.v32));
+            }
             if(h->opts.build_f32)
             {
                 LAL_TRY(to_f32(h, L.A.v, &L.A.v32, L.A.nnz));
                 if(l < h->levels)
                 {
-                    if(L.Q.rp)
-                        LAL_TRY(to_f32(h, L.Q.v, &L.Q.v32, L.Q.nnz));
                     LAL_TRY(to_f32(h, L.P.v, &L.P.v32, L.P.nnz));
                     LAL_TRY(to_f32(h, L.R.v, &L.R.v32, L.R.nnz));
                 }
@@ -1091,10 +1093,13 @@ namespace
         // it; the analysis describes the finest operator (a copy of the same
         // pattern), so the hierarchy keeps it for level 0
         auto* h = new lal_hierarchy_t;
-        // The whole hierarchy takes about 80 bytes per nonzero (120 with the
-        // FP32 levels) and 200 per row: the first chunk is half of that, and
-        // the arena grows by half its size.
-        h->mem.reserve((size_t)nnz * (o.build_f32 ? 60 : 40) + (size_t)m * 100);
+        // A hierarchy takes about 140 to 175 bytes per nonzero of a 7-point
+        // operator with the column lists and the FP32 levels, less without:
+        // the first chunk holds most of it (a hipMalloc and hipFree of
+        // hundreds of megabytes take 0.3 ms together), and the arena grows by
+        // half its size.
+        h->mem.reserve((size_t)nnz * ((o.exact ? 40 : 80) + (o.build_f32 ? 40 : 0)) +
+                       (size_t)m * (o.build_f32 ? 200 : 100));
         int s = lal::analyse(c, {{descr(h->L[0].A, m, nnz, n, o.exact), rp, ci, m, nnz,
                                   o.exact == 0, n}}, &h->mem, nullptr);
         if(s == LAL_OK)

@@ -64,10 +64,10 @@ namespace lal
     int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
                     const T* v, const T* e, const T* y, T* out);
     // AP's values become those of Q = P - D^-1 A P (pattern of A P, a superset
-    // of P's; both with ascending columns).
+    // of P's; both with ascending columns); v32 (or null): the same in FP32.
     int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
                              double* v, const int* prp, const int* pci, const double* pv,
-                             const double* dinv);
+                             const double* dinv, float* v32);
     template <typename T>
     int jacobi0_residual(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                          const int* ci, const T* v, const T* diag, const T* dinv, const T* b,

@@ -17,6 +17,8 @@
 // block in the same fixed order, so all blocks see bitwise the same value.
 #include "lal_vcycle.h"
 
+#include <type_traits>
+
 namespace
 {
     using lal::SPMV_THREADS;
@@ -439,32 +441,63 @@ namespace
             p[i] = beta == (T)0 ? (T)z[i] : (T)z[i] + beta * p[i];
     }
 
-    // One lane group per row: entry (i, c) of A P becomes P(i, c) - dinv_i (A P)(i, c).
+    // G lanes per row: entry (i, c) of A P becomes P(i, c) - dinv_i (A P)(i, c),
+    // in FP64 and, with v32, rounded to FP32 as well.  The row of P lies in the
+    // group's registers (up to G entries; a longer one is searched in memory)
+    // and is compared by shuffles, so a row's loads are one chain of two: a
+    // binary search in memory per entry, with 16 lanes on every row, took
+    // 452 us over the levels of a 121^3 diffusion hierarchy and the FP32 copy
+    // another pass (90 us); now 300 us with the copy.
+    template <int G>
     __global__ void __launch_bounds__(256)
         smoothed_prolongator_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                                     double* __restrict__ v, const int* __restrict__ prp,
                                     const int* __restrict__ pci, const double* __restrict__ pv,
-                                    const double* __restrict__ dinv)
+                                    const double* __restrict__ dinv, float* __restrict__ v32)
     {
-        const int i = blockIdx.x * 16 + (int)(threadIdx.x >> 4);
+        const int i = blockIdx.x * (256 / G) + (int)(threadIdx.x / G);
         if(i >= m)
             return;
+        const int    t  = (int)(threadIdx.x & (G - 1));
         const double di = dinv[i];
-        const int    ps = prp[i], pe = prp[i + 1];
-        for(int j = rp[i] + (int)(threadIdx.x & 15); j < rp[i + 1]; j += 16)
+        const int    ps = prp[i], pn = prp[i + 1] - ps;
+        const int    s = rp[i], e = rp[i + 1];
+        const int    pc = t < pn ? pci[ps + t] : -1;
+        const double pw = t < pn ? pv[ps + t] : 0.0;
+        for(int j0 = s; j0 < e; j0 += G)
         {
-            const int c  = ci[j];
-            int       lo = ps, hi = pe; // first entry of P's row at or after c
-            while(lo < hi)
+            const int    j = j0 + t;
+            const int    c = j < e ? ci[j] : -1;
+            const double a = j < e ? v[j] : 0.0;
+            double       p = 0.0;
+            if(pn <= G)
             {
-                const int mid = (lo + hi) >> 1;
-                if(pci[mid] < c)
-                    lo = mid + 1;
-                else
-                    hi = mid;
+                int hit = -1;
+                for(int u = 0; u < pn; u++)
+                    hit = __shfl(pc, u, G) == c ? u : hit;
+                p = __shfl(pw, hit < 0 ? 0 : hit, G);
+                p = hit < 0 ? 0.0 : p;
             }
-            const double p = lo < pe && pci[lo] == c ? pv[lo] : 0.0;
-            v[j]           = p - di * v[j];
+            else
+            {
+                int lo = ps, hi = ps + pn; // first entry of P's row at or after c
+                while(lo < hi)
+                {
+                    const int mid = (lo + hi) >> 1;
+                    if(pci[mid] < c)
+                        lo = mid + 1;
+                    else
+                        hi = mid;
+                }
+                p = lo < ps + pn && pci[lo] == c ? pv[lo] : 0.0;
+            }
+            if(j < e)
+            {
+                const double q = p - di * a;
+                v[j]           = q;
+                if(v32)
+                    v32[j] = (float)q;
+            }
         }
     }
 
@@ -564,12 +597,22 @@ namespace lal
 
     int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
                              double* v, const int* prp, const int* pci, const double* pv,
-                             const double* dinv)
+                             const double* dinv, float* v32)
     {
         if(m == 0 || nnz == 0)
             return LAL_OK;
-        smoothed_prolongator_kernel<<<grid_for(m, 16), 256, 0, c->stream>>>(m, rp, ci, v, prp,
-                                                                            pci, pv, dinv);
+        const auto go = [&](auto g) {
+            constexpr int G = decltype(g)::value;
+            smoothed_prolongator_kernel<G><<<grid_for(m, 256 / G), 256, 0, c->stream>>>(
+                m, rp, ci, v, prp, pci, pv, dinv, v32);
+        };
+        // about two steps of the group per row
+        if(nnz <= 16L * m)
+            go(std::integral_constant<int, 8>{});
+        else if(nnz <= 48L * m)
+            go(std::integral_constant<int, 16>{});
+        else
+            go(std::integral_constant<int, 64>{});
         LAL_LAUNCHED();
         return LAL_OK;
     }
