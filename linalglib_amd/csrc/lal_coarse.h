@@ -1,40 +1,46 @@
-// Single-workgroup coarse tail of the V-cycle (see lal_coarse.hip).
+// The small end of the V-cycle as one dense operator (see lal_coarse.hip).
 #pragma once
 
 #include "lal_internal.h"
 
 namespace lal
 {
-    // Levels the tail can hold, and the LDS it may use for them.
-    constexpr int TAIL_MAX_LEVELS = 12;
-    constexpr int TAIL_LDS_BYTES  = 64 * 1024;
+    // Rows of the largest level whose cycle is kept as a dense operator: 8 MB,
+    // which the eight L2s hold beside the level above.  Up to here it replaces
+    // four or more launches of 3 to 4 us (an iteration of PCG on 128^2 Poisson,
+    // where the level has 496 rows, 69 -> 52 us; on 64^3 with 1000 rows
+    // 208 -> 181 us with the hierarchy's build) for three launches a level in the
+    // setup, which the packing of the levels into an LDS image cost before.
+    // The operator grows with the square, its construction faster; the next
+    // larger levels of the grids measured (3,500 to 4,000 rows) would read 100 MB.
+    constexpr int CYCLE_ROWS = 1024;
 
-    // Word (4-byte) offsets of one level's arrays inside the tail's LDS
-    // image.  P and R are absent (-1) on the coarsest level.
-    struct tail_level
+    // One level as the construction reads it (FP64): A and 1/a_ii, the
+    // restriction R (mc x m) and Q = P - D^-1 A P (m x mc).
+    struct cycle_level
     {
-        int m;
-        int rp, ci, v, dinv;     // A and 1/a_ii
-        int prp, pci, pv;        // P (m x m_next)
-        int rrp, rci, rv;        // R (m_next x m)
-        int x, t, b, r;          // work vectors (LDS only, not in the image)
+        int           m, mc;
+        const int *   arp, *aci;
+        const double *av, *dinv;
+        const int *   rrp, *rci;
+        const double* rv;
+        const int *   qrp, *qci;
+        const double* qv;
     };
 
-    struct tail_desc
+    // Leading dimension of a level's operator.
+    __host__ __device__ inline int cycle_ld(int m)
     {
-        int        nl;        // levels in the tail, the last one the coarsest
-        int        kind;      // coarsest solve: 0 the 1x1 divide, 1 dense inverse
-        int        img_words; // words copied from the device image
-        int        lds_words; // image plus work vectors
-        int        inv;       // word offset of the dense inverse in LDS, -1: global
-        tail_level L[TAIL_MAX_LEVELS];
-    };
+        return (m + 1) & ~1;
+    }
 
-    // Runs the tail: the image (rp, ci, values, 1/a_ii, P, R of every tail
-    // level, optionally the coarsest dense inverse) is copied into LDS once,
-    // the first level's right-hand side comes from b_in, and the first
-    // level's post-smoothed result lands in `result`.
+    // M (m rows of cycle_ld(m)): the level's V-cycle from zero with one pre- and
+    // one post-sweep, given the next level's operator Mc (mc rows of ldc) or, for
+    // a 1x1 coarsest level, its entry a11.  S and U: mc x cycle_ld(m) scratch.
+    int cycle_matrix(lal_context* c, const cycle_level& L, const double* Mc, int ldc,
+                     const double* a11, double* S, double* U, double* M);
+
+    // x = M b
     template <typename T>
-    int coarse_tail(lal_context* c, const tail_desc& d, const int* image, const T* b_in,
-                    const double* inv, T* result);
+    int cycle_apply(lal_context* c, int m, const double* M, const T* b, T* x);
 }

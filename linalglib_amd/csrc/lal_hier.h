@@ -150,13 +150,10 @@ struct lal_hierarchy_t
     unsigned* d_seq      = nullptr;
     unsigned  seq        = 0;
     bool      has32      = false;
-    // coarse tail: levels tail_first..levels run in one workgroup out of LDS
-    // (fast path); one packed device image of their arrays per precision
-    int            tail_first = -1;
-    int*           tail_img64 = nullptr;
-    int*           tail_img32 = nullptr;
-    lal::tail_desc tail64{};
-    lal::tail_desc tail32{};
+    // levels cycle_first..levels of the fast path's V-cycle with one pre- and
+    // one post-sweep, as one dense operator (FP64)
+    int     cycle_first = -1;
+    double* cycle_op    = nullptr;
     // captured cycles (lal::captured): the multicolour smoothers' cycles
     // (kind = smoother 5 or 6) and the PCG preconditioner's V-cycle (kind
     // lal::KIND_PRECOND + 2 xinit + FP32), one per (x, b, sweeps, cycle, kind)

@@ -65,31 +65,6 @@ namespace
         return A.v32;
     }
 
-    template <typename T>
-    const lal::tail_desc& tail_of(const lal_hierarchy_t* h);
-    template <>
-    const lal::tail_desc& tail_of<double>(const lal_hierarchy_t* h)
-    {
-        return h->tail64;
-    }
-    template <>
-    const lal::tail_desc& tail_of<float>(const lal_hierarchy_t* h)
-    {
-        return h->tail32;
-    }
-    template <typename T>
-    const int* tail_image(const lal_hierarchy_t* h);
-    template <>
-    const int* tail_image<double>(const lal_hierarchy_t* h)
-    {
-        return h->tail_img64;
-    }
-    template <>
-    const int* tail_image<float>(const lal_hierarchy_t* h)
-    {
-        return h->tail_img32;
-    }
-
     // r = b - A x in the level's precision
     template <typename T>
     int residual_t(lal_context* c, const csr_dev& A, const T* Av, const T* x, const T* b, T* r)
@@ -152,103 +127,38 @@ namespace
         return true;
     }
 
-    // Layout of the coarse tail's LDS image for levels first..levels in
-    // precision T (word offsets; values 8-byte aligned for FP64).  With
-    // `img` the arrays are also copied into a fresh device image.  Returns
-    // false when the levels do not fit the tail's LDS.
-    template <typename T>
-    bool tail_layout(lal_hierarchy_t* h, int first, lal::tail_desc* d, int** img, int* status)
+    // The dense operator of the V-cycle's small end: the first level from
+    // `levels` - 1 down to 1 that is still within lal::CYCLE_ROWS rows, on the
+    // fast path with a direct coarsest solve.
+    int cycle_operator(lal_hierarchy_t* h, lal::arena* tmp)
     {
-        constexpr int S = (int)sizeof(T) / 4;
-        *status         = LAL_OK;
-        const int nl    = h->levels - first + 1;
-        if(first < 1 || nl < 2 || nl > lal::TAIL_MAX_LEVELS)
-            return false;
-        std::memset(d, 0, sizeof(*d));
-        d->nl   = nl;
-        d->kind = h->coarse_kind == 0 ? 0 : 1;
-        long w  = 0;
-        struct piece
+        lal_context* c     = h->c;
+        int          first = h->levels;
+        while(first > 1 && h->L[first - 1].A.m <= lal::CYCLE_ROWS)
+            first--;
+        const level_t& last = h->L[h->levels];
+        if(h->opts.exact || h->coarse_kind == 1 || first == h->levels ||
+           last.A.m > lal::CYCLE_ROWS)
+            return LAL_OK;
+        const double* Mc  = h->coarse_kind == 2 ? h->coarse_inv : nullptr;
+        int           ldc = last.A.m;
+        for(int l = h->levels - 1; l >= first; l--)
         {
-            long        off;
-            const void* src;
-            size_t      bytes;
-        };
-        std::vector<piece> pieces;
-        auto put = [&](const void* src, long words, int align) -> int {
-            w            = (w + align - 1) / align * align;
-            const long o = w;
-            if(words > 0)
-                pieces.push_back({o, src, (size_t)words * 4});
-            w += words;
-            return (int)o;
-        };
-        for(int k = 0; k < nl; k++)
-        {
-            const int       l  = first + k;
-            level_t&        L  = h->L[l];
-            work<T>&        W  = h->w<T>(l);
-            lal::tail_level& t = d->L[k];
-            t.m                = L.A.m;
-            t.rp               = put(L.A.rp, L.A.m + 1, 1);
-            t.ci               = put(L.A.ci, L.A.nnz, 1);
-            t.v                = put(vals<T>(L.A), (long)L.A.nnz * S, S);
-            t.dinv             = put(W.dinv, (long)L.A.m * S, S);
-            t.prp = t.pci = t.pv = t.rrp = t.rci = t.rv = -1;
-            if(l < h->levels)
-            {
-                t.prp = put(L.P.rp, L.P.m + 1, 1);
-                t.pci = put(L.P.ci, L.P.nnz, 1);
-                t.pv  = put(vals<T>(L.P), (long)L.P.nnz * S, S);
-                t.rrp = put(L.R.rp, L.R.m + 1, 1);
-                t.rci = put(L.R.ci, L.R.nnz, 1);
-                t.rv  = put(vals<T>(L.R), (long)L.R.nnz * S, S);
-            }
+            const level_t&   L  = h->L[l];
+            const size_t     ld = lal::cycle_ld(L.A.m);
+            lal::cycle_level in{L.A.m, L.R.m, L.A.rp, L.A.ci, L.A.v, L.w64.dinv, L.R.rp, L.R.ci,
+                                L.R.v, L.Q.rp, L.Q.ci, L.Q.v};
+            double *         S = nullptr, *U = nullptr, *M = nullptr;
+            LAL_TRY(tmp->get(&S, ld * L.R.m));
+            LAL_TRY(tmp->get(&U, ld * L.R.m));
+            LAL_TRY((l == first ? &h->mem : tmp)->get(&M, ld * L.A.m));
+            LAL_TRY(lal::cycle_matrix(c, in, Mc, ldc, last.A.v, S, U, M));
+            Mc  = M;
+            ldc = (int)ld;
         }
-        // the coarsest dense inverse joins the image when it fits
-        d->inv            = -1;
-        const long budget = lal::TAIL_LDS_BYTES / 4;
-        long       vec    = 0;
-        for(int k = 0; k < nl; k++)
-            vec += 4 * ((long)d->L[k].m * S + S);
-        const int mc = h->L[h->levels].A.m;
-        if(d->kind == 1 && h->coarse_inv)
-        {
-            const long inv_words = 2L * mc * mc;
-            if(((w + 1) / 2 * 2) + inv_words + vec + 8 <= budget)
-                d->inv = put(h->coarse_inv, inv_words, 2);
-        }
-        w            = (w + 3) / 4 * 4;
-        d->img_words = (int)w;
-        for(int k = 0; k < nl; k++)
-        {
-            lal::tail_level& t = d->L[k];
-            t.x                = put(nullptr, (long)t.m * S, S);
-            t.t                = put(nullptr, (long)t.m * S, S);
-            t.b                = put(nullptr, (long)t.m * S, S);
-            t.r                = put(nullptr, (long)t.m * S, S);
-        }
-        d->lds_words = (int)w;
-        if(w > budget)
-            return false;
-        if(img)
-        {
-            *status = h->mem.get(img, (size_t)d->img_words);
-            if(*status != LAL_OK)
-                return false;
-            for(const piece& p : pieces)
-                if(p.src)
-                {
-                    hipError_t e = hipMemcpyAsync(*img + p.off, p.src, p.bytes,
-                                                  hipMemcpyDeviceToDevice, h->c->stream);
-                    if(e != hipSuccess)
-                    {
-                        *status = lal::hip_status(e, "tail image", __FILE__, __LINE__);
-                        return false;
-                    }
-                }
-        }
-        return true;
+        h->cycle_first = first;
+        h->cycle_op    = const_cast<double*>(Mc);
+        return LAL_OK;
     }
 
     int to_f32(lal_hierarchy_t* h, const double* x, float** y, size_t n)
@@ -368,31 +278,7 @@ namespace
         else
             h->coarse_kind = 1;
 
-        // coarse tail: the deepest run of levels (at least two, never level 0)
-        // whose FP64 arrays fit the tail's LDS, on the fast path with a direct
-        // coarsest solve
-        if(!exact && h->coarse_kind != 1 && h->levels >= 2)
-        {
-            lal::tail_desc probe{};
-            int            st    = LAL_OK;
-            int            first = -1;
-            for(int f = h->levels - 1; f >= 1; f--)
-            {
-                if(!tail_layout<double>(h, f, &probe, nullptr, &st))
-                    break;
-                first = f;
-            }
-            if(first >= 1)
-            {
-                if(!tail_layout<double>(h, first, &h->tail64, &h->tail_img64, &st))
-                    return st != LAL_OK ? st : LAL_ERR_INVALID;
-                if(h->opts.build_f32 &&
-                   !tail_layout<float>(h, first, &h->tail32, &h->tail_img32, &st))
-                    return st != LAL_OK ? st : LAL_ERR_INVALID;
-                h->tail_first = first;
-                LAL_HIP(hipStreamSynchronize(h->c->stream));
-            }
-        }
+        LAL_TRY(cycle_operator(h, tmp));
 
         const int n = h->L[0].A.m;
         LAL_TRY(h->mem.get(&h->res, n));
@@ -531,11 +417,10 @@ namespace
         // update for level 0) when xinit is set; this level then only forms
         // r = b - A x.
         const bool fast = !h->opts.exact && n1 == 1;
-        if(fast && n2 == 1 && l == h->tail_first && tail_image<T>(h))
+        if(fast && n2 == 1 && l == h->cycle_first)
         {
             T* res = dst ? dst : W.t;
-            LAL_TRY(lal::coarse_tail<T>(c, tail_of<T>(h), tail_image<T>(h), b, h->coarse_inv,
-                                        res));
+            LAL_TRY(lal::cycle_apply<T>(c, A.m, h->cycle_op, b, res));
             *out = res;
             return LAL_OK;
         }
