@@ -512,11 +512,10 @@ namespace
     {
         lal_context*   c      = h->c;
         const csr_dev& A      = h->L[0].A;
-        double*        part_r = h->part + 3 * lal::PCG_BLOCKS;
         unsigned       seq    = 0;
         LAL_TRY(lal::residual_f64(c, A.d, A.m, A.n, A.nnz, A.rp, A.ci, A.v, x, b, h->res));
-        LAL_TRY(lal::norm_partials<double>(c, A.m, h->res, part_r));
-        LAL_TRY(lal::post_scalar(h, 1, part_r, slot, &seq));
+        LAL_TRY(lal::norm_partials<double>(c, A.m, h->res, h->part_r));
+        LAL_TRY(lal::post_norm(h, lal::PCG_BLOCKS, slot, &seq));
         return lal::wait_scalar(h, seq, slot, v);
     }
 }

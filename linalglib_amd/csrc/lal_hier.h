@@ -141,14 +141,18 @@ struct lal_hierarchy_t
     float*  q32   = nullptr;
     float*  d32   = nullptr;
     double* s     = nullptr; // LAL_SOLVER_SLOTS scalars
-    double* part  = nullptr; // 4 x PCG_BLOCKS reduction partials
+    // reduction partials: <q, p>, <z, r> (PCG_PARTS each), max|r| (PCG_BLOCKS)
+    double* part_pq = nullptr;
+    double* part_g  = nullptr;
+    double* part_r  = nullptr;
     // residual norms reach the host through mapped pinned memory: a value
     // and a sequence number the host polls
     double*   h_note     = nullptr;
     double*   d_note     = nullptr;
     unsigned* h_seq      = nullptr;
     unsigned* d_seq      = nullptr;
-    unsigned  seq        = 0;
+    unsigned  seq        = 0;       // the last note asked for
+    unsigned* d_count    = nullptr; // notes written (device)
     bool      has32      = false;
     // levels cycle_first..levels of the fast path's V-cycle with one pre- and
     // one post-sweep, as one dense operator (FP64)
@@ -156,7 +160,8 @@ struct lal_hierarchy_t
     double* cycle_op    = nullptr;
     // captured cycles (lal::captured): the multicolour smoothers' cycles
     // (kind = smoother 5 or 6) and the PCG preconditioner's V-cycle (kind
-    // lal::KIND_PRECOND + 2 xinit + FP32), one per (x, b, sweeps, cycle, kind)
+    // lal::KIND_PRECOND and what it does besides), one per (x, b, sweeps, cycle,
+    // kind)
     struct cycle_graph
     {
         const void*    x;
@@ -221,10 +226,12 @@ namespace lal
     // Records the reduction over the last step, clamped to [0.05, 1] (a NaN
     // norm gives 0.05), and the new norm.
     void observe_rate(double rn, double* r_prev, double* rate);
-    // Reduces PCG_BLOCKS partials (op 0 sum, 1 max) into the solver slot and
+    // Reduces max|r|'s `count` partials (h->part_r) into the solver slot and
     // hands the value to the host through the hierarchy's mapped note;
-    // returns the sequence number to wait for.
-    int post_scalar(lal_hierarchy_t* h, int op, const double* part, int slot, unsigned* seq);
+    // returns the sequence number to wait for.  With `later`, that reduction
+    // is left to the kernel which gets *later.
+    int post_norm(lal_hierarchy_t* h, int count, int slot, unsigned* seq,
+                  post_args* later = nullptr);
     // Waits for the note carrying `seq` (checks the stream now and then).
     int wait_scalar(lal_hierarchy_t* h, unsigned seq, int slot, double* v);
 

@@ -44,7 +44,7 @@ namespace lal
 }
 
 using lal::converges;
-using lal::post_scalar;
+using lal::post_norm;
 using lal::wait_scalar;
 using lal::csr_dev;
 using lal::level_t;
@@ -286,7 +286,11 @@ namespace
         LAL_TRY(h->mem.get(&h->p, n));
         LAL_TRY(h->mem.get(&h->q, n));
         LAL_TRY(h->mem.get(&h->s, lal::LAL_SOLVER_SLOTS));
-        LAL_TRY(h->mem.get(&h->part, 4 * lal::PCG_BLOCKS));
+        LAL_TRY(h->mem.get(&h->part_pq, lal::PCG_PARTS));
+        LAL_TRY(h->mem.get(&h->part_g, lal::PCG_PARTS));
+        LAL_TRY(h->mem.get(&h->part_r, lal::PCG_BLOCKS));
+        LAL_TRY(h->mem.get(&h->d_count, 1));
+        LAL_TRY(lal_fill_i32(c, (int*)h->d_count, 1, 0));
         LAL_HIP(hipHostMalloc((void**)&h->h_note, 64, hipHostMallocMapped | hipHostMallocCoherent));
         std::memset(h->h_note, 0, 64);
         h->h_seq = reinterpret_cast<unsigned*>(h->h_note + 1);
@@ -401,11 +405,27 @@ namespace
         return st;
     }
 
+    // What level 0's kernels do for the solver besides the cycle (merged()
+    // holds): the residual pass finishes the reduction `post`, the correction
+    // leaves <dot.w, z>'s partials in dot.part.
+    struct cycle_extra
+    {
+        lal::post_args post{};
+        lal::row_extra dot{};
+    };
+
+    // One pre-sweep and a post-sweep on the fast path: the residual pass also
+    // leaves y = x + r / a_ii, and the way up is y + Q e.
+    bool merged(const lal_hierarchy_t* h, int l, int n1, int n2)
+    {
+        return !h->opts.exact && n1 == 1 && n2 >= 1 && l < h->levels && h->L[l].Q.rp;
+    }
+
     // One V-cycle at level l for rhs b with the initial guess zero.  The
     // result lands in dst when given, else in a level buffer; *out gets it.
     template <typename T>
     int vcycle(lal_hierarchy_t* h, int l, const T* b, T* dst, int n1, int n2, bool xinit,
-               T** out)
+               T** out, const cycle_extra& ex = {})
     {
         lal_context* c = h->c;
         level_t&     L = h->L[l];
@@ -438,9 +458,7 @@ namespace
         }
         T* cur   = W.x;
         T* other = W.t;
-        // one pre-sweep and a post-sweep: the residual pass also leaves
-        // y = x + r / a_ii in W.t, and the way up is y + Q e
-        const bool merged = fast && n2 >= 1 && L.Q.rp;
+        const bool post_merged = merged(h, l, n1, n2); // y lies in W.t
         if(n1 == 0)
         {
             // x = 0 and r = b - A*0, which is b bit for bit
@@ -451,9 +469,9 @@ namespace
         {
             if(!xinit)
                 LAL_TRY(lal::mul_elem<T>(c, A.m, b, W.dinv, cur));
-            if(merged)
+            if(post_merged)
                 LAL_TRY(lal::residual_smoothed<T>(c, A.d, A.m, A.rp, A.ci, Av, cur, W.dinv, b, W.r,
-                                                  other));
+                                                  other, ex.post));
             else
                 LAL_TRY(residual_t<T>(c, A, Av, cur, b, W.r));
         }
@@ -484,12 +502,12 @@ namespace
         T* ec = nullptr;
         LAL_TRY(vcycle<T>(h, l + 1, Wc.b, nullptr, n1, n2, fast, &ec));
         int done = 0; // post-sweeps behind us
-        if(merged)
+        if(post_merged)
         {
             // other = y; the result may go straight to dst
             T* o = n2 == 1 && dst ? dst : cur;
             LAL_TRY(lal::add_product<T>(c, L.Q.d, L.Q.m, L.Q.rp, L.Q.ci, vals<T>(L.Q), ec, other,
-                                        o));
+                                        o, ex.dot));
             cur  = o;
             done = 1;
         }
@@ -519,10 +537,11 @@ namespace
     }
 
     template <typename T>
-    int precond(lal_hierarchy_t* h, const T* r, T* z, int n1, int n2, bool xinit = false)
+    int precond(lal_hierarchy_t* h, const T* r, T* z, int n1, int n2, bool xinit = false,
+                const cycle_extra& ex = {})
     {
         T* out = nullptr;
-        return vcycle<T>(h, 0, r, z, n1, n2, xinit, &out);
+        return vcycle<T>(h, 0, r, z, n1, n2, xinit, &out, ex);
     }
 
     // precond() for the solvers' own vectors (r, z fixed per hierarchy and
@@ -537,13 +556,41 @@ namespace
 
     template <typename T>
     int precond_graphed(lal_hierarchy_t* h, const T* r, T* z, int n1, int n2,
-                        bool xinit = false)
+                        bool xinit = false, const cycle_extra& ex = {})
     {
         if(n1 < 1 || h->L[0].A.m > GRAPH_MAX_ROWS)
-            return precond<T>(h, r, z, n1, n2, xinit);
-        const int kind = lal::KIND_PRECOND + 2 * (int)xinit + (sizeof(T) == 4 ? 1 : 0);
+            return precond<T>(h, r, z, n1, n2, xinit, ex);
+        // (ex is the same for every call with these flags: the solvers' own
+        // buffers; the inner product's other vector goes with the precision)
+        const int kind = lal::KIND_PRECOND + (sizeof(T) == 4 ? 1 : 0) + 2 * (int)xinit +
+                         (ex.post.part ? 4 : 0) + (ex.dot.part ? 8 : 0) + (ex.dot.wide ? 16 : 0);
         return lal::captured(h, z, r, n1, n2, 0, 0, kind,
-                             [&] { return precond<T>(h, r, z, n1, n2, xinit); });
+                             [&] { return precond<T>(h, r, z, n1, n2, xinit, ex); });
+    }
+
+    // z = one V-cycle on r, and the partials of <z, w> (w: the residual in the
+    // solver's precision) in h->part_g, *n_g of them.  seq given: the norm
+    // max|r| in h->part_r (n_r partials) is handed to the host on the way.
+    // Where the cycle's own kernels can do either, no launch of its own is spent.
+    template <typename T, typename W>
+    int apply_dot(lal_hierarchy_t* h, const T* r, T* z, const W* w, int n1, int n2, bool xinit,
+                  int n_r, unsigned* seq, int* n_g)
+    {
+        const csr_dev& Q    = h->L[0].Q;
+        const bool     fold = merged(h, 0, n1, n2);
+        cycle_extra    ex;
+        if(seq)
+            LAL_TRY(post_norm(h, n_r, lal::S_RNORM, seq, fold ? &ex.post : nullptr));
+        if(fold && n2 == 1 && lal::can_add_dot<T>(Q.d, Q.m, Q.rp, Q.ci, vals<T>(Q)))
+        {
+            ex.dot.part = h->part_g;
+            ex.dot.w    = w;
+            ex.dot.wide = sizeof(W) > sizeof(T);
+        }
+        LAL_TRY(precond_graphed<T>(h, r, z, n1, n2, xinit, ex));
+        *n_g = ex.dot.part ? Q.d->nblocks : lal::PCG_BLOCKS;
+        return ex.dot.part ? LAL_OK
+                           : lal::dot_partials<T, W>(h->c, h->L[0].A.m, z, w, h->part_g);
     }
 
     // cg_solver::solve_precond on the device.  T = double uses the FP64
@@ -566,50 +613,50 @@ namespace
         else
             LAL_TRY(lal::residual_f32(c, A.d, n, A.n, A.nnz, A.rp, A.ci, (const float*)Av,
                                       (const float*)x, (const float*)b, (float*)res));
-        // partial buffers: <q,p>, <z,r> (two generations), max|r|
-        double*  part_pq   = h->part;
-        double*  part_g[2] = {h->part + lal::PCG_BLOCKS, h->part + 2 * lal::PCG_BLOCKS};
-        double*  part_r    = h->part + 3 * lal::PCG_BLOCKS;
         unsigned seq       = 0;
         double   init      = 0.0;
-        LAL_TRY(lal::norm_partials<T>(c, n, res, part_r));
-        LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM0, &seq));
+        LAL_TRY(lal::norm_partials<T>(c, n, res, h->part_r));
+        LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM0, &seq));
         LAL_TRY(wait_scalar(h, seq, lal::S_RNORM0, &init));
         // the preconditioner: one V-cycle from zero, with the Jacobi fast path
         // or (smoother != 0, FP64 only) another smoother of the AMG cycles
-        auto apply = [&](bool xinit) -> int {
-            if(smoother != 0)
-                return lal::vcycle_smoothed(h, (const double*)res, (double*)z, n1, n2, smoother);
-            return precond_graphed<T>(h, res, z, n1, n2, xinit);
+        int        n_pq = 0, n_g = 0;
+        const int  n_r   = lal::update_blocks(n);
+        auto       apply = [&](bool xinit, unsigned* norm) -> int {
+            if(smoother == 0)
+                return apply_dot<T, T>(h, res, z, res, n1, n2, xinit, n_r, norm, &n_g);
+            if(norm)
+                LAL_TRY(post_norm(h, n_r, lal::S_RNORM, norm));
+            LAL_TRY(lal::vcycle_smoothed(h, (const double*)res, (double*)z, n1, n2, smoother));
+            n_g = lal::PCG_BLOCKS;
+            return lal::dot_partials<T, T>(c, n, z, res, h->part_g);
         };
-        LAL_TRY(apply(false));
+        LAL_TRY(apply(false, nullptr));
         LAL_HIP(hipMemcpyAsync(p, z, sizeof(T) * n, hipMemcpyDeviceToDevice, c->stream));
-        int cur = 0;
-        LAL_TRY(lal::dot_partials<T, T>(c, n, z, res, part_g[cur]));
+        int cur = 0; // generation of s[S_GAMMA]
+        LAL_TRY(lal::finish_partials(c, 0, {h->part_g, n_g, s + lal::S_GAMMA}));
         double rn   = init;
         int    iter = 0;
         bool   conv = false;
         double r_prev = init, rate = 0.5; // last norm, observed reduction per step
         while(!(iter > max_iter))
         {
-            LAL_TRY(lal::csrmv(c, A.d, n, A.n, A.nnz, 1.0, A.rp, A.ci, Av, p, 0.0, q));
-            LAL_TRY(lal::dot_partials<T, T>(c, n, q, p, part_pq));
+            LAL_TRY(lal::product_dot<T>(c, A.d, n, A.n, A.nnz, A.rp, A.ci, Av, p, q, h->part_pq,
+                                        &n_pq));
             // with one pre-sweep on the fast path, the update also writes the
             // V-cycle's first Jacobi iterate x0 = r / a_ii
             const bool fast = !h->opts.exact && n1 == 1 && h->levels > 0 && smoother == 0;
             work<T>&   W0   = h->w<T>(0);
-            LAL_TRY(lal::update_xr<T, T>(c, n, p, q, x, res, part_pq, part_g[cur], part_r,
-                                         s + lal::S_ALPHA, W0.dinv, fast ? W0.x : nullptr,
-                                         nullptr));
-            LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM, &seq));
+            LAL_TRY(lal::update_xr<T, T>(c, n, p, q, x, res, h->part_pq, n_pq,
+                                         s + lal::S_GAMMA + cur, h->part_r, s + lal::S_ALPHA,
+                                         W0.dinv, fast ? W0.x : nullptr, nullptr));
             // The next preconditioner application depends on r only: it is
             // queued before the host looks at the norm, so the GPU does not
             // wait for the convergence test -- unless the observed rate of
             // reduction predicts that this step converges, when the host
             // decides first so that no V-cycle is spent after the last step.
             const bool near = lal::near_tolerance(r_prev, rate, init, rel_tol, abs_tol);
-            if(!near)
-                LAL_TRY(apply(fast));
+            LAL_TRY(near ? post_norm(h, n_r, lal::S_RNORM, &seq) : apply(fast, &seq));
             LAL_TRY(wait_scalar(h, seq, lal::S_RNORM, &rn));
             lal::observe_rate(rn, &r_prev, &rate);
             if(std::isnan(rn))
@@ -620,9 +667,9 @@ namespace
                 break;
             }
             if(near)
-                LAL_TRY(apply(fast));
-            LAL_TRY(lal::dot_partials<T, T>(c, n, z, res, part_g[cur ^ 1]));
-            LAL_TRY(lal::update_p<T, T>(c, n, z, p, part_g[cur ^ 1], part_g[cur]));
+                LAL_TRY(apply(fast, nullptr));
+            LAL_TRY(lal::update_p<T, T>(c, n, z, p, h->part_g, n_g, s + lal::S_GAMMA + cur,
+                                        s + lal::S_GAMMA + (cur ^ 1)));
             cur ^= 1;
             iter++;
         }
@@ -660,21 +707,23 @@ namespace
         float*         r32 = h->res32;
         float*         z32 = h->z32;
         LAL_TRY(lal::residual_f64(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, x, b, res));
-        double*  part_pq   = h->part;
-        double*  part_g[2] = {h->part + lal::PCG_BLOCKS, h->part + 2 * lal::PCG_BLOCKS};
-        double*  part_r    = h->part + 3 * lal::PCG_BLOCKS;
         unsigned seq       = 0;
         double   init      = 0.0;
-        LAL_TRY(lal::norm_partials<double>(c, n, res, part_r));
-        LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM0, &seq));
+        LAL_TRY(lal::norm_partials<double>(c, n, res, h->part_r));
+        LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM0, &seq));
         LAL_TRY(wait_scalar(h, seq, lal::S_RNORM0, &init));
         const double sigma = init > 0.0 && std::isfinite(init) ? std::ldexp(1.0, -std::ilogb(init))
                                                                : 1.0;
         LAL_TRY(lal::scale_cast_f64_f32(c, n, res, sigma, r32));
-        LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2));
+        int       n_pq = 0, n_g = 0;
+        const int n_r   = lal::update_blocks(n);
+        auto      apply = [&](bool xinit, unsigned* norm) {
+            return apply_dot<float, double>(h, r32, z32, res, n1, n2, xinit, n_r, norm, &n_g);
+        };
+        LAL_TRY(apply(false, nullptr));
         LAL_TRY(lal_convert_f32_f64(c, z32, p, (size_t)n));
-        int cur = 0;
-        LAL_TRY(lal::dot_partials<float, double>(c, n, z32, res, part_g[cur]));
+        int cur = 0; // generation of s[S_GAMMA]
+        LAL_TRY(lal::finish_partials(c, 0, {h->part_g, n_g, s + lal::S_GAMMA}));
         double       rn   = init;
         int          iter = 0;
         bool         conv = false;
@@ -683,15 +732,14 @@ namespace
         double       r_prev = init, rate = 0.5;
         while(!(iter > max_iter))
         {
-            LAL_TRY(lal::csrmv(c, A.d, n, A.n, A.nnz, 1.0, A.rp, A.ci, A.v, p, 0.0, q));
-            LAL_TRY(lal::dot_partials<double, double>(c, n, q, p, part_pq));
-            LAL_TRY(lal::update_xr<double, float>(c, n, p, q, x, res, part_pq, part_g[cur],
-                                                  part_r, s + lal::S_ALPHA, W0.dinv,
+            LAL_TRY(lal::product_dot<double>(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, p, q,
+                                             h->part_pq, &n_pq));
+            LAL_TRY(lal::update_xr<double, float>(c, n, p, q, x, res, h->part_pq, n_pq,
+                                                  s + lal::S_GAMMA + cur, h->part_r,
+                                                  s + lal::S_ALPHA, W0.dinv,
                                                   fast ? W0.x : nullptr, r32, sigma));
-            LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM, &seq));
             const bool near = lal::near_tolerance(r_prev, rate, init, rel_tol, abs_tol);
-            if(!near)
-                LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2, fast));
+            LAL_TRY(near ? post_norm(h, n_r, lal::S_RNORM, &seq) : apply(fast, &seq));
             LAL_TRY(wait_scalar(h, seq, lal::S_RNORM, &rn));
             lal::observe_rate(rn, &r_prev, &rate);
             if(std::isnan(rn))
@@ -702,9 +750,10 @@ namespace
                 break;
             }
             if(near)
-                LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2, fast));
-            LAL_TRY(lal::dot_partials<float, double>(c, n, z32, res, part_g[cur ^ 1]));
-            LAL_TRY(lal::update_p<float, double>(c, n, z32, p, part_g[cur ^ 1], part_g[cur]));
+                LAL_TRY(apply(fast, nullptr));
+            LAL_TRY(lal::update_p<float, double>(c, n, z32, p, h->part_g, n_g,
+                                                 s + lal::S_GAMMA + cur,
+                                                 s + lal::S_GAMMA + (cur ^ 1)));
             cur ^= 1;
             iter++;
         }
@@ -750,14 +799,11 @@ namespace
         float*         p32   = h->p32;
         float*         q32   = h->q32;
         float*         y32   = h->d32;
-        double*        part_pq   = h->part;
-        double*        part_g[2] = {h->part + lal::PCG_BLOCKS, h->part + 2 * lal::PCG_BLOCKS};
-        double*        part_r    = h->part + 3 * lal::PCG_BLOCKS;
         unsigned       seq       = 0;
         double         init      = 0.0;
         LAL_TRY(lal::residual_f64(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, x, b, r64));
-        LAL_TRY(lal::norm_partials<double>(c, n, r64, part_r));
-        LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM0, &seq));
+        LAL_TRY(lal::norm_partials<double>(c, n, r64, h->part_r));
+        LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM0, &seq));
         LAL_TRY(wait_scalar(h, seq, lal::S_RNORM0, &init));
         double rn   = init; // true or recursive inf-norm, unscaled
         int    iter = 0, updates = 0;
@@ -767,24 +813,28 @@ namespace
             const double sigma = 1.0 / init;
             LAL_TRY(lal::scale_cast_f64_f32(c, n, r64, sigma, r32));
             LAL_HIP(hipMemsetAsync(y32, 0, sizeof(float) * n, c->stream));
-            LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2));
+            int       n_pq = 0, n_g = 0;
+            const int n_r   = lal::update_blocks(n);
+            auto      apply = [&](bool xinit, unsigned* norm) {
+                return apply_dot<float, float>(h, r32, z32, r32, n1, n2, xinit, n_r, norm, &n_g);
+            };
+            LAL_TRY(apply(false, nullptr));
             LAL_HIP(hipMemcpyAsync(p32, z32, sizeof(float) * n, hipMemcpyDeviceToDevice,
                                    c->stream));
-            int cur = 0;
-            LAL_TRY(lal::dot_partials<float, float>(c, n, z32, r32, part_g[cur]));
+            int cur = 0; // generation of s[S_GAMMA]
+            LAL_TRY(lal::finish_partials(c, 0, {h->part_g, n_g, s + lal::S_GAMMA}));
             const bool   fast  = !h->opts.exact && n1 == 1 && h->levels > 0;
             work<float>& W0    = h->w<float>(0);
             double       r_upd  = init; // true residual norm at the last update
             double       r_prev = init, rate = 0.5; // last norm, observed reduction per step
             while(!(iter > max_iter))
             {
-                LAL_TRY(lal::csrmv(c, A.d, n, A.n, A.nnz, 1.0, A.rp, A.ci, Av32, p32, 0.0,
-                                   q32));
-                LAL_TRY(lal::dot_partials<float, float>(c, n, q32, p32, part_pq));
-                LAL_TRY(lal::update_xr<float, float>(c, n, p32, q32, y32, r32, part_pq,
-                                                     part_g[cur], part_r, s + lal::S_ALPHA,
-                                                     W0.dinv, fast ? W0.x : nullptr, nullptr));
-                LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM, &seq));
+                LAL_TRY(lal::product_dot<float>(c, A.d, n, A.n, A.nnz, A.rp, A.ci, Av32, p32, q32,
+                                                h->part_pq, &n_pq));
+                LAL_TRY(lal::update_xr<float, float>(c, n, p32, q32, y32, r32, h->part_pq, n_pq,
+                                                     s + lal::S_GAMMA + cur, h->part_r,
+                                                     s + lal::S_ALPHA, W0.dinv,
+                                                     fast ? W0.x : nullptr, nullptr));
                 // The next V-cycle is queued before the host reads the norm,
                 // unless the observed rate of reduction predicts that this step
                 // crosses the update threshold: then the host decides first, so
@@ -792,8 +842,7 @@ namespace
                 const double threshold = std::max(std::max(delta * r_upd, rel_tol * init),
                                                   abs_tol);
                 const bool   near      = lal::near_threshold(r_prev, rate, threshold);
-                if(!near)
-                    LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2, fast));
+                LAL_TRY(near ? post_norm(h, n_r, lal::S_RNORM, &seq) : apply(fast, &seq));
                 double rs = 0.0;
                 LAL_TRY(wait_scalar(h, seq, lal::S_RNORM, &rs));
                 rn = rs * init;
@@ -809,8 +858,8 @@ namespace
                     LAL_HIP(hipMemsetAsync(y32, 0, sizeof(float) * n, c->stream));
                     LAL_TRY(lal::residual_f64(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, x, b,
                                               r64));
-                    LAL_TRY(lal::norm_partials<double>(c, n, r64, part_r));
-                    LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM, &seq));
+                    LAL_TRY(lal::norm_partials<double>(c, n, r64, h->part_r));
+                    LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM, &seq));
                     LAL_TRY(lal::scale_cast_f64_f32(c, n, r64, sigma, r32));
                     LAL_TRY(wait_scalar(h, seq, lal::S_RNORM, &rn));
                     updates++;
@@ -831,17 +880,21 @@ namespace
                         conv = true;
                         break;
                     }
-                    LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2));
+                    LAL_TRY(apply(false, nullptr));
                 }
                 else if(near)
-                    LAL_TRY(precond_graphed<float>(h, r32, z32, n1, n2, fast));
-                LAL_TRY(lal::dot_partials<float, float>(c, n, z32, r32, part_g[cur ^ 1]));
+                    LAL_TRY(apply(fast, nullptr));
                 if(restart)
+                {
                     LAL_HIP(hipMemcpyAsync(p32, z32, sizeof(float) * n, hipMemcpyDeviceToDevice,
                                            c->stream));
+                    LAL_TRY(lal::finish_partials(c, 0,
+                                                 {h->part_g, n_g, s + lal::S_GAMMA + (cur ^ 1)}));
+                }
                 else
-                    LAL_TRY(lal::update_p<float, float>(c, n, z32, p32, part_g[cur ^ 1],
-                                                        part_g[cur]));
+                    LAL_TRY(lal::update_p<float, float>(c, n, z32, p32, h->part_g, n_g,
+                                                        s + lal::S_GAMMA + cur,
+                                                        s + lal::S_GAMMA + (cur ^ 1)));
                 cur ^= 1;
                 iter++;
             }
@@ -891,13 +944,14 @@ namespace lal
         return false;
     }
 
-    // Reduces PCG_BLOCKS partials (op 0 sum, 1 max) into s[slot] and hands the
-    // value to the host through the mapped note; returns the sequence number
-    // to wait for.
-    int post_scalar(lal_hierarchy_t* h, int op, const double* part, int slot, unsigned* seq)
+    int post_norm(lal_hierarchy_t* h, int count, int slot, unsigned* seq, post_args* later)
     {
+        const post_args a{h->part_r, count, h->s + slot, h->d_note, h->d_seq, h->d_count};
         *seq = ++h->seq;
-        return lal::finish_partials(h->c, op, part, h->s + slot, h->d_note, h->d_seq, *seq);
+        if(later == nullptr)
+            return finish_partials(h->c, 1, a);
+        *later = a;
+        return LAL_OK;
     }
 
     // Waits until the note carries `seq`.  The host polls the mapped word
@@ -1191,11 +1245,10 @@ extern "C" int lal_ir_solve(lal_handle c, lal_hierarchy h, const double* b, doub
     const int      n = A.m;
     double*        r = h->q; // FP64 outer residual lives in the FP64 q buffer
     LAL_TRY(lal::residual_f64(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, x, b, r));
-    double*  part_r = h->part + 3 * lal::PCG_BLOCKS;
     unsigned seq    = 0;
     double   init   = 0.0;
-    LAL_TRY(lal::norm_partials<double>(c, n, r, part_r));
-    LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM0, &seq));
+    LAL_TRY(lal::norm_partials<double>(c, n, r, h->part_r));
+    LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM0, &seq));
     LAL_TRY(wait_scalar(h, seq, lal::S_RNORM0, &init));
     double rn    = init;
     int    outer = 0, inner_total = 0;
@@ -1221,8 +1274,8 @@ extern "C" int lal_ir_solve(lal_handle c, lal_hierarchy h, const double* b, doub
         // x += |r| d in FP64, then the true FP64 residual
         LAL_TRY(lal::axpy_f32_f64(c, n, rn, h->d32, x));
         LAL_TRY(lal::residual_f64(c, A.d, n, A.n, A.nnz, A.rp, A.ci, A.v, x, b, r));
-        LAL_TRY(lal::norm_partials<double>(c, n, r, part_r));
-        LAL_TRY(post_scalar(h, 1, part_r, lal::S_RNORM, &seq));
+        LAL_TRY(lal::norm_partials<double>(c, n, r, h->part_r));
+        LAL_TRY(post_norm(h, lal::PCG_BLOCKS, lal::S_RNORM, &seq));
         LAL_TRY(wait_scalar(h, seq, lal::S_RNORM, &rn));
         outer++;
         if(std::isnan(rn))

@@ -32,10 +32,12 @@
 //   SMOOTHED  y = b - A x and r = x + y * dinv  (residual, and the sweep that
 //                                           uses it)
 //   ADD       y = b + A x
+//   SPMV_DOT  y = A x, ADD_DOT  y = b + A x, and one partial of <w, y> per row
+//             block (PCG's inner products without a pass of their own)
 // dinv holds 1/a_ii, so no division is left in the inner loops.
 #pragma once
 
-#include "lal_spmv.h"
+#include "lal_reduce.h"
 
 namespace lal
 {
@@ -48,7 +50,28 @@ namespace lal
         RV_RESTRICT = 4, // y = A x and r = y * dinv: the coarse right-hand side
                          // and the first Jacobi iterate from zero on it
         RV_SMOOTHED = 5,
-        RV_ADD      = 6
+        RV_ADD      = 6,
+        RV_SPMV_DOT = 7,
+        RV_ADD_DOT  = 8
+    };
+
+    // Partials of one reduction at most: a product with more row blocks leaves
+    // its inner product to a kernel of its own.  Every block of the next kernel
+    // adds the partials up again; with fused products the solver saves a pass
+    // over two vectors and a launch (2.6 us each at 16,384 rows, 128^2 Poisson
+    // 52 -> 44 us per iteration together with the folded norm).  Up to 4096
+    // partials nothing measured is slower than with 512 (PCG on 64^3 16.15 ->
+    // 16.05 ms, on 101^3 even); 16384 cost 128^3 in FP32 1.3 %.
+    constexpr int PCG_PARTS = 4096;
+
+    // What a product does besides its own rows.
+    struct row_extra
+    {
+        double*     part = nullptr; // *_DOT: one partial of <w, y> per row block
+        const void* w    = nullptr; // m entries, FP64 with `wide`, else of the product's type
+        bool        wide = false;
+        // SMOOTHED: a last workgroup finishes the reduction before it
+        post_args post{};
     };
 
     struct rv_args
@@ -79,6 +102,7 @@ namespace lal
         const int*            lmeta    = nullptr;
         int                   list_max = 0;
         bool                  list_far = false;
+        row_extra             ex{};
     };
 
     // The descriptor's 16-bit columns and column lists into a's fields.
@@ -93,6 +117,9 @@ namespace lal
         a.list_far = d->list_far;
     }
 
+    int finish_partials(lal_context* c, int op, const post_args& a);
     template <typename T>
     int rowvec_launch(lal_context* c, int mode, const rv_args& a);
+    // True where rowvec_launch has a kernel for this *_DOT mode and matrix.
+    bool rowvec_can_dot(int mode, const rv_args& a);
 }

@@ -80,7 +80,8 @@ namespace
     template <typename T>
     struct row_operands
     {
-        T b = 0, d = 0, x = 0, y = 0;
+        T      b = 0, d = 0, x = 0, y = 0;
+        double w = 0;
     };
 
     template <typename T, int MODE>
@@ -88,13 +89,17 @@ namespace
                                                              const T* __restrict__ x,
                                                              const T* __restrict__ d,
                                                              const T* __restrict__ b, T beta,
-                                                             const T* __restrict__ y)
+                                                             const T* __restrict__ y,
+                                                             const lal::row_extra& ex = {})
     {
         row_operands<T> o;
         if(!on)
             return o;
+        if(MODE == lal::RV_SPMV_DOT || MODE == lal::RV_ADD_DOT)
+            o.w = ex.wide ? static_cast<const double*>(ex.w)[row]
+                          : (double)static_cast<const T*>(ex.w)[row];
         if(MODE == lal::RV_RESIDUAL || MODE == lal::RV_JACOBI || MODE == lal::RV_JACOBI0 ||
-           MODE == lal::RV_SMOOTHED || MODE == lal::RV_ADD)
+           MODE == lal::RV_SMOOTHED || MODE == lal::RV_ADD || MODE == lal::RV_ADD_DOT)
             o.b = b[row];
         if(MODE == lal::RV_JACOBI || MODE == lal::RV_JACOBI0 || MODE == lal::RV_RESTRICT ||
            MODE == lal::RV_SMOOTHED)
@@ -135,6 +140,21 @@ namespace
             y[row] = o.b * o.d;
             r[row] = o.b - acc;
         }
+    }
+
+    // The *_DOT epilogue, by the whole block: y of the lanes that end a row
+    // (`head`), and the block's partial of <w, y> in FP64.
+    template <typename T, int MODE>
+    __device__ __forceinline__ void dot_epilogue(bool head, int row, T acc,
+                                                 const row_operands<T>& o, T* __restrict__ y,
+                                                 double* __restrict__ part)
+    {
+        const T v = MODE == lal::RV_ADD_DOT ? o.b + acc : acc;
+        if(head)
+            y[row] = v;
+        const double t = lal::block_total<0>(head ? o.w * (double)v : 0.0);
+        if(threadIdx.x == 0)
+            *part = t;
     }
 
     template <typename T, int MODE>
@@ -282,8 +302,14 @@ namespace
                     const unsigned short* __restrict__ c16, const int* __restrict__ cbase,
                     const T* __restrict__ val, const T* __restrict__ x,
                     const T* __restrict__ d, const T* __restrict__ b, T alpha, T beta,
-                    T* __restrict__ y, T* __restrict__ r)
+                    T* __restrict__ y, T* __restrict__ r, lal::row_extra ex)
     {
+        if(MODE == lal::RV_SMOOTHED && (int)blockIdx.x == nb)
+        {
+            // (the grid has this workgroup only with ex.post)
+            lal::post_block<1>(ex.post);
+            return;
+        }
         // the block's row starts, then win entries of columns, then win
         // values (win: a multiple of 4)
         extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
@@ -312,7 +338,7 @@ namespace
         // descriptor's base and end, lane i loads rp[r0 + i] for 0 < i < nrows.
         const int rpv = (tid > 0 && tid < nrows) ? rp[r0 + tid] : 0;
         const row_operands<T> ops =
-            load_operands<T, MODE>(active && lig == 0, row, x, d, b, beta, y);
+            load_operands<T, MODE>(active && lig == 0, row, x, d, b, beta, y, ex);
         int       rs = 0, re = 0;
         bool      bounds = false;
 
@@ -380,6 +406,11 @@ namespace
         }
         if(g > 1)
             acc = lal::group_sum(acc, g);
+        if(MODE == lal::RV_SPMV_DOT)
+        {
+            dot_epilogue<T, MODE>(active && lig == 0, row, acc, ops, y, ex.part + tile);
+            return;
+        }
         if(!active || lig != 0)
             return;
         row_epilogue<T, MODE>(row, acc, ops, alpha, beta, y, r);
@@ -583,7 +614,7 @@ namespace
                     const unsigned short* __restrict__ list, const int* __restrict__ lmeta,
                     const T* __restrict__ val, const T* __restrict__ x, const T* __restrict__ d,
                     const T* __restrict__ b, T alpha, T beta, T* __restrict__ y,
-                    T* __restrict__ r)
+                    T* __restrict__ r, lal::row_extra ex)
     {
         typedef int int2v __attribute__((ext_vector_type(2)));
         // the block's row starts, its x entries, then its products
@@ -628,7 +659,7 @@ namespace
         const bool on   = lrow < nrows;
         const bool head = on && (tid & ((1u << lg) - 1u)) == 0;
         const int  rpv  = rp[r0 + min((int)tid, nrows)];
-        const row_operands<T> ops = load_operands<T, MODE>(head, r0 + lrow, x, d, b, beta, y);
+        const row_operands<T> ops = load_operands<T, MODE>(head, r0 + lrow, x, d, b, beta, y, ex);
         // (a list of odd length repeats its last column once more)
         T xv[LIST_U][2];
 #pragma unroll
@@ -681,63 +712,80 @@ namespace
                               s_rp[lrow + 1] - ws, 1 << lg);
         if(lg > 0)
             acc = lal::group_sum(acc, 1 << lg);
-        if(head)
+        if(MODE == lal::RV_ADD_DOT)
+            dot_epilogue<T, MODE>(head, r0 + lrow, acc, ops, y, ex.part + tile);
+        else if(head)
             row_epilogue<T, MODE>(r0 + lrow, acc, ops, alpha, beta, y, r);
     }
 
     template <typename T, int MODE, bool C16>
-    void launch_staged(lal_context* c, const lal::rv_args& a, int nb)
+    void launch_quad(lal_context* c, const lal::rv_args& a, int nb)
     {
         // LDS sized to the widest block window of this matrix, so that short
         // blocks leave room for more resident workgroups
         const int    win  = a.win;
         const size_t cbyt = C16 ? sizeof(unsigned short) : sizeof(int);
-        if(a.by_nnz)
-            quad_nnz_kernel<T, MODE, C16><<<nb, SPMV_THREADS, RP_LDS_BYTES + sizeof(T) * win,
-                                           c->stream>>>(
-                a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
-                (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y,
-                (T*)a.r);
-        else if(a.keep && (sizeof(T) + cbyt) * (size_t)a.nnz <= lal::CACHE_KEEP_BYTES)
-            quad_kernel<T, MODE, true, C16><<<nb, SPMV_THREADS,
-                                              RP_LDS_BYTES + (sizeof(int) + sizeof(T)) * win,
-                                              c->stream>>>(
-                a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
-                (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y,
-                (T*)a.r);
-        else
-            quad_kernel<T, MODE, false, C16><<<nb, SPMV_THREADS,
-                                               RP_LDS_BYTES + (sizeof(int) + sizeof(T)) * win,
-                                               c->stream>>>(
-                a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
-                (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y,
-                (T*)a.r);
+        const bool   keep = a.keep && (sizeof(T) + cbyt) * (size_t)a.nnz <= lal::CACHE_KEEP_BYTES;
+        auto*        fn   = keep ? quad_kernel<T, MODE, true, C16> : quad_kernel<T, MODE, false, C16>;
+        const int    more = MODE == lal::RV_SMOOTHED && a.ex.post.part ? 1 : 0;
+        fn<<<nb + more, SPMV_THREADS, RP_LDS_BYTES + (sizeof(int) + sizeof(T)) * win, c->stream>>>(
+            a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
+            (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r,
+            a.ex);
+    }
+
+    template <typename T, int MODE>
+    void launch_list(lal_context* c, const lal::rv_args& a, int nb)
+    {
+        const int    lm  = (a.list_max + 3) & ~3;
+        const size_t lds = RP_LDS_BYTES + sizeof(T) * (size_t)(lm + a.win);
+        auto* fn = a.list_far ? list_kernel<T, MODE, true> : list_kernel<T, MODE, false>;
+        fn<<<nb, SPMV_THREADS, lds, c->stream>>>(
+            a.blocks, nb, lm, a.rp, a.lpos, a.list, a.lmeta, (const T*)a.val, (const T*)a.x,
+            (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r, a.ex);
+    }
+
+    // Which kernel reads a matrix.
+    enum
+    {
+        BY_STAGED, // unaligned arrays
+        BY_LIST,   // x through LDS by column lists
+        BY_NNZ,    // gathers over consecutive nonzeros
+        BY_QUAD
+    };
+    int route(const lal::rv_args& a)
+    {
+        const bool val16 = (reinterpret_cast<uintptr_t>(a.val) & 15) == 0;
+        const bool cols  = (a.c16 && a.cbase) || (reinterpret_cast<uintptr_t>(a.ci) & 15) == 0;
+        if(!a.blocks || !val16)
+            return BY_STAGED;
+        if(a.list_max > 0)
+            return BY_LIST;
+        return !cols ? BY_STAGED : a.by_nnz ? BY_NNZ : BY_QUAD;
     }
 
     template <typename T, int MODE>
     int launch(lal_context* c, const lal::rv_args& a)
     {
-        const int nb = a.blocks ? a.nb : (a.m + SPMV_THREADS - 1) / SPMV_THREADS;
+        const int  nb  = a.blocks ? a.nb : (a.m + SPMV_THREADS - 1) / SPMV_THREADS;
+        const int  by  = route(a);
+        const bool c16 = a.c16 && a.cbase;
+        if(a.ex.post.part && (MODE != lal::RV_SMOOTHED || by != BY_QUAD || nb == 0))
+            LAL_TRY(lal::finish_partials(c, 1, a.ex.post));
         if(nb == 0)
             return LAL_OK;
-        const bool val16 = (reinterpret_cast<uintptr_t>(a.val) & 15) == 0;
-        if(a.blocks && val16 && a.list_max > 0)
+        if(by == BY_LIST)
+            launch_list<T, MODE>(c, a, nb);
+        else if(by == BY_QUAD)
+            c16 ? launch_quad<T, MODE, true>(c, a, nb) : launch_quad<T, MODE, false>(c, a, nb);
+        else if(by == BY_NNZ)
         {
-            const int    lm  = (a.list_max + 3) & ~3;
-            const size_t lds = RP_LDS_BYTES + sizeof(T) * (size_t)(lm + a.win);
-            auto*        fn  = a.list_far ? list_kernel<T, MODE, true>
-                                          : list_kernel<T, MODE, false>;
-            fn<<<nb, SPMV_THREADS, lds, c->stream>>>(
-                a.blocks, nb, lm, a.rp, a.lpos, a.list, a.lmeta, (const T*)a.val,
+            auto* fn = c16 ? quad_nnz_kernel<T, MODE, true> : quad_nnz_kernel<T, MODE, false>;
+            fn<<<nb, SPMV_THREADS, RP_LDS_BYTES + sizeof(T) * a.win, c->stream>>>(
+                a.m, a.nnz, a.blocks, nb, a.win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
                 (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y,
                 (T*)a.r);
-            LAL_LAUNCHED();
-            return LAL_OK;
         }
-        if(a.blocks && val16 && a.c16 && a.cbase)
-            launch_staged<T, MODE, true>(c, a, nb);
-        else if(a.blocks && val16 && (reinterpret_cast<uintptr_t>(a.ci) & 15) == 0)
-            launch_staged<T, MODE, false>(c, a, nb);
         else
             staged_kernel<T, MODE><<<nb, SPMV_THREADS, 0, c->stream>>>(
                 a.m, a.blocks, nb, a.rp, a.ci, (const T*)a.val, (const T*)a.x, (const T*)a.d,
@@ -745,10 +793,30 @@ namespace
         LAL_LAUNCHED();
         return LAL_OK;
     }
+
+    // (rowvec_can_dot holds)
+    template <typename T>
+    int launch_dot(lal_context* c, int mode, const lal::rv_args& a)
+    {
+        if(mode == lal::RV_ADD_DOT)
+            launch_list<T, lal::RV_ADD_DOT>(c, a, a.nb);
+        else if(a.c16 && a.cbase)
+            launch_quad<T, lal::RV_SPMV_DOT, true>(c, a, a.nb);
+        else
+            launch_quad<T, lal::RV_SPMV_DOT, false>(c, a, a.nb);
+        LAL_LAUNCHED();
+        return LAL_OK;
+    }
 }
 
 namespace lal
 {
+    bool rowvec_can_dot(int mode, const rv_args& a)
+    {
+        return a.blocks && a.nb > 0 && a.nb <= PCG_PARTS &&
+               route(a) == (mode == RV_ADD_DOT ? BY_LIST : BY_QUAD);
+    }
+
     template <typename T>
     int rowvec_launch(lal_context* c, int mode, const rv_args& a)
     {
@@ -760,6 +828,10 @@ namespace lal
         case RV_JACOBI: return launch<T, RV_JACOBI>(c, a);
         case RV_SMOOTHED: return launch<T, RV_SMOOTHED>(c, a);
         case RV_ADD: return launch<T, RV_ADD>(c, a);
+        case RV_SPMV_DOT:
+        case RV_ADD_DOT:
+            LAL_REQUIRE(rowvec_can_dot(mode, a) && a.ex.part != nullptr && a.ex.w != nullptr);
+            return launch_dot<T>(c, mode, a);
         default: return launch<T, RV_JACOBI0>(c, a);
         }
     }

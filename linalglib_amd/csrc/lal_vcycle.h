@@ -8,10 +8,8 @@ namespace lal
     // Device scalar slots of one solver (an array of LAL_SOLVER_SLOTS doubles).
     enum
     {
-        S_GAMMA  = 0, // <z, r>
-        S_PQ     = 1, // <A p, p>
+        S_GAMMA  = 0, // <z, r>, two generations
         S_ALPHA  = 2,
-        S_BETA   = 3,
         S_RNORM  = 4, // inf-norm of the recursively updated residual
         S_RNORM0 = 5,
         S_TMP    = 6,
@@ -46,8 +44,13 @@ namespace lal
         return csrmv_f32(c, d, m, n, nnz, (float)alpha, rp, ci, v, x, (float)beta, y);
     }
 
-    // Grid of the PCG reduction and update kernels (one partial per block).
+    // Grid of the PCG reduction kernels, and of the update kernels at most
+    // (one partial per block).
     constexpr int PCG_BLOCKS = 512;
+    inline int update_blocks(int n)
+    {
+        return grid_for(n, SPMV_THREADS, PCG_BLOCKS);
+    }
 
     template <typename T>
     int jacobi_sweep(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
@@ -58,11 +61,18 @@ namespace lal
     template <typename T>
     int residual_smoothed(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                           const int* ci, const T* v, const T* x, const T* dinv, const T* b, T* r,
-                          T* y);
-    // out = y + Q e (fast descriptors)
+                          T* y, const post_args& post = {});
+    // out = y + Q e (fast descriptors); with ex.part also <ex.w, out>'s partials
+    // (can_add_dot)
     template <typename T>
     int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
-                    const T* v, const T* e, const T* y, T* out);
+                    const T* v, const T* e, const T* y, T* out, const row_extra& ex = {});
+    template <typename T>
+    bool can_add_dot(const lal_csrmv_info* d, int m, const int* rp, const int* ci, const T* v);
+    // y = A x and *count partials of <y, x> in part (PCG_PARTS at most)
+    template <typename T>
+    int product_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, int nnz, const int* rp,
+                    const int* ci, const T* v, const T* x, T* y, double* part, int* count);
     // AP's values become those of Q = P - D^-1 A P (pattern of A P, a superset
     // of P's; both with ascending columns); v32 (or null): the same in FP32.
     int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
@@ -92,16 +102,15 @@ namespace lal
     int dot_partials(lal_context* c, int n, const TX* x, const TY* y, double* part);
     template <typename T>
     int norm_partials(lal_context* c, int n, const T* x, double* part);
-    // op 0: sum, 1: max of the partials into *slot (device) and, when host_val
-    // is given (mapped pinned memory), into *host_val then *host_seq = seq.
-    int finish_partials(lal_context* c, int op, const double* part, double* slot,
-                        double* host_val, unsigned* host_seq, unsigned seq);
-    // x += alpha p, r -= alpha q, partial max|r|; with x0 also
+    // op 0: sum, 1: max of a reduction's partials (post_args)
+    int finish_partials(lal_context* c, int op, const post_args& a);
+    // alpha = *gamma / sum of part_pq; x += alpha p, r -= alpha q,
+    // update_blocks(n) partials of max|r|; with x0 also
     // x0 = (S)(r * rs_scale) * dinv, with rs also rs = (S)(r * rs_scale) (the
     // preconditioner's precision S; rs_scale = 1 leaves r as it is).
     template <typename T, typename S>
     int update_xr(lal_context* c, int n, const T* p, const T* q, T* x, T* r,
-                  const double* part_pq, const double* part_gamma, double* part_r,
+                  const double* part_pq, int n_pq, const double* gamma, double* part_r,
                   double* s_alpha, const S* dinv, S* x0, S* rs, double rs_scale = 1.0);
     // x = b * dinv
     template <typename T>
@@ -110,9 +119,10 @@ namespace lal
     template <typename T>
     int restrict_init(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                       const int* ci, const T* v, const T* r, const T* dinv_c, T* b_c, T* x_c);
+    // *gamma_new = sum of part_new; p = z + (*gamma_new / *gamma_old) p
     template <typename TZ, typename T>
-    int update_p(lal_context* c, int n, const TZ* z, T* p, const double* part_new,
-                 const double* part_old);
+    int update_p(lal_context* c, int n, const TZ* z, T* p, const double* part_new, int n_new,
+                 const double* gamma_old, double* gamma_new);
     int scale_cast_f64_f32(lal_context* c, int n, const double* x, double scale, float* y);
     int axpy_f32_f64(lal_context* c, int n, double alpha, const float* d, double* x);
 }

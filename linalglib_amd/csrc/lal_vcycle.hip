@@ -262,41 +262,8 @@ namespace
     }
 
     // ---------------------------------------------------- PCG vector updates
-    // OP 0: sum; OP 1: maximum that keeps a NaN from either side, so that a
-    // NaN anywhere in a vector reaches the solver's norm (and stops it)
-    // whatever the order of the combination.
-    template <int OP>
-    __device__ __forceinline__ double combine(double a, double b)
-    {
-        return OP == 0 ? a + b : ((a != a || b < a) ? a : b);
-    }
-
-    // Block total of one value per lane (all lanes receive it).
-    template <int OP>
-    __device__ double block_total(double v)
-    {
-        __shared__ double sh[SPMV_THREADS / 64];
-        v = OP == 0 ? lal::wave_sum(v) : lal::wave_max_nan(v);
-        __syncthreads();
-        if((threadIdx.x & 63) == 0)
-            sh[threadIdx.x >> 6] = v;
-        __syncthreads();
-        double t = sh[0];
-#pragma unroll
-        for(int w = 1; w < SPMV_THREADS / 64; w++)
-            t = combine<OP>(t, sh[w]);
-        return t;
-    }
-
-    // Sum of the RB partials of a previous reduction, identical in every block.
-    __device__ double sum_partials(const double* __restrict__ part)
-    {
-        double v = 0.0;
-#pragma unroll
-        for(int k = threadIdx.x; k < RB; k += SPMV_THREADS)
-            v += part[k];
-        return block_total<0>(v);
-    }
+    using lal::block_total;
+    using lal::combine;
 
     // part[block] = partial of sum x_i*y_i (OP 0) or max |x_i| (OP 1); x and y
     // may differ in precision (FP32 preconditioned vector, FP64 residual).
@@ -330,26 +297,10 @@ namespace
             part[blockIdx.x] = t;
     }
 
-    // One block: total of RB partials into a device slot and, when given, a
-    // mapped host word (followed by a sequence number the host polls).
     template <int OP>
-    __global__ void __launch_bounds__(SPMV_THREADS)
-        finish_kernel(const double* __restrict__ part, double* __restrict__ slot,
-                      double* host_val, unsigned* host_seq, unsigned seq)
+    __global__ void __launch_bounds__(SPMV_THREADS) finish_kernel(lal::post_args a)
     {
-        double v = OP == 0 ? 0.0 : 0.0;
-        for(int k = threadIdx.x; k < RB; k += SPMV_THREADS)
-            v = combine<OP>(v, part[k]);
-        const double t = block_total<OP>(v);
-        if(threadIdx.x == 0)
-        {
-            *slot = t;
-            if(host_val)
-            {
-                __hip_atomic_store(host_val, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-        }
+        lal::post_block<OP>(a);
     }
 
     // alpha = gamma / <q, p>; x += alpha p; r += (-1*alpha) q (cg.cpp:185-193);
@@ -361,16 +312,15 @@ namespace
     __global__ void __launch_bounds__(SPMV_THREADS)
         update_xr_kernel(int n, const T* __restrict__ p, const T* __restrict__ q,
                          T* __restrict__ x, T* __restrict__ r,
-                         const double* __restrict__ part_pq,
-                         const double* __restrict__ part_gamma, double* __restrict__ part_r,
+                         const double* __restrict__ part_pq, int n_pq,
+                         const double* __restrict__ gamma, double* __restrict__ part_r,
                          double* __restrict__ s_alpha, const S* __restrict__ dinv,
                          S* __restrict__ x0, S* __restrict__ rs, T rs_scale)
     {
         const int stride = gridDim.x * SPMV_THREADS;
         int       i      = blockIdx.x * SPMV_THREADS + threadIdx.x;
-        const double pq    = sum_partials(part_pq);
-        const double gamma = sum_partials(part_gamma);
-        const double alpha = gamma / pq;
+        const double pq    = lal::total_of<0>(part_pq, n_pq);
+        const double alpha = *gamma / pq;
         if(blockIdx.x == 0 && threadIdx.x == 0)
             *s_alpha = alpha;
         const T a  = (T)alpha;
@@ -416,11 +366,13 @@ namespace
     template <typename TZ, typename T>
     __global__ void __launch_bounds__(SPMV_THREADS)
         update_p_kernel(int n, const TZ* __restrict__ z, T* __restrict__ p,
-                        const double* __restrict__ part_new,
-                        const double* __restrict__ part_old)
+                        const double* __restrict__ part_new, int n_new,
+                        const double* __restrict__ gamma_old, double* __restrict__ gamma_new)
     {
-        const double g_new = sum_partials(part_new);
-        const double g_old = sum_partials(part_old);
+        const double g_new = lal::total_of<0>(part_new, n_new);
+        const double g_old = *gamma_old;
+        if(blockIdx.x == 0 && threadIdx.x == 0)
+            *gamma_new = g_new;
         const T      beta  = (T)(g_new / g_old);
         const int    stride = gridDim.x * SPMV_THREADS;
         int          i      = blockIdx.x * SPMV_THREADS + threadIdx.x;
@@ -572,27 +524,66 @@ namespace lal
     template <typename T>
     int residual_smoothed(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                           const int* ci, const T* v, const T* x, const T* dinv, const T* b, T* r,
-                          T* y)
+                          T* y, const post_args& post)
     {
         if(m == 0)
             return LAL_OK;
         rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, x, dinv, b, r, y, 0.0,
                   0.0, d->win};
         lal::use_c16(a, d);
-        a.keep = d->keep;
+        a.keep    = d->keep;
+        a.ex.post = post;
         return rowvec_launch<T>(c, RV_SMOOTHED, a);
     }
 
     template <typename T>
-    int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
-                    const T* v, const T* e, const T* y, T* out)
+    static rv_args add_args(const lal_csrmv_info* d, int m, const int* rp, const int* ci,
+                            const T* v, const T* e, const T* y, T* out)
     {
-        if(m == 0)
-            return LAL_OK;
         rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, e, nullptr, y, out,
                   nullptr, 0.0, 0.0, d->win};
         lal::use_c16(a, d);
-        return rowvec_launch<T>(c, RV_ADD, a);
+        return a;
+    }
+
+    template <typename T>
+    bool can_add_dot(const lal_csrmv_info* d, int m, const int* rp, const int* ci, const T* v)
+    {
+        return rowvec_can_dot(RV_ADD_DOT, add_args<T>(d, m, rp, ci, v, nullptr, nullptr, nullptr));
+    }
+
+    template <typename T>
+    int add_product(lal_context* c, const lal_csrmv_info* d, int m, const int* rp, const int* ci,
+                    const T* v, const T* e, const T* y, T* out, const row_extra& ex)
+    {
+        if(m == 0)
+            return LAL_OK;
+        rv_args a = add_args<T>(d, m, rp, ci, v, e, y, out);
+        a.ex      = ex;
+        return rowvec_launch<T>(c, ex.part ? RV_ADD_DOT : RV_ADD, a);
+    }
+
+    template <typename T>
+    int product_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, int nnz, const int* rp,
+                    const int* ci, const T* v, const T* x, T* y, double* part, int* count)
+    {
+        if(d && !d->exact && m == n)
+        {
+            rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, x, nullptr,
+                      nullptr, y, nullptr, 1.0, 0.0, d->win};
+            lal::use_c16(a, d);
+            a.keep    = d->keep;
+            a.ex.part = part;
+            a.ex.w    = x;
+            if(rowvec_can_dot(RV_SPMV_DOT, a))
+            {
+                *count = d->nblocks;
+                return rowvec_launch<T>(c, RV_SPMV_DOT, a);
+            }
+        }
+        LAL_TRY(csrmv(c, d, m, n, nnz, 1.0, rp, ci, v, x, 0.0, y));
+        *count = PCG_BLOCKS;
+        return dot_partials<T, T>(c, m, y, x, part);
     }
 
     int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
@@ -704,26 +695,23 @@ namespace lal
         return LAL_OK;
     }
 
-    int finish_partials(lal_context* c, int op, const double* part, double* slot,
-                        double* host_val, unsigned* host_seq, unsigned seq)
+    int finish_partials(lal_context* c, int op, const post_args& a)
     {
         if(op == 0)
-            finish_kernel<0><<<1, SPMV_THREADS, 0, c->stream>>>(part, slot, host_val, host_seq,
-                                                                seq);
+            finish_kernel<0><<<1, SPMV_THREADS, 0, c->stream>>>(a);
         else
-            finish_kernel<1><<<1, SPMV_THREADS, 0, c->stream>>>(part, slot, host_val, host_seq,
-                                                                seq);
+            finish_kernel<1><<<1, SPMV_THREADS, 0, c->stream>>>(a);
         LAL_LAUNCHED();
         return LAL_OK;
     }
 
     template <typename T, typename S>
     int update_xr(lal_context* c, int n, const T* p, const T* q, T* x, T* r,
-                  const double* part_pq, const double* part_gamma, double* part_r,
+                  const double* part_pq, int n_pq, const double* gamma, double* part_r,
                   double* s_alpha, const S* dinv, S* x0, S* rs, double rs_scale)
     {
-        update_xr_kernel<T, S><<<RB, SPMV_THREADS, 0, c->stream>>>(
-            n, p, q, x, r, part_pq, part_gamma, part_r, s_alpha, dinv, x0, rs, (T)rs_scale);
+        update_xr_kernel<T, S><<<update_blocks(n), SPMV_THREADS, 0, c->stream>>>(
+            n, p, q, x, r, part_pq, n_pq, gamma, part_r, s_alpha, dinv, x0, rs, (T)rs_scale);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -751,11 +739,11 @@ namespace lal
     }
 
     template <typename TZ, typename T>
-    int update_p(lal_context* c, int n, const TZ* z, T* p, const double* part_new,
-                 const double* part_old)
+    int update_p(lal_context* c, int n, const TZ* z, T* p, const double* part_new, int n_new,
+                 const double* gamma_old, double* gamma_new)
     {
-        update_p_kernel<TZ, T><<<RB, SPMV_THREADS, 0, c->stream>>>(n, z, p, part_new,
-                                                                   part_old);
+        update_p_kernel<TZ, T><<<update_blocks(n), SPMV_THREADS, 0, c->stream>>>(
+            n, z, p, part_new, n_new, gamma_old, gamma_new);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -793,9 +781,15 @@ namespace lal
                                      T*);                                                    \
     template int residual_smoothed<T>(lal_context*, const lal_csrmv_info*, int, const int*,  \
                                       const int*, const T*, const T*, const T*, const T*,    \
-                                      T*, T*);                                               \
+                                      T*, T*, const post_args&);                             \
     template int add_product<T>(lal_context*, const lal_csrmv_info*, int, const int*,        \
-                                const int*, const T*, const T*, const T*, T*);               \
+                                const int*, const T*, const T*, const T*, T*,                \
+                                const row_extra&);                                           \
+    template bool can_add_dot<T>(const lal_csrmv_info*, int, const int*, const int*,         \
+                                 const T*);                                                  \
+    template int product_dot<T>(lal_context*, const lal_csrmv_info*, int, int, int,          \
+                                const int*, const int*, const T*, const T*, T*, double*,     \
+                                int*);                                                       \
     template int diag_inv<T>(lal_context*, int, const int*, const int*, const T*, T*, T*,   \
                              long);                                                          \
     template int coarse_scalar<T>(lal_context*, const T*, const T*, T*);                     \
@@ -805,10 +799,10 @@ namespace lal
     template int dot_partials<T, T>(lal_context*, int, const T*, const T*, double*);         \
     template int norm_partials<T>(lal_context*, int, const T*, double*);                     \
     template int update_xr<T, T>(lal_context*, int, const T*, const T*, T*, T*,              \
-                                 const double*, const double*, double*, double*, const T*,   \
-                                 T*, T*, double);                                                    \
-    template int update_p<T, T>(lal_context*, int, const T*, T*, const double*,              \
-                                const double*);                                              \
+                                 const double*, int, const double*, double*, double*,        \
+                                 const T*, T*, T*, double);                                  \
+    template int update_p<T, T>(lal_context*, int, const T*, T*, const double*, int,         \
+                                const double*, double*);                                     \
     template int mul_elem<T>(lal_context*, int, const T*, const T*, T*);                     \
     template int restrict_init<T>(lal_context*, const lal_csrmv_info*, int, const int*,      \
                                   const int*, const T*, const T*, const T*, T*, T*);
@@ -819,11 +813,11 @@ namespace lal
     template int dot_partials<float, double>(lal_context*, int, const float*, const double*,
                                              double*);
     template int update_xr<double, float>(lal_context*, int, const double*, const double*,
-                                          double*, double*, const double*, const double*,
-                                          double*, double*, const float*, float*, float*,
-                                          double);
+                                          double*, double*, const double*, int,
+                                          const double*, double*, double*, const float*, float*,
+                                          float*, double);
     template int update_p<float, double>(lal_context*, int, const float*, double*,
-                                         const double*, const double*);
+                                         const double*, int, const double*, double*);
 }
 
 extern "C" int lal_sddmm_f64(lal_handle c, int m, int nnz, const int* rp, const int* ci,
