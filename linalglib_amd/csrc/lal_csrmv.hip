@@ -549,10 +549,14 @@ namespace lal
     // matrices; for small ones it shrinks, down to 256, so that a launch still
     // has about 1024 workgroups: their time is one latency chain per
     // workgroup, and more, shorter chains spread over all CUs finish sooner.
-    static int block_cap(int nnz)
+    // With column lists a larger block also reads fewer columns of x per
+    // nonzero, and one workgroup per CU is enough (gradient on 64^3, whose
+    // second level holds 1.2 million nonzeros: 1024 workgroups 15.7 ms, 512
+    // 15.4, 256 15.2; 4096 17.6).
+    static int block_cap(int nnz, bool lists)
     {
-        int cap = spmv_cap<double>::value;
-        while(cap > 256 && nnz / 1024 < cap)
+        int cap = lists ? LIST_CAP : spmv_cap<double>::value;
+        while(cap > 256 && nnz / (lists ? 256 : 1024) < cap)
             cap >>= 1;
         return cap;
     }
@@ -574,7 +578,7 @@ namespace lal
                 o.m      = q.m;
                 o.nnz    = q.nnz;
                 // (the list kernel takes a block as 512 quads of four)
-                o.cap    = std::min(block_cap(q.nnz), q.want_list ? LIST_CAP : INT_MAX);
+                o.cap    = block_cap(q.nnz, q.want_list);
                 o.tile0  = tiles;
                 o.ntiles = std::max((q.m + RB_TILE - 1) / RB_TILE, 1);
                 o.blk0   = blocks;
