@@ -6,6 +6,7 @@
 // repeatable run to run (no floating-point atomics).
 #include "lal_internal.h"
 
+#include <cstring>
 #include <mutex>
 
 // Scratch of lal_exclusive_scan_i64_noalloc: the scan's tile sums, one int64
@@ -66,6 +67,26 @@ namespace
     }
 
     // ----------------------------------------------------------- reductions
+    // Where a reduction's result goes: a device scalar, or the context's note
+    // (mapped host memory, then the sequence number the host polls).
+    struct red_out
+    {
+        double*   value;
+        unsigned* seq_at; // null: a device scalar
+        unsigned  seq;
+    };
+
+    __device__ __forceinline__ void put_result(const red_out& o, double v)
+    {
+        if(o.seq_at == nullptr)
+        {
+            *o.value = v;
+            return;
+        }
+        __hip_atomic_store(o.value, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(o.seq_at, o.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+
     // OP 0: sum x_i*y_i ; OP 1: max |x_i| ; OP 2: y_i = alpha x_i + y_i (the
     // axpy kernel's arithmetic) then sum y_i*z_i, which is lal_axpy then
     // lal_dot in one pass with the same partition and order.  Accumulation is
@@ -73,8 +94,7 @@ namespace
     template <typename T, int OP>
     __global__ void __launch_bounds__(LAL_RED_THREADS)
         reduce_kernel(int n, const T* __restrict__ x, const T* y, double* __restrict__ part,
-                      unsigned* __restrict__ ticket, double* __restrict__ out, T alpha = 0,
-                      T* yw = nullptr, const T* z = nullptr)
+                      unsigned* __restrict__ ticket, red_out out, T alpha = 0, T* yw = nullptr, const T* z = nullptr)
     {
         __shared__ double sh[LAL_RED_THREADS / 64];
         __shared__ bool   last;
@@ -167,8 +187,8 @@ namespace
             double t = sh[0];
             for(int w = 1; w < LAL_RED_THREADS / 64; w++)
                 t = SUM ? t + sh[w] : ((sh[w] < t) ? t : sh[w]);
-            *out    = t;
             *ticket = 0u;
+            put_result(out, t);
         }
     }
 
@@ -180,7 +200,7 @@ namespace
 
     __global__ void __launch_bounds__(64)
         seq_dot_kernel(int n, const double* __restrict__ x, const double* __restrict__ y,
-                       double* __restrict__ out)
+                       red_out out)
     {
         __shared__ double sx[SEQ_DOT], sy[SEQ_DOT];
         for(int i = threadIdx.x; i < n; i += 64)
@@ -194,22 +214,23 @@ namespace
         double s = 0.0;
         for(int i = 0; i < n; i++)
             s = s + sx[i] * sy[i];
-        *out = s;
+        put_result(out, s);
     }
 
     template <typename T, int OP>
-    int reduce_dev(lal_context* c, int n, const T* x, const T* y, double* d_out)
+    int reduce_dev(lal_context* c, int n, const T* x, const T* y, const red_out& out,
+                   T alpha = 0, T* yw = nullptr, const T* z = nullptr)
     {
         if(OP == 0 && sizeof(T) == 8 && n > 0 && n <= SEQ_DOT)
         {
-            seq_dot_kernel<<<1, 64, 0, c->stream>>>(n, (const double*)x, (const double*)y,
-                                                    d_out);
+            seq_dot_kernel<<<1, 64, 0, c->stream>>>(n, (const double*)x, (const double*)y, out);
             LAL_LAUNCHED();
             return LAL_OK;
         }
         int g = n <= 0 ? 1 : lal::grid_for(n, LAL_RED_THREADS, LAL_RED_BLOCKS);
         reduce_kernel<T, OP>
-            <<<g, LAL_RED_THREADS, 0, c->stream>>>(n, x, y, c->d_part, c->d_ticket, d_out);
+            <<<g, LAL_RED_THREADS, 0, c->stream>>>(n, x, y, c->d_part, c->d_ticket, out, alpha, yw,
+                                                   z);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -413,15 +434,15 @@ namespace lal
 {
     int dot_f64_dev(lal_context* c, int n, const double* x, const double* y, double* d_out, int)
     {
-        return reduce_dev<double, 0>(c, n, x, y, d_out);
+        return reduce_dev<double, 0>(c, n, x, y, {d_out, nullptr, 0});
     }
     int dot_f32_dev(lal_context* c, int n, const float* x, const float* y, double* d_out, int)
     {
-        return reduce_dev<float, 0>(c, n, x, y, d_out);
+        return reduce_dev<float, 0>(c, n, x, y, {d_out, nullptr, 0});
     }
     int norm_inf_f64_dev(lal_context* c, int n, const double* x, double* d_out, int)
     {
-        return reduce_dev<double, 1>(c, n, x, x, d_out);
+        return reduce_dev<double, 1>(c, n, x, x, {d_out, nullptr, 0});
     }
     int scan_i32_dev(lal_context* c, int n, int32_t* x, arena* a)
     {
@@ -489,16 +510,25 @@ extern "C" int lal_axpbypgz_f64(lal_handle c, int n, double alpha, const double*
 
 namespace
 {
+    // The last block writes the result to the context's note, which the host
+    // polls (a CG step on 128^2 with four results, each by a copy to pinned
+    // memory and a stream synchronisation: 100 us, so: 79).  The block's release
+    // comes after every other block's through the ticket, so a vector that the
+    // same kernel wrote is complete when the host goes on.
     template <typename T, int OP>
-    int reduce_host(lal_context* c, int n, const T* x, const T* y, double* result)
+    int reduce_host(lal_context* c, int n, const T* x, const T* y, double* result, T alpha = 0,
+                    T* yw = nullptr, const T* z = nullptr)
     {
         LAL_REQUIRE(c != nullptr && n >= 0 && result != nullptr);
         LAL_REQUIRE(n == 0 || (x != nullptr && y != nullptr));
-        LAL_TRY((reduce_dev<T, OP>(c, n, x, y, c->d_slots)));
-        LAL_HIP(hipMemcpyAsync(c->h_slots, c->d_slots, sizeof(double), hipMemcpyDeviceToHost,
-                               c->stream));
-        LAL_HIP(hipStreamSynchronize(c->stream));
-        *result = c->h_slots[0];
+        const red_out out{reinterpret_cast<double*>(c->d_note),
+                          reinterpret_cast<unsigned*>(c->d_note + LAL_NOTE_INTS), ++c->note_seq};
+        LAL_TRY((reduce_dev<T, OP>(c, n, x, y, out, alpha, yw, z)));
+        LAL_TRY(lal::wait_note(c, out.seq));
+        const unsigned long long bits =
+            __atomic_load_n(reinterpret_cast<const unsigned long long*>(c->h_note),
+                            __ATOMIC_RELAXED);
+        std::memcpy(result, &bits, sizeof(double));
         return LAL_OK;
     }
 }
@@ -519,15 +549,7 @@ extern "C" int lal_axpy_dot_f64(lal_handle c, int n, double alpha, const double*
         LAL_TRY(axpy_t<double>(c, n, alpha, x, y));
         return reduce_host<double, 0>(c, n, y, z, result);
     }
-    const int g = n <= 0 ? 1 : lal::grid_for(n, LAL_RED_THREADS, LAL_RED_BLOCKS);
-    reduce_kernel<double, 2><<<g, LAL_RED_THREADS, 0, c->stream>>>(
-        n, x, y, c->d_part, c->d_ticket, c->d_slots, alpha, y, z);
-    LAL_LAUNCHED();
-    LAL_HIP(hipMemcpyAsync(c->h_slots, c->d_slots, sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    LAL_HIP(hipStreamSynchronize(c->stream));
-    *result = c->h_slots[0];
-    return LAL_OK;
+    return reduce_host<double, 2>(c, n, x, y, result, alpha, y, z);
 }
 extern "C" int lal_dot_f32(lal_handle c, int n, const float* x, const float* y, double* r)
 {

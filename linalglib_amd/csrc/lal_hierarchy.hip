@@ -954,35 +954,16 @@ namespace lal
         return LAL_OK;
     }
 
-    // Waits until the note carries `seq`.  The host polls the mapped word
-    // and checks the stream now and then so that a failed kernel turns into
-    // an error instead of a hang.
     int wait_scalar(lal_hierarchy_t* h, unsigned seq, int slot, double* v)
     {
-        for(long spins = 1;; spins++)
-        {
-            if(__atomic_load_n(h->h_seq, __ATOMIC_ACQUIRE) == seq)
-            {
-                *v = *reinterpret_cast<volatile double*>(h->h_note);
-                return LAL_OK;
-            }
-            if((spins & 1023) == 0)
-            {
-                hipError_t e = hipStreamQuery(h->c->stream);
-                if(e == hipSuccess)
-                {
-                    if(__atomic_load_n(h->h_seq, __ATOMIC_ACQUIRE) == seq)
-                        continue;
-                    // the stream has drained: read the device copy instead
-                    LAL_HIP(hipMemcpy(v, h->s + slot, sizeof(double), hipMemcpyDeviceToHost));
-                    return LAL_OK;
-                }
-                if(e != hipErrorNotReady)
-                    LAL_HIP(e);
-            }
-        }
+        bool there = false;
+        LAL_TRY(poll_word(h->c, h->h_seq, seq, &there));
+        if(there)
+            *v = *reinterpret_cast<volatile double*>(h->h_note);
+        else // the stream has drained: read the device copy instead
+            LAL_HIP(hipMemcpy(v, h->s + slot, sizeof(double), hipMemcpyDeviceToHost));
+        return LAL_OK;
     }
-
 }
 
 extern "C" void lal_saamg_default_options(lal_saamg_options* o)

@@ -12,7 +12,7 @@
 // Deterministic two-stage reductions use a fixed grid of this many blocks.
 #define LAL_RED_BLOCKS 1024
 #define LAL_RED_THREADS 256
-// Device result slots in the context (dot/norm outputs, solver scalars).
+// Pinned scalars in the context (solver flags and norms).
 #define LAL_NUM_SLOTS 64
 
 struct lal_hierarchy_t;
@@ -73,11 +73,10 @@ struct lal_context
                                       // captured on it
     int         device     = 0;
     int         num_cu     = 0;
-    // reduction workspace: partials, a ticket counter per reduction slot
+    // reduction workspace: partials and the ticket of the block that adds them up
     double*   d_part   = nullptr; // LAL_RED_BLOCKS * 2
-    unsigned* d_ticket = nullptr; // LAL_NUM_SLOTS
-    double*   d_slots  = nullptr; // LAL_NUM_SLOTS device scalars
-    double*   h_slots  = nullptr; // pinned mirror
+    unsigned* d_ticket = nullptr;
+    double*   h_slots  = nullptr; // LAL_NUM_SLOTS pinned scalars
     // flag words of the checks and setup passes: zero between calls (whoever
     // raises one reads it back with read_ints, which clears it)
     int*      d_flag   = nullptr;
@@ -294,6 +293,11 @@ namespace lal
     // Device address of the allocation-free scan's static scratch for
     // `device` (which must be current), looked up once per device.
     int noalloc_scratch_init(int device);
+    // Polls a mapped host word until it is `seq`; *there false: the stream has
+    // drained without it.
+    int poll_word(lal_context* c, const unsigned* word, unsigned seq, bool* there);
+    // Blocks until the context's note carries `seq`.
+    int wait_note(lal_context* c, unsigned seq);
     // The n ints at src once the stream has come to them (blocks); clear: they
     // are zeroed behind the read.
     int read_ints(lal_context* c, int* src, int n, int* out, bool clear);

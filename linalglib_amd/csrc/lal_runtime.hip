@@ -2,6 +2,7 @@
 #include "lal_internal.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -103,29 +104,51 @@ namespace
 
 namespace lal
 {
+    int poll_word(lal_context* c, const unsigned* word, unsigned seq, bool* there)
+    {
+        // A query puts a marker into the stream, which the kernels behind it
+        // then wait for: it is for a failed kernel to turn into an error instead
+        // of a hang, every two milliseconds.
+        using clock = std::chrono::steady_clock;
+        const auto every = std::chrono::milliseconds(2);
+        auto       next  = clock::now() + every;
+        *there           = true;
+        for(unsigned spins = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq; spins++)
+            if((spins & 255) == 0 && clock::now() >= next)
+            {
+                const hipError_t e = hipStreamQuery(c->stream);
+                if(e == hipSuccess) // drained: the word is there, or never will be
+                {
+                    *there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq;
+                    return LAL_OK;
+                }
+                if(e != hipErrorNotReady)
+                    LAL_HIP(e);
+                next = clock::now() + every;
+            }
+        return LAL_OK;
+    }
+
+    int wait_note(lal_context* c, unsigned seq)
+    {
+        bool there = false;
+        LAL_TRY(poll_word(c, reinterpret_cast<const unsigned*>(c->h_note + LAL_NOTE_INTS), seq,
+                          &there));
+        if(!there)
+        {
+            set_last_error("a result did not reach the host");
+            return LAL_ERR_HIP;
+        }
+        return LAL_OK;
+    }
+
     int read_ints(lal_context* c, int* src, int n, int* out, bool clear)
     {
         LAL_REQUIRE(n >= 0 && n <= LAL_NOTE_INTS);
         const unsigned seq = ++c->note_seq;
         note_kernel<<<1, 64, 0, c->stream>>>(src, n, clear ? 1 : 0, c->d_note, seq);
         LAL_LAUNCHED();
-        const unsigned* h_seq = reinterpret_cast<const unsigned*>(c->h_note + LAL_NOTE_INTS);
-        // poll, and look at the stream now and then so that a failed kernel
-        // turns into an error instead of a hang
-        for(long spins = 1; __atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq; spins++)
-            if((spins & 1023) == 0)
-            {
-                const hipError_t e = hipStreamQuery(c->stream);
-                if(e == hipSuccess)
-                    break; // drained: the note is there
-                if(e != hipErrorNotReady)
-                    LAL_HIP(e);
-            }
-        if(__atomic_load_n(h_seq, __ATOMIC_ACQUIRE) != seq)
-        {
-            set_last_error("a result did not reach the host");
-            return LAL_ERR_HIP;
-        }
+        LAL_TRY(wait_note(c, seq));
         for(int i = 0; i < n; i++)
             out[i] = __atomic_load_n(c->h_note + i, __ATOMIC_RELAXED);
         return LAL_OK;
@@ -188,16 +211,14 @@ extern "C" int lal_create(lal_handle* handle)
     LAL_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     c->stream = c->side;
     LAL_HIP(hipMalloc(&c->d_part, sizeof(double) * LAL_RED_BLOCKS * 2));
-    LAL_HIP(hipMalloc(&c->d_ticket, sizeof(unsigned) * LAL_NUM_SLOTS));
-    LAL_HIP(hipMalloc(&c->d_slots, sizeof(double) * LAL_NUM_SLOTS));
+    LAL_HIP(hipMalloc(&c->d_ticket, sizeof(unsigned)));
     LAL_HIP(hipMalloc(&c->d_flag, sizeof(int) * LAL_FLAGS));
     LAL_HIP(hipHostMalloc(&c->h_slots, sizeof(double) * LAL_NUM_SLOTS, hipHostMallocDefault));
     LAL_HIP(hipHostMalloc(&c->h_note, sizeof(int) * (LAL_NOTE_INTS + 1),
                           hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(c->h_note, 0, sizeof(int) * (LAL_NOTE_INTS + 1));
     LAL_HIP(hipHostGetDevicePointer((void**)&c->d_note, c->h_note, 0));
-    LAL_HIP(hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned) * LAL_NUM_SLOTS, c->stream));
-    LAL_HIP(hipMemsetAsync(c->d_slots, 0, sizeof(double) * LAL_NUM_SLOTS, c->stream));
+    LAL_HIP(hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned), c->stream));
     LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int) * LAL_FLAGS, c->stream));
     LAL_HIP(hipStreamSynchronize(c->stream));
     *handle = c;
@@ -212,7 +233,6 @@ extern "C" int lal_destroy(lal_handle c)
     lal::detach_hierarchies(c);
     (void)hipFree(c->d_part);
     (void)hipFree(c->d_ticket);
-    (void)hipFree(c->d_slots);
     (void)hipFree(c->d_flag);
     (void)hipHostFree(c->h_slots);
     (void)hipHostFree(c->h_note);
