@@ -151,12 +151,15 @@ namespace
     constexpr int PROLONG_KEEP = 4;
 
     template <int G>
-    __device__ __forceinline__ int group_min_i32(int v)
+    __device__ __forceinline__ int group_min(int v)
     {
-#pragma unroll
-        for(int o = G / 2; o > 0; o >>= 1)
-            v = min(v, __shfl_xor(v, o, 64));
-        return v;
+        return lal::group_fold<G>(v, [](int a, int b) { return min(a, b); });
+    }
+
+    template <int G>
+    __device__ __forceinline__ int group_max(int v)
+    {
+        return lal::group_fold<G>(v, [](int a, int b) { return max(a, b); });
     }
 
     // Aggregate of entry j's column when it is a candidate of row i (aggregate
@@ -184,11 +187,12 @@ namespace
     // Smallest aggregate id above `last` among the row's candidates (INT_MAX
     // when there is none); group-uniform.  key: the lane's first PROLONG_KEEP
     // entries; entries beyond them come from memory.
-    template <int G>
+    // (CI, CN: how a caller holds columns and connections)
+    template <int G, typename CI, typename CN>
     __device__ __forceinline__ int next_aggregate(int i, int rs, int re, int gl, bool more,
                                                   const int (&key)[PROLONG_KEEP],
-                                                  const int* __restrict__ ci,
-                                                  const int* __restrict__ conn,
+                                                  const CI* __restrict__ ci,
+                                                  const CN* __restrict__ conn,
                                                   const int64_t* __restrict__ agg, int last)
     {
         int best = INT_MAX;
@@ -203,25 +207,16 @@ namespace
                 if(a > last && a < best)
                     best = a;
             }
-        return group_min_i32<G>(best);
+        return group_min<G>(best);
     }
 
-    template <int G>
-    __global__ void __launch_bounds__(256)
-        prolong_count_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                                   const int* __restrict__ conn, const int64_t* __restrict__ agg,
-                                   int* __restrict__ count)
+    // Entries of row i of P (group-uniform).
+    template <int G, typename CI, typename CN>
+    __device__ __forceinline__ int prolong_count_row(int i, int gl, const int* __restrict__ rp,
+                                                     const CI* __restrict__ ci,
+                                                     const CN* __restrict__ conn,
+                                                     const int64_t* __restrict__ agg)
     {
-        const int gl = (int)threadIdx.x % G;
-        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        if(i > m)
-            return;
-        if(i == m)
-        {
-            if(gl == 0)
-                count[m] = 0;
-            return;
-        }
         const int rs = rp[i], re = rp[i + 1];
         int       key[PROLONG_KEEP];
 #pragma unroll
@@ -241,25 +236,34 @@ namespace
             k++;
             last = best;
         }
-        if(gl == 0)
-            count[i] = k;
+        return k;
     }
 
     template <int G>
     __global__ void __launch_bounds__(256)
-        prolong_fill_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                                  const double* __restrict__ val, const int* __restrict__ conn,
-                                  const int64_t* __restrict__ agg, double relax,
-                                  const int* __restrict__ prp, int* __restrict__ pci,
-                                  double* __restrict__ pv)
+        prolong_count_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
+                                   const int* __restrict__ conn, const int64_t* __restrict__ agg,
+                                   int* __restrict__ count)
     {
         const int gl = (int)threadIdx.x % G;
-        const int gb = ((int)threadIdx.x & 63) - gl; // the group's first lane
         const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        if(i >= m)
+        if(i > m)
             return;
+        const int k = i < m ? prolong_count_row<G>(i, gl, rp, ci, conn, agg) : 0;
+        if(gl == 0)
+            count[i] = k;
+    }
+
+    // Row i of P into pci/pv[p0 .. p1).
+    template <int G, typename CI, typename CN>
+    __device__ __forceinline__ void
+        prolong_fill_row(int i, int gl, const int* __restrict__ rp, const CI* __restrict__ ci,
+                         const double* __restrict__ val, const CN* __restrict__ conn,
+                         const int64_t* __restrict__ agg, double relax, int p0, int p1,
+                         int* __restrict__ pci, double* __restrict__ pv)
+    {
+        const int gb = ((int)threadIdx.x & 63) - gl; // the group's first lane
         const int rs = rp[i], re = rp[i + 1];
-        const int p0 = prp[i], p1 = prp[i + 1];
         int       key[PROLONG_KEEP];
         double    v[PROLONG_KEEP];
         int       kind[PROLONG_KEEP]; // 1: the diagonal, 2: weak, 0: strong or none
@@ -363,6 +367,20 @@ namespace
             last = best;
         }
     }
+
+    template <int G>
+    __global__ void __launch_bounds__(256)
+        prolong_fill_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
+                                  const double* __restrict__ val, const int* __restrict__ conn,
+                                  const int64_t* __restrict__ agg, double relax,
+                                  const int* __restrict__ prp, int* __restrict__ pci,
+                                  double* __restrict__ pv)
+    {
+        const int gl = (int)threadIdx.x % G;
+        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
+        if(i < m)
+            prolong_fill_row<G>(i, gl, rp, ci, val, conn, agg, relax, prp[i], prp[i + 1], pci, pv);
+    }
 }
 
 namespace
@@ -380,24 +398,6 @@ namespace
     {
         gl = (int)threadIdx.x % G;
         return blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-    }
-
-    template <int G>
-    __device__ __forceinline__ int group_min(int v)
-    {
-#pragma unroll
-        for(int o = G / 2; o > 0; o >>= 1)
-            v = min(v, __shfl_xor(v, o, 64));
-        return v;
-    }
-
-    template <int G>
-    __device__ __forceinline__ int group_max(int v)
-    {
-#pragma unroll
-        for(int o = G / 2; o > 0; o >>= 1)
-            v = max(v, __shfl_xor(v, o, 64));
-        return v;
     }
 
     // d[i] = the row's first diagonal entry (0 when it has none)
@@ -478,10 +478,10 @@ namespace
 
     // The best strong neighbour of row `row` across the group: each lane keeps
     // the first maximum of its entries, the group the earliest of the lanes'.
-    template <int G>
+    template <int G, typename CI, typename CN>
     __device__ __forceinline__ pmis_cand pmis_scan(int row, int gl, const int* __restrict__ rp,
-                                                   const int* __restrict__ ci,
-                                                   const int* __restrict__ conn,
+                                                   const CI* __restrict__ ci,
+                                                   const CN* __restrict__ conn,
                                                    const int* __restrict__ state,
                                                    const int* __restrict__ hash)
     {
@@ -495,12 +495,26 @@ namespace
                 if(sc > best.s || (sc == best.s && hc > best.h))
                     best = pmis_cand{sc, hc, c, j - rs};
             }
-#pragma unroll
-        for(int o = G / 2; o > 0; o >>= 1)
+        const auto take = [&](auto at) {
+            pmis_take(best, pmis_cand{at(best.s), at(best.h), at(best.r), at(best.pos)});
+        };
+        take([](int v) { return lal::partner<0>(v); });
+        take([](int v) { return lal::partner<1>(v); });
+        take([](int v) { return lal::partner<2>(v); });
+        if(G >= 16)
+            take([](int v) { return lal::partner<3>(v); });
+        if(G == 64)
         {
-            const pmis_cand other{__shfl_xor(best.s, o, 64), __shfl_xor(best.h, o, 64),
-                                  __shfl_xor(best.r, o, 64), __shfl_xor(best.pos, o, 64)};
-            pmis_take(best, other);
+            const pmis_cand mine = best;
+            const auto      row  = [&](int t) {
+                return pmis_cand{
+                    __builtin_amdgcn_readlane(mine.s, t), __builtin_amdgcn_readlane(mine.h, t),
+                    __builtin_amdgcn_readlane(mine.r, t), __builtin_amdgcn_readlane(mine.pos, t)};
+            };
+            best = row(0);
+            pmis_take(best, row(16));
+            pmis_take(best, row(32));
+            pmis_take(best, row(48));
         }
         return best;
     }
@@ -510,17 +524,13 @@ namespace
     // strong neighbours of the row that maximum names.
     // Every row's state goes to max_state, decided or not, so that the rounds
     // alternate two buffers.
-    template <int G>
-    __global__ void __launch_bounds__(256)
-        pmis_round_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                                const int* __restrict__ conn, const int* __restrict__ state,
-                                const int* __restrict__ hash, int64_t* __restrict__ agg,
-                                int* __restrict__ max_state, int* __restrict__ incomplete)
+    template <int G, typename CI, typename CN>
+    __device__ __forceinline__ void
+        pmis_round_row(int i, int gl, const int* __restrict__ rp, const CI* __restrict__ ci,
+                       const CN* __restrict__ conn, const int* __restrict__ state,
+                       const int* __restrict__ hash, int64_t* __restrict__ agg,
+                       int* __restrict__ max_state, int* __restrict__ incomplete)
     {
-        int       gl;
-        const int i = group_row<G>(gl);
-        if(i >= m)
-            return;
         const int si = state[i];
         if(si != 0)
         {
@@ -555,14 +565,23 @@ namespace
 
     template <int G>
     __global__ void __launch_bounds__(256)
-        pmis_join_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                               const int* __restrict__ conn, const int* __restrict__ state,
-                               int64_t* __restrict__ agg, int* __restrict__ max_state)
+        pmis_round_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
+                                const int* __restrict__ conn, const int* __restrict__ state,
+                                const int* __restrict__ hash, int64_t* __restrict__ agg,
+                                int* __restrict__ max_state, int* __restrict__ incomplete)
     {
         int       gl;
         const int i = group_row<G>(gl);
-        if(i >= m)
-            return;
+        if(i < m)
+            pmis_round_row<G>(i, gl, rp, ci, conn, state, hash, agg, max_state, incomplete);
+    }
+
+    template <int G, typename CI, typename CN>
+    __device__ __forceinline__ void
+        pmis_join_row(int i, int gl, const int* __restrict__ rp, const CI* __restrict__ ci,
+                      const CN* __restrict__ conn, const int* __restrict__ state, int64_t* agg,
+                      int* __restrict__ max_state)
+    {
         const int si = state[i];
         if(gl == 0)
             max_state[i] = si;
@@ -587,6 +606,225 @@ namespace
         }
         else if(si == -2 && gl == 0)
             agg[i] = -2;
+    }
+
+    template <int G>
+    __global__ void __launch_bounds__(256)
+        pmis_join_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
+                               const int* __restrict__ conn, const int* __restrict__ state,
+                               int64_t* __restrict__ agg, int* __restrict__ max_state)
+    {
+        int       gl;
+        const int i = group_row<G>(gl);
+        if(i < m)
+            pmis_join_row<G>(i, gl, rp, ci, conn, state, agg, max_state);
+    }
+
+    // A level from its operator to P and R = P^T in one workgroup.
+    struct small_level
+    {
+        int           m, nnz;
+        const int *   rp, *ci;
+        const double* v;
+        double        eps, relax;
+        bool          unsmoothed;
+        int*          place; // scratch, one per entry of P: its place in R's row,
+        int*          tci;   // and R's entries before they are in order
+        double*       tv;
+        int *         prp, *pci, *rrp, *rci;
+        double *      pv, *rv;
+    };
+    constexpr int SMALL_THREADS = 1024;
+    constexpr int SMALL_ROWS    = 1024; // (columns fit 16 bits)
+    constexpr int SMALL_NNZ     = 8192;
+
+    // Exclusive scan over the workgroup, one value per lane.
+    __device__ __forceinline__ int small_scan(int v, int* total)
+    {
+        __shared__ int s_w[SMALL_THREADS / 64];
+        const int      lane = (int)threadIdx.x & 63, wid = (int)threadIdx.x >> 6;
+        int            inc  = v;
+#pragma unroll
+        for(int o = 1; o < 64; o <<= 1)
+        {
+            const int q = __shfl_up(inc, o, 64);
+            inc += lane >= o ? q : 0;
+        }
+        __syncthreads();
+        if(lane == 63)
+            s_w[wid] = inc;
+        __syncthreads();
+        int at = inc - v, all = 0;
+        for(int w = 0; w < SMALL_THREADS / 64; w++)
+        {
+            at += w < wid ? s_w[w] : 0;
+            all += s_w[w];
+        }
+        *total = all;
+        return at;
+    }
+
+    // The steps of the passes above and of the transpose, row by row with the
+    // same functions, so the results are theirs bit for bit; states, hashes and
+    // aggregates lie in LDS.  Level after level these were 27 launches of a few
+    // microseconds and two waits for the host: the time of a small hierarchy.
+    // 25^3 diffusion, levels of 84, 12 and 3 rows, with the products' plans in
+    // one launch too: 318 launches and 2.36 ms -> 207 and 2.12.  One workgroup is
+    // slower per row than the chip (84 rows of 84 entries: 112 us), so a level
+    // comes here up to where its launches would take about as long.
+    // The note: columns of P, entries of P.
+    template <int G>
+    __global__ void __launch_bounds__(SMALL_THREADS)
+        small_level_kernel(small_level a, int* note, unsigned seq)
+    {
+        constexpr int             NG = SMALL_THREADS / G;
+        __shared__ double         s_d[SMALL_ROWS];
+        __shared__ int64_t        s_agg[SMALL_ROWS];
+        __shared__ int            s_state[2][SMALL_ROWS], s_hash[SMALL_ROWS], s_cnt[SMALL_ROWS];
+        __shared__ int            s_rp[SMALL_ROWS + 1];
+        __shared__ unsigned short s_ci[SMALL_NNZ];
+        __shared__ unsigned char  s_conn[SMALL_NNZ];
+        __shared__ int            s_flag, s_top;
+        const int                 tid = (int)threadIdx.x, gl = tid % G, g0 = tid / G, m = a.m;
+        if(tid == 0)
+        {
+            s_top   = -1;
+            s_rp[m] = a.nnz;
+        }
+        if(tid < m)
+            s_rp[tid] = a.rp[tid];
+        for(int e = tid; e < a.nnz; e += SMALL_THREADS)
+            s_ci[e] = (unsigned short)a.ci[e];
+        __syncthreads();
+        // the row's first diagonal entry (0 when it has none)
+        for(int i = g0; i < m; i += NG)
+        {
+            const int rs = s_rp[i], re = s_rp[i + 1];
+            int       first = INT_MAX;
+            for(int j = rs + gl; j < re; j += G)
+                if(s_ci[j] == i)
+                {
+                    first = j;
+                    break;
+                }
+            first = group_min<G>(first);
+            if(gl == 0)
+                s_d[i] = first != INT_MAX ? a.v[first] : 0.0;
+        }
+        __syncthreads();
+        for(int i = g0; i < m; i += NG)
+        {
+            const double di     = fabs(s_d[i]);
+            int          strong = 0;
+            for(int j = s_rp[i] + gl; j < s_rp[i + 1]; j += G)
+            {
+                const int c  = s_ci[j];
+                const int on = (c != i) && (fabs(a.v[j]) >= a.eps * sqrt(di * fabs(s_d[c])));
+                s_conn[j]    = (unsigned char)on;
+                strong |= on;
+            }
+            strong = group_max<G>(strong);
+            if(gl == 0)
+            {
+                s_state[0][i] = s_state[1][i] = strong ? 0 : -2;
+                s_hash[i]                     = hash1((unsigned)i);
+                s_agg[i]                      = 0;
+            }
+        }
+        int cur = 0;
+        for(int iter = 0; iter < 20; iter++)
+        {
+            __syncthreads();
+            if(tid == 0)
+                s_flag = 0;
+            __syncthreads();
+            for(int i = g0; i < m; i += NG)
+                pmis_round_row<G>(i, gl, s_rp, s_ci, s_conn, s_state[cur], s_hash, s_agg,
+                                  s_state[cur ^ 1], &s_flag);
+            cur ^= 1;
+            __syncthreads();
+            if(s_flag == 0)
+                break;
+        }
+        int       total = 0;
+        const int ahead = small_scan(tid < m ? (int)s_agg[tid] : 0, &total);
+        if(tid < m)
+            s_agg[tid] = ahead;
+        for(int k = 0; k < 2; k++, cur ^= 1)
+        {
+            __syncthreads();
+            for(int i = g0; i < m; i += NG)
+                pmis_join_row<G>(i, gl, s_rp, s_ci, s_conn, s_state[cur], s_agg,
+                                 s_state[cur ^ 1]);
+        }
+        __syncthreads();
+        // P's row pointer and columns
+        for(int i = g0; i < m; i += NG)
+        {
+            const int k = a.unsmoothed ? s_agg[i] >= 0
+                                       : prolong_count_row<G>(i, gl, s_rp, s_ci, s_conn, s_agg);
+            if(gl == 0)
+                s_cnt[i] = k;
+        }
+        if(tid < m)
+            atomicMax(&s_top, (int)s_agg[tid]);
+        __syncthreads();
+        int       nnz = 0;
+        const int p0  = small_scan(tid < m ? s_cnt[tid] : 0, &nnz);
+        if(tid < m)
+            a.prp[tid] = p0;
+        if(tid == 0)
+            a.prp[m] = nnz;
+        const int nc = s_top + 1;
+        __syncthreads();
+        for(int i = g0; i < m; i += NG)
+        {
+            const int at = a.prp[i], end = a.prp[i + 1];
+            if(!a.unsmoothed)
+                prolong_fill_row<G>(i, gl, s_rp, s_ci, a.v, s_conn, s_agg, a.relax, at, end, a.pci,
+                                    a.pv);
+            else if(gl == 0 && s_agg[i] >= 0)
+            {
+                a.pci[at] = (int)s_agg[i];
+                a.pv[at]  = 1.0;
+            }
+        }
+        // R = P^T: places by counting, then every row sorted by rank
+        s_cnt[tid] = 0;
+        __syncthreads();
+        for(int e = tid; e < nnz; e += SMALL_THREADS)
+            a.place[e] = atomicAdd(&s_cnt[a.pci[e]], 1);
+        __syncthreads();
+        int       same = 0;
+        const int r0   = small_scan(tid < nc ? s_cnt[tid] : 0, &same);
+        if(tid < nc)
+            a.rrp[tid] = r0;
+        if(tid == 0)
+            a.rrp[nc] = nnz;
+        __syncthreads();
+        for(int i = g0; i < m; i += NG)
+            for(int e = a.prp[i] + gl; e < a.prp[i + 1]; e += G)
+            {
+                const int at = a.rrp[a.pci[e]] + a.place[e];
+                a.tci[at]    = i;
+                a.tv[at]     = a.pv[e];
+            }
+        __syncthreads();
+        for(int c = g0; c < nc; c += NG)
+        {
+            const int rs = a.rrp[c], re = a.rrp[c + 1];
+            for(int e = rs + gl; e < re; e += G)
+            {
+                const int row  = a.tci[e];
+                int       rank = rs;
+                for(int q = rs; q < re; q++)
+                    rank += a.tci[q] < row;
+                a.rci[rank] = row;
+                a.rv[rank]  = a.tv[e];
+            }
+        }
+        if(tid < 64)
+            lal::put_note(note, 2, tid == 0 ? nc : nnz, seq);
     }
 
     __device__ __forceinline__ long long wave_max_i64(long long v)
@@ -764,6 +1002,42 @@ namespace lal
                     <<<gg, 256, 0, c->stream>>>(m, rp, ci, conn, in, agg, out);
             LAL_LAUNCHED();
         }
+        return LAL_OK;
+    }
+
+    // Levels that small_build takes: at most eight rows for each of the
+    // workgroup's lane groups.
+    bool small_fits(int m, long nnz)
+    {
+        return m > 0 && m <= SMALL_ROWS && nnz <= SMALL_NNZ &&
+               m * setup_row_lanes(nnz, m) <= 8 * SMALL_THREADS;
+    }
+
+    // Strength to R = P^T of one small level.  P's and R's arrays have room for
+    // max(m, nnz) entries, R's row pointer for m + 1.
+    int small_build(lal_context* c, int m, int nnz, const int* rp, const int* ci, const double* v,
+                    double eps, double relax, bool unsmoothed, int* prp, int* pci, double* pv,
+                    int* rrp, int* rci, double* rv, int* nnz_P, int* n_c, arena* a)
+    {
+        LAL_REQUIRE(small_fits(m, nnz));
+        temps       tmp(c, a);
+        const int   room = std::max(m, nnz);
+        small_level L{m,       nnz,     rp,  ci,  v,   eps, relax, unsmoothed, nullptr,
+                      nullptr, nullptr, prp, pci, rrp, rci, pv,    rv};
+        LAL_TRY(tmp.get(&L.place, room));
+        LAL_TRY(tmp.get(&L.tci, room));
+        LAL_TRY(tmp.get(&L.tv, room));
+        const int      lanes = setup_row_lanes(nnz, m);
+        const unsigned seq   = ++c->note_seq;
+        auto*          fn    = lanes == 64   ? small_level_kernel<64>
+                               : lanes == 16 ? small_level_kernel<16>
+                                             : small_level_kernel<8>;
+        fn<<<1, SMALL_THREADS, 0, c->stream>>>(L, c->d_note, seq);
+        LAL_LAUNCHED();
+        int got[2];
+        LAL_TRY(take_note(c, seq, 2, got));
+        *n_c   = got[0];
+        *nnz_P = got[1];
         return LAL_OK;
     }
 

@@ -31,6 +31,11 @@ namespace lal
     int sa_prolongator_fill(lal_context* c, int m, int nnz, const int* rp, const int* ci,
                             const double* v, const int* conn, const int64_t* agg, double relax,
                             const int* prp, int* pci, double* pv);
+    bool small_fits(int m, long nnz);
+    int  small_build(lal_context* c, int m, int nnz, const int* rp, const int* ci,
+                     const double* v, double eps, double relax, bool unsmoothed, int* prp,
+                     int* pci, double* pv, int* rrp, int* rci, double* rv, int* nnz_P, int* n_c,
+                     arena* a);
     int ua_prolongator_nnz(lal_context* c, int m, const int64_t* agg, int* prp, int* nnz_P,
                            int* n_c, arena* a);
     int ua_prolongator_fill(lal_context* c, int m, const int64_t* agg, const int* prp, int* pci,
@@ -345,44 +350,63 @@ namespace
             csr_dev& P  = h->L[level].P;
             csr_dev& R  = h->L[level].R;
             csr_dev& Ac = h->L[level + 1].A;
-            int*     conn = nullptr;
-            int64_t* agg  = nullptr;
             tmp.release(lal::arena::mark_t{});
-            LAL_TRY(tmp.get(&conn, Af.nnz));
-            LAL_TRY(tmp.get(&agg, Af.m));
-            LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn, &tmp));
-            LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, &tmp));
             LAL_TRY(h->mem.get(&P.rp, Af.m + 1));
             int nnzP = 0, nc = 0;
-            if(unsmoothed)
-                LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc, &tmp));
+            if(lal::small_fits(Af.m, Af.nnz))
+            {
+                const int room = std::max(Af.m, Af.nnz);
+                LAL_TRY(h->mem.get(&P.ci, room));
+                LAL_TRY(h->mem.get(&P.v, room));
+                LAL_TRY(h->mem.get(&R.rp, Af.m + 1));
+                LAL_TRY(h->mem.get(&R.ci, room));
+                LAL_TRY(h->mem.get(&R.v, room));
+                LAL_TRY(lal::small_build(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, o.relax,
+                                         unsmoothed, P.rp, P.ci, P.v, R.rp, R.ci, R.v, &nnzP, &nc,
+                                         &tmp));
+            }
             else
-                LAL_TRY(lal::sa_prolongator_nnz(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, P.rp,
-                                                &nnzP, &nc, &tmp));
+            {
+                int*     conn = nullptr;
+                int64_t* agg  = nullptr;
+                LAL_TRY(tmp.get(&conn, Af.nnz));
+                LAL_TRY(tmp.get(&agg, Af.m));
+                LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn, &tmp));
+                LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, &tmp));
+                if(unsmoothed)
+                    LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc, &tmp));
+                else
+                    LAL_TRY(lal::sa_prolongator_nnz(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg,
+                                                    P.rp, &nnzP, &nc, &tmp));
+                if(nc > 0)
+                {
+                    LAL_TRY(h->mem.get(&P.ci, nnzP));
+                    LAL_TRY(h->mem.get(&P.v, nnzP));
+                    if(unsmoothed)
+                        LAL_TRY(lal::ua_prolongator_fill(c, Af.m, agg, P.rp, P.ci, P.v));
+                    else
+                        LAL_TRY(lal::sa_prolongator_fill(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, conn,
+                                                         agg, o.relax, P.rp, P.ci, P.v));
+                    // R = P^T
+                    LAL_TRY(h->mem.get(&R.rp, nc + 1));
+                    LAL_TRY(h->mem.get(&R.ci, nnzP));
+                    LAL_TRY(h->mem.get(&R.v, nnzP));
+                    LAL_TRY(lal::transpose_f64(c, Af.m, nc, nnzP, P.rp, P.ci, P.v, R.rp, R.ci, R.v,
+                                               &tmp));
+                }
+            }
             if(nc == 0)
             {
                 P = csr_dev{};
+                R = csr_dev{};
                 break;
             }
             P.m   = Af.m;
             P.n   = nc;
             P.nnz = nnzP;
-            LAL_TRY(h->mem.get(&P.ci, nnzP));
-            LAL_TRY(h->mem.get(&P.v, nnzP));
-            if(unsmoothed)
-                LAL_TRY(lal::ua_prolongator_fill(c, Af.m, agg, P.rp, P.ci, P.v));
-            else
-                LAL_TRY(lal::sa_prolongator_fill(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, conn, agg,
-                                                 o.relax, P.rp, P.ci, P.v));
-            // R = P^T
             R.m   = nc;
             R.n   = Af.m;
             R.nnz = nnzP;
-            LAL_TRY(h->mem.get(&R.rp, nc + 1));
-            LAL_TRY(h->mem.get(&R.ci, nnzP));
-            LAL_TRY(h->mem.get(&R.v, nnzP));
-            LAL_TRY(lal::transpose_f64(c, P.m, P.n, P.nnz, P.rp, P.ci, P.v, R.rp, R.ci, R.v,
-                                       &tmp));
             // AP = A P (the fast path makes Q of it)
             csr_dev  ap_tmp;
             csr_dev& AP = o.exact ? ap_tmp : h->L[level].Q;

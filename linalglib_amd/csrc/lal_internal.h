@@ -156,6 +156,19 @@ namespace lal
         return x * per + (x < rem ? x : rem) + k;
     }
 
+    // By a whole wavefront: lane i < n's v into the note, then its sequence
+    // number.  The system-scope release waits for the wave's stores before it.
+    __device__ __forceinline__ void put_note(int* note, int n, int v, unsigned seq)
+    {
+        const int lane = (int)threadIdx.x & 63;
+        if(lane < n)
+            __hip_atomic_store(note + lane, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+        if(lane == 0)
+            __hip_atomic_store(reinterpret_cast<unsigned*>(note + LAL_NOTE_INTS), seq,
+                               __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+
     // v + the value of v in another lane of the same quad, half row or row
     // (DPP control CTRL: quad_perm, row_half_mirror 0x141, row_mirror 0x140).
     template <int CTRL>
@@ -171,6 +184,32 @@ namespace lal
     {
         const int o = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false);
         return v + __builtin_bit_cast(float, o);
+    }
+
+    // v of the partner lane in step STEP of a reduction over an aligned lane
+    // group: lane ^ 1, lane ^ 2, the half row's mirror image, the row's.  (A DPP
+    // move is an instruction or two; the shuffles they stand for go through LDS.)
+    template <int STEP>
+    __device__ __forceinline__ int partner(int v)
+    {
+        constexpr int CTRL = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : STEP == 2 ? 0x141 : 0x140;
+        return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+    }
+
+    // Reduction of an int over aligned groups of G = 8, 16 or 64 lanes, left in
+    // every lane; f is commutative, associative and f(a, a) = a.
+    template <int G, typename F>
+    __device__ __forceinline__ int group_fold(int v, F f)
+    {
+        v = f(v, partner<0>(v));
+        v = f(v, partner<1>(v));
+        v = f(v, partner<2>(v));
+        if(G >= 16)
+            v = f(v, partner<3>(v));
+        if(G == 64)
+            v = f(f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+                  f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+        return v;
     }
 
     // Sum over aligned groups of LANES (a power of two <= 64) lanes, left in
@@ -298,6 +337,9 @@ namespace lal
     int poll_word(lal_context* c, const unsigned* word, unsigned seq, bool* there);
     // Blocks until the context's note carries `seq`.
     int wait_note(lal_context* c, unsigned seq);
+    // The first n ints of the note carrying `seq` (blocks), for a kernel that
+    // was handed c->d_note and ++c->note_seq (put_note).
+    int take_note(lal_context* c, unsigned seq, int n, int* out);
     // The n ints at src once the stream has come to them (blocks); clear: they
     // are zeroed behind the read.
     int read_ints(lal_context* c, int* src, int n, int* out, bool clear);

@@ -142,16 +142,21 @@ namespace lal
         return LAL_OK;
     }
 
+    int take_note(lal_context* c, unsigned seq, int n, int* out)
+    {
+        LAL_TRY(wait_note(c, seq));
+        for(int i = 0; i < n; i++)
+            out[i] = __atomic_load_n(c->h_note + i, __ATOMIC_RELAXED);
+        return LAL_OK;
+    }
+
     int read_ints(lal_context* c, int* src, int n, int* out, bool clear)
     {
         LAL_REQUIRE(n >= 0 && n <= LAL_NOTE_INTS);
         const unsigned seq = ++c->note_seq;
         note_kernel<<<1, 64, 0, c->stream>>>(src, n, clear ? 1 : 0, c->d_note, seq);
         LAL_LAUNCHED();
-        LAL_TRY(wait_note(c, seq));
-        for(int i = 0; i < n; i++)
-            out[i] = __atomic_load_n(c->h_note + i, __ATOMIC_RELAXED);
-        return LAL_OK;
+        return take_note(c, seq, n, out);
     }
 }
 

@@ -665,10 +665,7 @@ namespace
     {
         const long long cap  = ncols > 1 ? ncols : 1;
         const long long need = 2LL * (prod < cap ? prod : cap);
-        long long       H    = 64;
-        while(H < need)
-            H <<= 1;
-        return H;
+        return need <= 64 ? 64 : 1LL << (64 - __clzll(need - 1));
     }
 
     // Rows of C grouped by hash-table size.
@@ -683,6 +680,7 @@ namespace
         int*              d_prod   = nullptr; // products per row (symbolic plan)
         int*              d_part   = nullptr; // row offsets per bin and workgroup
         int*              d_rows   = nullptr; // LDS-bin rows, then global rows
+        long long*        d_gsl    = nullptr; // table sizes of the global rows
         long long*        d_toff   = nullptr;
         int*              d_keys   = nullptr;
         double*           d_vals   = nullptr;
@@ -697,19 +695,21 @@ namespace
     // numeric pass sizes every row by its nonzero count from the symbolic
     // pass (`crp`), empty rows included, so that a row pointer which
     // undercounts them is detected.
+    __device__ __forceinline__ int size_bin(int p, bool skip_empty, int ncols, int max_h,
+                                            long long* slots)
+    {
+        if(skip_empty && p <= 0)
+            return -1;
+        const long long H = table_slots(p > 0 ? p : 0, ncols);
+        *slots            = H;
+        // (H is a power of two of 64 or more)
+        return H > max_h ? kBins : __ffsll(H) - 7;
+    }
     __device__ __forceinline__ int row_bin(int i, const int* __restrict__ prod,
                                            const int* __restrict__ crp, int ncols, int max_h,
                                            long long* slots)
     {
-        const int p = crp ? crp[i + 1] - crp[i] : prod[i];
-        if(!crp && p <= 0)
-            return -1;
-        const long long H = table_slots(p > 0 ? p : 0, ncols);
-        *slots            = H;
-        int b             = 0;
-        while((64LL << b) < H && b < kBins)
-            b++;
-        return H > max_h ? kBins : b;
+        return size_bin(crp ? crp[i + 1] - crp[i] : prod[i], !crp, ncols, max_h, slots);
     }
 
     // Rows of a workgroup of the binning kernels (each takes one contiguous
@@ -749,11 +749,11 @@ namespace
     }
 
     // One workgroup: the counts, bin after bin, become row offsets (one scan
-    // over all of them); out[b] = rows of bin b, out[kBins + 1] = *tail when
-    // given.
+    // over all of them).  The host's note: the rows of every bin, then *tail
+    // (when given).
     __global__ void __launch_bounds__(1024)
-        bin_scan_kernel(int groups, int* __restrict__ part, int* __restrict__ out,
-                        const int* __restrict__ tail)
+        bin_scan_kernel(int groups, int* __restrict__ part, const int* __restrict__ tail,
+                        int* note, unsigned seq)
     {
         __shared__ int s_w[16];
         __shared__ int s_first[kBins + 2]; // offset of each bin's first row
@@ -792,10 +792,12 @@ namespace
         if(threadIdx.x == 0)
             s_first[kBins + 1] = carry;
         __syncthreads();
-        if(threadIdx.x <= kBins)
-            out[threadIdx.x] = s_first[threadIdx.x + 1] - s_first[threadIdx.x];
-        if(threadIdx.x == 0)
-            out[kBins + 1] = tail ? *tail : 0;
+        if(wid == 0)
+            lal::put_note(note, kBins + 2,
+                          lane <= kBins                ? s_first[lane + 1] - s_first[lane]
+                          : lane == kBins + 1 && tail ? *tail
+                                                      : 0,
+                          seq);
     }
 
     // Rows into their bins, at the workgroup's offsets (each row of C is
@@ -826,30 +828,140 @@ namespace
         }
     }
 
-    // Rows of C binned by table size on the device: counts the rows of each
-    // bin and hands the host the eleven counts (and, for the numeric plan,
-    // *tail, which it wants at the same time).
-    int plan_count(lal_context* c, int m, int n, const int* crp, bool numeric, spgemm_plan& P,
-                   lal::temps& tmp, int* clear, const int* tail, int* tail_out)
+    // The whole plan of up to PLAN_SMALL rows in one workgroup: a small
+    // product's time is its launches (a 25^3 hierarchy build: 318 launches in
+    // 2.5 ms).  Row sizes from prod (crp null), from the row pointer crp, or,
+    // with SCAN, from the counts in crp, which become the row pointer (m + 1
+    // entries).  rows gets the rows bin by bin, gslots the table sizes of those
+    // in the last bin, the note what bin_scan_kernel's gets.
+    constexpr int PLAN_CHUNKS = 16;
+    constexpr int PLAN_SMALL  = PLAN_CHUNKS * 1024 - 1;
+
+    template <bool SCAN>
+    __global__ void __launch_bounds__(1024)
+        plan_small_kernel(int m, const int* __restrict__ prod, int* __restrict__ crp, int ncols,
+                          int max_h, int* __restrict__ rows, long long* __restrict__ gslots,
+                          int* __restrict__ clear, int* note, unsigned seq)
+    {
+        __shared__ int s_w[2][16];
+        __shared__ int s_n[kBins + 1], s_at[kBins + 1];
+        const int      tid = (int)threadIdx.x, lane = tid & 63, wid = tid >> 6;
+        if(tid <= kBins)
+            s_n[tid] = 0;
+        // (chunks past the last row are skipped by the whole workgroup)
+        int p[PLAN_CHUNKS];
+#pragma unroll
+        for(int k = 0; k < PLAN_CHUNKS; k++)
+            if(k * 1024 <= m)
+            {
+                const int i = k * 1024 + tid;
+                p[k]        = i >= m ? 0 : SCAN ? crp[i] : crp ? crp[i + 1] - crp[i] : prod[i];
+                if(clear && i <= m)
+                    clear[i] = 0;
+            }
+        __syncthreads();
+        int total = 0;
+#pragma unroll
+        for(int k = 0; k < PLAN_CHUNKS; k++)
+            if(k * 1024 <= m)
+            {
+                const int i = k * 1024 + tid;
+                if(SCAN)
+                {
+                    int inc = p[k];
+#pragma unroll
+                    for(int o = 1; o < 64; o <<= 1)
+                    {
+                        const int q = __shfl_up(inc, o, 64);
+                        inc += lane >= o ? q : 0;
+                    }
+                    if(lane == 63)
+                        s_w[k & 1][wid] = inc;
+                    __syncthreads();
+                    int at = total + inc - p[k];
+                    for(int w = 0; w < 16; w++)
+                    {
+                        at += w < wid ? s_w[k & 1][w] : 0;
+                        total += s_w[k & 1][w];
+                    }
+                    if(i <= m)
+                        crp[i] = at;
+                }
+                long long H = 0;
+                const int b = i < m ? size_bin(p[k], !SCAN && !crp, ncols, max_h, &H) : -1;
+                if(b >= 0)
+                    atomicAdd(&s_n[b], 1);
+            }
+        __syncthreads();
+        if(tid <= kBins)
+        {
+            int at = 0;
+            for(int b = 0; b < tid; b++)
+                at += s_n[b];
+            s_at[tid] = at;
+        }
+        __syncthreads();
+        const int g0 = s_at[kBins];
+        __syncthreads();
+#pragma unroll
+        for(int k = 0; k < PLAN_CHUNKS; k++)
+            if(k * 1024 < m)
+            {
+                long long H = 0;
+                const int i = k * 1024 + tid;
+                const int b = i < m ? size_bin(p[k], !SCAN && !crp, ncols, max_h, &H) : -1;
+                if(b < 0)
+                    continue;
+                const int pos = atomicAdd(&s_at[b], 1);
+                rows[pos]     = i;
+                if(b == kBins)
+                    gslots[pos - g0] = H;
+            }
+        if(wid == 0)
+            lal::put_note(note, kBins + 2,
+                          lane <= kBins ? s_n[lane] : lane == kBins + 1 ? total : 0, seq);
+    }
+
+    // Rows of C binned by table size on the device; the host gets the eleven
+    // counts and, with `scan` (crp holds the rows' counts and becomes the row
+    // pointer), the number of C's entries.  Up to PLAN_SMALL rows are in their
+    // lists after one launch, larger products' go there in plan_rows.
+    int plan_count(lal_context* c, int m, int n, int* crp, bool numeric, spgemm_plan& P,
+                   lal::temps& tmp, int* clear, bool scan, int* total_out, lal::arena* a)
     {
         constexpr int nb = kBins + 1;
         P.bin_start.assign(nb, 0);
         P.n_lds = P.n_global = 0;
         if(m <= 0)
             return LAL_OK;
-        const int per    = bin_rows(m);
-        const int groups = (m + per - 1) / per;
-        int*      out    = nullptr;
-        LAL_TRY(tmp.get(&P.d_part, (size_t)nb * groups));
-        LAL_TRY(tmp.get(&out, nb + 1));
-        bin_count_kernel<<<groups, 256, 0, c->stream>>>(m, per, P.d_prod, numeric ? crp : nullptr,
-                                                        n, numeric ? kLdsMaxH : kLdsMaxHSym,
-                                                        P.d_part, clear);
-        LAL_LAUNCHED();
-        bin_scan_kernel<<<1, 1024, 0, c->stream>>>(groups, P.d_part, out, tail);
+        const int max_h = numeric ? kLdsMaxH : kLdsMaxHSym;
+        unsigned  seq   = 0;
+        if(m <= PLAN_SMALL)
+        {
+            LAL_TRY(tmp.get(&P.d_rows, m));
+            LAL_TRY(tmp.get(&P.d_gsl, m));
+            seq      = ++c->note_seq;
+            auto* fn = scan ? plan_small_kernel<true> : plan_small_kernel<false>;
+            fn<<<1, 1024, 0, c->stream>>>(m, P.d_prod, numeric ? crp : nullptr, n, max_h, P.d_rows,
+                                          P.d_gsl, clear, c->d_note, seq);
+        }
+        else
+        {
+            if(scan)
+                LAL_TRY(lal::scan_i32_dev(c, m + 1, crp, a));
+            const int per    = bin_rows(m);
+            const int groups = (m + per - 1) / per;
+            LAL_TRY(tmp.get(&P.d_part, (size_t)nb * groups));
+            bin_count_kernel<<<groups, 256, 0, c->stream>>>(
+                m, per, P.d_prod, numeric ? crp : nullptr, n, max_h, P.d_part, clear);
+            LAL_LAUNCHED();
+            seq = ++c->note_seq;
+            bin_scan_kernel<<<1, 1024, 0, c->stream>>>(groups, P.d_part, scan ? crp + m : nullptr,
+                                                       c->d_note, seq);
+        }
         LAL_LAUNCHED();
         int got[nb + 1];
-        LAL_TRY(lal::read_ints(c, out, nb + 1, got, false));
+        LAL_TRY(lal::take_note(c, seq, nb + 1, got));
         int total = 0;
         for(int b = 0; b < nb; b++)
         {
@@ -858,32 +970,35 @@ namespace
         }
         P.n_lds    = P.bin_start[kBins];
         P.n_global = got[kBins];
-        if(tail_out)
-            *tail_out = got[kBins + 1];
+        if(total_out)
+            *total_out = got[kBins + 1];
         return LAL_OK;
     }
 
-    // The rows' lists, and the tables of those that need global memory.
+    // The rows' lists where they are not there yet, and the tables of those
+    // that need global memory.
     int plan_rows(lal_context* c, int m, int n, const int* crp, bool numeric, spgemm_plan& P,
                   lal::temps& tmp)
     {
         const int total = P.n_lds + P.n_global;
         if(total == 0)
             return LAL_OK;
-        const int  per    = bin_rows(m);
-        const int  groups = (m + per - 1) / per;
-        long long* d_gsl  = nullptr;
-        LAL_TRY(tmp.get(&P.d_rows, total));
-        if(P.n_global)
-            LAL_TRY(tmp.get(&d_gsl, P.n_global));
-        bin_scatter_kernel<<<groups, 256, 0, c->stream>>>(
-            m, per, P.d_prod, numeric ? crp : nullptr, n, numeric ? kLdsMaxH : kLdsMaxHSym,
-            P.d_part, P.d_rows, P.n_lds, d_gsl);
-        LAL_LAUNCHED();
+        if(m > PLAN_SMALL)
+        {
+            const int per    = bin_rows(m);
+            const int groups = (m + per - 1) / per;
+            LAL_TRY(tmp.get(&P.d_rows, total));
+            if(P.n_global)
+                LAL_TRY(tmp.get(&P.d_gsl, P.n_global));
+            bin_scatter_kernel<<<groups, 256, 0, c->stream>>>(
+                m, per, P.d_prod, numeric ? crp : nullptr, n, numeric ? kLdsMaxH : kLdsMaxHSym,
+                P.d_part, P.d_rows, P.n_lds, P.d_gsl);
+            LAL_LAUNCHED();
+        }
         if(P.n_global)
         {
             P.toff.assign(P.n_global + 1, 0);
-            LAL_HIP(hipMemcpyAsync(P.toff.data() + 1, d_gsl, sizeof(long long) * P.n_global,
+            LAL_HIP(hipMemcpyAsync(P.toff.data() + 1, P.d_gsl, sizeof(long long) * P.n_global,
                                    hipMemcpyDeviceToHost, c->stream));
             LAL_HIP(hipStreamSynchronize(c->stream));
             for(int r = 0; r < P.n_global; r++)
@@ -1074,14 +1189,13 @@ namespace lal
         P.g = g;
         P.l = l;
         LAL_TRY(count_products(c, m, arp, aci, brp, nnz_a, P, tmp));
-        LAL_TRY(plan_count(c, m, n, nullptr, false, P, tmp, crp, nullptr, nullptr));
+        LAL_TRY(plan_count(c, m, n, nullptr, false, P, tmp, crp, false, nullptr, a));
         LAL_TRY(plan_rows(c, m, n, nullptr, false, P, tmp));
         LAL_TRY(run_plan<false>(c, P, arp, aci, nullptr, brp, bci, nullptr, nullptr, crp,
                                 nullptr));
-        LAL_TRY(scan_i32_dev(c, m + 1, crp, a));
         num.g = g;
         num.l = l;
-        return plan_count(c, m, n, crp, true, num, tmp, nullptr, crp + m, nnz_c);
+        return plan_count(c, m, n, crp, true, num, tmp, nullptr, true, nnz_c, a);
     }
 
     int csrgemm_nnz(lal_context* c, int m, int k, int n, const int* arp, const int* aci,
@@ -1101,7 +1215,8 @@ namespace lal
         spgemm_plan P;
         P.g = lanes_for(m > 0 ? nnz_a / m : 0);
         P.l = lanes_for(k > 0 ? nnz_b / k : 0);
-        LAL_TRY(plan_count(c, m, n, crp, true, P, tmp, nullptr, nullptr, nullptr));
+        LAL_TRY(plan_count(c, m, n, const_cast<int*>(crp), true, P, tmp, nullptr, false, nullptr,
+                           nullptr));
         LAL_TRY(plan_rows(c, m, n, crp, true, P, tmp));
         LAL_TRY(run_plan<true>(c, P, arp, aci, av, brp, bci, bv, crp, cci, cv));
         int bad = 0;
