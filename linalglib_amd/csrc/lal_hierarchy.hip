@@ -185,6 +185,46 @@ namespace
         return A.d;
     }
 
+    // Which operators are read with cache-allocating loads, per precision of the
+    // cycle: they share lal::CACHE_KEEP_BYTES of the Infinity Cache.  The finest
+    // one comes first (a PCG iteration reads it three times), then, beside eight
+    // of the iteration's vectors, whole levels from the coarsest up.  Gradient on 64^3, where everything fits: 14.1 ms
+    // with the finest alone, 13.25 with all; PCG on 101^3 (FP64), where levels 3
+    // and up fit: 8.65 and 8.54 ms, but 9.03 with level 2 and 9.05 with all,
+    // since what overflows evicts the rest; in FP32 on 128^3 levels 3 and up
+    // (61 MB, of which 37 are free by this count) cost 0.6 %.
+    void choose_kept(lal_hierarchy_t* h)
+    {
+        for(const size_t prec : {sizeof(double), sizeof(float)})
+        {
+            const int bit  = prec == sizeof(double) ? 1 : 2;
+            size_t    room = lal::CACHE_KEEP_BYTES;
+            auto      size = [&](const csr_dev& M) {
+                // (a column list adds about a third of an entry per nonzero)
+                return !M.d ? 0
+                            : (size_t)M.nnz * (prec + (M.d->list_max ? 3 : M.d->d_c16 ? 2 : 4));
+            };
+            auto take = [&](std::initializer_list<csr_dev*> ops) {
+                size_t all = 0;
+                for(const csr_dev* M : ops)
+                    all += size(*M);
+                if(all > room)
+                    return false;
+                room -= all;
+                for(csr_dev* M : ops)
+                    if(M->d)
+                        M->d->keep |= bit;
+                return true;
+            };
+            if(!take({&h->L[0].A}))
+                continue;
+            room -= std::min(room, 8 * prec * (size_t)h->L[0].A.m);
+            int l = h->levels;
+            while(l > 0 && take({&h->L[l].A, &h->L[l - 1].R, &h->L[l - 1].Q}))
+                l--;
+        }
+    }
+
     int finish_setup(lal_hierarchy_t* h, lal::arena* tmp)
     {
         lal_context* c     = h->c;
@@ -202,15 +242,11 @@ namespace
                                    A->nnz, exact == 0, -1,
                                    A == &h->L[l].Q || A == &h->L[l].A || A == &h->L[l].R});
         LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
+        if(!exact)
+            choose_kept(h);
         for(int l = 0; l <= h->levels; l++)
         {
             level_t& L = h->L[l];
-            // The finest operator is read three times per PCG iteration
-            // (residual, post-sweep, the Krylov product), the last two with
-            // only vector passes between them: it may stay in the Infinity
-            // Cache when it fits (decided per precision at launch).  Keeping
-            // a coarser level as well overflows the cache and slows the solve.
-            L.A.d->keep = l == 0;
             LAL_TRY(h->mem.get(&L.w64.x, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.t, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.b, L.A.m));

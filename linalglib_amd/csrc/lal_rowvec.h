@@ -14,10 +14,9 @@
 // Unaligned arrays take the product-staging kernel: lanes gather x for
 // consecutive nonzeros and stage a_ij * x_j in LDS before the row sums.
 // Column indices and values are read once per call, so they are streamed
-// (non-temporal) and x keeps the caches -- except for an operator marked
-// `keep` that fits lal::CACHE_KEEP_BYTES (a hierarchy's finest level, read
-// several times per solver iteration), whose ordinary loads let it stay in
-// the Infinity Cache between calls.  The sum order differs from the
+// (non-temporal) and x keeps the caches -- except for operators marked `keep`
+// (a hierarchy's, as many as share the Infinity Cache), whose ordinary loads
+// let them stay there between calls.  The sum order differs from the
 // host's sequential fma, so results agree to rounding, deterministically; the
 // bit-exact path is the row-block kernel of lal_csrmv.hip.
 //

@@ -578,9 +578,11 @@ namespace
     {
         return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + byte);
     }
-    template <typename V, typename T>
+    template <typename V, bool KEEP, typename T>
     __device__ __forceinline__ V stream_at(const T* p, unsigned byte)
     {
+        if(KEEP)
+            return load_at<V>(p, byte);
         return __builtin_nontemporal_load(
             reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + byte));
     }
@@ -605,9 +607,10 @@ namespace
     constexpr int LIST_U = 4; // list pairs per lane: a list has at most 2044 entries
 
     //
+    // KEEP: the matrix is read with cache-allocating loads (lal_csrmv_info::keep).
     // FAR: some block's columns span more than 65536 (the finest restriction
     // of a large grid), and its list's entries from `split` on are 65536 further.
-    template <typename T, int MODE, bool FAR>
+    template <typename T, int MODE, bool FAR, bool KEEP>
     __global__ void __launch_bounds__(SPMV_THREADS)
         list_kernel(const int* __restrict__ blocks, int nb, int list_max,
                     const int* __restrict__ rp, const unsigned short* __restrict__ lpos,
@@ -643,7 +646,7 @@ namespace
 #pragma unroll
         for(int u = 0; u < LIST_U; u++)
             if(SPMV_THREADS * u < np) // (uniform)
-                lo[u] = stream_at<unsigned>(lb, 4u * min(tid + SPMV_THREADS * u, np - 1));
+                lo[u] = stream_at<unsigned, KEEP>(lb, 4u * min(tid + SPMV_THREADS * u, np - 1));
         us4v    pq[2];
         quad<T> vq[2];
 #pragma unroll
@@ -651,9 +654,9 @@ namespace
             if(SPMV_THREADS * u < nq) // (uniform)
             {
                 const unsigned q = min(tid + SPMV_THREADS * u, nq - 1);
-                pq[u]            = stream_at<us4v>(pb, 8u * q);
-                vq[u].load(reinterpret_cast<const T*>(reinterpret_cast<const char*>(vb) +
-                                                      4u * sizeof(T) * q));
+                pq[u]            = stream_at<us4v, KEEP>(pb, 8u * q);
+                vq[u].template load<KEEP>(reinterpret_cast<const T*>(
+                    reinterpret_cast<const char*>(vb) + 4u * sizeof(T) * q));
             }
         const int  lrow = (int)tid >> lg;
         const bool on   = lrow < nrows;
@@ -718,15 +721,19 @@ namespace
             row_epilogue<T, MODE>(r0 + lrow, acc, ops, alpha, beta, y, r);
     }
 
+    template <typename T>
+    bool kept(const lal::rv_args& a)
+    {
+        return a.keep & (sizeof(T) == sizeof(double) ? 1 : 2);
+    }
+
     template <typename T, int MODE, bool C16>
     void launch_quad(lal_context* c, const lal::rv_args& a, int nb)
     {
         // LDS sized to the widest block window of this matrix, so that short
         // blocks leave room for more resident workgroups
         const int    win  = a.win;
-        const size_t cbyt = C16 ? sizeof(unsigned short) : sizeof(int);
-        const bool   keep = a.keep && (sizeof(T) + cbyt) * (size_t)a.nnz <= lal::CACHE_KEEP_BYTES;
-        auto*        fn   = keep ? quad_kernel<T, MODE, true, C16> : quad_kernel<T, MODE, false, C16>;
+        auto*        fn   = kept<T>(a) ? quad_kernel<T, MODE, true, C16> : quad_kernel<T, MODE, false, C16>;
         const int    more = MODE == lal::RV_SMOOTHED && a.ex.post.part ? 1 : 0;
         fn<<<nb + more, SPMV_THREADS, RP_LDS_BYTES + (sizeof(int) + sizeof(T)) * win, c->stream>>>(
             a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
@@ -739,7 +746,10 @@ namespace
     {
         const int    lm  = (a.list_max + 3) & ~3;
         const size_t lds = RP_LDS_BYTES + sizeof(T) * (size_t)(lm + a.win);
-        auto* fn = a.list_far ? list_kernel<T, MODE, true> : list_kernel<T, MODE, false>;
+        auto* fn = kept<T>(a) ? (a.list_far ? list_kernel<T, MODE, true, true>
+                                        : list_kernel<T, MODE, false, true>)
+                          : (a.list_far ? list_kernel<T, MODE, true, false>
+                                        : list_kernel<T, MODE, false, false>);
         fn<<<nb, SPMV_THREADS, lds, c->stream>>>(
             a.blocks, nb, lm, a.rp, a.lpos, a.list, a.lmeta, (const T*)a.val, (const T*)a.x,
             (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r, a.ex);

@@ -543,6 +543,7 @@ namespace lal
         rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, e, nullptr, y, out,
                   nullptr, 0.0, 0.0, d->win};
         lal::use_c16(a, d);
+        a.keep = d->keep;
         return a;
     }
 
