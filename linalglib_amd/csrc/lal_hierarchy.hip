@@ -166,14 +166,6 @@ namespace
         return LAL_OK;
     }
 
-    int to_f32(lal_hierarchy_t* h, const double* x, float** y, size_t n)
-    {
-        LAL_TRY(h->mem.get(y, n));
-        if(n)
-            LAL_TRY(lal_convert_f64_f32(h->c, x, *y, n));
-        return LAL_OK;
-    }
-
     // A fresh descriptor for an m x n operator of a hierarchy.
     lal_csrmv_info* descr(csr_dev& A, int m, int nnz, int n, int exact)
     {
@@ -188,11 +180,10 @@ namespace
     // Which operators are read with cache-allocating loads, per precision of the
     // cycle: they share lal::CACHE_KEEP_BYTES of the Infinity Cache.  The finest
     // one comes first (a PCG iteration reads it three times), then, beside eight
-    // of the iteration's vectors, whole levels from the coarsest up.  Gradient on 64^3, where everything fits: 14.1 ms
-    // with the finest alone, 13.25 with all; PCG on 101^3 (FP64), where levels 3
-    // and up fit: 8.65 and 8.54 ms, but 9.03 with level 2 and 9.05 with all,
-    // since what overflows evicts the rest; in FP32 on 128^3 levels 3 and up
-    // (61 MB, of which 37 are free by this count) cost 0.6 %.
+    // of the iteration's vectors, whole levels from the coarsest up.  Gradient on
+    // 64^3, where everything fits: 14.1 ms with the finest alone, 13.25 with all;
+    // PCG on 101^3 (FP64), where levels 3 and up fit: 8.65 and 8.54 ms, but 9.03
+    // with level 2 and 9.05 with all, since what overflows evicts the rest.
     void choose_kept(lal_hierarchy_t* h)
     {
         for(const size_t prec : {sizeof(double), sizeof(float)})
@@ -244,6 +235,7 @@ namespace
         LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
         if(!exact)
             choose_kept(h);
+        lal::f32_copies copies;
         for(int l = 0; l <= h->levels; l++)
         {
             level_t& L = h->L[l];
@@ -253,33 +245,42 @@ namespace
             LAL_TRY(h->mem.get(&L.w64.r, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.diag, L.A.m));
             LAL_TRY(h->mem.get(&L.w64.dinv, L.A.m));
-            LAL_TRY(lal::diag_inv<double>(c, L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag,
-                                          L.w64.dinv, L.A.nnz));
-            if(L.Q.rp && l < h->levels)
+            const bool       up = l < h->levels, f32 = h->opts.build_f32, q = up && L.Q.rp;
+            lal::ready_level r{L.A.m, L.A.rp, L.A.ci, L.A.v, L.w64.diag, L.w64.dinv};
+            if(f32)
             {
-                if(h->opts.build_f32)
-                    LAL_TRY(h->mem.get(&L.Q.v32, L.Q.nnz));
-                LAL_TRY(lal::smoothed_prolongator(c, L.Q.m, L.Q.nnz, L.Q.rp, L.Q.ci, L.Q.v, L.P.rp,
-                                                  L.P.ci, L.P.v, L.w64.dinv, L.Q.v32));
-            }
-            if(h->opts.build_f32)
-            {
-                LAL_TRY(to_f32(h, L.A.v, &L.A.v32, L.A.nnz));
-                if(l < h->levels)
-                {
-                    LAL_TRY(to_f32(h, L.P.v, &L.P.v32, L.P.nnz));
-                    LAL_TRY(to_f32(h, L.R.v, &L.R.v32, L.R.nnz));
-                }
+                LAL_TRY(h->mem.get(&L.A.v32, L.A.nnz));
+                for(csr_dev* M : {&L.P, &L.R})
+                    if(up)
+                    {
+                        LAL_TRY(h->mem.get(&M->v32, M->nnz));
+                        copies.add(M->v, M->v32, M->nnz);
+                    }
                 LAL_TRY(h->mem.get(&L.w32.x, L.A.m));
                 LAL_TRY(h->mem.get(&L.w32.t, L.A.m));
                 LAL_TRY(h->mem.get(&L.w32.b, L.A.m));
                 LAL_TRY(h->mem.get(&L.w32.r, L.A.m));
                 LAL_TRY(h->mem.get(&L.w32.diag, L.A.m));
                 LAL_TRY(h->mem.get(&L.w32.dinv, L.A.m));
-                LAL_TRY(lal::diag_inv<float>(c, L.A.m, L.A.rp, L.A.ci, L.A.v32, L.w32.diag,
-                                             L.w32.dinv, L.A.nnz));
+                r.v32    = L.A.v32;
+                r.d32    = L.w32.diag;
+                r.dinv32 = L.w32.dinv;
+                if(q)
+                    LAL_TRY(h->mem.get(&L.Q.v32, L.Q.nnz));
             }
+            if(q)
+            {
+                r.qrp  = L.Q.rp;
+                r.qci  = L.Q.ci;
+                r.qv   = L.Q.v;
+                r.qv32 = L.Q.v32;
+                r.prp  = L.P.rp;
+                r.pci  = L.P.ci;
+                r.pv   = L.P.v;
+            }
+            LAL_TRY(lal::make_ready(c, r, q ? std::max(L.A.nnz, L.Q.nnz) : L.A.nnz));
         }
+        LAL_TRY(lal::copy_f32(c, copies));
         // coarsest level
         csr_dev& Ac = h->L[h->levels].A;
         if(Ac.m == 1)

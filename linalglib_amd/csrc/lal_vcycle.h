@@ -73,20 +73,51 @@ namespace lal
     template <typename T>
     int product_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, int nnz, const int* rp,
                     const int* ci, const T* v, const T* x, T* y, double* part, int* count);
-    // AP's values become those of Q = P - D^-1 A P (pattern of A P, a superset
-    // of P's; both with ascending columns); v32 (or null): the same in FP32.
-    int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
-                             double* v, const int* prp, const int* pci, const double* pv,
-                             const double* dinv, float* v32);
+    // A level's arrays for make_ready: from A, d (the last diagonal entry of each
+    // row), dinv = 1/d and, with v32, the FP32 copies of A's values, d and 1/d;
+    // with qv, A P's values become those of Q = P - D^-1 A P (pattern of A P, a
+    // superset of P's; both with ascending columns), in qv32 (or null) in FP32.
+    struct ready_level
+    {
+        int           m;
+        const int *   rp, *ci;
+        const double* v;
+        double *      d, *dinv;
+        float *       v32, *d32, *dinv32;
+        const int *   qrp, *qci;
+        double*       qv;
+        float*        qv32;
+        const int *   prp, *pci;
+        const double* pv;
+    };
+    // nnz: the longer of A's and Q's, which picks the lanes per row
+    int make_ready(lal_context* c, const ready_level& a, long nnz);
+    // y = (float) x for the arrays added.
+    struct f32_copies
+    {
+        static constexpr int PER = 2048; // entries per workgroup
+        struct one
+        {
+            const double* x;
+            float*        y;
+            size_t        len;
+            int           block0;
+        };
+        one  c[40]; // (P and R of up to 20 levels)
+        int  n = 0, blocks = 0;
+        void add(const double* x, float* y, size_t len)
+        {
+            if(len == 0)
+                return;
+            c[n++] = {x, y, len, blocks};
+            blocks += (int)((len + PER - 1) / PER);
+        }
+    };
+    int copy_f32(lal_context* c, const f32_copies& a);
     template <typename T>
     int jacobi0_residual(lal_context* c, const lal_csrmv_info* d, int m, const int* rp,
                          const int* ci, const T* v, const T* diag, const T* dinv, const T* b,
                          T* x, T* r);
-    // d = the last diagonal entry of each row, dinv = 1/d.
-    template <typename T>
-    // nnz: the operator's nonzeros, which pick a lane or a wavefront per row
-    int diag_inv(lal_context* c, int m, const int* rp, const int* ci, const T* v, T* d, T* dinv,
-                 long nnz = 0);
     template <typename T>
     int coarse_scalar(lal_context* c, const T* v, const T* b, T* x);
     template <typename T>

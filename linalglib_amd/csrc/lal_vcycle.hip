@@ -113,48 +113,6 @@ namespace
         }
     }
 
-    // a_ii as the Jacobi sweep sees it (the last diagonal entry of the row)
-    // and its reciprocal for the fast path.
-    template <typename T>
-    __global__ void __launch_bounds__(256)
-        diag_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                    const T* __restrict__ val, T* __restrict__ d, T* __restrict__ dinv)
-    {
-        int i = blockIdx.x * 256 + threadIdx.x;
-        if(i >= m)
-            return;
-        T a = 0;
-        for(int j = rp[i]; j < rp[i + 1]; j++)
-            if(ci[j] == i)
-                a = val[j];
-        d[i]    = a;
-        dinv[i] = (T)1 / a;
-    }
-
-    // diag_kernel with 64 lanes per row, for long rows: the row's last
-    // diagonal entry is the group's largest matching position.
-    template <typename T>
-    __global__ void __launch_bounds__(256)
-        diag_wave_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                         const T* __restrict__ val, T* __restrict__ d, T* __restrict__ dinv)
-    {
-        const int lane = (int)threadIdx.x & 63;
-        const int i    = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-        if(i >= m)
-            return;
-        int last = -1;
-        for(int j = rp[i] + lane; j < rp[i + 1]; j += 64)
-            if(ci[j] == i)
-                last = j;
-        last = lal::wave_max(last);
-        if(lane == 0)
-        {
-            const T a = last >= 0 ? val[last] : (T)0;
-            d[i]      = a;
-            dinv[i]   = (T)1 / a;
-        }
-    }
-
     // Coarsest level with one unknown: x = b / a (amg.cpp:211-216).
     template <typename T>
     __global__ void scalar_solve_kernel(const T* __restrict__ val, const T* __restrict__ b,
@@ -393,34 +351,53 @@ namespace
             p[i] = beta == (T)0 ? (T)z[i] : (T)z[i] + beta * p[i];
     }
 
-    // G lanes per row: entry (i, c) of A P becomes P(i, c) - dinv_i (A P)(i, c),
-    // in FP64 and, with v32, rounded to FP32 as well.  The row of P lies in the
-    // group's registers (up to G entries; a longer one is searched in memory)
-    // and is compared by shuffles, so a row's loads are one chain of two: a
-    // binary search in memory per entry, with 16 lanes on every row, took
-    // 452 us over the levels of a 121^3 diffusion hierarchy and the FP32 copy
-    // another pass (90 us); now 300 us with the copy.
+    // A level's operator made ready for the cycle, G lanes per row in one pass:
+    // the row's last diagonal entry d and 1/d; with A P given, its entry (i, c)
+    // becomes Q's, P(i, c) - 1/d (A P)(i, c); all of it in FP32 too where asked
+    // for.  The row of P lies in the group's registers (up to G entries; a longer
+    // one is searched in memory) and is compared by shuffles, so a row's loads
+    // are two short chains.  Bound by memory and, on small levels, by the launch:
+    // as six passes per level (two diagonals, Q, three FP32 copies) it took
+    // 0.82 ms over a 121^3 diffusion hierarchy, as this one and one for all the
+    // copies of P and R 0.52.
     template <int G>
-    __global__ void __launch_bounds__(256)
-        smoothed_prolongator_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
-                                    double* __restrict__ v, const int* __restrict__ prp,
-                                    const int* __restrict__ pci, const double* __restrict__ pv,
-                                    const double* __restrict__ dinv, float* __restrict__ v32)
+    __global__ void __launch_bounds__(256) ready_kernel(lal::ready_level a)
     {
         const int i = blockIdx.x * (256 / G) + (int)(threadIdx.x / G);
-        if(i >= m)
+        if(i >= a.m)
             return;
-        const int    t  = (int)(threadIdx.x & (G - 1));
-        const double di = dinv[i];
-        const int    ps = prp[i], pn = prp[i + 1] - ps;
-        const int    s = rp[i], e = rp[i + 1];
-        const int    pc = t < pn ? pci[ps + t] : -1;
-        const double pw = t < pn ? pv[ps + t] : 0.0;
+        const int t  = (int)(threadIdx.x & (G - 1));
+        const int rs = a.rp[i], re = a.rp[i + 1];
+        const int s = a.qv ? a.qrp[i] : 0, e = a.qv ? a.qrp[i + 1] : 0;
+        const int    ps = a.qv ? a.prp[i] : 0, pn = a.qv ? a.prp[i + 1] - ps : 0;
+        const int    pc = t < pn ? a.pci[ps + t] : -1;
+        const double pw = t < pn ? a.pv[ps + t] : 0.0;
+        int          last = -1;
+        for(int j = rs + t; j < re; j += G)
+        {
+            if(a.ci[j] == i)
+                last = j;
+            if(a.v32)
+                a.v32[j] = (float)a.v[j];
+        }
+        last            = lal::group_fold<G>(last, [](int x, int y) { return max(x, y); });
+        const double d  = last >= 0 ? a.v[last] : 0.0;
+        const double di = 1.0 / d;
+        if(t == 0)
+        {
+            a.d[i]    = d;
+            a.dinv[i] = di;
+            if(a.v32)
+            {
+                a.d32[i]    = (float)d;
+                a.dinv32[i] = 1.0f / (float)d;
+            }
+        }
         for(int j0 = s; j0 < e; j0 += G)
         {
             const int    j = j0 + t;
-            const int    c = j < e ? ci[j] : -1;
-            const double a = j < e ? v[j] : 0.0;
+            const int    c = j < e ? a.qci[j] : -1;
+            const double w = j < e ? a.qv[j] : 0.0;
             double       p = 0.0;
             if(pn <= G)
             {
@@ -436,21 +413,35 @@ namespace
                 while(lo < hi)
                 {
                     const int mid = (lo + hi) >> 1;
-                    if(pci[mid] < c)
+                    if(a.pci[mid] < c)
                         lo = mid + 1;
                     else
                         hi = mid;
                 }
-                p = lo < ps + pn && pci[lo] == c ? pv[lo] : 0.0;
+                p = lo < ps + pn && a.pci[lo] == c ? a.pv[lo] : 0.0;
             }
             if(j < e)
             {
-                const double q = p - di * a;
-                v[j]           = q;
-                if(v32)
-                    v32[j] = (float)q;
+                const double q = p - di * w;
+                a.qv[j]        = q;
+                if(a.qv32)
+                    a.qv32[j] = (float)q;
             }
         }
+    }
+
+    // FP32 copies of several arrays, one after the other in the grid.
+    __global__ void __launch_bounds__(256) copies_kernel(lal::f32_copies a)
+    {
+        int k = 0;
+        while(k + 1 < a.n && a.c[k + 1].block0 <= (int)blockIdx.x)
+            k++;
+        const lal::f32_copies::one o = a.c[k];
+        const size_t at = (size_t)(blockIdx.x - o.block0) * lal::f32_copies::PER + threadIdx.x;
+#pragma unroll
+        for(int u = 0; u < lal::f32_copies::PER / 256; u++)
+            if(at + 256 * u < o.len)
+                o.y[at + 256 * u] = (float)o.x[at + 256 * u];
     }
 
     // x = b * dinv (first Jacobi iterate from zero)
@@ -587,24 +578,30 @@ namespace lal
         return dot_partials<T, T>(c, m, y, x, part);
     }
 
-    int smoothed_prolongator(lal_context* c, int m, long nnz, const int* rp, const int* ci,
-                             double* v, const int* prp, const int* pci, const double* pv,
-                             const double* dinv, float* v32)
+    int make_ready(lal_context* c, const ready_level& a, long nnz)
     {
-        if(m == 0 || nnz == 0)
+        if(a.m == 0)
             return LAL_OK;
         const auto go = [&](auto g) {
             constexpr int G = decltype(g)::value;
-            smoothed_prolongator_kernel<G><<<grid_for(m, 256 / G), 256, 0, c->stream>>>(
-                m, rp, ci, v, prp, pci, pv, dinv, v32);
+            ready_kernel<G><<<grid_for(a.m, 256 / G), 256, 0, c->stream>>>(a);
         };
         // about two steps of the group per row
-        if(nnz <= 16L * m)
+        if(nnz <= 16L * a.m)
             go(std::integral_constant<int, 8>{});
-        else if(nnz <= 48L * m)
+        else if(nnz <= 48L * a.m)
             go(std::integral_constant<int, 16>{});
         else
             go(std::integral_constant<int, 64>{});
+        LAL_LAUNCHED();
+        return LAL_OK;
+    }
+
+    int copy_f32(lal_context* c, const f32_copies& a)
+    {
+        if(a.blocks == 0)
+            return LAL_OK;
+        copies_kernel<<<a.blocks, 256, 0, c->stream>>>(a);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -627,22 +624,6 @@ namespace lal
         jacobi_kernel<T, 1><<<nb, SPMV_THREADS, 0, c->stream>>>(
             d ? d->d_blocks : nullptr, nb, m, rp, ci, v, nullptr, diag, b, x, r,
             1); // no fast descriptor: one lane per row
-        LAL_LAUNCHED();
-        return LAL_OK;
-    }
-
-    template <typename T>
-    int diag_inv(lal_context* c, int m, const int* rp, const int* ci, const T* v, T* d, T* dinv,
-                 long nnz)
-    {
-        if(m == 0)
-            return LAL_OK;
-        // a lane per row walks the row alone: rows of 24 or more entries take
-        // a wavefront each
-        if(nnz >= 24L * m)
-            diag_wave_kernel<T><<<(m + 3) / 4, 256, 0, c->stream>>>(m, rp, ci, v, d, dinv);
-        else
-            diag_kernel<T><<<grid_for(m, 256), 256, 0, c->stream>>>(m, rp, ci, v, d, dinv);
         LAL_LAUNCHED();
         return LAL_OK;
     }
@@ -791,8 +772,6 @@ namespace lal
     template int product_dot<T>(lal_context*, const lal_csrmv_info*, int, int, int,          \
                                 const int*, const int*, const T*, const T*, T*, double*,     \
                                 int*);                                                       \
-    template int diag_inv<T>(lal_context*, int, const int*, const int*, const T*, T*, T*,   \
-                             long);                                                          \
     template int coarse_scalar<T>(lal_context*, const T*, const T*, T*);                     \
     template int coarse_gs<T>(lal_context*, int, const int*, const int*, const T*, const T*, \
                               T*);                                                           \
