@@ -147,6 +147,7 @@ struct lal_hierarchy_t
     double* part_r  = nullptr;
     // residual norms reach the host through mapped pinned memory: a value
     // and a sequence number the host polls
+    std::shared_ptr<lal::chunk_pool> pool; // the note's owner, or null: its own memory
     double*   h_note     = nullptr;
     double*   d_note     = nullptr;
     unsigned* h_seq      = nullptr;
@@ -192,7 +193,9 @@ struct lal_hierarchy_t
                 if(ptr)
                     (void)hipFree(ptr);
         }
-        if(h_note)
+        if(pool)
+            pool->give_note(h_note);
+        else if(h_note)
             (void)hipHostFree(h_note);
     }
 

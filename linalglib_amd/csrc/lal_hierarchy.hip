@@ -333,10 +333,16 @@ namespace
         LAL_TRY(h->mem.get(&h->part_r, lal::PCG_BLOCKS));
         LAL_TRY(h->mem.get(&h->d_count, 1));
         LAL_TRY(lal_fill_i32(c, (int*)h->d_count, 1, 0));
-        LAL_HIP(hipHostMalloc((void**)&h->h_note, 64, hipHostMallocMapped | hipHostMallocCoherent));
-        std::memset(h->h_note, 0, 64);
+        if(c->pool->take_note((void**)&h->h_note, (void**)&h->d_note))
+            h->pool = c->pool;
+        else
+        {
+            LAL_HIP(hipHostMalloc((void**)&h->h_note, 64,
+                                  hipHostMallocMapped | hipHostMallocCoherent));
+            std::memset(h->h_note, 0, 64);
+            LAL_HIP(hipHostGetDevicePointer((void**)&h->d_note, h->h_note, 0));
+        }
         h->h_seq = reinterpret_cast<unsigned*>(h->h_note + 1);
-        LAL_HIP(hipHostGetDevicePointer((void**)&h->d_note, h->h_note, 0));
         h->d_seq = reinterpret_cast<unsigned*>(h->d_note + 1);
         if(h->opts.build_f32)
         {
@@ -365,6 +371,7 @@ namespace
         A0.n = n;
         A0.nnz = nnz;
         lal::arena tmp; // a level's temporary arrays
+        tmp.use(c->pool);
         tmp.reserve((size_t)nnz * 30 + (size_t)m * 60);
         LAL_TRY(h->mem.get(&A0.rp, m + 1));
         LAL_TRY(h->mem.get(&A0.ci, nnz));
@@ -1079,6 +1086,7 @@ namespace
         // the first chunk holds most of it (a hipMalloc and hipFree of
         // hundreds of megabytes take 0.3 ms together), and the arena grows by
         // half its size.
+        h->mem.use(c->pool);
         h->mem.reserve((size_t)nnz * ((o.exact ? 40 : 80) + (o.build_f32 ? 40 : 0)) +
                        (size_t)m * (o.build_f32 ? 200 : 100));
         int s = lal::analyse(c, {{descr(h->L[0].A, m, nnz, n, o.exact), rp, ci, m, nnz,

@@ -16,10 +16,121 @@ namespace lal
         g_last_error = msg;
     }
 
+    chunk_pool::~chunk_pool()
+    {
+        clear();
+        if(notes_)
+            (void)hipHostFree(notes_);
+    }
+
+    bool chunk_pool::take_note(void** host, void** dev)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if(notes_ == nullptr)
+        {
+            void *h = nullptr, *d = nullptr;
+            if(hipHostMalloc(&h, 64 * NOTES, hipHostMallocMapped | hipHostMallocCoherent) !=
+               hipSuccess)
+            {
+                (void)hipGetLastError();
+                return false;
+            }
+            if(hipHostGetDevicePointer(&d, h, 0) != hipSuccess)
+            {
+                (void)hipGetLastError();
+                (void)hipHostFree(h);
+                return false;
+            }
+            notes_     = static_cast<char*>(h);
+            notes_dev_ = static_cast<char*>(d);
+        }
+        if(~noted_ == 0)
+            return false;
+        const int k = __builtin_ctzll(~noted_);
+        noted_ |= 1ull << k;
+        *host = notes_ + 64 * k;
+        *dev  = notes_dev_ + 64 * k;
+        std::memset(*host, 0, 64);
+        return true;
+    }
+
+    void chunk_pool::give_note(void* host)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        noted_ &= ~(1ull << ((static_cast<char*>(host) - notes_) / 64));
+    }
+
+    chunk_pool::chunk chunk_pool::take(size_t want)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        size_t best = spare_.size();
+        for(size_t k = 0; k < spare_.size(); k++)
+            if(spare_[k].cap >= want && spare_[k].cap / 4 <= want &&
+               (best == spare_.size() || spare_[k].cap < spare_[best].cap))
+                best = k;
+        if(best == spare_.size())
+            return {nullptr, 0};
+        const chunk k = spare_[best];
+        spare_.erase(spare_.begin() + best);
+        held_ -= k.cap;
+        return k;
+    }
+
+    void chunk_pool::give(const chunk& k)
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if(k.cap > limit_)
+        {
+            (void)hipFree(k.p);
+            return;
+        }
+        size_t drop = 0; // the oldest make room
+        for(; held_ + k.cap > limit_; drop++)
+        {
+            held_ -= spare_[drop].cap;
+            (void)hipFree(spare_[drop].p);
+        }
+        spare_.erase(spare_.begin(), spare_.begin() + drop);
+        spare_.push_back(k);
+        held_ += k.cap;
+    }
+
+    void chunk_pool::clear()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        for(const chunk& k : spare_)
+            (void)hipFree(k.p);
+        spare_.clear();
+        held_ = 0;
+    }
+
+    void chunk_pool::close()
+    {
+        clear();
+        std::lock_guard<std::mutex> lock(mu_);
+        limit_ = 0;
+    }
+
+    void chunk_pool::settle()
+    {
+        int now = device_;
+        (void)hipGetDevice(&now);
+        if(now != device_)
+            (void)hipSetDevice(device_);
+        (void)hipDeviceSynchronize();
+        if(now != device_)
+            (void)hipSetDevice(now);
+    }
+
     arena::~arena()
     {
+        if(pool_ && !chunks_.empty())
+            pool_->settle();
         for(chunk& k : chunks_)
-            (void)hipFree(k.p);
+            if(pool_)
+                pool_->give({k.p, k.cap});
+            else
+                (void)hipFree(k.p);
     }
 
     int arena::get_bytes(void** p, size_t bytes)
@@ -42,11 +153,19 @@ namespace lal
         cap        = std::max((cap + 255) & ~(size_t)255, bytes);
         next_      = 0;
         char* q    = nullptr;
-        if(cap > bytes && hipMalloc(&q, cap) != hipSuccess)
+        if(pool_)
+        {
+            const chunk_pool::chunk k = pool_->take(cap);
+            q                         = k.p;
+            cap                       = q ? k.cap : cap;
+        }
+        if(q == nullptr && hipMalloc(&q, cap) != hipSuccess)
         {
             (void)hipGetLastError(); // no room to spare: just this array
             q   = nullptr;
             cap = bytes;
+            if(pool_)
+                pool_->clear();
         }
         if(q == nullptr)
             LAL_HIP(hipMalloc(&q, cap));
@@ -226,6 +345,7 @@ extern "C" int lal_create(lal_handle* handle)
     LAL_HIP(hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned), c->stream));
     LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int) * LAL_FLAGS, c->stream));
     LAL_HIP(hipStreamSynchronize(c->stream));
+    c->pool = std::make_shared<lal::chunk_pool>(c->device, prop.totalGlobalMem / 32);
     *handle = c;
     return LAL_OK;
 }
@@ -236,6 +356,7 @@ extern "C" int lal_destroy(lal_handle c)
         return LAL_OK;
     (void)hipStreamSynchronize(c->stream);
     lal::detach_hierarchies(c);
+    c->pool->close();
     (void)hipFree(c->d_part);
     (void)hipFree(c->d_ticket);
     (void)hipFree(c->d_flag);
