@@ -340,8 +340,26 @@ namespace
         }
     }
 
-    // Rows of C in LDS tables of H slots (a power of two, at least 64): G lanes
-    // per row, L of them per B row.
+    // The bins of one launch: nr rows with tables of H slots (a power of two, at
+    // least 64) from workgroup `first` on.
+    struct group_bins
+    {
+        struct one
+        {
+            const int* rows;
+            int        nr, H, first;
+        };
+        one b[10];
+        int n = 0, blocks = 0, max_h = 0;
+        void add(const int* rows, int nr, int H, int rpb)
+        {
+            b[n++] = {rows, nr, H, blocks};
+            blocks += (nr + rpb - 1) / rpb;
+            max_h = std::max(max_h, H);
+        }
+    };
+
+    // Rows of C in LDS tables: G lanes per row, L of them per B row.
     //
     // Bound by latency: a step (one A entry and its B row) is a chain of
     // dependent loads and LDS round trips, and the coarse levels have few and
@@ -361,8 +379,8 @@ namespace
     // it is for launches of few rows (launch_group).
     template <int G, int L, bool NUMERIC, bool AHEAD>
     __global__ void __launch_bounds__(256)
-        spgemm_group_kernel(int nrows, int H, const int* __restrict__ rows,
-                            const int* __restrict__ arp, const int* __restrict__ aci,
+        spgemm_group_kernel(group_bins bins, const int* __restrict__ arp,
+                            const int* __restrict__ aci,
                             const double* __restrict__ av, const int* __restrict__ brp,
                             const int* __restrict__ bci, const double* __restrict__ bv,
                             const int* __restrict__ crp, int* __restrict__ cout_,
@@ -374,16 +392,20 @@ namespace
         typedef int   int4v __attribute__((ext_vector_type(4)));
         // per row of the workgroup: H values (numeric pass), H keys
         extern __shared__ __attribute__((aligned(16))) unsigned char s_tab[];
+        int bin = 0;
+        while(bin + 1 < bins.n && bins.b[bin + 1].first <= (int)blockIdx.x)
+            bin++;
+        const int H     = bins.b[bin].H;
         const int hmask = H - 1;
         const int rpb   = (int)blockDim.x / G;
         const int grp   = (int)threadIdx.x / G;
         const int gl    = (int)threadIdx.x % G;         // lane in the group
         const int gb    = ((int)threadIdx.x & 63) - gl; // the group's first lane
         const int sl    = gl % L, sg = gl / L;          // lane of the step, step of the batch
-        const int r     = blockIdx.x * rpb + grp;
-        if(r >= nrows)
+        const int r     = ((int)blockIdx.x - bins.b[bin].first) * rpb + grp;
+        if(r >= bins.b[bin].nr)
             return;
-        const int row  = rows[r];
+        const int row  = bins.b[bin].rows[r];
         double*   vals = NUMERIC ? reinterpret_cast<double*>(s_tab) + (size_t)grp * H : nullptr;
         int*      keys = reinterpret_cast<int*>(s_tab + (NUMERIC ? sizeof(double) * rpb * H : 0)) +
                     (size_t)grp * H;
@@ -1086,34 +1108,48 @@ namespace
         return g;
     }
 
-    // Rows of C with H-slot tables: l lanes take a B row (its mean length),
-    // g lanes the A row (its mean length).  Below 262,144 such lanes (half of
+    // Rows of C in their tables: l lanes take a B row (its mean length), g lanes
+    // the A row (its mean length).  Below 262,144 such lanes (half of
     // what the chip holds) the rows' own chains are the time: they take a
     // wavefront each and load a batch ahead.  121^3 diffusion, numeric pass:
     // level 3's R (A P), 4,400 rows, takes 502 us with the batch ahead and 648
     // without (960 with one step at a time); level 0's, 300,000 rows, 606 with
     // and 484 without (790 with one step at a time).
-    template <bool NUMERIC>
-    void launch_group(lal_context* c, int nr, int H, int g, int l, const int* rows,
-                      const int* arp, const int* aci, const double* av, const int* brp,
-                      const int* bci, const double* bv, const int* crp, int* cout_, double* cval)
+    inline bool few_rows(int nr, int g)
     {
-        const bool few = (long)nr * g < 256L * 1024;
+        return (long)nr * g < 256L * 1024;
+    }
+    inline size_t table_bytes(int H, bool numeric)
+    {
+        return (size_t)H * (numeric ? 12 : 4);
+    }
+
+    // (one bin, or several of few rows)
+    template <bool NUMERIC>
+    void launch_group(lal_context* c, const int* const* rows, const int* nr, const int* H, int n,
+                      int g, int l, const int* arp, const int* aci, const double* av,
+                      const int* brp, const int* bci, const double* bv, const int* crp,
+                      int* cout_, double* cval)
+    {
+        const bool few = n > 1 || few_rows(nr[0], g);
         if(few)
             g = 64;
         g = std::max(g, l);
-        // up to 256 lanes and 48 KB of tables per workgroup
-        const size_t row_bytes = (size_t)H * (NUMERIC ? 12 : 4);
-        int          nt        = 256;
-        while(nt > 64 && row_bytes * (nt / g) > 48 * 1024)
+        // up to 256 lanes and 48 KB of tables per workgroup; a row for each
+        // where several bins share the launch
+        int nt = n > 1 ? 64 : 256;
+        while(nt > 64 && table_bytes(H[0], NUMERIC) * (nt / g) > 48 * 1024)
             nt >>= 1;
-        const int    rpb = nt / g;
-        const size_t lds = row_bytes * rpb;
-        const int    nb  = (nr + rpb - 1) / rpb;
+        const int  rpb = nt / g;
+        group_bins bins;
+        for(int k = 0; k < n; k++)
+            bins.add(rows[k], nr[k], H[k], rpb);
+        const size_t lds = table_bytes(bins.max_h, NUMERIC) * rpb;
+        const int    nb  = bins.blocks;
 #define LAL_SPGEMM_GROUP(GG, LL, AHEAD)                                                      \
     case (AHEAD ? 65536 : 0) + GG * 128 + LL:                                                \
         spgemm_group_kernel<GG, LL, NUMERIC, AHEAD><<<nb, nt, lds, c->stream>>>(             \
-            nr, H, rows, arp, aci, av, brp, bci, bv, crp, cout_, cval, c->d_flag);           \
+            bins, arp, aci, av, brp, bci, bv, crp, cout_, cval, c->d_flag);                  \
         break;
         switch((few ? 65536 : 0) + g * 128 + l)
         {
@@ -1140,19 +1176,38 @@ namespace
                  const double* av, const int* brp, const int* bci, const double* bv,
                  const int* crp, int* cout_, double* cval)
     {
-        for(int b = 0; b < kBins; b++)
+        // Bins of few rows share a launch, longest rows first: one after the
+        // other, each is as long as its longest row and leaves most of the chip
+        // idle (level 4 of a 121^3 diffusion hierarchy, 464 rows in four bins:
+        // 450 us apart, 175 together).  Every workgroup then has room for the
+        // largest table, so a launch takes rows up to four times what the chip
+        // holds at once (once: 10.65 ms for the whole build, four times: 10.51).
+        const int* rows[kBins];
+        int        nrs[kBins], hs[kBins], n = 0;
+        long       joined = 0;
+        const auto flush  = [&]() -> int {
+            if(n == 0)
+                return LAL_OK;
+            launch_group<NUMERIC>(c, rows, nrs, hs, n, P.g, P.l, arp, aci, av, brp, bci, bv, crp,
+                                  cout_, cval);
+            n      = 0;
+            joined = 0;
+            LAL_LAUNCHED();
+            return LAL_OK;
+        };
+        for(int b = kBins - 1; b >= 0; b--)
         {
-            int n0 = P.bin_start[b], nr = P.bin_start[b + 1] - n0;
+            const int n0 = P.bin_start[b], nr = P.bin_start[b + 1] - n0, H = 64 << b;
             if(nr == 0)
                 continue;
-            const int* rows = P.d_rows + n0;
-            const int H = 64 << b;
 #define LAL_SPGEMM_COUNT(HH)                                                                 \
-    spgemm_count_kernel<HH><<<nr, 256, 0, c->stream>>>(rows, arp, aci, brp, bci, cout_, c->d_flag)
+    spgemm_count_kernel<HH><<<nr, 256, 0, c->stream>>>(P.d_rows + n0, arp, aci, brp, bci,     \
+                                                       cout_, c->d_flag)
             // the symbolic pass's tables of 2048 slots and more (alone beyond
             // 4096), and smaller ones of so few rows that the chip holds a
             // workgroup for each: a workgroup per row
             if(!NUMERIC && (H >= 2048 || (H >= 512 && nr <= 2048)))
+            {
                 switch(b)
                 {
                 case 3: LAL_SPGEMM_COUNT(512); break;
@@ -1163,12 +1218,24 @@ namespace
                 case 8: LAL_SPGEMM_COUNT(16384); break;
                 default: LAL_SPGEMM_COUNT(32768); break;
                 }
-            else
-                launch_group<NUMERIC>(c, nr, H, P.g, P.l, rows, arp, aci, av, brp, bci, bv, crp,
-                                      cout_, cval);
+                LAL_LAUNCHED();
+                continue;
+            }
 #undef LAL_SPGEMM_COUNT
-            LAL_LAUNCHED();
+            const int  largest = n > 0 ? hs[0] : H;
+            const long held =
+                4L * c->num_cu * (long)(160 * 1024 / table_bytes(largest, NUMERIC));
+            if(n > 0 && (!few_rows(nr, P.g) || joined + nr > held))
+                LAL_TRY(flush());
+            rows[n] = P.d_rows + n0;
+            nrs[n]  = nr;
+            hs[n]   = H;
+            n++;
+            joined += nr;
+            if(!few_rows(nr, P.g))
+                LAL_TRY(flush());
         }
+        LAL_TRY(flush());
         if(P.n_global)
         {
             spgemm_global_kernel<NUMERIC><<<P.n_global, 64, 0, c->stream>>>(
