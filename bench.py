@@ -81,7 +81,11 @@ def solve_bytes(levels, iters, vbytes):
     one V-cycle, two dot products, one inf-norm and three axpy-class updates
     (vectors of vbytes each); levels = [(m, nnz_A, nnz_P, cA, cP, cR)] finest
     first (cX: bytes per column index the kernels read for A, P and R =
-    P^T), the last entry being the coarsest operator."""
+    P^T), the last entry being the coarsest operator.  These are the bytes of the
+    cycle as the reference states it (residual, restriction, prolongation, a
+    post-sweep with A), which keeps the rate comparable; the fast path replaces
+    the last two by one product with Q = P - D^-1 A P, the levels of up to 1024
+    rows by one dense product, and reads no vector again for the inner products."""
     v = vbytes
     m0, nnz0, _, c0, _, _ = levels[0]
     prec = 0
