@@ -142,6 +142,8 @@ struct lal_hierarchy_t
     float*  d32   = nullptr;
     double* s     = nullptr; // LAL_SOLVER_SLOTS scalars
     // reduction partials: <q, p>, <z, r> (PCG_PARTS each), max|r| (PCG_BLOCKS)
+    double* p2      = nullptr; // small problems: the direction's other buffer
+    float*  p2_32   = nullptr;
     double* part_pq = nullptr;
     double* part_g  = nullptr;
     double* part_r  = nullptr;

@@ -33,6 +33,8 @@
 //   ADD       y = b + A x
 //   SPMV_DOT  y = A x, ADD_DOT  y = b + A x, and one partial of <w, y> per row
 //             block (PCG's inner products without a pass of their own)
+//   STEP_DOT  p' = x + beta p, y = A p' and <p', y>'s partials: PCG's next
+//             direction formed by the product that needs it
 // dinv holds 1/a_ii, so no division is left in the inner loops.
 #pragma once
 
@@ -51,7 +53,8 @@ namespace lal
         RV_SMOOTHED = 5,
         RV_ADD      = 6,
         RV_SPMV_DOT = 7,
-        RV_ADD_DOT  = 8
+        RV_ADD_DOT  = 8,
+        RV_STEP_DOT = 9
     };
 
     // Partials of one reduction at most: a product with more row blocks leaves
@@ -69,6 +72,12 @@ namespace lal
         double*     part = nullptr; // *_DOT: one partial of <w, y> per row block
         const void* w    = nullptr; // m entries, FP64 with `wide`, else of the product's type
         bool        wide = false;
+        // STEP_DOT: beta = (sum of the gamma_count partials at gamma_part) / *gamma_old,
+        // whose numerator also goes to *gamma_new
+        const double* gamma_part  = nullptr;
+        int           gamma_count = 0;
+        const double* gamma_old   = nullptr;
+        double*       gamma_new   = nullptr;
         // SMOOTHED: a last workgroup finishes the reduction before it
         post_args post{};
     };

@@ -67,10 +67,12 @@ namespace
 
     template <typename T, int MODE>
     __device__ __forceinline__ T gather(const T* __restrict__ x, const T* __restrict__ d,
-                                        const T* __restrict__ b, int c)
+                                        const T* __restrict__ b, int c, T beta = 0)
     {
         if(MODE == lal::RV_JACOBI0)
             return b[c] * d[c];
+        if(MODE == lal::RV_STEP_DOT) // (as update_p_kernel)
+            return beta == (T)0 ? x[c] : x[c] + beta * d[c];
         return x[c];
     }
 
@@ -234,7 +236,7 @@ namespace
     __device__ __forceinline__ T staged_row_sum(const int* s_c, const T* s_v, int j, int e, int g,
                                                 const T* __restrict__ x,
                                                 const T* __restrict__ d,
-                                                const T* __restrict__ b)
+                                                const T* __restrict__ b, T beta)
     {
         T acc = 0;
         if(j >= e)
@@ -254,7 +256,7 @@ namespace
             }
 #pragma unroll
             for(int u = 0; u < UR; u++)
-                xx[u] = gather<T, MODE>(x, d, b, cc[u]);
+                xx[u] = gather<T, MODE>(x, d, b, cc[u], beta);
 #pragma unroll
             for(int u = 0; u < UR; u++)
             {
@@ -309,6 +311,13 @@ namespace
             // (the grid has this workgroup only with ex.post)
             lal::post_block<1>(ex.post);
             return;
+        }
+        if(MODE == lal::RV_STEP_DOT)
+        {
+            const double g_new = lal::total_of<0>(ex.gamma_part, ex.gamma_count);
+            if(blockIdx.x == 0 && threadIdx.x == 0)
+                *ex.gamma_new = g_new;
+            beta = (T)(g_new / *ex.gamma_old);
         }
         // the block's row starts, then win entries of columns, then win
         // values (win: a multiple of 4)
@@ -399,13 +408,26 @@ namespace
             {
                 const int a = max(rs, ws) - ws + lig;
                 const int e = min(re, we) - ws;
-                acc += g == 1 ? staged_row_sum<T, MODE, 8>(s_c, s_v, a, e, 1, x, d, b)
-                              : staged_row_sum<T, MODE, 4>(s_c, s_v, a, e, g, x, d, b);
+                acc += g == 1 ? staged_row_sum<T, MODE, 8>(s_c, s_v, a, e, 1, x, d, b, beta)
+                              : staged_row_sum<T, MODE, 4>(s_c, s_v, a, e, g, x, d, b, beta);
             }
             __syncthreads();
         }
         if(g > 1)
             acc = lal::group_sum(acc, g);
+        if(MODE == lal::RV_STEP_DOT)
+        {
+            const bool head = active && lig == 0;
+            row_operands<T> o;
+            if(head)
+            {
+                const T p = gather<T, MODE>(x, d, b, row, beta);
+                r[row]    = p;
+                o.w       = (double)p;
+            }
+            dot_epilogue<T, MODE>(head, row, acc, o, y, ex.part + tile);
+            return;
+        }
         if(MODE == lal::RV_SPMV_DOT)
         {
             dot_epilogue<T, MODE>(active && lig == 0, row, acc, ops, y, ex.part + tile);
@@ -810,6 +832,10 @@ namespace
     {
         if(mode == lal::RV_ADD_DOT)
             launch_list<T, lal::RV_ADD_DOT>(c, a, a.nb);
+        else if(mode == lal::RV_STEP_DOT && a.c16 && a.cbase)
+            launch_quad<T, lal::RV_STEP_DOT, true>(c, a, a.nb);
+        else if(mode == lal::RV_STEP_DOT)
+            launch_quad<T, lal::RV_STEP_DOT, false>(c, a, a.nb);
         else if(a.c16 && a.cbase)
             launch_quad<T, lal::RV_SPMV_DOT, true>(c, a, a.nb);
         else
@@ -840,7 +866,9 @@ namespace lal
         case RV_ADD: return launch<T, RV_ADD>(c, a);
         case RV_SPMV_DOT:
         case RV_ADD_DOT:
-            LAL_REQUIRE(rowvec_can_dot(mode, a) && a.ex.part != nullptr && a.ex.w != nullptr);
+        case RV_STEP_DOT:
+            LAL_REQUIRE(rowvec_can_dot(mode, a) && a.ex.part != nullptr &&
+                        (mode == RV_STEP_DOT ? a.ex.gamma_part != nullptr : a.ex.w != nullptr));
             return launch_dot<T>(c, mode, a);
         default: return launch<T, RV_JACOBI0>(c, a);
         }

@@ -69,6 +69,14 @@ namespace lal
                     const T* v, const T* e, const T* y, T* out, const row_extra& ex = {});
     template <typename T>
     bool can_add_dot(const lal_csrmv_info* d, int m, const int* rp, const int* ci, const T* v);
+    // p' = z + beta p, y = A p' and *count partials of <y, p'>, beta = gamma_new /
+    // gamma_old with gamma_new from its partials (as update_p, then product_dot);
+    // *done false: not a matrix the one kernel takes, nothing was launched.
+    template <typename T>
+    int step_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, const int* rp,
+                 const int* ci, const T* v, const T* z, const T* p, T* p_new, T* y,
+                 const double* part_g, int n_g, const double* gamma_old, double* gamma_new,
+                 double* part, int* count, bool* done);
     // y = A x and *count partials of <y, x> in part (PCG_PARTS at most)
     template <typename T>
     int product_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, int nnz, const int* rp,

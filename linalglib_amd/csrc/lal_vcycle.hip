@@ -556,6 +556,31 @@ namespace lal
     }
 
     template <typename T>
+    int step_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, const int* rp,
+                 const int* ci, const T* v, const T* z, const T* p, T* p_new, T* y,
+                 const double* part_g, int n_g, const double* gamma_old, double* gamma_new,
+                 double* part, int* count, bool* done)
+    {
+        *done = false;
+        if(!d || d->exact || m != n)
+            return LAL_OK;
+        rv_args a{m, d->nnz, d->by_nnz, d->d_blocks, d->nblocks, rp, ci, v, z, p, nullptr, y,
+                  p_new, 1.0, 0.0, d->win};
+        lal::use_c16(a, d);
+        a.keep           = d->keep;
+        a.ex.part        = part;
+        a.ex.gamma_part  = part_g;
+        a.ex.gamma_count = n_g;
+        a.ex.gamma_old   = gamma_old;
+        a.ex.gamma_new   = gamma_new;
+        if(!rowvec_can_dot(RV_STEP_DOT, a))
+            return LAL_OK;
+        *done  = true;
+        *count = d->nblocks;
+        return rowvec_launch<T>(c, RV_STEP_DOT, a);
+    }
+
+    template <typename T>
     int product_dot(lal_context* c, const lal_csrmv_info* d, int m, int n, int nnz, const int* rp,
                     const int* ci, const T* v, const T* x, T* y, double* part, int* count)
     {
@@ -769,6 +794,10 @@ namespace lal
                                 const row_extra&);                                           \
     template bool can_add_dot<T>(const lal_csrmv_info*, int, const int*, const int*,         \
                                  const T*);                                                  \
+    template int step_dot<T>(lal_context*, const lal_csrmv_info*, int, int, const int*,     \
+                             const int*, const T*, const T*, const T*, T*, T*,              \
+                             const double*, int, const double*, double*, double*, int*,      \
+                             bool*);                                                         \
     template int product_dot<T>(lal_context*, const lal_csrmv_info*, int, int, int,          \
                                 const int*, const int*, const T*, const T*, T*, double*,     \
                                 int*);                                                       \
