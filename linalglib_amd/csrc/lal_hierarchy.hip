@@ -626,12 +626,13 @@ namespace
     // precond() for the solvers' own vectors (r, z fixed per hierarchy and
     // precision): with at least one pre-sweep the V-cycle is kernels and
     // device copies only.  On a small finest level (at most GRAPH_MAX_ROWS
-    // rows), where every kernel is short and the launches bound the cycle, it
-    // is captured as a HIP graph on its second use and replayed after
-    // (lal::captured): 2D Poisson 128^2 solves in 2.83 ms against 2.99.  On
-    // larger ones the graph's replay costs more than it saves (3D Poisson
-    // 128^3: FP64 15.37 against 15.13 ms), so they launch eagerly.
-    constexpr int GRAPH_MAX_ROWS = 262144;
+    // rows), where every kernel is short and the host's launches bound the cycle,
+    // it is captured as a HIP graph on its second use and replayed after
+    // (lal::captured): PCG on 2D Poisson 128^2, 16,384 rows, 1.37 ms against 1.51
+    // to 1.56 launched eagerly by a busy host.  On larger ones the graph's replay
+    // costs more than it saves (gradient on 64^3, 262,144 rows: 12.2 against
+    // 11.5 ms; 101^3: 8.70 against 8.53), so they launch eagerly.
+    constexpr int GRAPH_MAX_ROWS = 65536;
 
     template <typename T>
     int precond_graphed(lal_hierarchy_t* h, const T* r, T* z, int n1, int n2,

@@ -16,8 +16,9 @@ pytestmark = pytest.mark.gpu
 SIZES = {
     "one_block": lambda: pb.poisson2d(9, 7),
     "blocks_512": lambda: pb.poisson2d(360, 362),   # about 510 blocks of 256 rows
-    "graph_limit": lambda: pb.poisson2d(512, 512),  # replayed as a graph
-    "beyond_graph": lambda: pb.poisson2d(513, 512),
+    "graph_limit": lambda: pb.poisson2d(256, 256),  # replayed as a graph
+    "beyond_graph": lambda: pb.poisson2d(257, 256),
+    "rows_262144": lambda: pb.poisson2d(512, 512),
     "beyond_parts": lambda: pb.poisson3d(102),      # 4146 blocks of 256 rows
 }
 
