@@ -272,7 +272,9 @@ int lal_saamg_setup(lal_handle h, int m, int n, int nnz, const int* row_ptr,
                     const int* col_ind, const double* val, const lal_saamg_options* opts,
                     lal_hierarchy* out);
 /* May also be called after lal_destroy of the context it was built on (the
- * hierarchy is then only freed); no other call takes such a hierarchy. */
+ * hierarchy is then only freed); no other call takes such a hierarchy.  Waits
+ * for the device's work; the context keeps up to 1/32 of the device's memory of
+ * destroyed hierarchies for its next ones, until lal_destroy. */
 int lal_hierarchy_destroy(lal_hierarchy hier);
 int lal_hierarchy_levels(lal_hierarchy hier, int* total_levels);
 /* kind: 0 = A, 1 = P, 2 = R.  Device pointers stay owned by the hierarchy. */
