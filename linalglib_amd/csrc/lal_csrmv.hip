@@ -489,13 +489,14 @@ namespace
             if(carry & 1)
                 s_list[carry] = (unsigned short)span; // (its low 16 bits)
             // (words from 2048 on start the offsets of 65536 and more)
-            const int split    = words > 2048 ? s_place[2048] : carry;
+            const int near     = words > 2048 ? s_place[2048] : carry;
+            const int split    = lal::list_split(carry, near);
             o.lmeta[2 * b]     = carry | split << 12 | lal::spmv_group_log(mt.y - mt.x) << 24;
             o.lmeta[2 * b + 1] = base;
             // (one address for all blocks: few of them raise it)
             if(carry > *(volatile int*)(out + RB_LMAX))
                 atomicMax(out + RB_LMAX, carry);
-            if(split < carry && *(volatile int*)(out + RB_FAR) == 0)
+            if(near < carry && *(volatile int*)(out + RB_FAR) == 0)
                 atomicOr(out + RB_FAR, 1);
         }
         __syncthreads();

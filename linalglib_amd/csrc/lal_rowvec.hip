@@ -695,8 +695,8 @@ namespace
                 if(FAR)
                 {
                     const unsigned i = 2u * min(tid + SPMV_THREADS * u, np - 1);
-                    o0 += i >= split ? 65536u : 0u;
-                    o1 += i + 1 >= split ? 65536u : 0u;
+                    o0               = lal::list_offset(o0, i, split);
+                    o1               = lal::list_offset(o1, i + 1, split);
                 }
                 xv[u][0] = load_at<T>(xb, (unsigned)sizeof(T) * o0);
                 xv[u][1] = load_at<T>(xb, (unsigned)sizeof(T) * o1);

@@ -10,6 +10,7 @@
 // group of G lanes and combine the partial sums with a fixed butterfly.
 #pragma once
 
+#include "lal_columns.h"
 #include "lal_internal.h"
 
 #include <vector>
@@ -37,10 +38,10 @@ struct lal_csrmv_info
     // Gathered x through LDS (operators a hierarchy asks it for): every block's
     // distinct columns, ascending, as 16-bit offsets from its smallest one from
     // d_list[lal::list_start()] on (an odd list's last one twice); per nonzero four times its
-    // column's place in that list; per block {list length | first entry whose
-    // offset is 65536 more than stored << 12 | log2 of the lanes per row << 24,
-    // smallest column}.  list_max: the longest list; 0 when not built (a block
-    // spans more than 131,072 columns or holds more than 2044 nonzeros).
+    // column's place in that list; per block {list length | lal::list_split() << 12 |
+    // log2 of the lanes per row << 24, smallest column}.  list_max: the longest
+    // list; 0 when not built (a block spans more than 131,072 columns or holds
+    // more than 2044 nonzeros).
     unsigned short* d_lpos   = nullptr;
     unsigned short* d_list   = nullptr;
     int*            d_lmeta  = nullptr;
