@@ -658,7 +658,10 @@ namespace
         const int      lg    = lm.x >> 24;                    // log2 of the lanes per row
         const int      ws  = base & ~3;
         const unsigned nq  = (unsigned)(end - ws + 3) >> 2;
-        const T*              xb = x + lm.y;
+        // (JACOBI0's x is b d, as in gather())
+        constexpr bool        ZERO = MODE == lal::RV_JACOBI0;
+        const T*              xb = (ZERO ? b : x) + lm.y;
+        const T*              db = ZERO ? d + lm.y : nullptr;
         const T*              vb = val + ws;
         const unsigned short* pb = lpos + ws;
         const unsigned short* lb = list + lal::list_start(base, tile);
@@ -685,6 +688,10 @@ namespace
         const bool head = on && (tid & ((1u << lg) - 1u)) == 0;
         const int  rpv  = rp[r0 + min((int)tid, nrows)];
         const row_operands<T> ops = load_operands<T, MODE>(head, r0 + lrow, x, d, b, beta, y, ex);
+        const auto x_at = [&](unsigned at) {
+            const unsigned byte = (unsigned)sizeof(T) * at;
+            return ZERO ? load_at<T>(xb, byte) * load_at<T>(db, byte) : load_at<T>(xb, byte);
+        };
         // (a list of odd length repeats its last column once more)
         T xv[LIST_U][2];
 #pragma unroll
@@ -698,8 +705,8 @@ namespace
                     o0               = lal::list_offset(o0, i, split);
                     o1               = lal::list_offset(o1, i + 1, split);
                 }
-                xv[u][0] = load_at<T>(xb, (unsigned)sizeof(T) * o0);
-                xv[u][1] = load_at<T>(xb, (unsigned)sizeof(T) * o1);
+                xv[u][0] = x_at(o0);
+                xv[u][1] = x_at(o1);
             }
 #pragma unroll
         for(int u = 0; u < LIST_U; u++)
@@ -856,6 +863,8 @@ namespace lal
     template <typename T>
     int rowvec_launch(lal_context* c, int mode, const rv_args& a)
     {
+        // what the mode's kernels gather
+        LAL_REQUIRE(a.nnz == 0 || (mode == RV_JACOBI0 ? a.b && a.d : a.x != nullptr));
         switch(mode)
         {
         case RV_SPMV: return launch<T, RV_SPMV>(c, a);
