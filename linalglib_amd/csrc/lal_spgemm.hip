@@ -1136,10 +1136,15 @@ namespace
             g = 64;
         g = std::max(g, l);
         // up to 256 lanes and 48 KB of tables per workgroup; a row for each
-        // where several bins share the launch
-        int nt = n > 1 ? 64 : 256;
-        while(nt > 64 && table_bytes(H[0], NUMERIC) * (nt / g) > 48 * 1024)
+        // where several bins share the launch.  Rows much longer than the mean
+        // that chose g (a matrix of few long rows among many short ones) get as
+        // many lanes as leave room for their tables.
+        int        nt  = n > 1 ? 64 : 256;
+        const auto big = [&] { return table_bytes(H[0], NUMERIC) * (nt / g) > 48 * 1024; };
+        while(nt > 64 && big())
             nt >>= 1;
+        while(g < nt && big())
+            g <<= 1;
         const int  rpb = nt / g;
         group_bins bins;
         for(int k = 0; k < n; k++)
