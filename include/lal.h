@@ -273,8 +273,11 @@ int lal_saamg_setup(lal_handle h, int m, int n, int nnz, const int* row_ptr,
                     lal_hierarchy* out);
 /* May also be called after lal_destroy of the context it was built on (the
  * hierarchy is then only freed); no other call takes such a hierarchy.  Waits
- * for the device's work; the context keeps up to 1/32 of the device's memory of
- * destroyed hierarchies for its next ones, until lal_destroy. */
+ * for the device's work.  Contexts keep memory of destroyed hierarchies for their
+ * next ones: at most 1/32 of the device's in all contexts together, until
+ * lal_destroy or until an allocation of this library on the device fails; nothing
+ * large while less than an eighth of the device's memory is free.  Other allocators
+ * in the process get it back with lal_destroy only. */
 int lal_hierarchy_destroy(lal_hierarchy hier);
 int lal_hierarchy_levels(lal_hierarchy hier, int* total_levels);
 /* kind: 0 = A, 1 = P, 2 = R.  Device pointers stay owned by the hierarchy. */

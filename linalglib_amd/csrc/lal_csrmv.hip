@@ -729,8 +729,7 @@ int lal_csrmv_info::arrays(lal::arena* mem, int nb)
     owned             = mem == nullptr;
     if(mem)
         return mem->get(&d_blocks, ints);
-    LAL_HIP(hipMalloc(&d_blocks, sizeof(int) * ints));
-    return LAL_OK;
+    return lal::device_malloc(reinterpret_cast<void**>(&d_blocks), sizeof(int) * ints);
 }
 
 extern "C" int lal_csrmv_analysis(lal_handle c, int m, int n, int nnz, const int* row_ptr,

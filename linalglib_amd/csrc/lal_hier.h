@@ -107,8 +107,7 @@ namespace lal
         *p = nullptr;
         if(bytes == 0)
             return LAL_OK;
-        LAL_HIP(hipMalloc(p, bytes));
-        return LAL_OK;
+        return device_malloc(p, bytes);
     }
 
     template <typename T>

@@ -25,8 +25,11 @@ namespace lal
     // next ones.  The driver takes freed memory back at a bounded rate: programs
     // that build hierarchies one after the other (121^3: 2.9 GB each) run dry
     // after about a second and then wait for it, in steps of 10 ms (500 builds
-    // took 78 ms each on average, of which 12.5 are work; now 11.2).  At most 1/32 of the
-    // device's memory; given back when an allocation fails and with the context.
+    // took 78 ms each on average, of which 12.5 are work; now 11.2).  At most 1/32
+    // of the device's memory in all contexts' pools together; given back with the
+    // context, and by every pool of the device when an allocation of this library
+    // fails (device_malloc); nothing large is taken in while less than an eighth
+    // of the device's memory is free.
     struct chunk_pool
     {
         struct chunk
@@ -34,7 +37,7 @@ namespace lal
             char*  p;
             size_t cap;
         };
-        chunk_pool(int device, size_t limit) : device_(device), limit_(limit) {}
+        chunk_pool(int device, size_t total);
         ~chunk_pool();
         chunk_pool(const chunk_pool&) = delete;
         chunk_pool& operator=(const chunk_pool&) = delete;
@@ -42,24 +45,36 @@ namespace lal
         chunk take(size_t want);
         // after every kernel that uses it has ended (any thread)
         void give(const chunk& k);
-        void clear();
+        // true: something went back to the driver
+        bool clear();
         void close(); // the context is gone: what is given from now on is freed
-        // waits for the device's work, as a hipFree would
-        void settle();
+        // Waits for the device's work, as a hipFree would; false: the `bytes` to
+        // be given are better freed, the device is short of memory.
+        bool settle(size_t bytes);
         // 64 bytes of zeroed mapped host memory (a solver's note); false: none left
         bool take_note(void** host, void** dev);
         void give_note(void* host);
+        // clear() for every pool of the device
+        static bool clear_all(int device);
 
     private:
         static constexpr int NOTES = 64;
+        // arenas of less are given without a look at the device's free memory
+        // (5 us; the build of a 25^3 hierarchy takes 1.7 ms)
+        static constexpr size_t LARGE = (size_t)64 << 20;
         std::mutex           mu_;
         std::vector<chunk>   spare_; // oldest first
         size_t               held_ = 0;
         int                  device_;
-        size_t               limit_;
+        size_t               limit_; // of all the device's pools together
         char *               notes_ = nullptr, *notes_dev_ = nullptr;
         unsigned long long   noted_ = 0; // a bit per note in use
     };
+
+    // hipMalloc, and hipMallocAsync on a stream; when the device is out of
+    // memory, its pools are emptied and the allocation is tried once more.
+    int device_malloc(void** p, size_t bytes);
+    int device_malloc(void** p, size_t bytes, hipStream_t stream);
 
     // Device memory handed out from a few large allocations and freed with
     // the object, or kept by the pool it uses.  A hierarchy build makes several
@@ -357,8 +372,8 @@ namespace lal
             if(a_)
                 return a_->get(p, n);
             *p = nullptr;
-            LAL_HIP(hipMallocAsync(reinterpret_cast<void**>(p), sizeof(T) * (n > 0 ? n : 1),
-                                   c_->stream));
+            LAL_TRY(device_malloc(reinterpret_cast<void**>(p), sizeof(T) * (n > 0 ? n : 1),
+                                  c_->stream));
             own_.push_back(*p);
             return LAL_OK;
         }

@@ -240,7 +240,8 @@ namespace
         int get(double** p, size_t n)
         {
             *p = nullptr;
-            LAL_HIP(hipMallocAsync((void**)p, sizeof(double) * std::max<size_t>(n, 1), c->stream));
+            LAL_TRY(lal::device_malloc((void**)p, sizeof(double) * std::max<size_t>(n, 1),
+                                       c->stream));
             bufs.push_back(*p);
             return LAL_OK;
         }

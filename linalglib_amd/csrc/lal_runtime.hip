@@ -2,6 +2,7 @@
 #include "lal_internal.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <mutex>
@@ -16,8 +17,36 @@ namespace lal
         g_last_error = msg;
     }
 
+    namespace
+    {
+        // The process's pools, and what those of a device hold together.
+        struct pool_list
+        {
+            std::mutex               mu;
+            std::vector<chunk_pool*> pools;
+            std::atomic<size_t>      held[LAL_MAX_DEVICES] = {};
+        };
+        pool_list& all_pools()
+        {
+            static pool_list* l = new pool_list; // (outlives every context)
+            return *l;
+        }
+    }
+
+    chunk_pool::chunk_pool(int device, size_t total)
+        : device_(device), limit_(device < LAL_MAX_DEVICES ? total / 32 : 0)
+    {
+        std::lock_guard<std::mutex> lock(all_pools().mu);
+        all_pools().pools.push_back(this);
+    }
+
     chunk_pool::~chunk_pool()
     {
+        {
+            std::lock_guard<std::mutex> lock(all_pools().mu);
+            auto&                       v = all_pools().pools;
+            v.erase(std::remove(v.begin(), v.end(), this), v.end());
+        }
         clear();
         if(notes_)
             (void)hipHostFree(notes_);
@@ -73,61 +102,130 @@ namespace lal
         const chunk k = spare_[best];
         spare_.erase(spare_.begin() + best);
         held_ -= k.cap;
+        all_pools().held[device_] -= k.cap;
         return k;
     }
 
     void chunk_pool::give(const chunk& k)
     {
         std::lock_guard<std::mutex> lock(mu_);
-        if(k.cap > limit_)
-        {
-            (void)hipFree(k.p);
-            return;
-        }
-        size_t drop = 0; // the oldest make room
-        for(; held_ + k.cap > limit_; drop++)
-        {
-            held_ -= spare_[drop].cap;
-            (void)hipFree(spare_[drop].p);
-        }
+        size_t                      drop = 0; // the oldest make room
+        const auto                  room = [&] {
+            if(k.cap > limit_)
+                return false;
+            std::atomic<size_t>& held = all_pools().held[device_];
+            for(size_t now = held;;)
+                if(now + k.cap <= limit_)
+                {
+                    if(held.compare_exchange_weak(now, now + k.cap))
+                        return true;
+                }
+                else if(drop == spare_.size())
+                    return false;
+                else
+                {
+                    const chunk& old = spare_[drop++];
+                    (void)hipFree(old.p);
+                    held_ -= old.cap;
+                    held -= old.cap;
+                    now = held;
+                }
+        };
+        const bool kept = room();
         spare_.erase(spare_.begin(), spare_.begin() + drop);
-        spare_.push_back(k);
-        held_ += k.cap;
+        if(kept)
+        {
+            spare_.push_back(k);
+            held_ += k.cap;
+        }
+        else
+            (void)hipFree(k.p);
     }
 
-    void chunk_pool::clear()
+    bool chunk_pool::clear()
     {
         std::lock_guard<std::mutex> lock(mu_);
         for(const chunk& k : spare_)
             (void)hipFree(k.p);
         spare_.clear();
+        const bool any = held_ > 0;
+        if(any)
+            all_pools().held[device_] -= held_;
         held_ = 0;
+        return any;
+    }
+
+    bool chunk_pool::clear_all(int device)
+    {
+        std::lock_guard<std::mutex> lock(all_pools().mu);
+        bool                        any = false;
+        for(chunk_pool* p : all_pools().pools)
+            if(p->device_ == device)
+                any |= p->clear();
+        return any;
     }
 
     void chunk_pool::close()
     {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            limit_ = 0;
+        }
         clear();
-        std::lock_guard<std::mutex> lock(mu_);
-        limit_ = 0;
     }
 
-    void chunk_pool::settle()
+    bool chunk_pool::settle(size_t bytes)
     {
         int now = device_;
         (void)hipGetDevice(&now);
         if(now != device_)
             (void)hipSetDevice(device_);
         (void)hipDeviceSynchronize();
+        size_t free = 0, total = 0;
+        bool   ample = true;
+        if(bytes >= LARGE)
+            ample = hipMemGetInfo(&free, &total) == hipSuccess && free >= total / 8;
         if(now != device_)
             (void)hipSetDevice(now);
+        return ample;
+    }
+
+    namespace
+    {
+        template <typename F>
+        int with_room(F&& alloc, const char* what, int line)
+        {
+            hipError_t e   = alloc();
+            int        dev = 0;
+            if(e == hipErrorOutOfMemory)
+            {
+                (void)hipGetLastError();
+                if(hipGetDevice(&dev) == hipSuccess && chunk_pool::clear_all(dev))
+                    e = alloc();
+            }
+            if(e == hipSuccess)
+                return LAL_OK;
+            (void)hipGetLastError();
+            return hip_status(e, what, __FILE__, line);
+        }
+    }
+
+    int device_malloc(void** p, size_t bytes)
+    {
+        return with_room([&] { return hipMalloc(p, bytes); }, "hipMalloc", __LINE__);
+    }
+
+    int device_malloc(void** p, size_t bytes, hipStream_t stream)
+    {
+        return with_room([&] { return hipMallocAsync(p, bytes, stream); }, "hipMallocAsync",
+                         __LINE__);
     }
 
     arena::~arena()
     {
-        if(pool_ && !chunks_.empty())
-            pool_->settle();
+        const bool keep = pool_ && !chunks_.empty() && pool_->settle(total_);
         for(chunk& k : chunks_)
-            if(pool_)
+            if(keep)
                 pool_->give({k.p, k.cap});
             else
                 (void)hipFree(k.p);
@@ -164,11 +262,9 @@ namespace lal
             (void)hipGetLastError(); // no room to spare: just this array
             q   = nullptr;
             cap = bytes;
-            if(pool_)
-                pool_->clear();
         }
         if(q == nullptr)
-            LAL_HIP(hipMalloc(&q, cap));
+            LAL_TRY(device_malloc(reinterpret_cast<void**>(&q), cap));
         chunks_.push_back({q, cap, bytes});
         total_ += cap;
         *p = q;
@@ -334,9 +430,9 @@ extern "C" int lal_create(lal_handle* handle)
     }
     LAL_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     c->stream = c->side;
-    LAL_HIP(hipMalloc(&c->d_part, sizeof(double) * LAL_RED_BLOCKS * 2));
-    LAL_HIP(hipMalloc(&c->d_ticket, sizeof(unsigned)));
-    LAL_HIP(hipMalloc(&c->d_flag, sizeof(int) * LAL_FLAGS));
+    LAL_TRY(lal::device_malloc((void**)&c->d_part, sizeof(double) * LAL_RED_BLOCKS * 2));
+    LAL_TRY(lal::device_malloc((void**)&c->d_ticket, sizeof(unsigned)));
+    LAL_TRY(lal::device_malloc((void**)&c->d_flag, sizeof(int) * LAL_FLAGS));
     LAL_HIP(hipHostMalloc(&c->h_slots, sizeof(double) * LAL_NUM_SLOTS, hipHostMallocDefault));
     LAL_HIP(hipHostMalloc(&c->h_note, sizeof(int) * (LAL_NOTE_INTS + 1),
                           hipHostMallocMapped | hipHostMallocCoherent));
@@ -345,7 +441,7 @@ extern "C" int lal_create(lal_handle* handle)
     LAL_HIP(hipMemsetAsync(c->d_ticket, 0, sizeof(unsigned), c->stream));
     LAL_HIP(hipMemsetAsync(c->d_flag, 0, sizeof(int) * LAL_FLAGS, c->stream));
     LAL_HIP(hipStreamSynchronize(c->stream));
-    c->pool = std::make_shared<lal::chunk_pool>(c->device, prop.totalGlobalMem / 32);
+    c->pool = std::make_shared<lal::chunk_pool>(c->device, prop.totalGlobalMem);
     *handle = c;
     return LAL_OK;
 }
@@ -395,8 +491,7 @@ extern "C" int lal_alloc(void** ptr, size_t bytes)
     *ptr = nullptr;
     if(bytes == 0)
         return LAL_OK;
-    LAL_HIP(hipMalloc(ptr, bytes));
-    return LAL_OK;
+    return lal::device_malloc(ptr, bytes);
 }
 
 extern "C" int lal_free(void* ptr)
