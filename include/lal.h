@@ -267,7 +267,9 @@ int  lal_uaamg_setup(lal_handle h, int m, int n, int nnz, const int* row_ptr, co
                      const double* val, const lal_saamg_options* opts, lal_hierarchy* hier);
 
 /* Builds the hierarchy on the device from a device-resident CSR matrix. The
- * hierarchy keeps its own copy of A. */
+ * hierarchy keeps its own copy of A.  Where the device's memory does not hold the
+ * arrays that are there for speed alone (about half of it), the hierarchy is built
+ * without them: the same operators, a slower cycle. */
 int lal_saamg_setup(lal_handle h, int m, int n, int nnz, const int* row_ptr,
                     const int* col_ind, const double* val, const lal_saamg_options* opts,
                     lal_hierarchy* out);

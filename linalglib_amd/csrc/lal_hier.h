@@ -156,6 +156,11 @@ struct lal_hierarchy_t
     unsigned  seq        = 0;       // the last note asked for
     unsigned* d_count    = nullptr; // notes written (device)
     bool      has32      = false;
+    // Built without Q, the column lists and the dense cycle operator, which are
+    // there for speed and more than double the hierarchy: 180^3 Poisson takes 146
+    // bytes per nonzero with them and 74 without.  A build that runs out of
+    // memory is done again so.
+    bool      lean       = false;
     // levels cycle_first..levels of the fast path's V-cycle with one pre- and
     // one post-sweep, as one dense operator (FP64)
     int     cycle_first = -1;

@@ -142,7 +142,7 @@ namespace
         while(first > 1 && h->L[first - 1].A.m <= lal::CYCLE_ROWS)
             first--;
         const level_t& last = h->L[h->levels];
-        if(h->opts.exact || h->coarse_kind == 1 || first == h->levels ||
+        if(h->opts.exact || h->lean || h->coarse_kind == 1 || first == h->levels ||
            last.A.m > lal::CYCLE_ROWS)
             return LAL_OK;
         const double* Mc  = h->coarse_kind == 2 ? h->coarse_inv : nullptr;
@@ -237,8 +237,7 @@ namespace
             for(csr_dev* A : {&h->L[l].A, &h->L[l].P, &h->L[l].R, &h->L[l].Q})
                 if(A->d == nullptr && (A == &h->L[l].A || (l < h->levels && A->rp)))
                     req.push_back({descr(*A, A->m, A->nnz, A->n, exact), A->rp, A->ci, A->m,
-                                   A->nnz, exact == 0, -1,
-                                   A == &h->L[l].Q || A == &h->L[l].A || A == &h->L[l].R});
+                                   A->nnz, exact == 0, -1, !h->lean && A != &h->L[l].P});
         LAL_TRY(lal::analyse(c, req, &h->mem, tmp));
         if(!exact)
             choose_kept(h);
@@ -381,9 +380,29 @@ namespace
         A0.m = m;
         A0.n = n;
         A0.nnz = nnz;
-        lal::arena tmp; // a level's temporary arrays
-        tmp.use(c->pool);
-        tmp.reserve((size_t)nnz * 30 + (size_t)m * 60);
+        // a level's temporary arrays; a lean build gives them back as soon as they
+        // are done with, and lets every step free its own
+        std::unique_ptr<lal::arena> tmp;
+        auto fresh = [&]() -> int {
+            if(tmp && !h->lean)
+            {
+                tmp->release(lal::arena::mark_t{});
+                return LAL_OK;
+            }
+            if(tmp)
+                LAL_HIP(hipStreamSynchronize(c->stream));
+            tmp.reset(new lal::arena);
+            if(h->lean)
+                tmp->tight();
+            else
+            {
+                tmp->use(c->pool);
+                tmp->reserve((size_t)nnz * 30 + (size_t)m * 60);
+            }
+            return LAL_OK;
+        };
+        LAL_TRY(fresh());
+        lal::arena* const work = h->lean ? nullptr : tmp.get();
         LAL_TRY(h->mem.get(&A0.rp, m + 1));
         LAL_TRY(h->mem.get(&A0.ci, nnz));
         LAL_TRY(h->mem.get(&A0.v, nnz));
@@ -405,7 +424,7 @@ namespace
             csr_dev& P  = h->L[level].P;
             csr_dev& R  = h->L[level].R;
             csr_dev& Ac = h->L[level + 1].A;
-            tmp.release(lal::arena::mark_t{});
+            LAL_TRY(fresh());
             LAL_TRY(h->mem.get(&P.rp, Af.m + 1));
             int nnzP = 0, nc = 0;
             if(lal::small_fits(Af.m, Af.nnz))
@@ -418,21 +437,21 @@ namespace
                 LAL_TRY(h->mem.get(&R.v, room));
                 LAL_TRY(lal::small_build(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, o.relax,
                                          unsmoothed, P.rp, P.ci, P.v, R.rp, R.ci, R.v, &nnzP, &nc,
-                                         &tmp));
+                                         work));
             }
             else
             {
                 int*     conn = nullptr;
                 int64_t* agg  = nullptr;
-                LAL_TRY(tmp.get(&conn, Af.nnz));
-                LAL_TRY(tmp.get(&agg, Af.m));
-                LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn, &tmp));
-                LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, &tmp));
+                LAL_TRY(tmp->get(&conn, Af.nnz));
+                LAL_TRY(tmp->get(&agg, Af.m));
+                LAL_TRY(lal::sa_strength(c, Af.m, Af.nnz, Af.rp, Af.ci, Af.v, eps, conn, work));
+                LAL_TRY(lal::pmis_aggregate(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg, work));
                 if(unsmoothed)
-                    LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc, &tmp));
+                    LAL_TRY(lal::ua_prolongator_nnz(c, Af.m, agg, P.rp, &nnzP, &nc, work));
                 else
                     LAL_TRY(lal::sa_prolongator_nnz(c, Af.m, Af.nnz, Af.rp, Af.ci, conn, agg,
-                                                    P.rp, &nnzP, &nc, &tmp));
+                                                    P.rp, &nnzP, &nc, work));
                 if(nc > 0)
                 {
                     LAL_TRY(h->mem.get(&P.ci, nnzP));
@@ -447,7 +466,7 @@ namespace
                     LAL_TRY(h->mem.get(&R.ci, nnzP));
                     LAL_TRY(h->mem.get(&R.v, nnzP));
                     LAL_TRY(lal::transpose_f64(c, Af.m, nc, nnzP, P.rp, P.ci, P.v, R.rp, R.ci, R.v,
-                                               &tmp));
+                                               work));
                 }
             }
             if(nc == 0)
@@ -462,25 +481,29 @@ namespace
             R.m   = nc;
             R.n   = Af.m;
             R.nnz = nnzP;
+            if(h->lean)
+                LAL_TRY(fresh());
             // AP = A P (the fast path makes Q of it)
             csr_dev  ap_tmp;
-            csr_dev& AP = o.exact ? ap_tmp : h->L[level].Q;
+            csr_dev& AP = o.exact || h->lean ? ap_tmp : h->L[level].Q;
             AP.m        = Af.m;
             AP.n        = nc;
             LAL_TRY(lal::product(c, Af.m, Af.n, nc, Af.nnz, Af.rp, Af.ci, Af.v, P.nnz, P.rp,
                                  P.ci, P.v, &AP.rp, &AP.ci, &AP.v, &AP.nnz,
-                                 o.exact ? &tmp : &h->mem, &tmp));
+                                 &AP == &ap_tmp ? tmp.get() : &h->mem, work));
             // A_c = R (A P)
             Ac.m = nc;
             Ac.n = nc;
             LAL_TRY(lal::product(c, nc, Af.m, nc, R.nnz, R.rp, R.ci, R.v, AP.nnz, AP.rp, AP.ci,
-                                 AP.v, &Ac.rp, &Ac.ci, &Ac.v, &Ac.nnz, &h->mem, &tmp));
+                                 AP.v, &Ac.rp, &Ac.ci, &Ac.v, &Ac.nnz, &h->mem, work));
             level++;
             eps *= 0.5;
         }
-        h->levels    = level;
-        const int st = finish_setup(h, &tmp);
-        (void)hipStreamSynchronize(c->stream); // before tmp goes
+        h->levels = level;
+        if(h->lean)
+            LAL_TRY(fresh());
+        const int st = finish_setup(h, tmp.get());
+        (void)hipStreamSynchronize(c->stream); // before the arrays go
         return st;
     }
 
@@ -1117,28 +1140,37 @@ namespace
         // validate the input pattern before any setup kernel gathers through
         // it; the analysis describes the finest operator (a copy of the same
         // pattern), so the hierarchy keeps it for level 0
-        auto* h = new lal_hierarchy_t;
-        // A hierarchy takes about 140 to 175 bytes per nonzero of a 7-point
-        // operator with the column lists and the FP32 levels, less without:
-        // the first chunk holds most of it (a hipMalloc and hipFree of
-        // hundreds of megabytes take 0.3 ms together), and the arena grows by
-        // half its size.
-        h->mem.use(c->pool);
-        h->mem.reserve((size_t)nnz * ((o.exact ? 40 : 80) + (o.build_f32 ? 40 : 0)) +
-                       (size_t)m * (o.build_f32 ? 200 : 100));
-        int s = lal::analyse(c, {{descr(h->L[0].A, m, nnz, n, o.exact), rp, ci, m, nnz,
-                                  o.exact == 0, n}}, &h->mem, nullptr);
-        if(s == LAL_OK)
-            s = setup(c, m, n, nnz, rp, ci, v, o, h, unsmoothed);
-        if(s != LAL_OK)
+        for(const bool lean : {false, true})
         {
+            auto* h = new lal_hierarchy_t;
+            h->lean = lean;
+            // A hierarchy takes about 140 to 175 bytes per nonzero of a 7-point
+            // operator with the column lists and the FP32 levels, less without:
+            // the first chunk holds most of it (a hipMalloc and hipFree of
+            // hundreds of megabytes take 0.3 ms together), and the arena grows by
+            // half its size.
+            h->mem.use(c->pool);
+            if(lean)
+                h->mem.tight();
+            else
+                h->mem.reserve((size_t)nnz * ((o.exact ? 40 : 80) + (o.build_f32 ? 40 : 0)) +
+                               (size_t)m * (o.build_f32 ? 200 : 100));
+            int s = lal::analyse(c, {{descr(h->L[0].A, m, nnz, n, o.exact), rp, ci, m, nnz,
+                                      o.exact == 0, n}}, &h->mem, nullptr);
+            if(s == LAL_OK)
+                s = setup(c, m, n, nnz, rp, ci, v, o, h, unsmoothed);
+            if(s == LAL_OK)
+            {
+                c->hierarchies.push_back(h);
+                *out = h;
+                return LAL_OK;
+            }
             (void)hipStreamSynchronize(c->stream);
             delete h;
-            return s;
+            if(s != LAL_ERR_OOM)
+                return s;
         }
-        c->hierarchies.push_back(h);
-        *out = h;
-        return LAL_OK;
+        return LAL_ERR_OOM;
     }
 }
 

@@ -99,6 +99,11 @@ namespace lal
         {
             next_ = first;
         }
+        // no allocation beyond what is asked for (of 1 MiB at least)
+        void tight()
+        {
+            tight_ = true;
+        }
         int get_bytes(void** p, size_t bytes);
         template <typename T>
         int get(T** p, size_t n)
@@ -118,6 +123,7 @@ namespace lal
         };
         std::vector<chunk>          chunks_;
         size_t                      cur_ = 0, next_ = 0, total_ = 0;
+        bool                        tight_ = false;
         std::shared_ptr<chunk_pool> pool_;
     };
 }

@@ -246,8 +246,8 @@ namespace lal
             }
         }
         // a new chunk: half of what there is, within 1 MiB .. 512 MiB
-        size_t cap = std::max(next_, std::min(std::max(total_ / 2, (size_t)1 << 20),
-                                              (size_t)512 << 20));
+        const size_t half = tight_ ? 0 : total_ / 2;
+        size_t cap = std::max(next_, std::min(std::max(half, (size_t)1 << 20), (size_t)512 << 20));
         cap        = std::max((cap + 255) & ~(size_t)255, bytes);
         next_      = 0;
         char* q    = nullptr;
