@@ -95,47 +95,15 @@ namespace
         }
     }
 
-    // Sorts each row by column, stably, with G lanes per row (16 for rows of up
-    // to 32 entries on average, else a wavefront): each lane ranks its entries
-    // (up to K) by counting the row's smaller columns, ties broken by position;
-    // the columns pass from lane to lane in registers, and every load of the
-    // row completes before the first store, so the row is permuted in place.
-    // Rows longer than K G entries take the group's first lane's insertion sort.
-    // Bound by the ranking's instructions: rows of 22 entries (121^3 diffusion's
-    // R, 341,000 rows) took 236 us with a wavefront each, 125 with 16 lanes.
+    // Sorts a row of n <= K G entries by column, stably, with the G lanes from gb
+    // on: each lane ranks its entries by counting the row's smaller columns, ties
+    // broken by position; the columns pass from lane to lane in registers, and
+    // every load of the row completes before the first store, so the row is
+    // permuted in place.
     template <int G, int K, typename T>
-    __global__ void __launch_bounds__(256)
-        row_sort_kernel(int m, const int* __restrict__ rp, int* __restrict__ ci,
-                        T* __restrict__ v)
+    __device__ __forceinline__ void rank_row(int s, int n, int gl, int gb, int* __restrict__ ci,
+                                             T* __restrict__ v)
     {
-        const int gl = (int)threadIdx.x % G;
-        const int gb = ((int)threadIdx.x & 63) - gl;
-        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        if(i >= m)
-            return;
-        const int s = rp[i], n = rp[i + 1] - s;
-        if(n <= 1)
-            return;
-        if(n > K * G)
-        {
-            if(gl != 0)
-                return;
-            for(int j = s + 1; j < s + n; j++)
-            {
-                int kc = ci[j];
-                T   kv = v[j];
-                int t  = j - 1;
-                while(t >= s && ci[t] > kc)
-                {
-                    ci[t + 1] = ci[t];
-                    v[t + 1]  = v[t];
-                    t--;
-                }
-                ci[t + 1] = kc;
-                v[t + 1]  = kv;
-            }
-            return;
-        }
         int key[K], rank[K];
         T   val[K];
 #pragma unroll
@@ -172,6 +140,50 @@ namespace
             {
                 ci[s + rank[u]] = key[u];
                 v[s + rank[u]]  = val[u];
+            }
+    }
+
+    // Sorts each row by column with G lanes per row (16 for rows of up to 32
+    // entries on average, else a wavefront).  Rows of more than K G entries and up
+    // to 256 are ranked by the whole wavefront, its rows one after the other;
+    // longer ones take the insertion sort of one lane.
+    // Bound by the ranking's instructions: rows of 22 entries (121^3 diffusion's
+    // R, 341,000 rows) took 236 us with a wavefront each, 125 with 16 lanes.  A
+    // transpose with 2000 rows of 200 entries among 98,000 of 8: 202 us (with the
+    // insertion sort from 129 entries on 3170, with a wavefront for every row 258).
+    template <int G, int K, typename T>
+    __global__ void __launch_bounds__(256)
+        row_sort_kernel(int m, const int* __restrict__ rp, int* __restrict__ ci,
+                        T* __restrict__ v)
+    {
+        constexpr int WAVE_ROW = 256;
+        const int     lane = (int)threadIdx.x & 63, gl = (int)threadIdx.x % G;
+        const int     i = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
+        const int     s = i < m ? rp[i] : 0, n = i < m ? rp[i + 1] - s : 0;
+        if(n > 1 && n <= K * G)
+            rank_row<G, K>(s, n, gl, lane - gl, ci, v);
+        else if(n > WAVE_ROW && gl == 0)
+            for(int j = s + 1; j < s + n; j++)
+            {
+                int kc = ci[j];
+                T   kv = v[j];
+                int t  = j - 1;
+                while(t >= s && ci[t] > kc)
+                {
+                    ci[t + 1] = ci[t];
+                    v[t + 1]  = v[t];
+                    t--;
+                }
+                ci[t + 1] = kc;
+                v[t + 1]  = kv;
+            }
+        if constexpr(K * G < WAVE_ROW)
+            for(unsigned long long todo = __ballot(gl == 0 && n > K * G && n <= WAVE_ROW);
+                todo != 0; todo &= todo - 1)
+            {
+                const int t = __ffsll((long long)todo) - 1;
+                rank_row<64, WAVE_ROW / 64>(__builtin_amdgcn_readlane(s, t),
+                                            __builtin_amdgcn_readlane(n, t), lane, 0, ci, v);
             }
     }
 
