@@ -166,12 +166,22 @@ namespace
         return LAL_OK;
     }
 
-    // Finest levels up to here form PCG's next direction p = z + beta p inside the
-    // product that needs it, for every gathered entry, and spare the pass between:
-    // 128^2 Poisson 4.2 + 3.8 us -> 6.4 (PCG 1.52 -> 1.38 ms), 64^3 7.1 + 4.8 ->
-    // 12.5 with a launch less (gradient 12.5 -> 12.3 ms).  Beyond, the second
-    // gathered vector costs more than the pass.
-    constexpr int STEP_MAX_ROWS = 262144;
+    // PCG forms its next direction p = z + beta p inside the product that needs it,
+    // for every gathered entry, and spares the pass between (128^2 Poisson 4.2 + 3.8
+    // us -> 6.4), where that pays: a second gathered vector costs more the more
+    // entries there are, and the more of them a row's neighbours do not share.
+    // Whole FP64 and reliable solves, seven pairs in turn, gain of forming it so:
+    //   grids, 5 to 7 per row, 8,000 to 65,000 rows 1.05 .. 1.17, 130,000 1.05 .. 1.18,
+    //     262,144 (64^3, 512^2) 1.03 .. 1.12, 327,680 1.02 .. 1.04
+    //   graphs, 6 to 13 per row, up to 131,072 rows 1.02 .. 1.07; 262,144 rows (1.5 to
+    //     3.3 million entries) 1.02 .. 1.04, 0.98, 1.02, 0.96 .. 1.00
+    //   graphs, 15 per row, up to 48,000 rows (706,000 entries) 1.01 .. 1.08, 65,536 rows
+    //     0.99 .. 1.00, 131,072 0.97 .. 1.03, 250,000 0.93 .. 0.99
+    // (pairs of one case differ by 1 to 4 %)
+    bool step_pays(const csr_dev& A)
+    {
+        return A.nnz <= (A.nnz <= 13L * A.m ? 2 << 20 : 706000);
+    }
 
     // A fresh descriptor for an m x n operator of a hierarchy.
     lal_csrmv_info* descr(csr_dev& A, int m, int nnz, int n, int exact)
@@ -334,7 +344,7 @@ namespace
         LAL_TRY(h->mem.get(&h->p, n));
         LAL_TRY(h->mem.get(&h->q, n));
         LAL_TRY(h->mem.get(&h->s, lal::LAL_SOLVER_SLOTS));
-        if(n <= STEP_MAX_ROWS)
+        if(step_pays(h->L[0].A))
             LAL_TRY(h->mem.get(&h->p2, n));
         LAL_TRY(h->mem.get(&h->part_pq, lal::PCG_PARTS));
         LAL_TRY(h->mem.get(&h->part_g, lal::PCG_PARTS));
@@ -357,7 +367,7 @@ namespace
             LAL_TRY(h->mem.get(&h->res32, n));
             LAL_TRY(h->mem.get(&h->z32, n));
             LAL_TRY(h->mem.get(&h->p32, n));
-            if(n <= STEP_MAX_ROWS)
+            if(step_pays(h->L[0].A))
                 LAL_TRY(h->mem.get(&h->p2_32, n));
             LAL_TRY(h->mem.get(&h->q32, n));
             LAL_TRY(h->mem.get(&h->d32, n));
@@ -708,7 +718,7 @@ namespace
         double*      prev = h->s + lal::S_GAMMA + (cur ^ 1);
         double*      now  = h->s + lal::S_GAMMA + cur;
         bool         done = false;
-        if(stale && *p_other != nullptr)
+        if(stale && *p_other != nullptr && step_pays(A))
             LAL_TRY(lal::step_dot<T>(c, A.d, A.m, A.n, A.rp, A.ci, Av, z, *p, *p_other, q,
                                      h->part_g, n_g, prev, now, h->part_pq, n_pq, &done));
         if(done)
