@@ -66,10 +66,10 @@ namespace lal
     // 16.05 ms, on 101^3 even); 16384 cost 128^3 in FP32 1.3 %.
     constexpr int PCG_PARTS = 4096;
 
-    // What a product does besides its own rows.
-    struct row_extra
+    // What a product does besides its own rows: the *_DOT modes...
+    struct row_dot
     {
-        double*     part = nullptr; // *_DOT: one partial of <w, y> per row block
+        double*     part = nullptr; // one partial of <w, y> per row block
         const void* w    = nullptr; // m entries, FP64 with `wide`, else of the product's type
         bool        wide = false;
         // STEP_DOT: beta = (sum of the gamma_count partials at gamma_part) / *gamma_old,
@@ -78,7 +78,10 @@ namespace lal
         int           gamma_count = 0;
         const double* gamma_old   = nullptr;
         double*       gamma_new   = nullptr;
-        // SMOOTHED: a last workgroup finishes the reduction before it
+    };
+    // ... and SMOOTHED, whose last workgroup finishes the reduction before it.
+    struct row_extra : row_dot
+    {
         post_args post{};
     };
 

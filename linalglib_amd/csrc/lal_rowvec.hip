@@ -5,6 +5,47 @@ namespace
 {
     using lal::SPMV_THREADS;
 
+    // The kernels' last argument: what its mode uses of a row_extra and no more.  A
+    // launch copies its arguments to the device, and a small grid's V-cycle is its
+    // launches: with 110 bytes more that nothing read, two pre-sweeps on 128^2
+    // Poisson (31 launches) took 116 to 126 us in ten of eleven processes, without
+    // them 94 to 96 in four of seven and 110 to 120 in the others; 20^2 Poisson 92 to
+    // 102 and 71.
+    struct no_extra
+    {
+    };
+    template <int MODE>
+    struct extra_for
+    {
+        using type = no_extra;
+        static type of(const lal::row_extra&) { return {}; }
+    };
+    template <>
+    struct extra_for<lal::RV_SMOOTHED>
+    {
+        using type = lal::post_args;
+        static type of(const lal::row_extra& ex) { return ex.post; }
+    };
+    struct dot_extra
+    {
+        using type = lal::row_dot;
+        static type of(const lal::row_extra& ex) { return ex; }
+    };
+    template <>
+    struct extra_for<lal::RV_SPMV_DOT> : dot_extra
+    {
+    };
+    template <>
+    struct extra_for<lal::RV_ADD_DOT> : dot_extra
+    {
+    };
+    template <>
+    struct extra_for<lal::RV_STEP_DOT> : dot_extra
+    {
+    };
+    template <int MODE>
+    using mode_extra = typename extra_for<MODE>::type;
+
     // LDS bytes of a block's row starts (nrows + 1 <= SPMV_THREADS + 1 ints,
     // rounded up to 16 bytes so that the staged window stays aligned).
     constexpr int RP_LDS_BYTES = (int)(((SPMV_THREADS + 1) * sizeof(int) + 15) & ~15);
@@ -92,12 +133,12 @@ namespace
                                                              const T* __restrict__ d,
                                                              const T* __restrict__ b, T beta,
                                                              const T* __restrict__ y,
-                                                             const lal::row_extra& ex = {})
+                                                             const mode_extra<MODE>& ex = {})
     {
         row_operands<T> o;
         if(!on)
             return o;
-        if(MODE == lal::RV_SPMV_DOT || MODE == lal::RV_ADD_DOT)
+        if constexpr(MODE == lal::RV_SPMV_DOT || MODE == lal::RV_ADD_DOT)
             o.w = ex.wide ? static_cast<const double*>(ex.w)[row]
                           : (double)static_cast<const T*>(ex.w)[row];
         if(MODE == lal::RV_RESIDUAL || MODE == lal::RV_JACOBI || MODE == lal::RV_JACOBI0 ||
@@ -304,15 +345,16 @@ namespace
                     const unsigned short* __restrict__ c16, const int* __restrict__ cbase,
                     const T* __restrict__ val, const T* __restrict__ x,
                     const T* __restrict__ d, const T* __restrict__ b, T alpha, T beta,
-                    T* __restrict__ y, T* __restrict__ r, lal::row_extra ex)
+                    T* __restrict__ y, T* __restrict__ r, mode_extra<MODE> ex)
     {
-        if(MODE == lal::RV_SMOOTHED && (int)blockIdx.x == nb)
-        {
-            // (the grid has this workgroup only with ex.post)
-            lal::post_block<1>(ex.post);
-            return;
-        }
-        if(MODE == lal::RV_STEP_DOT)
+        if constexpr(MODE == lal::RV_SMOOTHED)
+            if((int)blockIdx.x == nb)
+            {
+                // (the grid has this workgroup only with a reduction to finish)
+                lal::post_block<1>(ex);
+                return;
+            }
+        if constexpr(MODE == lal::RV_STEP_DOT)
         {
             const double g_new = lal::total_of<0>(ex.gamma_part, ex.gamma_count);
             if(blockIdx.x == 0 && threadIdx.x == 0)
@@ -415,7 +457,7 @@ namespace
         }
         if(g > 1)
             acc = lal::group_sum(acc, g);
-        if(MODE == lal::RV_STEP_DOT)
+        if constexpr(MODE == lal::RV_STEP_DOT)
         {
             const bool head = active && lig == 0;
             row_operands<T> o;
@@ -428,7 +470,7 @@ namespace
             dot_epilogue<T, MODE>(head, row, acc, o, y, ex.part + tile);
             return;
         }
-        if(MODE == lal::RV_SPMV_DOT)
+        if constexpr(MODE == lal::RV_SPMV_DOT)
         {
             dot_epilogue<T, MODE>(active && lig == 0, row, acc, ops, y, ex.part + tile);
             return;
@@ -639,7 +681,7 @@ namespace
                     const unsigned short* __restrict__ list, const int* __restrict__ lmeta,
                     const T* __restrict__ val, const T* __restrict__ x, const T* __restrict__ d,
                     const T* __restrict__ b, T alpha, T beta, T* __restrict__ y,
-                    T* __restrict__ r, lal::row_extra ex)
+                    T* __restrict__ r, mode_extra<MODE> ex)
     {
         typedef int int2v __attribute__((ext_vector_type(2)));
         // the block's row starts, its x entries, then its products
@@ -744,7 +786,7 @@ namespace
                               s_rp[lrow + 1] - ws, 1 << lg);
         if(lg > 0)
             acc = lal::group_sum(acc, 1 << lg);
-        if(MODE == lal::RV_ADD_DOT)
+        if constexpr(MODE == lal::RV_ADD_DOT)
             dot_epilogue<T, MODE>(head, r0 + lrow, acc, ops, y, ex.part + tile);
         else if(head)
             row_epilogue<T, MODE>(r0 + lrow, acc, ops, alpha, beta, y, r);
@@ -767,7 +809,7 @@ namespace
         fn<<<nb + more, SPMV_THREADS, RP_LDS_BYTES + (sizeof(int) + sizeof(T)) * win, c->stream>>>(
             a.m, a.nnz, a.blocks, nb, win, a.rp, a.ci, a.c16, a.cbase, (const T*)a.val,
             (const T*)a.x, (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r,
-            a.ex);
+            extra_for<MODE>::of(a.ex));
     }
 
     template <typename T, int MODE>
@@ -781,7 +823,8 @@ namespace
                                         : list_kernel<T, MODE, false, false>);
         fn<<<nb, SPMV_THREADS, lds, c->stream>>>(
             a.blocks, nb, lm, a.rp, a.lpos, a.list, a.lmeta, (const T*)a.val, (const T*)a.x,
-            (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r, a.ex);
+            (const T*)a.d, (const T*)a.b, (T)a.alpha, (T)a.beta, (T*)a.y, (T*)a.r,
+            extra_for<MODE>::of(a.ex));
     }
 
     // Which kernel reads a matrix.
