@@ -127,10 +127,12 @@ namespace
     constexpr int RB_TILE  = 2048;
     constexpr int RB_BATCH = 24; // operators per launch (their table is a kernel argument)
 
+    // (a descriptor's own analysis has one: a launch copies its arguments)
+    template <int MAX>
     struct rb_table
     {
-        int           n;
-        lal::rb_op op[RB_BATCH];
+        int        n;
+        lal::rb_op op[MAX];
     };
 
     // results of one operator, in the order read back
@@ -147,8 +149,8 @@ namespace
     };
 
     // Position of `at` among the operators' starts (ascending).
-    template <typename F>
-    __device__ __forceinline__ int rb_find(const rb_table& t, int at, F start)
+    template <int MAX, typename F>
+    __device__ __forceinline__ int rb_find(const rb_table<MAX>& t, int at, F start)
     {
         int k = 0;
         while(k + 1 < t.n && start(t.op[k + 1]) <= at)
@@ -156,22 +158,50 @@ namespace
         return k;
     }
 
+    // Tiles of one operator that the second pass scans by itself.
+    constexpr int RB_SCAN = 256;
+
     // WRITE false: blocks per tile into tcount, the widest window and the row
     // pointer's faults into res.  WRITE true: the block table, at the tile's
-    // offset that the scan left in tcount.
-    template <bool WRITE>
+    // offset that the scan left in tcount; with `scan` (one operator of at most
+    // RB_SCAN tiles) every workgroup adds up the counts before its own.
+    template <bool WRITE, int MAX>
     __global__ void __launch_bounds__(256)
-        rb_tile_kernel(rb_table tab, int* __restrict__ tcount, int* __restrict__ res)
+        rb_tile_kernel(rb_table<MAX> tab, int* __restrict__ tcount, int* __restrict__ res, bool scan)
     {
         __shared__ int            s_rp[RB_TILE + 1];
         __shared__ unsigned short s_next[RB_TILE];
-        __shared__ int            s_n;
+        __shared__ int            s_n, s_sum[2][4];
         const int    k   = rb_find(tab, (int)blockIdx.x, [](const lal::rb_op& o) { return o.tile0; });
         const lal::rb_op o = tab.op[k];
         int*         out = res + RB_RES * k;
-        if(WRITE && (out[RB_BAD] != 0 || out[RB_NBLOCKS] > o.ub))
+        const int    tid = (int)threadIdx.x;
+        int          all = 0, at = 0; // blocks of the operator, and before this tile
+        if(WRITE && scan)
+        {
+            const int v = tid < o.ntiles ? tcount[tid] : 0;
+            const int a = lal::wave_sum(v), b = lal::wave_sum(tid < (int)blockIdx.x ? v : 0);
+            if((tid & 63) == 0)
+            {
+                s_sum[0][tid >> 6] = a;
+                s_sum[1][tid >> 6] = b;
+            }
+            __syncthreads();
+            for(int w = 0; w < 4; w++)
+            {
+                all += s_sum[0][w];
+                at += s_sum[1][w];
+            }
+            if(blockIdx.x == 0 && tid == 0)
+                out[RB_NBLOCKS] = all;
+        }
+        else if(WRITE)
+        {
+            all = out[RB_NBLOCKS];
+            at  = tcount[blockIdx.x];
+        }
+        if(WRITE && (out[RB_BAD] != 0 || all > o.ub))
             return;
-        const int tid = (int)threadIdx.x;
         const int r0  = ((int)blockIdx.x - o.tile0) * RB_TILE;
         const int n   = min(RB_TILE, o.m - r0);
         for(int i = tid; i <= n; i += 256)
@@ -206,30 +236,34 @@ namespace
         __syncthreads();
         if(tid == 0)
         {
-            int cnt = 0, win = 4;
+            // reached rows are read once: the list of block starts replaces the
+            // links behind the walk
+            int cnt = 0;
             for(int r = 0; r < n;)
             {
-                const int nx   = s_next[r];
-                const int span = ((s_rp[nx] + 3) & ~3) - (s_rp[r] & ~3);
-                win            = max(win, min(span, 2052));
-                // reached rows are read once: the list of block starts
-                // replaces the links behind the walk
-                s_next[cnt++] = (unsigned short)r;
-                r             = nx;
+                const int next = s_next[r];
+                s_next[cnt++]  = (unsigned short)r;
+                r              = next;
             }
             s_n = cnt;
-            if(!WRITE)
-            {
-                tcount[blockIdx.x] = cnt;
-                atomicMax(out + RB_WIN, win);
-            }
         }
-        if(!WRITE)
-            return;
         __syncthreads();
-        const int nb   = s_n;
-        const int at   = tcount[blockIdx.x];
-        const int all  = out[RB_NBLOCKS];
+        const int nb = s_n;
+        if(!WRITE)
+        {
+            int win = 4;
+            for(int b = tid; b < nb; b += 256)
+            {
+                const int i = s_next[b], e = b + 1 < nb ? (int)s_next[b + 1] : n;
+                win         = max(win, min(((s_rp[e] + 3) & ~3) - (s_rp[i] & ~3), 2052));
+            }
+            win = lal::wave_max(win);
+            if((tid & 63) == 0 && win > 4)
+                atomicMax(out + RB_WIN, win);
+            if(tid == 0)
+                tcount[blockIdx.x] = nb;
+            return;
+        }
         int*      meta = o.blocks + lal::block_meta_offset(all);
         for(int b = tid; b < nb; b += 256)
         {
@@ -245,8 +279,9 @@ namespace
     }
 
     // One workgroup per operator: its tiles' block counts become offsets.
+    template <int MAX>
     __global__ void __launch_bounds__(256)
-        rb_scan_kernel(rb_table tab, int* __restrict__ tcount, int* __restrict__ res)
+        rb_scan_kernel(rb_table<MAX> tab, int* __restrict__ tcount, int* __restrict__ res)
     {
         __shared__ int  s_w[4];
         const int       k    = (int)blockIdx.x;
@@ -307,8 +342,9 @@ namespace
     // entry and one lane unpacking a bitmap word took 770 us over the operators
     // of a 121^3 diffusion hierarchy; now 460 us, bound by the chain of
     // barriers).
+    template <int MAX>
     __global__ void __launch_bounds__(256)
-        rb_columns_kernel(rb_table tab, int* __restrict__ res)
+        rb_columns_kernel(rb_table<MAX> tab, int* __restrict__ res)
     {
         typedef int            int4v __attribute__((ext_vector_type(4)));
         typedef unsigned       uint4v __attribute__((ext_vector_type(4)));
@@ -562,103 +598,132 @@ namespace lal
         return cap;
     }
 
-    int analyse(lal_context* c, const std::vector<rb_request>& req, arena* mem, arena* tmp)
+    // Requests [first, ...) in one pass, MAX of them at most.
+    template <int MAX>
+    static int analyse_some(lal_context* c, const std::vector<rb_request>& req, size_t first,
+                            arena* mem, arena* tmp)
     {
-        for(size_t first = 0; first < req.size(); first += RB_BATCH)
+        temps         t(c, tmp);
+        rb_table<MAX> tab{};
+        int           tiles = 0, blocks = 0;
+        tab.n               = (int)std::min(req.size() - first, (size_t)MAX);
+        for(int k = 0; k < tab.n; k++)
         {
-            temps    t(c, tmp);
-            rb_table tab{};
-            int      tiles = 0, blocks = 0;
-            tab.n          = (int)std::min(req.size() - first, (size_t)RB_BATCH);
-            for(int k = 0; k < tab.n; k++)
+            const rb_request& q = req[first + k];
+            rb_op&            o = tab.op[k];
+            o.rp     = q.rp;
+            o.ci     = q.ci;
+            o.m      = q.m;
+            o.nnz    = q.nnz;
+            // (the list kernel takes a block as 512 quads of four)
+            o.cap    = block_cap(q.nnz, q.want_list);
+            o.tile0  = tiles;
+            o.ntiles = std::max((q.m + RB_TILE - 1) / RB_TILE, 1);
+            o.blk0   = blocks;
+            // a block that is neither of 256 rows nor a tile's last holds
+            // more than cap nonzeros together with its successor
+            o.ub = q.m / SPMV_THREADS + (int)(2LL * q.nnz / o.cap) + o.ntiles + 1;
+            tiles += o.ntiles;
+            blocks += o.ub;
+            LAL_TRY(q.d->arrays(mem, o.ub));
+            o.blocks = q.d->d_blocks;
+            if(mem && q.want16 && q.nnz > 0)
             {
-                const rb_request& q = req[first + k];
-                rb_op&            o = tab.op[k];
-                o.rp     = q.rp;
-                o.ci     = q.ci;
-                o.m      = q.m;
-                o.nnz    = q.nnz;
-                // (the list kernel takes a block as 512 quads of four)
-                o.cap    = block_cap(q.nnz, q.want_list);
-                o.tile0  = tiles;
-                o.ntiles = std::max((q.m + RB_TILE - 1) / RB_TILE, 1);
-                o.blk0   = blocks;
-                // a block that is neither of 256 rows nor a tile's last holds
-                // more than cap nonzeros together with its successor
-                o.ub = q.m / SPMV_THREADS + (int)(2LL * q.nnz / o.cap) + o.ntiles + 1;
-                tiles += o.ntiles;
-                blocks += o.ub;
-                LAL_TRY(q.d->arrays(mem, o.ub));
-                o.blocks = q.d->d_blocks;
-                if(mem && q.want16 && q.nnz > 0)
+                // whole 16-byte lines: the kernels load four entries at a time
+                LAL_TRY(mem->get(&q.d->d_c16, ((size_t)q.nnz + 7) & ~(size_t)7));
+                LAL_TRY(mem->get(&q.d->d_cbase, o.ub));
+                o.c16   = q.d->d_c16;
+                o.cbase = q.d->d_cbase;
+                if(q.want_list)
                 {
-                    // whole 16-byte lines: the kernels load four entries at a time
-                    LAL_TRY(mem->get(&q.d->d_c16, ((size_t)q.nnz + 7) & ~(size_t)7));
-                    LAL_TRY(mem->get(&q.d->d_cbase, o.ub));
-                    o.c16   = q.d->d_c16;
-                    o.cbase = q.d->d_cbase;
-                    if(q.want_list)
-                    {
-                        LAL_TRY(mem->get(&q.d->d_lpos, ((size_t)q.nnz + 7) & ~(size_t)7));
-                        LAL_TRY(mem->get(&q.d->d_list, list_start(q.nnz, o.ub) + 4));
-                        LAL_TRY(mem->get(&q.d->d_lmeta, 2 * (size_t)o.ub));
-                        o.lpos  = q.d->d_lpos;
-                        o.list  = q.d->d_list;
-                        o.lmeta = q.d->d_lmeta;
-                    }
+                    LAL_TRY(mem->get(&q.d->d_lpos, ((size_t)q.nnz + 7) & ~(size_t)7));
+                    LAL_TRY(mem->get(&q.d->d_list, list_start(q.nnz, o.ub) + 4));
+                    LAL_TRY(mem->get(&q.d->d_lmeta, 2 * (size_t)o.ub));
+                    o.lpos  = q.d->d_lpos;
+                    o.list  = q.d->d_list;
+                    o.lmeta = q.d->d_lmeta;
                 }
-            }
-            int *tcount = nullptr, *res = nullptr;
-            int  h[RB_RES * RB_BATCH] = {};
-            LAL_TRY(t.get(&res, RB_RES * RB_BATCH));
-            LAL_TRY(t.get(&tcount, tiles));
-            LAL_TRY(lal_fill_i32(c, res, RB_RES * RB_BATCH, 0));
-            rb_tile_kernel<false><<<tiles, 256, 0, c->stream>>>(tab, tcount, res);
-            LAL_LAUNCHED();
-            rb_scan_kernel<<<tab.n, 256, 0, c->stream>>>(tab, tcount, res);
-            LAL_LAUNCHED();
-            rb_tile_kernel<true><<<tiles, 256, 0, c->stream>>>(tab, tcount, res);
-            LAL_LAUNCHED();
-            if(mem)
-            {
-                rb_columns_kernel<<<blocks, 256, 0, c->stream>>>(tab, res);
-                LAL_LAUNCHED();
-            }
-            for(int k = 0; k < tab.n; k++)
-                if(req[first + k].check_n >= 0 && tab.op[k].nnz > 0)
-                {
-                    check_cols_kernel<<<grid_for(tab.op[k].nnz, 256, 4096), 256, 0, c->stream>>>(
-                        tab.op[k].nnz, req[first + k].check_n, tab.op[k].ci,
-                        res + RB_RES * k + RB_BAD, 4);
-                    LAL_LAUNCHED();
-                }
-            LAL_TRY(read_ints(c, res, RB_RES * tab.n, h, false));
-            for(int k = 0; k < tab.n; k++)
-            {
-                const rb_request& q = req[first + k];
-                const int*        r = h + RB_RES * k;
-                if(r[RB_BAD] & 4)
-                    set_last_error("column index outside [0, n)");
-                else if(r[RB_BAD] & 1)
-                    set_last_error("row_ptr does not start at 0 or end at nnz");
-                else if(r[RB_BAD] & 2 || r[RB_NBLOCKS] > tab.op[k].ub)
-                    set_last_error("row_ptr is not monotone");
-                else
-                {
-                    q.d->nblocks = r[RB_NBLOCKS];
-                    q.d->win     = std::max(r[RB_WIN], 4);
-                    if(r[RB_WIDE])
-                        q.d->d_c16 = nullptr;
-                    if(q.d->d_lpos && !r[RB_LONG])
-                    {
-                        q.d->list_max = r[RB_LMAX];
-                        q.d->list_far = r[RB_FAR] != 0;
-                    }
-                    continue;
-                }
-                return LAL_ERR_INVALID;
             }
         }
+        // A single operator of few tiles, as a caller's descriptor mostly is,
+        // takes the context's flags (zero between calls) and reduction
+        // workspace for its results and counts: no allocation, no clearing and
+        // no scan of its own.  128^2 Poisson: 88 to 99 us without this and with a
+        // table of 24 operators among the arguments, 40 so, 58 on the host; 5000
+        // rows of up to 2500 entries 115, 55, 58; 100^3 (the general way) 89 and
+        // 640 on the host.
+        const bool few    = tab.n == 1 && tiles <= RB_SCAN;
+        int *      tcount = nullptr, *res = nullptr;
+        int        h[RB_RES * MAX] = {};
+        static_assert(RB_RES <= LAL_FLAGS && RB_SCAN <= 2 * LAL_RED_BLOCKS);
+        if(few)
+        {
+            res    = c->d_flag;
+            tcount = reinterpret_cast<int*>(c->d_part);
+        }
+        else
+        {
+            LAL_TRY(t.get(&res, RB_RES * MAX));
+            LAL_TRY(t.get(&tcount, tiles));
+            LAL_TRY(lal_fill_i32(c, res, RB_RES * MAX, 0));
+        }
+        rb_tile_kernel<false, MAX><<<tiles, 256, 0, c->stream>>>(tab, tcount, res, few);
+        LAL_LAUNCHED();
+        if(!few)
+        {
+            rb_scan_kernel<MAX><<<tab.n, 256, 0, c->stream>>>(tab, tcount, res);
+            LAL_LAUNCHED();
+        }
+        rb_tile_kernel<true, MAX><<<tiles, 256, 0, c->stream>>>(tab, tcount, res, few);
+        LAL_LAUNCHED();
+        if(mem)
+        {
+            rb_columns_kernel<MAX><<<blocks, 256, 0, c->stream>>>(tab, res);
+            LAL_LAUNCHED();
+        }
+        for(int k = 0; k < tab.n; k++)
+            if(req[first + k].check_n >= 0 && tab.op[k].nnz > 0)
+            {
+                check_cols_kernel<<<grid_for(tab.op[k].nnz, 256, 4096), 256, 0, c->stream>>>(
+                    tab.op[k].nnz, req[first + k].check_n, tab.op[k].ci,
+                    res + RB_RES * k + RB_BAD, 4);
+                LAL_LAUNCHED();
+            }
+        LAL_TRY(read_ints(c, res, RB_RES * tab.n, h, few));
+        for(int k = 0; k < tab.n; k++)
+        {
+            const rb_request& q = req[first + k];
+            const int*        r = h + RB_RES * k;
+            if(r[RB_BAD] & 4)
+                set_last_error("column index outside [0, n)");
+            else if(r[RB_BAD] & 1)
+                set_last_error("row_ptr does not start at 0 or end at nnz");
+            else if(r[RB_BAD] & 2 || r[RB_NBLOCKS] > tab.op[k].ub)
+                set_last_error("row_ptr is not monotone");
+            else
+            {
+                q.d->nblocks = r[RB_NBLOCKS];
+                q.d->win     = std::max(r[RB_WIN], 4);
+                if(r[RB_WIDE])
+                    q.d->d_c16 = nullptr;
+                if(q.d->d_lpos && !r[RB_LONG])
+                {
+                    q.d->list_max = r[RB_LMAX];
+                    q.d->list_far = r[RB_FAR] != 0;
+                }
+                continue;
+            }
+            return LAL_ERR_INVALID;
+        }
+        return LAL_OK;
+    }
+
+    int analyse(lal_context* c, const std::vector<rb_request>& req, arena* mem, arena* tmp)
+    {
+        if(req.size() == 1)
+            return analyse_some<1>(c, req, 0, mem, tmp);
+        for(size_t first = 0; first < req.size(); first += RB_BATCH)
+            LAL_TRY(analyse_some<RB_BATCH>(c, req, first, mem, tmp));
         return LAL_OK;
     }
 
