@@ -239,19 +239,44 @@ namespace
         return k;
     }
 
+    // f(row, lane) by the whole wavefront, for every row of its groups that holds
+    // more entries than a group's registers (`len`, -1: no row).  Such a row is read
+    // again for every output column, and the lanes per row follow the mean length.
+    // Power law, 5000 rows of up to 2500 entries, 28 on average: counts 4.1 ms with
+    // a wavefront for every row, 14.0 with 16 lanes, 3.5 so; fills 9.5, 36.3, 9.2.
+    // 400,000 rows of up to 3000, 8 lanes for the others: 265 -> 36 and 690 -> 88 ms.
+    template <int G, typename F>
+    __device__ __forceinline__ void long_rows(int i, int len, F f)
+    {
+        if constexpr(G < 64)
+        {
+            const int lane = (int)threadIdx.x & 63;
+            for(unsigned long long todo = __ballot(lane % G == 0 && len > G * PROLONG_KEEP);
+                todo != 0; todo &= todo - 1)
+                f(__builtin_amdgcn_readlane(i, __ffsll((long long)todo) - 1), lane);
+        }
+    }
+
     template <int G>
     __global__ void __launch_bounds__(256)
         prolong_count_group_kernel(int m, const int* __restrict__ rp, const int* __restrict__ ci,
                                    const int* __restrict__ conn, const int64_t* __restrict__ agg,
                                    int* __restrict__ count)
     {
-        const int gl = (int)threadIdx.x % G;
-        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        if(i > m)
-            return;
-        const int k = i < m ? prolong_count_row<G>(i, gl, rp, ci, conn, agg) : 0;
-        if(gl == 0)
-            count[i] = k;
+        const int gl  = (int)threadIdx.x % G;
+        const int i   = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
+        const int len = i < m ? rp[i + 1] - rp[i] : -1;
+        if(i <= m && (G == 64 || len <= G * PROLONG_KEEP))
+        {
+            const int k = i < m ? prolong_count_row<G>(i, gl, rp, ci, conn, agg) : 0;
+            if(gl == 0)
+                count[i] = k;
+        }
+        long_rows<G>(i, len, [&](int row, int lane) {
+            const int k = prolong_count_row<64>(row, lane, rp, ci, conn, agg);
+            if(lane == 0)
+                count[row] = k;
+        });
     }
 
     // Row i of P into pci/pv[p0 .. p1).
@@ -376,10 +401,15 @@ namespace
                                   const int* __restrict__ prp, int* __restrict__ pci,
                                   double* __restrict__ pv)
     {
-        const int gl = (int)threadIdx.x % G;
-        const int i  = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        if(i < m)
+        const int gl  = (int)threadIdx.x % G;
+        const int i   = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
+        const int len = i < m ? rp[i + 1] - rp[i] : -1;
+        if(i < m && (G == 64 || len <= G * PROLONG_KEEP))
             prolong_fill_row<G>(i, gl, rp, ci, val, conn, agg, relax, prp[i], prp[i + 1], pci, pv);
+        long_rows<G>(i, len, [&](int row, int lane) {
+            prolong_fill_row<64>(row, lane, rp, ci, val, conn, agg, relax, prp[row], prp[row + 1],
+                                 pci, pv);
+        });
     }
 }
 
