@@ -1147,6 +1147,14 @@ namespace
         if(few)
             g = 64;
         g = std::max(g, l);
+        // The counting pass, whose order does not matter: twice the lanes where the
+        // tables of 256 would not let eight workgroups share a CU's LDS.  kNN
+        // graphs, 12 neighbours (512 and 1024 slots, 16 lanes by the mean), kernel
+        // time: 60,000 points 56 -> 42 us, 150,001 184 -> 127, 300,000 334 -> 233
+        // (four times the lanes 45, 134, 251).  7-point operators (128 slots, 8
+        // lanes, 16 KB) stay: 100^3 91 us, 199 with four times.
+        if(!NUMERIC && !few && g < 64 && table_bytes(H[0], false) * (256 / g) > 20 * 1024)
+            g <<= 1;
         // up to 256 lanes and 48 KB of tables per workgroup; a row for each
         // where several bins share the launch.  Rows much longer than the mean
         // that chose g (a matrix of few long rows among many short ones) get as

@@ -4,7 +4,7 @@ tables within a workgroup's share of LDS; bit for bit against the oracle."""
 import numpy as np
 import pytest
 
-from linalglib_amd import lal
+from linalglib_amd import lal, problems as pb
 from oracle.oracle import CSR
 from tests.gpu_util import log
 from tests.test_gpu_amg import _gpu_spgemm, csr_equal
@@ -48,3 +48,17 @@ def test_long_rows_among_short_ones(oracle, m, long_rows, length, slots):
     lanes = 8 if A.nnz <= 8 * m else 16
     assert slots // 4 < most <= slots // 2 and (per_row > slots // 4).sum() * lanes >= 262144
     assert csr_equal(_gpu_spgemm(lal.Handle(), A, B), C)
+
+
+@pytest.mark.parametrize("k,tables", [(4, 128), (9, 512), (14, 1024)])
+def test_counting_lanes(oracle, k, tables):
+    """Square products of graphs on either side of the line where the counting pass
+    doubles its lanes (8 lanes a row and 128 slots; 16 and 512 or 1024)."""
+    n = 34000
+    rp, ci, m, edges, entry, edge, sign, dpos = pb.knn_laplacian(n, k=k, seed=3)
+    v = np.random.default_rng(k).uniform(-1, 1, len(ci))
+    A = CSR(rp, ci, v, m, m)
+    products = np.add.reduceat(np.diff(rp)[ci], rp[:-1])
+    log(f"counting lanes: {len(ci) / m:.1f} per row, {products.mean():.0f} products")
+    assert tables // 2 < 2 * np.median(products) <= tables
+    assert csr_equal(_gpu_spgemm(lal.Handle(), A, A), oracle.csrgemm(A, A))
