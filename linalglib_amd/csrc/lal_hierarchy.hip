@@ -662,10 +662,16 @@ namespace
     // rows), where every kernel is short and the host's launches bound the cycle,
     // it is captured as a HIP graph on its second use and replayed after
     // (lal::captured): PCG on 2D Poisson 128^2, 16,384 rows, 1.37 ms against 1.51
-    // to 1.56 launched eagerly by a busy host.  On larger ones the graph's replay
-    // costs more than it saves (gradient on 64^3, 262,144 rows: 12.2 against
-    // 11.5 ms; 101^3: 8.70 against 8.53), so they launch eagerly.
-    constexpr int GRAPH_MAX_ROWS = 65536;
+    // to 1.56 launched eagerly by a busy host.  The host launches at one of two
+    // speeds, by process; a graph takes the same time in both.  Whole solves,
+    // graph / eager fast / eager slow (us): 2D 66,049 rows 2050 / 1970 / 2210 to
+    // 2460, 131,044 rows 2270 to 2360 / 2120 to 2160 / 2430 to 2620, 261,632 rows
+    // 2770 to 2920 / 2560 to 2750 / 2840 to 3010; 3D diffusion 91,125 rows 1510 /
+    // 1390 to 1440 / 1550 to 1690, 166,375 rows 1790 / 1670 to 1690 / 1810 to 1900,
+    // 262,144 rows 1980 to 2070 / 1870 to 1980 / 2000 to 2060 (gradient on 64^3:
+    // 11.9 and 12.4 against 11.3 and 11.8 ms).  The line is where what the slow
+    // speed loses no longer outweighs what the fast one gains.
+    constexpr int GRAPH_MAX_ROWS = 131072;
 
     template <typename T>
     int precond_graphed(lal_hierarchy_t* h, const T* r, T* z, int n1, int n2,
