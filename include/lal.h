@@ -85,7 +85,8 @@ int lal_axpbypgz_f64(lal_handle h, int n, double alpha, const double* x, double 
                      const double* y, double gamma, double* z);
 int lal_axpy_f32(lal_handle h, int n, float alpha, const float* x, float* y);
 int lal_axpby_f32(lal_handle h, int n, float alpha, const float* x, float beta, float* y);
-/* Result returned to host memory (blocks until ready). FP64 accumulation.
+/* Result returned to host memory (blocks until it is there; the stream may still be
+ * ending the launch that wrote it).  FP64 accumulation.
  * lal_dot_f64 with n <= 1024 sums in index order (bit-identical to the host
  * loop at one OpenMP thread); longer vectors use a fixed-order tree. */
 int lal_dot_f64(lal_handle h, int n, const double* x, const double* y, double* result);

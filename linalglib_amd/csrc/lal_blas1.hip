@@ -512,7 +512,12 @@ namespace
 {
     // The last block writes the result to the context's note, which the host
     // polls (a CG step on 128^2 with four results, each by a copy to pinned
-    // memory and a stream synchronisation: 100 us, so: 79).  The block's release
+    // memory and a stream synchronisation: 98 to 100 us, so: 74 to 77).  The
+    // runtime has not seen the launches end then: a wait for the device right
+    // behind costs 9 us, 25 with eight or more of them, so that step and such a
+    // wait take 119 us instead of 103.  Every form that spares it (a stream
+    // synchronisation for each result or for every second, stop events) costs a
+    // loop 9 to 20 us a step.  The block's release
     // comes after every other block's through the ticket, so a vector that the
     // same kernel wrote is complete when the host goes on.
     template <typename T, int OP>
