@@ -143,48 +143,134 @@ namespace
             }
     }
 
-    // Sorts each row by column with G lanes per row (16 for rows of up to 32
-    // entries on average, else a wavefront).  Rows of more than K G entries and up
-    // to 256 are ranked by the whole wavefront, its rows one after the other;
-    // longer ones take the insertion sort of one lane.
+    constexpr int WAVE_ROW = 256;  // entries of a row that a wavefront ranks
+    constexpr int LONG_RUN = 4096; // keys sorted in LDS at a time
+
+    // Row c of the transpose, n entries from s on, by the whole workgroup: its
+    // columns are sorted in LDS runs, which are merged pairwise between tci and
+    // tmp (every key finds its place in the other run by binary search); the
+    // values then come from the matrix itself, the d-th of several equal columns
+    // from the d-th entry of column c in that row.
+    template <typename T>
+    __device__ void long_row(int c, int s, int n, int* s_key, int* tci, T* tv, int* tmp,
+                             const int* __restrict__ rp, const int* __restrict__ ci,
+                             const T* __restrict__ v)
+    {
+        const int tid = (int)threadIdx.x;
+        for(int r0 = 0; r0 < n; r0 += LONG_RUN)
+        {
+            const int len = min(LONG_RUN, n - r0);
+            int       pow = 256;
+            while(pow < len)
+                pow <<= 1;
+            for(int t = tid; t < pow; t += 256)
+                s_key[t] = t < len ? tci[s + r0 + t] : INT_MAX;
+            __syncthreads();
+            for(int k = 2; k <= pow; k <<= 1)
+                for(int j = k >> 1; j > 0; j >>= 1)
+                {
+                    for(int t = tid; t < pow / 2; t += 256)
+                    {
+                        const int at = 2 * t - (t & (j - 1)), x = s_key[at], y = s_key[at + j];
+                        if((x > y) == ((at & k) == 0))
+                        {
+                            s_key[at]     = y;
+                            s_key[at + j] = x;
+                        }
+                    }
+                    __syncthreads();
+                }
+            for(int t = tid; t < len; t += 256)
+                tci[s + r0 + t] = s_key[t];
+            __syncthreads();
+        }
+        int *src = tci + s, *dst = tmp + s;
+        for(unsigned run = LONG_RUN; run < (unsigned)n; run <<= 1)
+        {
+            for(unsigned e = tid; e < (unsigned)n; e += 256)
+            {
+                const int      key  = src[e];
+                const unsigned pair = e & ~(2 * run - 1), mid = min(pair + run, (unsigned)n);
+                const bool     left = e < mid;
+                // the other run's keys that come before this one
+                unsigned lo = left ? mid : pair, hi = left ? min(pair + 2 * run, (unsigned)n) : mid;
+                const unsigned first = lo;
+                while(lo < hi)
+                {
+                    const unsigned m = (lo + hi) >> 1;
+                    if(left ? src[m] < key : src[m] <= key)
+                        lo = m + 1;
+                    else
+                        hi = m;
+                }
+                dst[(left ? e : pair + (e - mid)) + (lo - first)] = key;
+            }
+            __syncthreads();
+            int* const t = src;
+            src          = dst;
+            dst          = t;
+        }
+        if(src != tci + s)
+        {
+            for(int e = tid; e < n; e += 256)
+                tci[s + e] = src[e];
+            __syncthreads();
+        }
+        for(int e = tid; e < n; e += 256)
+        {
+            const int i = tci[s + e];
+            int       d = 0;
+            while(d < e && tci[s + e - d - 1] == i)
+                d++;
+            for(int j = rp[i]; j < rp[i + 1]; j++)
+                if(ci[j] == c && d-- == 0)
+                {
+                    tv[s + e] = v[j];
+                    break;
+                }
+        }
+        __syncthreads();
+    }
+
+    // Sorts each row of the transpose by column with G lanes per row (16 for rows
+    // of up to 32 entries on average, else a wavefront).  Rows of more than K G
+    // entries and up to 256 are ranked by the whole wavefront, longer ones sorted
+    // by the workgroup, its rows one after the other (tmp: an int per entry; rp,
+    // ci, v: the matrix).
     // Bound by the ranking's instructions: rows of 22 entries (121^3 diffusion's
     // R, 341,000 rows) took 236 us with a wavefront each, 125 with 16 lanes.  A
     // transpose with 2000 rows of 200 entries among 98,000 of 8: 202 us (with the
     // insertion sort from 129 entries on 3170, with a wavefront for every row 258).
+    // Graph of 60,000 rows, one of 28,000 entries: 3.9 ms, 56 s with one lane's
+    // insertion sort (42 s while the entries arrived in another order).
     template <int G, int K, typename T>
     __global__ void __launch_bounds__(256)
-        row_sort_kernel(int m, const int* __restrict__ rp, int* __restrict__ ci,
-                        T* __restrict__ v)
+        row_sort_kernel(int m, const int* __restrict__ trp, int* tci, T* tv, int* tmp,
+                        const int* __restrict__ rp, const int* __restrict__ ci,
+                        const T* __restrict__ v)
     {
-        constexpr int WAVE_ROW = 256;
-        const int     lane = (int)threadIdx.x & 63, gl = (int)threadIdx.x % G;
-        const int     i = blockIdx.x * (256 / G) + (int)threadIdx.x / G;
-        const int     s = i < m ? rp[i] : 0, n = i < m ? rp[i + 1] - s : 0;
+        __shared__ int s_key[LONG_RUN];
+        const int      lane = (int)threadIdx.x & 63, gl = (int)threadIdx.x % G;
+        const int      first = blockIdx.x * (256 / G), i = first + (int)threadIdx.x / G;
+        const int      s = i < m ? trp[i] : 0, n = i < m ? trp[i + 1] - s : 0;
         if(n > 1 && n <= K * G)
-            rank_row<G, K>(s, n, gl, lane - gl, ci, v);
-        else if(n > WAVE_ROW && gl == 0)
-            for(int j = s + 1; j < s + n; j++)
-            {
-                int kc = ci[j];
-                T   kv = v[j];
-                int t  = j - 1;
-                while(t >= s && ci[t] > kc)
-                {
-                    ci[t + 1] = ci[t];
-                    v[t + 1]  = v[t];
-                    t--;
-                }
-                ci[t + 1] = kc;
-                v[t + 1]  = kv;
-            }
+            rank_row<G, K>(s, n, gl, lane - gl, tci, tv);
         if constexpr(K * G < WAVE_ROW)
             for(unsigned long long todo = __ballot(gl == 0 && n > K * G && n <= WAVE_ROW);
                 todo != 0; todo &= todo - 1)
             {
                 const int t = __ffsll((long long)todo) - 1;
                 rank_row<64, WAVE_ROW / 64>(__builtin_amdgcn_readlane(s, t),
-                                            __builtin_amdgcn_readlane(n, t), lane, 0, ci, v);
+                                            __builtin_amdgcn_readlane(n, t), lane, 0, tci, tv);
             }
+        if(!__syncthreads_or(n > WAVE_ROW))
+            return;
+        for(int c = first; c < min(m, first + 256 / G); c++)
+        {
+            const int at = trp[c], len = trp[c + 1] - at; // (uniform)
+            if(len > WAVE_ROW)
+                long_row(c, at, len, s_key, tci, tv, tmp, rp, ci, v);
+        }
     }
 
     // -------------------------------------------------------------- SpGEMM
@@ -1295,9 +1381,11 @@ namespace lal
                                                                             place, tci, tv);
         LAL_LAUNCHED();
         if(nnz <= 32L * n)
-            row_sort_kernel<16, 8, T><<<(n + 15) / 16, 256, 0, c->stream>>>(n, trp, tci, tv);
+            row_sort_kernel<16, 8, T><<<(n + 15) / 16, 256, 0, c->stream>>>(n, trp, tci, tv, place, rp,
+                                                                            ci, v);
         else
-            row_sort_kernel<64, 4, T><<<(n + 3) / 4, 256, 0, c->stream>>>(n, trp, tci, tv);
+            row_sort_kernel<64, 4, T><<<(n + 3) / 4, 256, 0, c->stream>>>(n, trp, tci, tv, place, rp,
+                                                                          ci, v);
         LAL_LAUNCHED();
         return LAL_OK;
     }
