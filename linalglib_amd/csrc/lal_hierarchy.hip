@@ -974,6 +974,7 @@ namespace
             bool         stale   = false; // p32 is still the last direction
             double       r_upd  = init; // true residual norm at the last update
             double       r_prev = init, rate = 0.5; // last norm, observed reduction per step
+            int          since  = 0, longest = 0; // steps since the last update; between two at most
             while(!(iter > max_iter))
             {
                 LAL_TRY(next_product<float>(h, A, Av32, z32, stale, &p32, &p_other, q32, n_g, cur,
@@ -996,7 +997,16 @@ namespace
                 lal::observe_rate(rn, &r_prev, &rate);
                 if(std::isnan(rn))
                     break;
-                const bool update = rn <= delta * r_upd || converges(rn, init, rel_tol, abs_tol);
+                // A recurrence whose kept direction no longer fits its replaced
+                // residual can drift above the last update's norm for thousands of
+                // steps (face diffusion 96^3, 1e-12: a true residual of 1.6e-12
+                // after 360 steps, the next update 1900 later).  One that takes
+                // four times as long as any before it is taken for such: the
+                // update comes now, and restarts.
+                since++;
+                const bool lost   = updates > 0 && since > 4 * std::max(longest, 25);
+                const bool update = lost || rn <= delta * r_upd ||
+                                    converges(rn, init, rel_tol, abs_tol);
                 bool       restart = false;
                 if(update)
                 {
@@ -1017,7 +1027,9 @@ namespace
                     // restarts from it (p = z), as iterative refinement would.
                     // Healthy runs (a reduction near delta per update) never
                     // restart and keep their iterates.
-                    restart = rn > 0.1 * r_upd;
+                    restart = lost || rn > 0.1 * r_upd;
+                    longest = std::max(longest, since);
+                    since   = 0;
                     r_upd   = rn;
                     r_prev  = rn;
                     if(std::isnan(rn))
