@@ -362,7 +362,9 @@ int lal_pcg_solve_mixed(lal_handle h, lal_hierarchy hier, const double* b, doubl
  * (1e-2 when opts is NULL; the default options' 1e-4 suits well-conditioned
  * operators only) since the last update, or meets the tolerance, x += y in
  * FP64 and the residual is
- * replaced by the true FP64 b - A x.  Convergence (rel_tol / abs_tol on the
+ * replaced by the true FP64 b - A x.  The Krylov space restarts when an update
+ * has not cut that residual tenfold, or did not come within four times the
+ * longest interval before it (at least 100 iterations).  Convergence (rel_tol / abs_tol on the
  * inf-norm) is tested on that true residual only; info->iterations counts CG
  * iterations as cg_solver does, info->outer_iterations the updates.  Needs
  * build_f32.  No reference counterpart beyond cg.cpp: the reference has no
